@@ -45,58 +45,114 @@ struct SFields {
 #define D4B(b1, b2, m2, m1, c0, p1) ((b1) * ((c0) - (m1)) + (b2) * ((p1) - (m2)))
 
 // ---------------------------------------------------------------------------
-// velocity: CPML corrections of the 9 stress derivatives of one cell
-// (update_v_ssg_CPML.c:84-130: x with K/a/b_x(_half), y, z)
-__device__ inline void v_cpml(const DevGeom &g, const Prof &P, const Psi9 &psi, int j, int i, int k,
-                              int hx, int hy, int hz, float &sxx_x, float &sxy_x, float &sxz_x,
-                              float &sxy_y, float &syy_y, float &syz_y, float &sxz_z, float &syz_z,
-                              float &szz_z)
+// CPML memory variables of a cell.  The variables of the axes whose layer
+// the cell lies in are loaded together, before the derivatives they correct
+// are formed, and updated and stored afterwards: a cell of a layer then waits
+// one memory latency per plane.  Reading, updating and storing one variable
+// after the other (the compiler keeps a load behind a store to an array it
+// may alias) waited one latency each, up to nine per plane.  Buffer accesses
+// (one 32-bit offset per axis) keep the LDS marches at 5 waves per SIMD (v 97,
+// s 91 VGPRs; with 64-bit addresses 111 and 107).  v / s march, serial ->
+// this: 84^3 97 / 102 -> 78 / 83 us (one shot, 32-plane chunks), 536 x 280 x
+// 536 1249 / 1547 -> 1224 / 1528 us, 4 shots at 276^3 1201 / 1467 -> 1207 /
+// 1453 us.
+// m[0..2], m[3..5], m[6..8]: x, y, z variables, as Psi9 orders them.
+struct PsiCell {
+    float m[9];
+    uint32_t o[3];  // byte offset of the cell in the x, y and z arrays
+};
+// one array of axis ax (smaller than a field, so a 32-bit offset reaches it)
+__device__ inline rsrc_t psi_rsrc(const DevGeom &g, const float *p, int ax)
+{
+    const uint32_t f2 = 2u * (uint32_t)g.fw * 4u;
+    return make_rsrc(p, ax == 0 ? f2 * g.ny * g.nz : ax == 1 ? f2 * g.nx * g.nz : f2 * g.ny * g.nx);
+}
+__device__ inline void psi_load(const DevGeom &g, const Psi9 &psi, int j, int i, int k, int hx, int hy, int hz,
+                                PsiCell &c)
 {
     if (hx) {
-        int64_t a = psi_x_at(g, j, hx, k);
-        cpml_apply(psi.p[0], a, sxx_x, P.KH(0, hx), P.AH(0, hx), P.BH(0, hx));
-        cpml_apply(psi.p[1], a, sxy_x, P.K(0, hx), P.A(0, hx), P.B(0, hx));
-        cpml_apply(psi.p[2], a, sxz_x, P.K(0, hx), P.A(0, hx), P.B(0, hx));
+        c.o[0] = (uint32_t)psi_x_at(g, j, hx, k) * 4u;
+#pragma unroll
+        for (int n = 0; n < 3; ++n) c.m[n] = bload(psi_rsrc(g, psi.p[n], 0), c.o[0], 0);
     }
     if (hy) {
-        int64_t a = psi_y_at(g, hy, i, k);
-        cpml_apply(psi.p[3], a, sxy_y, P.K(1, hy), P.A(1, hy), P.B(1, hy));
-        cpml_apply(psi.p[4], a, syy_y, P.KH(1, hy), P.AH(1, hy), P.BH(1, hy));
-        cpml_apply(psi.p[5], a, syz_y, P.K(1, hy), P.A(1, hy), P.B(1, hy));
+        c.o[1] = (uint32_t)psi_y_at(g, hy, i, k) * 4u;
+#pragma unroll
+        for (int n = 3; n < 6; ++n) c.m[n] = bload(psi_rsrc(g, psi.p[n], 1), c.o[1], 0);
     }
     if (hz) {
-        int64_t a = psi_z_at(g, j, i, hz);
-        cpml_apply(psi.p[6], a, sxz_z, P.K(2, hz), P.A(2, hz), P.B(2, hz));
-        cpml_apply(psi.p[7], a, syz_z, P.K(2, hz), P.A(2, hz), P.B(2, hz));
-        cpml_apply(psi.p[8], a, szz_z, P.KH(2, hz), P.AH(2, hz), P.BH(2, hz));
+        c.o[2] = (uint32_t)psi_z_at(g, j, i, hz) * 4u;
+#pragma unroll
+        for (int n = 6; n < 9; ++n) c.m[n] = bload(psi_rsrc(g, psi.p[n], 2), c.o[2], 0);
+    }
+}
+// the three variables of one axis: psi <- b psi + a d, d <- d / K + psi
+// (update_v_ssg_CPML.c:85-90), q-th with the profile (K, a, b)[q]
+struct Coef3 {
+    float K, a, b;
+};
+__device__ inline void psi_axis(const DevGeom &g, const Psi9 &psi, PsiCell &c, int ax, const Coef3 &c0, const Coef3 &c1,
+                                const Coef3 &c2, float &d0, float &d1, float &d2)
+{
+    float *m = c.m + 3 * ax;
+    m[0] = c0.b * m[0] + c0.a * d0;
+    m[1] = c1.b * m[1] + c1.a * d1;
+    m[2] = c2.b * m[2] + c2.a * d2;
+    d0 = d0 / c0.K + m[0];
+    d1 = d1 / c1.K + m[1];
+    d2 = d2 / c2.K + m[2];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) bstore(m[n], psi_rsrc(g, psi.p[3 * ax + n], ax), c.o[ax], 0);
+}
+// cell and half-cell profiles of an axis; kax: the axis K comes from
+__device__ inline Coef3 coef_c(const Prof &P, int kax, int ax, int h)
+{
+    return Coef3{P.K(kax, h), P.A(ax, h), P.B(ax, h)};
+}
+__device__ inline Coef3 coef_h(const Prof &P, int kax, int ax, int h)
+{
+    return Coef3{P.KH(kax, h), P.AH(ax, h), P.BH(ax, h)};
+}
+
+// velocity: CPML corrections of the 9 stress derivatives of one cell
+// (update_v_ssg_CPML.c:84-130: x with K/a/b_x(_half), y, z)
+__device__ inline void v_cpml(const DevGeom &g, const Prof &P, const Psi9 &psi, PsiCell &c, int hx, int hy, int hz, float &sxx_x,
+                              float &sxy_x, float &sxz_x, float &sxy_y, float &syy_y, float &syz_y, float &sxz_z,
+                              float &syz_z, float &szz_z)
+{
+    if (hx) {
+        const Coef3 q = coef_c(P, 0, 0, hx), h = coef_h(P, 0, 0, hx);
+        psi_axis(g, psi, c, 0, h, q, q, sxx_x, sxy_x, sxz_x);
+    }
+    if (hy) {
+        const Coef3 q = coef_c(P, 1, 1, hy), h = coef_h(P, 1, 1, hy);
+        psi_axis(g, psi, c, 1, q, h, q, sxy_y, syy_y, syz_y);
+    }
+    if (hz) {
+        const Coef3 q = coef_c(P, 2, 2, hz), h = coef_h(P, 2, 2, hz);
+        psi_axis(g, psi, c, 2, q, q, h, sxz_z, syz_z, szz_z);
     }
 }
 
 // stress: CPML corrections of the 9 velocity derivatives
 // (update_s_ssg_CPML_elastic.c:72-115; the low-z layer divides by the y-axis
 // K profile, :104-108)
-__device__ inline void s_cpml(const DevGeom &g, const Prof &P, const Psi9 &psi, int j, int i, int k,
-                              int hx, int hy, int hz, float &vxx, float &vyx, float &vzx, float &vxy,
-                              float &vyy, float &vzy, float &vxz, float &vyz, float &vzz)
+__device__ inline void s_cpml(const DevGeom &g, const Prof &P, const Psi9 &psi, PsiCell &c, int k, int hx, int hy,
+                              int hz, float &vxx, float &vyx, float &vzx, float &vxy, float &vyy, float &vzy,
+                              float &vxz, float &vyz, float &vzz)
 {
     if (hx) {
-        int64_t a = psi_x_at(g, j, hx, k);
-        cpml_apply(psi.p[0], a, vxx, P.K(0, hx), P.A(0, hx), P.B(0, hx));
-        cpml_apply(psi.p[1], a, vyx, P.KH(0, hx), P.AH(0, hx), P.BH(0, hx));
-        cpml_apply(psi.p[2], a, vzx, P.KH(0, hx), P.AH(0, hx), P.BH(0, hx));
+        const Coef3 q = coef_c(P, 0, 0, hx), h = coef_h(P, 0, 0, hx);
+        psi_axis(g, psi, c, 0, q, h, h, vxx, vyx, vzx);
     }
     if (hy) {
-        int64_t a = psi_y_at(g, hy, i, k);
-        cpml_apply(psi.p[3], a, vxy, P.KH(1, hy), P.AH(1, hy), P.BH(1, hy));
-        cpml_apply(psi.p[4], a, vyy, P.K(1, hy), P.A(1, hy), P.B(1, hy));
-        cpml_apply(psi.p[5], a, vzy, P.KH(1, hy), P.AH(1, hy), P.BH(1, hy));
+        const Coef3 q = coef_c(P, 1, 1, hy), h = coef_h(P, 1, 1, hy);
+        psi_axis(g, psi, c, 1, h, q, h, vxy, vyy, vzy);
     }
     if (hz) {
-        int64_t a = psi_z_at(g, j, i, hz);
         const int kax = (k <= g.fw) ? 1 : 2;
-        cpml_apply(psi.p[6], a, vxz, P.KH(kax, hz), P.AH(2, hz), P.BH(2, hz));
-        cpml_apply(psi.p[7], a, vyz, P.KH(kax, hz), P.AH(2, hz), P.BH(2, hz));
-        cpml_apply(psi.p[8], a, vzz, P.K(kax, hz), P.A(2, hz), P.B(2, hz));
+        const Coef3 q = coef_c(P, kax, 2, hz), h = coef_h(P, kax, 2, hz);
+        psi_axis(g, psi, c, 2, h, h, q, vxz, vyz, vzz);
     }
 }
 
@@ -425,6 +481,9 @@ __global__ __launch_bounds__(64 * TI) void k_v_march(DevGeom g, MTiles T, VField
             cur.syz_za = b.m2; cur.syz_zb = b.m1; cur.syz_zd = b.p1;
             cur.szz_a = c.m1; cur.szz_c = c.p1; cur.szz_d = c.p2;
         }
+        PsiCell pc;
+        const int hy = CPML ? slab_h(j, g.ny, g.fw, !g.free_surf) : 0;
+        if (CPML) psi_load(g, psi, j, i, k, hx, hy, hz, pc);
         float sxx_x = g.dtdx * D4F(b1, b2, cur.sxx_a, cur.sxx_b, cur.sxx_c, cur.sxx_d);
         float sxy_y = g.dtdy * D4B(b1, b2, sxy_m2, sxy_m1, sxy_0, cur.sxy_n);
         float sxz_z = g.dtdz * D4B(b1, b2, cur.sxz_za, cur.sxz_zb, cur.sxz_0, cur.sxz_zd);
@@ -434,11 +493,7 @@ __global__ __launch_bounds__(64 * TI) void k_v_march(DevGeom g, MTiles T, VField
         float szz_z = g.dtdz * D4F(b1, b2, cur.szz_a, cur.szz_b, cur.szz_c, cur.szz_d);
         float sxz_x = g.dtdx * D4B(b1, b2, cur.sxz_xa, cur.sxz_xb, cur.sxz_0, cur.sxz_xd);
         float syz_y = g.dtdy * D4B(b1, b2, syz_m2, syz_m1, syz_0, cur.syz_n);
-        if (CPML) {
-            const int hy = slab_h(j, g.ny, g.fw, !g.free_surf);
-            v_cpml(g, P, psi, j, i, k, hx, hy, hz, sxx_x, sxy_x, sxz_x, sxy_y, syy_y, syz_y, sxz_z, syz_z,
-                   szz_z);
-        }
+        if (CPML) v_cpml(g, P, psi, pc, hx, hy, hz, sxx_x, sxy_x, sxz_x, sxy_y, syy_y, syz_y, sxz_z, syz_z, szz_z);
         const float nvx = cur.vx0 + (sxx_x + sxy_y + sxz_z) / cur.rip;
         const float nvy = cur.vy0 + (syy_y + sxy_x + syz_z) / cur.rjp;
         const float nvz = cur.vz0 + (szz_z + sxz_x + syz_y) / cur.rkp;
@@ -592,6 +647,9 @@ __global__ __launch_bounds__(64 * TI) void k_v_lds(DevGeom g, MTiles T, VFields 
             const float(*YZ)[68] = sh[p][3];
             const float(*ZZ)[68] = sh[p][4];
             const int c0 = lane + 2, r0_ = y + 2;
+            PsiCell pc;
+            const int hy = CPML ? slab_h(j, g.ny, g.fw, !g.free_surf) : 0;
+            if (CPML) psi_load(g, psi, j, i, k, hx, hy, hz, pc);
             float sxx_x = g.dtdx * D4F(b1, b2, XX[r0_ - 1][c0], cur.sxx, XX[r0_ + 1][c0], XX[r0_ + 2][c0]);
             float sxy_y = g.dtdy * D4B(b1, b2, sxy_m2, sxy_m1, sxy_0, sxy_p1);
             float sxz_z = g.dtdz * D4B(b1, b2, XZ[r0_][c0 - 2], XZ[r0_][c0 - 1], cur.sxz, XZ[r0_][c0 + 1]);
@@ -601,11 +659,8 @@ __global__ __launch_bounds__(64 * TI) void k_v_lds(DevGeom g, MTiles T, VFields 
             float szz_z = g.dtdz * D4F(b1, b2, ZZ[r0_][c0 - 1], cur.szz, ZZ[r0_][c0 + 1], ZZ[r0_][c0 + 2]);
             float sxz_x = g.dtdx * D4B(b1, b2, XZ[r0_ - 2][c0], XZ[r0_ - 1][c0], cur.sxz, XZ[r0_ + 1][c0]);
             float syz_y = g.dtdy * D4B(b1, b2, syz_m2, syz_m1, syz_0, syz_p1);
-            if (CPML) {
-                const int hy = slab_h(j, g.ny, g.fw, !g.free_surf);
-                v_cpml(g, P, psi, j, i, k, hx, hy, hz, sxx_x, sxy_x, sxz_x, sxy_y, syy_y, syz_y, sxz_z, syz_z,
-                       szz_z);
-            }
+            if (CPML)
+                v_cpml(g, P, psi, pc, hx, hy, hz, sxx_x, sxy_x, sxz_x, sxy_y, syy_y, syz_y, sxz_z, syz_z, szz_z);
             const float nvx = cur.vx0 + (sxx_x + sxy_y + sxz_z) / cur.rip;
             const float nvy = cur.vy0 + (syy_y + sxy_x + syz_z) / cur.rjp;
             const float nvz = cur.vz0 + (szz_z + sxz_x + syz_y) / cur.rkp;
@@ -716,6 +771,9 @@ __global__ __launch_bounds__(64 * TI) void k_s_march(DevGeom g, MTiles T, SField
             cur.vy_zb = b.m1; cur.vy_zc = b.p1; cur.vy_zd = b.p2;
             cur.vz_za = c.m2; cur.vz_zb = c.m1; cur.vz_zd = c.p1;
         }
+        PsiCell pc;
+        const int hy = CPML ? slab_h(j, g.ny, g.fw, !g.free_surf) : 0;
+        if (CPML) psi_load(g, psi, j, i, k, hx, hy, hz, pc);
         float vxx = D4B(b1, b2, cur.vx_xa, cur.vx_xb, vx_0, cur.vx_xd);
         float vxy = D4F(b1, b2, vx_m1, vx_0, vx_p1, cur.vx_n);
         float vxz = D4F(b1, b2, cur.vx_zb, vx_0, cur.vx_zc, cur.vx_zd);
@@ -726,10 +784,7 @@ __global__ __launch_bounds__(64 * TI) void k_s_march(DevGeom g, MTiles T, SField
         float vzy = D4F(b1, b2, vz_m1, vz_0, vz_p1, cur.vz_n);
         float vzz = D4B(b1, b2, cur.vz_za, cur.vz_zb, vz_0, cur.vz_zd);
         div_spacing(g, vxx, vxy, vxz, vyx, vyy, vyz, vzx, vzy, vzz);
-        if (CPML) {
-            const int hy = slab_h(j, g.ny, g.fw, !g.free_surf);
-            s_cpml(g, P, psi, j, i, k, hx, hy, hz, vxx, vyx, vzx, vxy, vyy, vzy, vxz, vyz, vzz);
-        }
+        if (CPML) s_cpml(g, P, psi, pc, k, hx, hy, hz, vxx, vyx, vzx, vxy, vyy, vzy, vxz, vyz, vzz);
         const float vxyyx = vxy + vyx, vyzzy = vyz + vzy, vxzzx = vxz + vzx;
         const float vxxyyzz = vxx + vyy + vzz;
         const float vyyzz = vyy + vzz, vxxzz = vxx + vzz, vxxyy = vxx + vyy;
@@ -960,6 +1015,9 @@ __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields 
             const float(*Y)[68] = sh[p][1];
             const float(*Z)[68] = sh[p][2];
             const int c0 = lane + 2, r0_ = y + 2;
+            PsiCell pc;
+            const int hy = CPML ? slab_h(j, g.ny, g.fw, !g.free_surf) : 0;
+            if (CPML) psi_load(g, psi, j, i, k, hx, hy, hz, pc);
             float vxx = D4B(b1, b2, X[r0_ - 2][c0], X[r0_ - 1][c0], vx_0, X[r0_ + 1][c0]);
             float vxy = D4F(b1, b2, vx_m1, vx_0, vx_p1, vx_p2);
             float vxz = D4F(b1, b2, X[r0_][c0 - 1], vx_0, X[r0_][c0 + 1], X[r0_][c0 + 2]);
@@ -970,10 +1028,7 @@ __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields 
             float vzy = D4F(b1, b2, vz_m1, vz_0, vz_p1, vz_p2);
             float vzz = D4B(b1, b2, Z[r0_][c0 - 2], Z[r0_][c0 - 1], vz_0, Z[r0_][c0 + 1]);
             div_spacing(g, vxx, vxy, vxz, vyx, vyy, vyz, vzx, vzy, vzz);
-            if (CPML) {
-                const int hy = slab_h(j, g.ny, g.fw, !g.free_surf);
-                s_cpml(g, P, psi, j, i, k, hx, hy, hz, vxx, vyx, vzx, vxy, vyy, vzy, vxz, vyz, vzz);
-            }
+            if (CPML) s_cpml(g, P, psi, pc, k, hx, hy, hz, vxx, vyx, vzx, vxy, vyy, vzy, vxz, vyz, vzz);
             const float vxyyx = vxy + vyx, vyzzy = vyz + vzy, vxzzx = vxz + vzx;
             const float vxxyyzz = vxx + vyy + vzz;
             const float vyyzz = vyy + vzz, vxxzz = vxx + vzz, vxxyy = vxx + vyy;
@@ -1212,6 +1267,11 @@ __global__ __launch_bounds__(256) void k_v_slabs(DevGeom g, BoxList L, VFields F
     if (!slab_cell(L, t, j, i, k)) return;
     const int64_t c = at(g, j, i, k), sj = g.sj, si = g.si;
     const float b1 = g.b1, b2 = g.b2;
+    const int hx = slab_h(i, g.nx, g.fw, 1);
+    const int hy = slab_h(j, g.ny, g.fw, !g.free_surf);
+    const int hz = slab_h(k, g.nz, g.fw, 1);
+    PsiCell pc;
+    psi_load(g, psi, j, i, k, hx, hy, hz, pc);
     float sxx_x = g.dtdx * D4F(b1, b2, F.sxx[c - si], F.sxx[c], F.sxx[c + si], F.sxx[c + 2 * si]);
     float sxy_x = g.dtdx * D4B(b1, b2, F.sxy[c - 2 * si], F.sxy[c - si], F.sxy[c], F.sxy[c + si]);
     float sxz_x = g.dtdx * D4B(b1, b2, F.sxz[c - 2 * si], F.sxz[c - si], F.sxz[c], F.sxz[c + si]);
@@ -1221,10 +1281,7 @@ __global__ __launch_bounds__(256) void k_v_slabs(DevGeom g, BoxList L, VFields F
     float sxz_z = g.dtdz * D4B(b1, b2, F.sxz[c - 2], F.sxz[c - 1], F.sxz[c], F.sxz[c + 1]);
     float syz_z = g.dtdz * D4B(b1, b2, F.syz[c - 2], F.syz[c - 1], F.syz[c], F.syz[c + 1]);
     float szz_z = g.dtdz * D4F(b1, b2, F.szz[c - 1], F.szz[c], F.szz[c + 1], F.szz[c + 2]);
-    const int hx = slab_h(i, g.nx, g.fw, 1);
-    const int hy = slab_h(j, g.ny, g.fw, !g.free_surf);
-    const int hz = slab_h(k, g.nz, g.fw, 1);
-    v_cpml(g, P, psi, j, i, k, hx, hy, hz, sxx_x, sxy_x, sxz_x, sxy_y, syy_y, syz_y, sxz_z, syz_z, szz_z);
+    v_cpml(g, P, psi, pc, hx, hy, hz, sxx_x, sxy_x, sxz_x, sxy_y, syy_y, syz_y, sxz_z, syz_z, szz_z);
     F.vx[c] += (sxx_x + sxy_y + sxz_z) / F.rip[c];
     F.vy[c] += (syy_y + sxy_x + syz_z) / F.rjp[c];
     F.vz[c] += (szz_z + sxz_x + syz_y) / F.rkp[c];
@@ -1239,6 +1296,11 @@ __global__ __launch_bounds__(256) void k_s_slabs(DevGeom g, BoxList L, SFields F
     const int64_t c = at(g, j, i, k), sj = g.sj, si = g.si;
     const float b1 = g.b1, b2 = g.b2;
 
+    const int hx = slab_h(i, g.nx, g.fw, 1);
+    const int hy = slab_h(j, g.ny, g.fw, !g.free_surf);
+    const int hz = slab_h(k, g.nz, g.fw, 1);
+    PsiCell pc;
+    psi_load(g, psi, j, i, k, hx, hy, hz, pc);
     float vxx = D4B(b1, b2, F.vx[c - 2 * si], F.vx[c - si], F.vx[c], F.vx[c + si]);
     float vxy = D4F(b1, b2, F.vx[c - sj], F.vx[c], F.vx[c + sj], F.vx[c + 2 * sj]);
     float vxz = D4F(b1, b2, F.vx[c - 1], F.vx[c], F.vx[c + 1], F.vx[c + 2]);
@@ -1249,10 +1311,7 @@ __global__ __launch_bounds__(256) void k_s_slabs(DevGeom g, BoxList L, SFields F
     float vzy = D4F(b1, b2, F.vz[c - sj], F.vz[c], F.vz[c + sj], F.vz[c + 2 * sj]);
     float vzz = D4B(b1, b2, F.vz[c - 2], F.vz[c - 1], F.vz[c], F.vz[c + 1]);
     div_spacing(g, vxx, vxy, vxz, vyx, vyy, vyz, vzx, vzy, vzz);
-    const int hx = slab_h(i, g.nx, g.fw, 1);
-    const int hy = slab_h(j, g.ny, g.fw, !g.free_surf);
-    const int hz = slab_h(k, g.nz, g.fw, 1);
-    s_cpml(g, P, psi, j, i, k, hx, hy, hz, vxx, vyx, vzx, vxy, vyy, vzy, vxz, vyz, vzz);
+    s_cpml(g, P, psi, pc, k, hx, hy, hz, vxx, vyx, vzx, vxy, vyy, vzy, vxz, vyz, vzz);
     if (!VM) {
         s_apply(g, F, c, vxx, vxy, vxz, vyx, vyy, vyz, vzx, vzy, vzz);
         return;
@@ -2036,9 +2095,11 @@ __global__ __launch_bounds__(64 * TI) void k_vs_fused(DevGeom g, FTiles T, Fused
             float sxz_x = g.dtdx * D4B(b1, b2, XZ[ty - 2][lx], XZ[ty - 1][lx], sxz_0, XZ[ty + 1][lx]);
             float syz_y = g.dtdy * D4B(b1, b2, qyz[0], qyz[1], syz_0, qyz[3]);
             const int hy = slab_h(jv, g.ny, g.fw, !g.free_surf);
-            if (hx | hy | hz)
-                v_cpml(g, P, pss, jv, i, k, hx, hy, hz, sxx_x, sxy_x, sxz_x, sxy_y, syy_y, syz_y, sxz_z, syz_z,
-                       szz_z);
+            if (hx | hy | hz) {
+                PsiCell pc;
+                psi_load(g, pss, jv, i, k, hx, hy, hz, pc);
+                v_cpml(g, P, pss, pc, hx, hy, hz, sxx_x, sxy_x, sxz_x, sxy_y, syy_y, syz_y, sxz_z, syz_z, szz_z);
+            }
             const float rip = LDJ(rrip, jv, 0, 0), rjp = LDJ(rrjp, jv, 0, 0), rkp = LDJ(rrkp, jv, 0, 0);
             const float nvx = qvx[0] + (sxx_x + sxy_y + sxz_z) / rip;
             const float nvy = qvy[0] + (syy_y + sxy_x + syz_z) / rjp;
