@@ -1395,8 +1395,7 @@ static Box region_box(const ifos_geom *g, int region)
     return B;
 }
 
-// tiles of boxes for TI i-rows per block; jc <= 0 picks the j chunk so a
-// launch has >= 4096 workgroups (16 per CU) when the boxes allow it
+// tiles of boxes for TI i-rows per block and at most jc j-planes (<= 0: 64)
 static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, int ns, int group, int kb = 1, int sb = 1)
 {
     MTiles T = {};
@@ -1431,10 +1430,19 @@ static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, int ns, int g
             tot += (int64_t)T.ntk[q] * T.nti[q] * ((T.b[q].j1 - T.b[q].j0 + 1 + c - 1) / c);
         return tot;
     };
-    if (jc <= 0) {
-        jc = 64;
-        while (jc > 8 && count(jc) * T.nsg < 4096) jc /= 2;
-    }
+    // A tile's march over jc planes is a serial chain (a plane takes 1-2.5 us,
+    // a memory latency and some 400 instructions), and the chip holds some
+    // 1300 workgroups at once: with fewer than a few rounds of them the launch
+    // time is the chain and the last round's idle CUs, so the chunk is halved
+    // until the launch has kTileMin workgroups, down to 4 planes (below, the
+    // 4-6 extra planes a tile loads cost what the shorter chain gains).
+    // One shot, v / s march, chunk 32 -> this rule: 84^3 97 / 102 -> 25 / 27
+    // us (chunk 4), 148^3 117 / 130 -> 65 / 71 us (4), 276^3 404 / 485 ->
+    // 345 / 417 us (8).  4 shots at 276^3 and 536 x 280 x 536 have the
+    // workgroups and keep 32 planes (8-16 planes: 0-9 % slower there).
+    constexpr int64_t kTileMin = 8192;
+    if (jc <= 0) jc = 64;
+    while (jc > 4 && count(jc) * T.nsg < kTileMin) jc = jc / 2 > 4 ? jc / 2 : 4;
     T.jc = jc;
     for (int q = 0; q < T.nb; ++q)
         T.start[q + 1] = T.start[q] + T.ntk[q] * T.nti[q] * ((T.b[q].j1 - T.b[q].j0 + 1 + jc - 1) / jc);

@@ -406,7 +406,8 @@ int ifos_levels_run(ifos_batch *const *lv, int nlev, const ifos_shot *const *sho
                     float *const *d_syn, int use_graph);
 /* tile shapes of the velocity and stress march launches, each
  * {TI, jc, group, split, pipe, kb, sb, lds}: TI wavefronts per workgroup (1, 2, 4, 8);
- * jc j-planes per tile (<= 0: automatic); group: tiles of one shot before
+ * at most jc j-planes per tile (<= 0: 64), halved down to 4 where the launch
+ * would leave the chip short of workgroups (results do not depend on it); group: tiles of one shot before
  * the next shot (1: shots fastest, <= 0: one shot after the other); split:
  * 1 = interior box and CPML slabs in separate launches, 0 = one CPML-aware
  * launch; pipe: 1 = the next plane's operands are loaded one plane ahead;
