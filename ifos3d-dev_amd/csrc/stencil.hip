@@ -25,6 +25,7 @@
 // (update_v_ssg.c:106-125, update_v_ssg_CPML.c:73-100,
 //  update_s_ssg_elastic.c:106-138, update_s_ssg_CPML_elastic.c:63-140).
 #include <algorithm>
+#include <type_traits>
 
 #include "ifos_dev.h"
 
@@ -399,11 +400,9 @@ __device__ inline void shift_psi(Psi9 &psi, const Shots &S, int shot)
 #define LD(r, dj, di, dk) bload(r, vo + ((dk) + 2) * 4, ((dj) + 2) * SJ + ((di) + 2) * SI)
 #define LDH(r, dj) bload(r, vo + khv, ((dj) + 2) * SJ + 2 * SI)
 // words a march touches once (its own cell's old value, its stores) carry
-// the policy CPN, the streaming hint in the whole-domain launches (CPML
-// template true: the batched path, whose fields are far larger than the
-// 256 MB Infinity Cache) and the default policy in the interior launches of
-// the plain path (measured: streaming there makes them 10-25 % slower, as
-// the next launches re-read those words from the Infinity Cache)
+// the policy CPN: the streaming hint where the launch is whole-domain and its
+// working set is larger than the Infinity Cache (launch_v / launch_s pass NT),
+// the default policy elsewhere
 #define LDN(r, dj, di, dk) bload_cp<CPN>(r, vo + ((dk) + 2) * 4, ((dj) + 2) * SJ + ((di) + 2) * SI)
 #define STN(v, r) bstore_cp<CPN>(v, r, vo + 8, 2 * SJ + 2 * SI)
 #define ST(v, r) bstore(v, r, vo + 8, 2 * SJ + 2 * SI)
@@ -438,7 +437,7 @@ struct VPlane {
         P.sxy_n = LD(rsxy, (D) + 1, 0, 0); P.syz_n = LD(rsyz, (D) + 1, 0, 0); P.syy_n = LD(rsyy, (D) + 2, 0, 0); \
     } while (0)
 
-template <int TI, bool CPML, bool SNAP, bool PIPE>
+template <int TI, bool CPML, bool SNAP, bool PIPE, bool NT>
 __global__ __launch_bounds__(64 * TI) void k_v_march(DevGeom g, MTiles T, VFields F, Prof P, Psi9 psi, Shots S,
                                                     Snap N)
 {
@@ -447,7 +446,7 @@ __global__ __launch_bounds__(64 * TI) void k_v_march(DevGeom g, MTiles T, VField
     bool krow;
     if (!decode_tile(T, TI, k, i, jb, je, shot, R, &krow)) return;
     const uint32_t khv = khalo_off();
-    constexpr int CPN = CPML ? IFOS_CPOL_NT : 0;
+    constexpr int CPN = NT ? IFOS_CPOL_NT : 0;
     const uint32_t SJ = (uint32_t)g.sj * 4u, SI = (uint32_t)g.si * 4u;
     const float b1 = g.b1, b2 = g.b2;
     const int64_t so = (int64_t)shot * S.fstride;
@@ -522,13 +521,13 @@ __global__ __launch_bounds__(64 * TI) void k_v_march(DevGeom g, MTiles T, VField
 // i0+TI), sxz, syz and szz for their k-neighbours (the row's halo words).
 // sxx, sxz and szz are read at the plane itself, sxy and syz come from the
 // j-queues.  Same arithmetic, in the same order, as k_v_march.
-template <int TI, bool CPML, bool SNAP>
+template <int TI, bool CPML, bool SNAP, bool NT>
 __global__ __launch_bounds__(64 * TI) void k_v_lds(DevGeom g, MTiles T, VFields F, Prof P, Psi9 psi, Shots S,
                                                   Snap N)
 {
     constexpr int RW = TI + 4;
     constexpr int NH = (9 + TI - 1) / TI;
-    constexpr int CPN = CPML ? IFOS_CPOL_NT : 0;
+    constexpr int CPN = NT ? IFOS_CPOL_NT : 0;
     __shared__ float sh[2][5][RW][68];  // sxx, sxy, sxz, syz, szz
     const int b = blockIdx.x;
     const int L = (b & 7) * T.per + (b >> 3);
@@ -718,7 +717,7 @@ struct SPlane {
 
 // VM: 0 elastic, 1 one relaxation mechanism (the reference's update_s),
 // 2 V.L >= 1 mechanisms (stress_visco_n)
-template <int TI, bool CPML, int VM, bool PIPE>
+template <int TI, bool CPML, int VM, bool PIPE, bool NT>
 __global__ __launch_bounds__(64 * TI) void k_s_march(DevGeom g, MTiles T, SFields F, Prof P, Psi9 psi, Shots S,
                                                     ViscoF V)
 {
@@ -727,7 +726,7 @@ __global__ __launch_bounds__(64 * TI) void k_s_march(DevGeom g, MTiles T, SField
     bool krow;
     if (!decode_tile(T, TI, k, i, jb, je, shot, R, &krow)) return;
     const uint32_t khv = khalo_off();
-    constexpr int CPN = CPML ? IFOS_CPOL_NT : 0;
+    constexpr int CPN = NT ? IFOS_CPOL_NT : 0;
     const uint32_t SJ = (uint32_t)g.sj * 4u, SI = (uint32_t)g.si * 4u;
     const float b1 = g.b1, b2 = g.b2;
     const float DT = g.dt;
@@ -862,13 +861,13 @@ __global__ __launch_bounds__(64 * TI) void k_s_march(DevGeom g, MTiles T, SField
 // update and store.  The barrier waits for LDS only (s_waitcnt lgkmcnt(0)):
 // the loads in flight for the next plane stay in flight across it.  Same
 // arithmetic, in the same order, as k_s_march.
-template <int TI, bool CPML, int VM>
+template <int TI, bool CPML, int VM, bool NT>
 __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields F, Prof P, Psi9 psi, Shots S,
                                                   ViscoF V)
 {
     constexpr int RW = TI + 4;              // LDS rows: i0-2 .. i0+TI+1
     constexpr int NH = (9 + TI - 1) / TI;   // outside rows per wavefront (9 per workgroup)
-    constexpr int CPN = CPML ? IFOS_CPOL_NT : 0;
+    constexpr int CPN = NT ? IFOS_CPOL_NT : 0;
     __shared__ float sh[2][3][RW][68];
     const int b = blockIdx.x;
     const int L = (b & 7) * T.per + (b >> 3);
@@ -1460,7 +1459,7 @@ static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, int ns, int g
 // the batched path's autotuner overrides it per kernel.  On the 256^3
 // interior of a 276^3 grid the LDS marches with 32-plane chunks run 4-8 %
 // faster than the register marches over the whole j extent.
-static MarchCfg g_default_cfg = {4, 32, 0, 0, 0, 1, 1, 1};
+static MarchCfg g_default_cfg = {4, 32, 0, 0, 0, 1, 1, 1, 1};
 
 // the shape checks of ifos_batch_set_tiles and ifos_set_plain_tiles
 int check_tile_cfg(const int *c, const char *who)
@@ -1476,17 +1475,11 @@ int check_tile_cfg(const int *c, const char *who)
     return IFOS_OK;
 }
 
-template <bool CPML, bool SNAP, bool PIPE>
-static void launch_v_ti(int ti, dim3 grid, const MTiles &T, const DevGeom &G, const VFields &F, const Prof &P,
-                        const Psi9 &psi, const Shots &S, const Snap &N, hipStream_t s)
-{
-    switch (ti) {
-    case 1: hipLaunchKernelGGL((k_v_march<1, CPML, SNAP, PIPE>), grid, dim3(64, 1), 0, s, G, T, F, P, psi, S, N); break;
-    case 2: hipLaunchKernelGGL((k_v_march<2, CPML, SNAP, PIPE>), grid, dim3(64, 2), 0, s, G, T, F, P, psi, S, N); break;
-    case 4: hipLaunchKernelGGL((k_v_march<4, CPML, SNAP, PIPE>), grid, dim3(64, 4), 0, s, G, T, F, P, psi, S, N); break;
-    default: hipLaunchKernelGGL((k_v_march<8, CPML, SNAP, PIPE>), grid, dim3(64, 8), 0, s, G, T, F, P, psi, S, N); break;
-    }
-}
+// shape of a launch beyond its tiles: register marches one plane ahead
+// (pipe), LDS staging, streaming policy
+struct MarchMode {
+    bool lds, pipe, nt;
+};
 
 // the LDS-staged marches need 64-lane rows (every box at least 64 cells deep
 // in k), one k column and one shot per workgroup, and TI >= 2
@@ -1498,15 +1491,37 @@ static bool lds_ok(const MarchCfg &c, const MTiles &T)
     return true;
 }
 
-template <bool CPML, bool SNAP>
-static void launch_v_lds_ti(int ti, dim3 grid, const MTiles &T, const DevGeom &G, const VFields &F, const Prof &P,
-                            const Psi9 &psi, const Shots &S, const Snap &N, hipStream_t s)
+// A time step reads 9 fields of every shot and 8 of the model.  While these
+// fit the 256 MB Infinity Cache the next launch finds this launch's words
+// there: the streaming hint then only costs, and the register marches, whose
+// neighbour loads are cache hits, beat the LDS staging and its barrier; past
+// it the LDS marches with streamed own words win.  v / s whole-domain
+// marches, LDS + streaming -> register + default policy: one shot at 84^3
+// (10 MB) 24.3 / 25.8 -> 18.9 / 19.5 us, 148^3 (220 MB) 66.4 / 70.8 -> 56.4 /
+// 64.2, 202 x 106 x 202 (294 MB) 89.6 / 96.2 -> 93.7 / 109.2, 4 shots at 84^3
+// (104 MB) 63.2 / 67.2 -> 53.7 / 55.0, 3 at 148^3 (454 MB) with LDS 195 / 196
+// -> 197 / 208.  A tile shape that a caller or the autotuner set keeps its
+// lds choice.
+static MarchMode march_mode(const MarchCfg &c, const MTiles &T, const DevGeom &g, int ns, bool whole, int L = 0)
 {
-    switch (ti) {
-    case 2: hipLaunchKernelGGL((k_v_lds<2, CPML, SNAP>), grid, dim3(64, 2), 0, s, G, T, F, P, psi, S, N); break;
-    case 4: hipLaunchKernelGGL((k_v_lds<4, CPML, SNAP>), grid, dim3(64, 4), 0, s, G, T, F, P, psi, S, N); break;
-    default: hipLaunchKernelGGL((k_v_lds<8, CPML, SNAP>), grid, dim3(64, 8), 0, s, G, T, F, P, psi, S, N); break;
-    }
+    const double set = 4.0 * g.nx * g.ny * g.nz * ((9.0 + 6.0 * L) * ns + (L ? 13.0 : 8.0));
+    const bool cached = set <= 256e6;
+    return MarchMode{lds_ok(c, T) && !(c.dflt && cached), c.pipe != 0, whole && !cached};
+}
+
+template <int TI, bool CPML, bool SNAP, bool NT>
+static void launch_v_one(const MarchMode &m, dim3 grid, const MTiles &T, const DevGeom &G, const VFields &F,
+                         const Prof &P, const Psi9 &psi, const Shots &S, const Snap &N, hipStream_t s)
+{
+    if constexpr (TI >= 2)
+        if (m.lds) {
+            hipLaunchKernelGGL((k_v_lds<TI, CPML, SNAP, NT>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, N);
+            return;
+        }
+    if (m.pipe)
+        hipLaunchKernelGGL((k_v_march<TI, CPML, SNAP, true, NT>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, N);
+    else
+        hipLaunchKernelGGL((k_v_march<TI, CPML, SNAP, false, NT>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, N);
 }
 
 template <bool CPML, bool SNAP>
@@ -1514,41 +1529,40 @@ static int launch_v(const MarchCfg &c, const MTiles &T, const DevGeom &G, const 
                     const Psi9 &psi, const Shots &S, const Snap &N, hipStream_t s)
 {
     if (T.total == 0) return IFOS_OK;
-    if (c.ti != 1 && c.ti != 2 && c.ti != 4 && c.ti != 8) {
-        set_error("march: TI=%d not in {1,2,4,8}", c.ti);
-        return IFOS_EINVAL;
-    }
     const dim3 grid((unsigned)(T.per * 8));
-    if (lds_ok(c, T)) {
-        launch_v_lds_ti<CPML, SNAP>(c.ti, grid, T, G, F, P, psi, S, N, s);
-        return hip_check(hipGetLastError(), "k_v_lds");
+    const MarchMode m = march_mode(c, T, G, S.n, CPML);
+    auto go = [&](auto ti) {
+        constexpr int TI = decltype(ti)::value;
+        if constexpr (CPML)
+            if (m.nt) {
+                launch_v_one<TI, CPML, SNAP, true>(m, grid, T, G, F, P, psi, S, N, s);
+                return;
+            }
+        launch_v_one<TI, CPML, SNAP, false>(m, grid, T, G, F, P, psi, S, N, s);
+    };
+    switch (c.ti) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 8: go(std::integral_constant<int, 8>{}); break;
+    default: set_error("march: TI=%d not in {1,2,4,8}", c.ti); return IFOS_EINVAL;
     }
-    if (c.pipe) launch_v_ti<CPML, SNAP, true>(c.ti, grid, T, G, F, P, psi, S, N, s);
-    else launch_v_ti<CPML, SNAP, false>(c.ti, grid, T, G, F, P, psi, S, N, s);
-    return hip_check(hipGetLastError(), "k_v_march");
+    return hip_check(hipGetLastError(), "velocity march");
 }
 
-template <bool CPML, int VM, bool PIPE>
-static void launch_s_ti(int ti, dim3 grid, const MTiles &T, const DevGeom &G, const SFields &F, const Prof &P,
-                        const Psi9 &psi, const Shots &S, const ViscoF &V, hipStream_t s)
+template <int TI, bool CPML, int VM, bool NT>
+static void launch_s_one(const MarchMode &m, dim3 grid, const MTiles &T, const DevGeom &G, const SFields &F,
+                         const Prof &P, const Psi9 &psi, const Shots &S, const ViscoF &V, hipStream_t s)
 {
-    switch (ti) {
-    case 1: hipLaunchKernelGGL((k_s_march<1, CPML, VM, PIPE>), grid, dim3(64, 1), 0, s, G, T, F, P, psi, S, V); break;
-    case 2: hipLaunchKernelGGL((k_s_march<2, CPML, VM, PIPE>), grid, dim3(64, 2), 0, s, G, T, F, P, psi, S, V); break;
-    case 4: hipLaunchKernelGGL((k_s_march<4, CPML, VM, PIPE>), grid, dim3(64, 4), 0, s, G, T, F, P, psi, S, V); break;
-    default: hipLaunchKernelGGL((k_s_march<8, CPML, VM, PIPE>), grid, dim3(64, 8), 0, s, G, T, F, P, psi, S, V); break;
-    }
-}
-
-template <bool CPML, int VM>
-static void launch_s_lds_ti(int ti, dim3 grid, const MTiles &T, const DevGeom &G, const SFields &F, const Prof &P,
-                            const Psi9 &psi, const Shots &S, const ViscoF &V, hipStream_t s)
-{
-    switch (ti) {
-    case 2: hipLaunchKernelGGL((k_s_lds<2, CPML, VM>), grid, dim3(64, 2), 0, s, G, T, F, P, psi, S, V); break;
-    case 4: hipLaunchKernelGGL((k_s_lds<4, CPML, VM>), grid, dim3(64, 4), 0, s, G, T, F, P, psi, S, V); break;
-    default: hipLaunchKernelGGL((k_s_lds<8, CPML, VM>), grid, dim3(64, 8), 0, s, G, T, F, P, psi, S, V); break;
-    }
+    if constexpr (TI >= 2)
+        if (m.lds) {
+            hipLaunchKernelGGL((k_s_lds<TI, CPML, VM, NT>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, V);
+            return;
+        }
+    if (m.pipe)
+        hipLaunchKernelGGL((k_s_march<TI, CPML, VM, true, NT>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, V);
+    else
+        hipLaunchKernelGGL((k_s_march<TI, CPML, VM, false, NT>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, V);
 }
 
 template <bool CPML, int VM = 0>
@@ -1556,18 +1570,25 @@ static int launch_s(const MarchCfg &c, const MTiles &T, const DevGeom &G, const 
                     const Psi9 &psi, const Shots &S, hipStream_t s, const ViscoF &V = ViscoF{})
 {
     if (T.total == 0) return IFOS_OK;
-    if (c.ti != 1 && c.ti != 2 && c.ti != 4 && c.ti != 8) {
-        set_error("march: TI=%d not in {1,2,4,8}", c.ti);
-        return IFOS_EINVAL;
-    }
     const dim3 grid((unsigned)(T.per * 8));
-    if (lds_ok(c, T)) {
-        launch_s_lds_ti<CPML, VM>(c.ti, grid, T, G, F, P, psi, S, V, s);
-        return hip_check(hipGetLastError(), "k_s_lds");
+    const MarchMode m = march_mode(c, T, G, S.n, CPML, VM ? V.L : 0);
+    auto go = [&](auto ti) {
+        constexpr int TI = decltype(ti)::value;
+        if constexpr (CPML)
+            if (m.nt) {
+                launch_s_one<TI, CPML, VM, true>(m, grid, T, G, F, P, psi, S, V, s);
+                return;
+            }
+        launch_s_one<TI, CPML, VM, false>(m, grid, T, G, F, P, psi, S, V, s);
+    };
+    switch (c.ti) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 8: go(std::integral_constant<int, 8>{}); break;
+    default: set_error("march: TI=%d not in {1,2,4,8}", c.ti); return IFOS_EINVAL;
     }
-    if (c.pipe) launch_s_ti<CPML, VM, true>(c.ti, grid, T, G, F, P, psi, S, V, s);
-    else launch_s_ti<CPML, VM, false>(c.ti, grid, T, G, F, P, psi, S, V, s);
-    return hip_check(hipGetLastError(), "k_s_march");
+    return hip_check(hipGetLastError(), "stress march");
 }
 
 static VFields vfields(const ifos_fields *f, const ifos_model *m)
