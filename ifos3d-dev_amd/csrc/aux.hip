@@ -392,6 +392,30 @@ __global__ void k_fill(float *d, int64_t n, float v)
     for (; t < n; t += stride) d[t] = v;
 }
 
+// one workgroup moves kMoveElems floats of one array of the list
+constexpr int kMoveElems = 4096;
+__global__ __launch_bounds__(256) void k_moves(MoveList L)
+{
+    int q = 0;
+    while (q + 1 < L.n && (int)blockIdx.x >= L.start[q + 1]) ++q;
+    const int64_t b = (int64_t)((int)blockIdx.x - L.start[q]) * kMoveElems;
+    const float *src = L.src[q];
+    float *dst = L.dst[q];
+    const int64_t n = L.len[q];
+    if (b + kMoveElems <= n) {  // every array starts on a 16-byte boundary
+        v4f v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t t = b / 4 + u * 256 + threadIdx.x;
+            v[u] = src ? ((const v4f *)src)[t] : v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) ((v4f *)dst)[b / 4 + u * 256 + threadIdx.x] = v[u];
+    } else {
+        for (int64_t t = b + threadIdx.x; t < n; t += 256) dst[t] = src ? src[t] : 0.0f;
+    }
+}
+
 // time-domain gradient: running time integrals u += v dt of three
 // components over the whole device layout (halos stay 0: v is 0 there)
 __global__ void k_td_integrate(float *u0, float *u1, float *u2, const float *v0, const float *v1, const float *v2,
@@ -865,6 +889,28 @@ extern "C" int ifos_residual_noalloc(const ifos_geom *g, const float *d_obs, con
 }
 
 namespace ifos {
+int launch_moves(MoveList &L, hipStream_t st)
+{
+    int64_t blocks = 0;
+    for (int q = 0; q < L.n; ++q) {
+        if (((uintptr_t)L.dst[q] | (uintptr_t)L.src[q]) % 16) {
+            set_error("launch_moves: array %d is not 16-byte aligned", q);
+            return IFOS_EINVAL;
+        }
+        L.start[q] = (int)blocks;
+        blocks += (L.len[q] + kMoveElems - 1) / kMoveElems;
+    }
+    L.start[L.n] = (int)blocks;
+    if (blocks == 0) return IFOS_OK;
+    if (blocks > 2147483647) {
+        set_error("launch_moves: %lld workgroups", (long long)blocks);
+        return IFOS_EINVAL;
+    }
+    ProfScope ps_(IFOS_K_OTHER, st);
+    hipLaunchKernelGGL(k_moves, dim3((unsigned)blocks), dim3(256), 0, st, L);
+    return hip_check(hipGetLastError(), "k_moves");
+}
+
 int launch_td_integrate(const ifos_geom *g, float *const u[3], const float *const v[3], float dt, hipStream_t s)
 {
     const size_t n = ifos_field_elems(g);

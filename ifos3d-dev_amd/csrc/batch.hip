@@ -29,6 +29,7 @@
 #include <atomic>
 #include <map>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "ifos_dev.h"
@@ -37,8 +38,7 @@ namespace ifos {
 
 #define IFOS_CHUNK_MAX 32
 
-// class of a point: 1 = in a CPML slab, 0 = in the interior box
-static int point_class(const ifos_geom *g, int i, int j, int k)
+int point_class(const ifos_geom *g, int i, int j, int k)
 {
     return (slab_h(i, g->nx, g->fw, 1) || slab_h(j, g->ny, g->fw, !g->free_surf) || slab_h(k, g->nz, g->fw, 1)) ? 1
                                                                                                               : 0;
@@ -86,31 +86,35 @@ __global__ void k_bforces(DevGeom g, BFields F, const float *rip, const float *r
     }
 }
 
-// adjoint traces (update_v_ssg.c:512-522): thread per (receiver, shot); the
-// first receiver of a cell applies its whole same-cell chain in order.
-// cls: 0 interior cells only, 1 slab cells only, 2 all.
+// adjoint traces (update_v_ssg.c:512-522, update_v_ssg_CPML.c:384-393): thread
+// per (receiver, shot); the first receiver of a cell applies its whole
+// same-cell chain in order.  before = 1: the cells of CPML slabs, ahead of the
+// velocity update; before = 0, after it: once more for those, and both
+// additions of the interior cells.
 __global__ __launch_bounds__(256) void k_badjoint(DevGeom g, BFields F, const int *rec, const int *chain,
                                                  const int *rcls, const float *adj, int ntr, int nt, int ldadj,
-                                                 int cls, Snap N)
+                                                 int before, Snap N)
 {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     const int s = blockIdx.y;
     if (r >= ntr) return;
     const int64_t rs = (int64_t)s * ntr;
     if (!chain[2 * (rs + r)]) return;
-    if (cls != 2 && rcls[rs + r] != cls) return;
+    const int cls = rcls[rs + r];
+    if (before && !cls) return;
     const int *p = rec + 3 * (rs + r);
     const int64_t c = at(g, p[1], p[0], p[2]);
     const int64_t so = (int64_t)s * F.fstride;
     const int64_t comp = (int64_t)ntr * ldadj;
     const float *a = adj + (int64_t)s * 3 * comp;
     float x = F.vx[so + c], y = F.vy[so + c], z = F.vz[so + c];
-    for (int q = r; q >= 0 && q < ntr; q = chain[2 * (rs + q) + 1]) {
-        const int64_t o = (int64_t)q * ldadj + nt;
-        x += a[o];
-        z += a[2 * comp + o];
-        y += a[comp + o];
-    }
+    for (int times = before || cls ? 1 : 2; times > 0; --times)
+        for (int q = r; q >= 0 && q < ntr; q = chain[2 * (rs + q) + 1]) {
+            const int64_t o = (int64_t)q * ldadj + nt;
+            x += a[o];
+            z += a[2 * comp + o];
+            y += a[comp + o];
+        }
     F.vx[so + c] = x;
     F.vy[so + c] = y;
     F.vz[so + c] = z;
@@ -123,13 +127,27 @@ __global__ __launch_bounds__(256) void k_badjoint(DevGeom g, BFields F, const in
     }
 }
 
-// explosive sources (psource.c:26-54), one thread per shot
-__global__ void k_bpsource(DevGeom g, BFields F, const int *src, const float *sig, int nsrc, int nt, int ntall,
-                           int ldsig)
+// explosive sources (psource.c:26-54, the first thread of each shot, sources
+// in order) and seismograms (seismo_ssg.c:51-53, thread per receiver and
+// shot; sec [S][3][ntr][ldsec], or null) in one launch: the one writes
+// stresses, the other reads velocities
+__global__ __launch_bounds__(256) void k_bpoints(DevGeom g, BFields F, const int *src, const float *sig, int nsrc,
+                                                int nt, int ntall, int ldsig, const int *rec, int ntr, int ldsec,
+                                                float *sec)
 {
-    const int s = blockIdx.x;
-    if (threadIdx.x != 0) return;
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    const int s = blockIdx.y;
     const int64_t so = (int64_t)s * F.fstride;
+    if (sec && r < ntr) {
+        const int *p = rec + 3 * ((int64_t)s * ntr + r);
+        const int64_t c = so + at(g, p[1], p[0], p[2]);
+        const int64_t comp = (int64_t)ntr * ldsec;
+        float *o = sec + (int64_t)s * 3 * comp + (int64_t)r * ldsec + nt;
+        o[0] = F.vx[c];
+        o[comp] = F.vy[c];
+        o[2 * comp] = F.vz[c];
+    }
+    if (r != 0) return;
     float amp = 0.0f;
     const double den = 2.0 * g.dx * g.dy * g.dz;
     for (int l = 0; l < nsrc; ++l) {
@@ -144,22 +162,6 @@ __global__ void k_bpsource(DevGeom g, BFields F, const int *src, const float *si
         F.syy[c] += amp;
         F.szz[c] += amp;
     }
-}
-
-// seismo_ssg.c:51-53, thread per (receiver, shot); sec [S][3][ntr][ldsec]
-__global__ __launch_bounds__(256) void k_bseismo(DevGeom g, BFields F, const int *rec, int ntr, int ins, int ldsec,
-                                                float *sec)
-{
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    const int s = blockIdx.y;
-    if (r >= ntr) return;
-    const int *p = rec + 3 * ((int64_t)s * ntr + r);
-    const int64_t c = (int64_t)s * F.fstride + at(g, p[1], p[0], p[2]);
-    const int64_t comp = (int64_t)ntr * ldsec;
-    float *o = sec + (int64_t)s * 3 * comp + (int64_t)r * ldsec + ins;
-    o[0] = F.vx[c];
-    o[comp] = F.vy[c];
-    o[2 * comp] = F.vz[c];
 }
 
 // surface_ssg_elastic.c:78-112 for every shot (blockIdx.z)
@@ -190,21 +192,22 @@ __global__ void k_bsurface(DevGeom g, BFields F, float *sxy, float *syz, const f
 }
 
 // chunked DFT: nsnap (<= CH) snapshots of one shot's v, every accumulator
-// of the cell updated nsnap times in registers.  trig[(c*NF + l)*2 + {0,1}]
-// are the cos/sin factors of snapshot c (disc_fourier.c:42-44).  One thread
+// of the cell updated nsnap times in registers.  trig[(c*tstride + l)*2 +
+// {0,1}] are the cos/sin factors of snapshot c (disc_fourier.c:42-44).  One thread
 // per cell of [1..N]^3, shot and velocity component (blockIdx.z = shot * ny
 // + j - 1, blockIdx.y = 3 * (i row block) + component), so a thread holds
 // one component's snapshots and its two accumulators; the frequencies are
 // walked in order with the next frequency's accumulators loaded while the
-// current one is updated.
+// current one is updated.  FIRST: the accumulators start at 0 and are not
+// read, which saves their zeroing as well.
 struct FBase {
     float *p[6];
 };
 
-template <int NF, int CH, bool KAHAN>
+template <int NF, int CH, bool KAHAN, bool FIRST>
 __global__ __launch_bounds__(256) void k_dft_chunk(DevGeom g, const float *ring, int64_t rstride, int nsnap,
                                                   FBase F, FBase Cc, int64_t fshot, uint32_t tot,
-                                                  const double *__restrict__ trig)
+                                                  const double *__restrict__ trig, int tstride)
 {
     const int q = (int)(blockIdx.y % 3u);  // velocity component: accumulators q (Re) and 3 + q (Im)
     const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
@@ -229,16 +232,16 @@ __global__ __launch_bounds__(256) void k_dft_chunk(DevGeom g, const float *ring,
     float a[2], cm[2], an[2], cn[2];
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
-        a[n] = bload(r[n], vo, 0);
-        cm[n] = KAHAN ? bload(rc[n], vo, 0) : 0.0f;
+        a[n] = FIRST ? 0.0f : bload(r[n], vo, 0);
+        cm[n] = KAHAN && !FIRST ? bload(rc[n], vo, 0) : 0.0f;
     }
 #pragma unroll
     for (int l = 0; l < NF; ++l) {
         if (l + 1 < NF) {
 #pragma unroll
             for (int n = 0; n < 2; ++n) {
-                an[n] = bload(r[n], vo, (uint32_t)(l + 1) * g.fbytes);
-                cn[n] = KAHAN ? bload(rc[n], vo, (uint32_t)(l + 1) * g.fbytes) : 0.0f;
+                an[n] = FIRST ? 0.0f : bload(r[n], vo, (uint32_t)(l + 1) * g.fbytes);
+                cn[n] = KAHAN && !FIRST ? bload(rc[n], vo, (uint32_t)(l + 1) * g.fbytes) : 0.0f;
             }
         }
 #pragma unroll
@@ -247,7 +250,7 @@ __global__ __launch_bounds__(256) void k_dft_chunk(DevGeom g, const float *ring,
 #pragma unroll
             for (int c = 0; c < CH; ++c)
                 if (c < nsnap) {
-                    const double term = (double)v[c] * trig[(c * NF + l) * 2 + n];
+                    const double term = (double)v[c] * trig[(c * tstride + l) * 2 + n];
                     if (KAHAN) {
                         const float yv = (float)(term - (double)cmp);
                         const float t = acc + yv;
@@ -275,6 +278,138 @@ static __global__ void k_bfill(float *d, int64_t n, float v)
     int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (; t < n; t += stride) d[t] = v;
+}
+
+int dft_trig(const ifos_geom *g, const float *finv, int nf, int ntast, double *out)
+{
+    const int nsamp = g->nt / ntast;
+    for (int back = 0; back < 2; ++back)
+        for (int q = 0; q < nsamp; ++q) {
+            const int nt = (q + 1) * ntast;
+            float t = 0.0f;
+            if (back == 0) t = nt * g->dt;
+            if (back == 1) t = g->time - nt * g->dt;
+            double *o = out + ((size_t)back * nsamp + q) * nf * 2;
+            for (int l = 0; l < nf; ++l) {
+                o[2 * l + 0] = cos(2.0 * t * finv[l] * M_PI) * g->dt * ntast;
+                o[2 * l + 1] = sin(2.0 * t * finv[l] * M_PI) * g->dt * ntast;
+            }
+        }
+    return nsamp;
+}
+
+template <int NF>
+static void dft_chunk_nf(int chunk, bool kahan, bool first, dim3 grid, dim3 block, hipStream_t st, const DevGeom &G,
+                         const float *ring, int64_t rstride, int nsnap, const FBase &F, const FBase &C,
+                         int64_t fshot, uint32_t tot, const double *trig, int tstride)
+{
+    auto go = [&](auto ch) {
+        constexpr int CH = decltype(ch)::value;
+        if (kahan && first)
+            hipLaunchKernelGGL((k_dft_chunk<NF, CH, true, true>), grid, block, 0, st, G, ring, rstride, nsnap, F, C,
+                               fshot, tot, trig, tstride);
+        else if (kahan)
+            hipLaunchKernelGGL((k_dft_chunk<NF, CH, true, false>), grid, block, 0, st, G, ring, rstride, nsnap, F, C,
+                               fshot, tot, trig, tstride);
+        else if (first)
+            hipLaunchKernelGGL((k_dft_chunk<NF, CH, false, true>), grid, block, 0, st, G, ring, rstride, nsnap, F, C,
+                               fshot, tot, trig, tstride);
+        else
+            hipLaunchKernelGGL((k_dft_chunk<NF, CH, false, false>), grid, block, 0, st, G, ring, rstride, nsnap, F,
+                               C, fshot, tot, trig, tstride);
+    };
+    if (chunk <= 4) go(std::integral_constant<int, 4>{});
+    else if (chunk <= 8) go(std::integral_constant<int, 8>{});
+    else if (chunk <= 16) go(std::integral_constant<int, 16>{});
+    else if (chunk <= 24) go(std::integral_constant<int, 24>{});
+    else go(std::integral_constant<int, 32>{});
+}
+
+int launch_dft_chunk(const ifos_geom *g, int ns, const float *ring, int chunk, int nsnap, float *const Fp[6],
+                     float *const Cp[6], int64_t fshot, const double *trig, int nf, bool first, hipStream_t st)
+{
+    DevGeom G = make_dev_geom(g);
+    const size_t fe = ifos_field_elems(g);
+    const int64_t rstride = (int64_t)chunk * 3 * (int64_t)fe;
+    dim3 block(64, 4), grid((unsigned)((g->nz + 63) / 64), (unsigned)(3 * ((g->nx + 3) / 4)), (unsigned)(ns * g->ny));
+    ProfScope ps_(IFOS_K_DFT, st);
+    // up to 8 frequencies a launch, and their fields below 4 GiB (the
+    // accumulators' buffer offsets are 32-bit)
+    const int most = (int)std::min<size_t>(8, 4294967295u / (fe * 4));
+    for (int l0 = 0; l0 < nf; l0 += most) {
+        const int n = std::min(most, nf - l0);
+        FBase F, C = {};
+        for (int q = 0; q < 6; ++q) {
+            F.p[q] = Fp[q] + (size_t)l0 * fe;
+            if (Cp) C.p[q] = Cp[q] + (size_t)l0 * fe;
+        }
+        const uint32_t tot = (uint32_t)(n * fe * 4);
+        const double *tr = trig + 2 * l0;
+#define IFOS_CHUNK_CASE(NFV)                                                                                    \
+    case NFV:                                                                                                   \
+        dft_chunk_nf<NFV>(chunk, Cp != nullptr, first, grid, block, st, G, ring, rstride, nsnap, F, C, fshot,    \
+                          tot, tr, nf);                                                                         \
+        break;
+        switch (n) {
+            IFOS_CHUNK_CASE(1)
+            IFOS_CHUNK_CASE(2)
+            IFOS_CHUNK_CASE(3)
+            IFOS_CHUNK_CASE(4)
+            IFOS_CHUNK_CASE(5)
+            IFOS_CHUNK_CASE(6)
+            IFOS_CHUNK_CASE(7)
+            IFOS_CHUNK_CASE(8)
+        default: set_error("dft_chunk: nf=%d", n); return IFOS_EINVAL;
+        }
+#undef IFOS_CHUNK_CASE
+        const int rc = hip_check(hipGetLastError(), "k_dft_chunk");
+        if (rc) return rc;
+    }
+    return IFOS_OK;
+}
+
+int launch_step(const StepArgs &A, int back, int nt, const Snap *N, bool seis, hipStream_t st)
+{
+    const ifos_geom *g = A.g;
+    const DevGeom G = make_dev_geom(g);
+    const ifos_fields &f = A.f;
+    const BFields BF = {f.vx, f.vy, f.vz, f.sxx, f.syy, f.szz, A.S.fstride};
+    const int nt2 = g->nt + 2;
+    const dim3 rgrid((unsigned)((A.ntr + 255) / 256), (unsigned)A.ns);
+    const Snap none = {nullptr, 0, 0, 0};
+    auto forces = [&](int cls, const Snap &snap) {
+        ProfScope ps_(IFOS_K_SOURCES, st);
+        hipLaunchKernelGGL(k_bforces, dim3(A.ns), dim3(64), 0, st, G, BF, A.m.rip, A.m.rjp, A.m.rkp, A.src,
+                           A.srccls, A.sig, 1, nt, nt2, cls, snap);
+        return hip_check(hipGetLastError(), "k_bforces");
+    };
+    auto adjoint = [&](int before, const Snap &snap) {
+        ProfScope ps_(IFOS_K_SOURCES, st);
+        hipLaunchKernelGGL(k_badjoint, rgrid, dim3(256), 0, st, G, BF, A.rec, A.chain, A.rcls, A.adj, A.ntr, nt,
+                           nt2, before, snap);
+        return hip_check(hipGetLastError(), "k_badjoint");
+    };
+    int rc = IFOS_OK;
+    // points in CPML cells: before the fused update
+    if (!back && A.force_slab) rc = forces(1, none);
+    if (!rc && back && A.slab_rec && A.ntr > 0) rc = adjoint(1, none);
+    if (!rc) rc = launch_v_shots(g, &f, &A.m, A.prof, &A.ps, A.S, N, A.cfg_v, st);
+    if (!rc && !back && A.force_in) rc = forces(0, N ? *N : none);
+    if (!rc && back && A.ntr > 0) rc = adjoint(0, N ? *N : none);
+    if (!rc) rc = launch_s_shots(g, &f, &A.m, A.prof, &A.pv, A.S, A.cfg_s, st, A.V);
+    if (!rc && !back && (A.explosive || (seis && A.ntr > 0))) {
+        ProfScope ps_(IFOS_K_SOURCES, st);
+        const bool sec = seis && A.ntr > 0;
+        hipLaunchKernelGGL(k_bpoints, sec ? rgrid : dim3(1, (unsigned)A.ns), dim3(256), 0, st, G, BF, A.src, A.sig,
+                           1, nt, g->nt, nt2, A.rec, A.ntr, g->nt + 1, sec ? A.syn : nullptr);
+        rc = hip_check(hipGetLastError(), "k_bpoints");
+    }
+    if (!rc && g->free_surf) {
+        hipLaunchKernelGGL(k_bsurface, dim3((unsigned)((g->nz + 63) / 64), (unsigned)g->nx, (unsigned)A.ns),
+                           dim3(64), 0, st, G, BF, f.sxy, f.syz, A.m.u, A.m.pi);
+        rc = hip_check(hipGetLastError(), "k_bsurface");
+    }
+    return rc;
 }
 
 }  // namespace ifos
@@ -311,6 +446,7 @@ struct ifos_batch {
     int nf, tast, ntast, nsamp;
     int ntr;                   // receivers of the current batch
     bool any_slab_src, any_slab_rec;
+    bool any_force, any_explosive;  // a body force in the interior, an explosive source
     MarchCfg cfg_v, cfg_s;     // tile shapes of the two march launches
     // viscoelastic (L mechanisms): memory variables [S][L][fe] x 6, shared
     // relaxation ratios and their averages
@@ -320,7 +456,7 @@ struct ifos_batch {
     hipStream_t st;
     std::vector<void *> allocs;
     // captured time loops with the buffer set (cur_set) each leaves current
-    std::map<std::tuple<int, int, int, int, int, int, int>, std::pair<hipGraphExec_t, int>> graphs;
+    std::map<std::tuple<int, int, int, int, int, int>, std::pair<hipGraphExec_t, int>> graphs;
     // identity of this context (never reused) and of its launch state
     // (bumped whenever cached graphs are dropped): the key of multi-level
     // graphs that include this context
@@ -546,26 +682,19 @@ extern "C" int ifos_batch_set_freqs(ifos_batch *b, const float *finv, int nf, in
     b->tast = tast;
     b->ntast = ifos_ntast(finv[nf - 1], tast, g->dt);
     b->nsamp = g->nt / b->ntast;
-    std::vector<double> h((size_t)(b->nsamp > 0 ? b->nsamp : 1) * nf * 2);
+    const size_t half = (size_t)b->nsamp * nf * 2;
+    std::vector<double> h(2 * half + 1);
+    dft_trig(g, finv, nf, b->ntast, h.data());
     for (int back = 0; back < 2; ++back) {
-        for (int q = 0; q < b->nsamp; ++q) {
-            const int nt = (q + 1) * b->ntast;
-            float t = 0.0f;
-            if (back == 0) t = nt * g->dt;
-            if (back == 1) t = g->time - nt * g->dt;
-            for (int l = 0; l < nf; ++l) {
-                h[((size_t)q * nf + l) * 2 + 0] = cos(2.0 * t * finv[l] * M_PI) * g->dt * b->ntast;
-                h[((size_t)q * nf + l) * 2 + 1] = sin(2.0 * t * finv[l] * M_PI) * g->dt * b->ntast;
-            }
-        }
         if (b->trig[back]) (void)hipFree(b->trig[back]);
         b->trig[back] = nullptr;
-        hipError_t e = hipMalloc((void **)&b->trig[back], h.size() * sizeof(double));
+        hipError_t e = hipMalloc((void **)&b->trig[back], std::max<size_t>(half, 1) * sizeof(double));
         if (e != hipSuccess) {
             set_error("hipMalloc(trig): %s", hipGetErrorString(e));
             return IFOS_ENOMEM;
         }
-        int rc = hip_check(hipMemcpy(b->trig[back], h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice),
+        int rc = hip_check(hipMemcpy(b->trig[back], h.data() + back * half, half * sizeof(double),
+                                     hipMemcpyHostToDevice),
                            "upload trig");
         if (rc) return rc;
     }
@@ -607,73 +736,28 @@ static int fill(float *d, size_t n, hipStream_t st)
 
 static int dft_chunk(ifos_batch *b, int back, int ns, int q0, int nsnap, hipStream_t st)
 {
-    const ifos_geom *g = &b->g;
-    DevGeom G = make_dev_geom(g);
-    FBase F, Cc = {};
-    for (int n = 0; n < 6; ++n) {
-        F.p[n] = b->F[(back ? 6 : 0) + n];
-        if (b->C[0]) Cc.p[n] = b->C[(back ? 6 : 0) + n];
-    }
-    const int64_t rstride = (int64_t)b->chunk * 3 * b->fe;
-    const int64_t fshot = (int64_t)b->nf_max * b->fe;
-    const uint32_t tot = (uint32_t)((size_t)b->nf * b->fe * 4);
-    const double *tr = b->trig[back] + (size_t)q0 * b->nf * 2;
-    dim3 block(64, 4), grid((unsigned)((g->nz + 63) / 64), (unsigned)(3 * ((g->nx + 3) / 4)), (unsigned)(ns * g->ny));
-    const bool kahan = b->prec == IFOS_DFT_KAHAN;
-    ProfScope ps_(IFOS_K_DFT, st);
-#define IFOS_CHUNK_LAUNCH(NFV, CHV)                                                                             \
-    do {                                                                                                        \
-        if (kahan)                                                                                              \
-            hipLaunchKernelGGL((k_dft_chunk<NFV, CHV, true>), grid, block, 0, st, G, b->ring, rstride, nsnap, F, \
-                               Cc, fshot, tot, tr);                                                             \
-        else                                                                                                    \
-            hipLaunchKernelGGL((k_dft_chunk<NFV, CHV, false>), grid, block, 0, st, G, b->ring, rstride, nsnap,   \
-                               F, Cc, fshot, tot, tr);                                                          \
-    } while (0)
-#define IFOS_CHUNK_CASE(NFV)                                                                                    \
-    case NFV:                                                                                                   \
-        if (b->chunk <= 4) IFOS_CHUNK_LAUNCH(NFV, 4);                                                           \
-        else if (b->chunk <= 8) IFOS_CHUNK_LAUNCH(NFV, 8);                                                      \
-        else if (b->chunk <= 16) IFOS_CHUNK_LAUNCH(NFV, 16);                                                    \
-        else if (b->chunk <= 24) IFOS_CHUNK_LAUNCH(NFV, 24);                                                    \
-        else IFOS_CHUNK_LAUNCH(NFV, 32);                                                                        \
-        break;
-    switch (b->nf) {
-        IFOS_CHUNK_CASE(1)
-        IFOS_CHUNK_CASE(2)
-        IFOS_CHUNK_CASE(3)
-        IFOS_CHUNK_CASE(4)
-        IFOS_CHUNK_CASE(5)
-        IFOS_CHUNK_CASE(6)
-        IFOS_CHUNK_CASE(7)
-        IFOS_CHUNK_CASE(8)
-    default: set_error("dft_chunk: nf=%d", b->nf); return IFOS_EINVAL;
-    }
-#undef IFOS_CHUNK_LAUNCH
-#undef IFOS_CHUNK_CASE
-    return hip_check(hipGetLastError(), "k_dft_chunk");
+    float *const *C = b->prec == IFOS_DFT_KAHAN ? b->C + (back ? 6 : 0) : nullptr;
+    return launch_dft_chunk(&b->g, ns, b->ring, b->chunk, nsnap, b->F + (back ? 6 : 0), C,
+                            (int64_t)b->nf_max * (int64_t)b->fe, b->trig[back] + (size_t)q0 * b->nf * 2, b->nf,
+                            q0 == 0, st);
 }
 
 // one propagation of NT steps for shots [0, ns); back = 0 forward, 1 adjoint
-static int bpass(ifos_batch *b, int back, int ns, int dft, int seis, hipStream_t st)
+static StepArgs step_args(const ifos_batch *b, int ns, ViscoF &V)
 {
-    const ifos_geom *g = &b->g;
-    DevGeom G = make_dev_geom(g);
-    ifos_fields f = bfields(b);
-    ifos_model m = bmodel(b);
-    ifos_psi ps, pv;
+    StepArgs A = {};
+    A.g = &b->g;
+    A.ns = ns;
+    A.f = bfields(b);
+    A.m = bmodel(b);
     for (int n = 0; n < 9; ++n) {
-        ps.p[n] = b->psi_s[n];
-        pv.p[n] = b->psi_v[n];
+        A.ps.p[n] = b->psi_s[n];
+        A.pv.p[n] = b->psi_v[n];
     }
-    const Shots S = {ns, (int64_t)b->fe, {b->pe[0], b->pe[1], b->pe[2]}};
-    const BFields BF = {f.vx, f.vy, f.vz, f.sxx, f.syy, f.szz, (int64_t)b->fe};
-    const int64_t rstride = (int64_t)b->chunk * 3 * b->fe;
-    const int ntr = b->ntr, nt2 = g->nt + 2;
-    const dim3 rgrid((unsigned)((ntr + 255) / 256), (unsigned)ns);
-    const Snap nosnap = {nullptr, 0, 0, 0};
-    ViscoF V = {};
+    A.prof = b->prof;
+    A.S = Shots{ns, (int64_t)b->fe, {b->pe[0], b->pe[1], b->pe[2]}};
     if (b->L) {
+        V = ViscoF{};
         for (int n = 0; n < 6; ++n) V.r[n] = b->r[n];
         V.taus = b->taus;
         V.taup = b->taup;
@@ -683,62 +767,42 @@ static int bpass(ifos_batch *b, int back, int ns, int dft, int seis, hipStream_t
         for (int l = 0; l < IFOS_MAX_L; ++l) V.eta[l] = b->eta[l];
         V.L = b->L;
         V.lstride = (int64_t)b->fe;
+        A.V = &V;
     }
+    A.src = b->src;
+    A.srccls = b->srccls;
+    A.sig = b->sig;
+    A.force_slab = b->any_slab_src;
+    A.force_in = b->any_force;
+    A.explosive = b->any_explosive;
+    A.rec = b->rec;
+    A.chain = b->chain;
+    A.rcls = b->rcls;
+    A.adj = b->adj;
+    A.syn = b->syn;
+    A.ntr = b->ntr;
+    A.slab_rec = b->any_slab_rec;
+    A.cfg_v = b->cfg_v;
+    A.cfg_s = b->cfg_s;
+    return A;
+}
+
+static int bpass(ifos_batch *b, int back, int ns, int dft, int seis, hipStream_t st)
+{
+    const ifos_geom *g = &b->g;
+    ViscoF V;
+    const StepArgs A = step_args(b, ns, V);
+    const int64_t rstride = (int64_t)b->chunk * 3 * b->fe;
     int nsnap = 0, q0 = 0;
     for (int nt = 1; nt <= g->nt; ++nt) {
         const bool samp = dft && nt % b->ntast == 0 && (nt / b->ntast) <= b->nsamp;
-        Snap N = nosnap;
+        Snap N = {nullptr, 0, 0, 0};
         if (samp) N = Snap{b->ring + (size_t)nsnap * 3 * b->fe, rstride, (uint32_t)(3 * (size_t)b->fe * 4), 0};
-        int rc = 0;
-        // sources in CPML cells: before the fused update
-        if (!back && b->any_slab_src) {
-            hipLaunchKernelGGL(k_bforces, dim3(ns), dim3(64), 0, st, G, BF, m.rip, m.rjp, m.rkp, b->src, b->srccls,
-                               b->sig, 1, nt, nt2, 1, nosnap);
-            rc = hip_check(hipGetLastError(), "k_bforces");
-        }
-        if (!rc && back && b->any_slab_rec && ntr > 0) {
-            hipLaunchKernelGGL(k_badjoint, rgrid, dim3(256), 0, st, G, BF, b->rec, b->chain, b->rcls, b->adj, ntr,
-                               nt, nt2, 1, nosnap);
-            rc = hip_check(hipGetLastError(), "k_badjoint");
-        }
-        if (!rc) rc = launch_v_shots(g, &f, &m, b->prof, &ps, S, samp ? &N : nullptr, b->cfg_v, st);
-        if (!rc && !back) {
-            ProfScope ps_(IFOS_K_SOURCES, st);
-            hipLaunchKernelGGL(k_bforces, dim3(ns), dim3(64), 0, st, G, BF, m.rip, m.rjp, m.rkp, b->src, b->srccls,
-                               b->sig, 1, nt, nt2, 0, N);
-            rc = hip_check(hipGetLastError(), "k_bforces");
-        }
-        if (!rc && back && ntr > 0) {
-            ProfScope ps_(IFOS_K_SOURCES, st);
-            hipLaunchKernelGGL(k_badjoint, rgrid, dim3(256), 0, st, G, BF, b->rec, b->chain, b->rcls, b->adj, ntr,
-                               nt, nt2, 0, N);
-            hipLaunchKernelGGL(k_badjoint, rgrid, dim3(256), 0, st, G, BF, b->rec, b->chain, b->rcls, b->adj, ntr,
-                               nt, nt2, 2, N);
-            rc = hip_check(hipGetLastError(), "k_badjoint");
-        }
-        if (!rc) rc = launch_s_shots(g, &f, &m, b->prof, &pv, S, b->cfg_s, st, b->L ? &V : nullptr);
-        if (!rc && !back) {
-            ProfScope ps_(IFOS_K_SOURCES, st);
-            hipLaunchKernelGGL(k_bpsource, dim3(ns), dim3(64), 0, st, G, BF, b->src, b->sig, 1, nt, g->nt, nt2);
-            rc = hip_check(hipGetLastError(), "k_bpsource");
-        }
-        if (!rc && samp) {
-            ++nsnap;
-            if (nsnap == b->chunk) {
-                rc = dft_chunk(b, back, ns, q0, nsnap, st);
-                q0 += nsnap;
-                nsnap = 0;
-            }
-        }
-        if (!rc && g->free_surf) {
-            hipLaunchKernelGGL(k_bsurface, dim3((unsigned)((g->nz + 63) / 64), (unsigned)g->nx, (unsigned)ns),
-                               dim3(64), 0, st, G, BF, f.sxy, f.syz, m.u, m.pi);
-            rc = hip_check(hipGetLastError(), "k_bsurface");
-        }
-        if (!rc && !back && seis && ntr > 0) {
-            ProfScope ps_(IFOS_K_SOURCES, st);
-            hipLaunchKernelGGL(k_bseismo, rgrid, dim3(256), 0, st, G, BF, b->rec, ntr, nt, g->nt + 1, b->syn);
-            rc = hip_check(hipGetLastError(), "k_bseismo");
+        int rc = launch_step(A, back, nt, samp ? &N : nullptr, seis != 0, st);
+        if (!rc && samp && ++nsnap == b->chunk) {
+            rc = dft_chunk(b, back, ns, q0, nsnap, st);
+            q0 += nsnap;
+            nsnap = 0;
         }
         if (rc) return rc;
     }
@@ -809,7 +873,7 @@ static int bpass_fused(ifos_batch *b, int back, int ns, int dft, int seis, hipSt
             set ^= 1;
         }
         const BFields BF = {cur[0], cur[1], cur[2], cur[3], cur[4], cur[5], (int64_t)b->fe};
-        if (!rc && !back) {
+        if (!rc && !back && b->any_force) {
             ProfScope ps_(IFOS_K_SOURCES, st);
             hipLaunchKernelGGL(k_bforces, dim3(ns), dim3(64), 0, st, G, BF, m.rip, m.rjp, m.rkp, b->src, b->srccls,
                                b->sig, 1, nt, nt2, 0, N);
@@ -819,8 +883,6 @@ static int bpass_fused(ifos_batch *b, int back, int ns, int dft, int seis, hipSt
             ProfScope ps_(IFOS_K_SOURCES, st);
             hipLaunchKernelGGL(k_badjoint, rgrid, dim3(256), 0, st, G, BF, b->rec, b->chain, b->rcls, b->adj, ntr,
                                nt, nt2, 0, N);
-            hipLaunchKernelGGL(k_badjoint, rgrid, dim3(256), 0, st, G, BF, b->rec, b->chain, b->rcls, b->adj, ntr,
-                               nt, nt2, 2, N);
             rc = hip_check(hipGetLastError(), "k_badjoint");
         }
         if (!rc && samp) {
@@ -833,8 +895,9 @@ static int bpass_fused(ifos_batch *b, int back, int ns, int dft, int seis, hipSt
         }
         if (!rc && !back && seis && ntr > 0) {
             ProfScope ps_(IFOS_K_SOURCES, st);
-            hipLaunchKernelGGL(k_bseismo, rgrid, dim3(256), 0, st, G, BF, b->rec, ntr, nt, g->nt + 1, b->syn);
-            rc = hip_check(hipGetLastError(), "k_bseismo");
+            hipLaunchKernelGGL(k_bpoints, rgrid, dim3(256), 0, st, G, BF, b->src, b->sig, 0, nt, g->nt, nt2, b->rec,
+                               ntr, g->nt + 1, b->syn);
+            rc = hip_check(hipGetLastError(), "k_bpoints");
         }
         if (rc) return rc;
     }
@@ -849,12 +912,20 @@ static int zero_state(ifos_batch *b, int ns, hipStream_t st)
     for (int n = 0; n < 9 && !rc; ++n) rc = fill(b->fields[n], (size_t)ns * b->fe, st);
     for (int n = 0; n < 9 && !rc; ++n) rc = fill(b->psi_s[n], (size_t)ns * b->pe[n / 3], st);
     for (int n = 0; n < 9 && !rc; ++n) rc = fill(b->psi_v[n], (size_t)ns * b->pe[n / 3], st);
-    for (int n = 0; n < 9 && !rc; ++n) rc = fill(b->fields_alt[n], (size_t)ns * b->fe, st);
-    for (int n = 0; n < 9 && !rc; ++n) rc = fill(b->psi_v_alt[n], (size_t)ns * b->pe[n / 3], st);
+    if (fused_ok(b)) {  // the second buffer set
+        for (int n = 0; n < 9 && !rc; ++n) rc = fill(b->fields_alt[n], (size_t)ns * b->fe, st);
+        for (int n = 0; n < 9 && !rc; ++n) rc = fill(b->psi_v_alt[n], (size_t)ns * b->pe[n / 3], st);
+    }
     b->cur_set = 0;
     if (b->L)  // zero_wavefield.c:80-95
         for (int n = 0; n < 6 && !rc; ++n) rc = fill(b->r[n], (size_t)ns * b->L * b->fe, st);
     return rc;
+}
+
+// the point operations a captured time loop holds
+static int point_key(const ifos_batch *b)
+{
+    return b->any_slab_src | b->any_slab_rec << 1 | b->any_force << 2 | b->any_explosive << 3;
 }
 
 // runs the pass, through a cached graph when use_graph
@@ -865,7 +936,7 @@ static int run_pass(ifos_batch *b, int back, int ns, int dft, int seis, int use_
     b->last_fused = fz;
     auto pass = [&](hipStream_t s) { return fz ? bpass_fused(b, back, ns, dft, seis, s) : bpass(b, back, ns, dft, seis, s); };
     if (!use_graph) return pass(st);
-    auto key = std::make_tuple(back, ns, dft, seis, b->ntr, (int)b->any_slab_src, (int)b->any_slab_rec);
+    auto key = std::make_tuple(back, ns, dft, seis, b->ntr, point_key(b));
     auto it = b->graphs.find(key);
     if (it == b->graphs.end()) {
         hipGraph_t graph;
@@ -954,7 +1025,7 @@ static int batch_prepare(ifos_batch *b, const ifos_shot *shots, int ns, const ch
     std::vector<float> sig((size_t)ns * nt2);
     std::vector<int> src(4 * (size_t)ns), srccls(ns), rec(3 * (size_t)ns * ntrs), chain(2 * (size_t)ns * ntrs),
         rcls((size_t)ns * ntrs);
-    b->any_slab_src = b->any_slab_rec = false;
+    b->any_slab_src = b->any_slab_rec = b->any_force = b->any_explosive = false;
     for (int s = 0; s < ns; ++s) {
         const ifos_shot &sh = shots[s];
         int rc = ifos_wavelet(g, sh.source_shape, sh.tshift, sh.fc, sh.amp, sig.data() + (size_t)s * nt2);
@@ -964,7 +1035,8 @@ static int batch_prepare(ifos_batch *b, const ifos_shot *shots, int ns, const ch
         src[4 * s + 2] = sh.src_k;
         src[4 * s + 3] = sh.src_type;
         srccls[s] = point_class(g, sh.src_i, sh.src_j, sh.src_k);
-        if (srccls[s] && sh.src_type >= 2 && sh.src_type <= 5) b->any_slab_src = true;
+        if (sh.src_type == 1) b->any_explosive = true;
+        if (sh.src_type >= 2 && sh.src_type <= 5) (srccls[s] ? b->any_slab_src : b->any_force) = true;
         if (ntr > 0) {
             rc = ifos_rec_chain(sh.rec_ijk, ntr, chain.data() + 2 * (size_t)s * ntr);
             if (rc) return rc;
@@ -993,8 +1065,10 @@ static int batch_prepare(ifos_batch *b, const ifos_shot *shots, int ns, const ch
     }
     // ifos3d.c:738-739: zero wavefields and the accumulators of these shots
     if (!rc) rc = zero_state(b, ns, st);
+    // (the first chunk of a pass writes the frequencies in use without reading
+    // them; without a sample, or with frequencies not in use, fill)
     const size_t fshot = (size_t)b->nf_max * b->fe;
-    for (int n = 0; n < 12 && !rc && want_adj; ++n) {
+    for (int n = 0; n < 12 && !rc && want_adj && (b->nsamp < 1 || b->nf < b->nf_max); ++n) {
         rc = fill(b->F[n], (size_t)ns * fshot, st);
         if (!rc && b->C[n]) rc = fill(b->C[n], (size_t)ns * fshot, st);
     }
@@ -1141,8 +1215,7 @@ extern "C" int ifos_levels_run(ifos_batch *const *lv, int nlev, const ifos_shot 
         std::vector<long long> key;
         for (int l = 0; l < nlev; ++l) {
             const ifos_batch *b = lv[l];
-            key.insert(key.end(), {b->gen, b->ver, ns[l], b->ntr, (long long)b->any_slab_src,
-                                   (long long)b->any_slab_rec, (long long)fused_ok(b)});
+            key.insert(key.end(), {b->gen, b->ver, ns[l], b->ntr, (long long)point_key(b), (long long)fused_ok(b)});
         }
         ifos_batch *b0 = lv[0];
         if (!b0->lv_exec || b0->lv_key != key) {

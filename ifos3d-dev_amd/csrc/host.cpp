@@ -352,7 +352,13 @@ struct ifos_ctx {
     int *src;              // [4]
     int *rec;              // [ntr][3]
     int *chain;            // [ntr][2] same-cell chain of the receivers
+    int *srccls, *rcls;    // [1], [ntr] point_class of the source and the receivers
+    bool slab_src, slab_rec;
     float *adj;            // [3][ntr][nt+2]
+    float *ring;           // [chunk][3][fe] velocity snapshots of the chunked DFT
+    int chunk;             // snapshots of the ring; 0: one DFT pass per sample; -1: not decided
+    double *trig;          // [2][nsamp][nf][2] (dft_trig)
+    int nsamp;
     float finv[IFOS_MAX_NF];
     int nf, tast;
     // viscoelastic (L mechanisms): memory variables (L fields per component),
@@ -420,11 +426,18 @@ extern "C" int ifos_ctx_create(ifos_ctx **out, const ifos_geom *g, int nf_max, i
     if (!rc) rc = dalloc(c, (void **)&c->src, 4 * sizeof(int));
     if (!rc) rc = dalloc(c, (void **)&c->rec, 3 * sizeof(int) * (size_t)(ntr_max > 0 ? ntr_max : 1));
     if (!rc) rc = dalloc(c, (void **)&c->chain, 2 * sizeof(int) * (size_t)(ntr_max > 0 ? ntr_max : 1));
+    if (!rc) rc = dalloc(c, (void **)&c->srccls, sizeof(int));
+    if (!rc) rc = dalloc(c, (void **)&c->rcls, sizeof(int) * (size_t)(ntr_max > 0 ? ntr_max : 1));
+    if (!rc) rc = dalloc(c, (void **)&c->trig, 4 * sizeof(double) * (size_t)g->nt * (size_t)nf_max);
     if (!rc) rc = dalloc(c, (void **)&c->adj, 3 * (size_t)(ntr_max > 0 ? ntr_max : 1) * (g->nt + 2) * 4);
     if (rc) {
         ifos_ctx_destroy(c);
         return rc;
     }
+    c->ring = nullptr;
+    c->chunk = -1;
+    c->nsamp = 0;
+    c->slab_src = c->slab_rec = false;
     c->nf = 0;
     c->tast = 100;
     c->L = 0;
@@ -564,63 +577,61 @@ static ShotState ctx_state(const ifos_ctx *c)
     return S;
 }
 
-// time step nt of a propagation of state S in the order of ifos3d.c:754-814
-// (back = 0: forward with the source) and ifos3d.c:905-960 (back = 1:
-// adjoint with the receivers injecting): velocity update with its
-// injections, stress update, explosive source, the DFT sample (dft), free
-// surface, seismograms (d_syn, forward only)
-static int step(ifos_ctx *c, const ShotState &S, int back, const ifos_shot *s, int nt, bool dft, int ntast,
-                float *d_syn, hipStream_t st)
-{
-    const ifos_geom *g = &c->g;
-    ifos_fields f = {S.fields[0], S.fields[1], S.fields[2], S.fields[3], S.fields[4],
-                     S.fields[5], S.fields[6], S.fields[7], S.fields[8]};
-    ifos_model m = ctx_model(c);
-    ifos_psi ps, pv;
-    for (int n = 0; n < 9; ++n) {
-        ps.p[n] = S.psi_s[n];
-        pv.p[n] = S.psi_v[n];
-    }
-    int rc = ifos_update_v(g, IFOS_REGION_INTERIOR, &f, &m, c->prof, &ps, st);
-    if (!rc) {
-        if (!back)
-            rc = ifos_add_forces(g, &f, &m, c->src, c->sig, 1, nt, 0.0f, 0.0f, st);
-        else
-            rc = ifos_add_adjoint(g, &f, c->rec, c->chain, c->adj, s->ntr, nt, st);
-    }
-    if (!rc) rc = ifos_update_v(g, IFOS_REGION_CPML, &f, &m, c->prof, &ps, st);
-    if (!rc && back) rc = ifos_add_adjoint(g, &f, c->rec, c->chain, c->adj, s->ntr, nt, st);
-    if (c->L) {
-        ifos_visco V;
-        for (int n = 0; n < 6; ++n) V.r[n] = S.r[n];
-        V.taus = c->taus;
-        V.taup = c->taup;
-        V.tausipjp = c->tavg[0];
-        V.tausjpkp = c->tavg[1];
-        V.tausipkp = c->tavg[2];
-        V.eta = c->eta[0];
-        for (int l = 1; l < IFOS_MAX_L; ++l) V.eta_more[l - 1] = c->eta[l];
-        V.L = c->L;
-        if (!rc) rc = ifos_update_s_visco(g, IFOS_REGION_INTERIOR, &f, &m, &V, c->prof, &pv, st);
-        if (!rc) rc = ifos_update_s_visco(g, IFOS_REGION_CPML, &f, &m, &V, c->prof, &pv, st);
-    } else {
-        if (!rc) rc = ifos_update_s(g, IFOS_REGION_INTERIOR, &f, &m, c->prof, &pv, st);
-        if (!rc) rc = ifos_update_s(g, IFOS_REGION_CPML, &f, &m, c->prof, &pv, st);
-    }
-    if (!rc && !back) rc = ifos_psource(g, &f, c->src, c->sig, 1, nt, st);
-    if (!rc && dft && nt % ntast == 0) {
-        float *Fp[6], *Cp[6];
-        for (int n = 0; n < 6; ++n) {
-            Fp[n] = c->F[(back ? 6 : 0) + n];
-            Cp[n] = c->C[(back ? 6 : 0) + n];
+// one time step of a state of the context (launch_step): the whole-domain
+// marches, each one launch for the interior and the CPML slabs
+struct CtxStep {
+    ViscoF V;
+    StepArgs A;
+    CtxStep(const ifos_ctx *c, const ShotState &S, const ifos_shot *s, float *d_syn) : V{}, A{}
+    {
+        A.g = &c->g;
+        A.ns = 1;
+        A.f = ifos_fields{S.fields[0], S.fields[1], S.fields[2], S.fields[3], S.fields[4],
+                          S.fields[5], S.fields[6], S.fields[7], S.fields[8]};
+        for (int n = 0; n < 9; ++n) {
+            A.ps.p[n] = S.psi_s[n];
+            A.pv.p[n] = S.psi_v[n];
         }
-        rc = ifos_discfourier(g, &f, Fp, c->prec == IFOS_DFT_KAHAN ? Cp : nullptr, c->finv, c->nf, nt, ntast, back,
-                              c->prec, st);
+        A.m = ctx_model(c);
+        A.prof = c->prof;
+        A.S = Shots{1, 0, {0, 0, 0}};
+        if (c->L) {
+            for (int n = 0; n < 6; ++n) V.r[n] = S.r[n];
+            V.taus = c->taus;
+            V.taup = c->taup;
+            V.tausipjp = c->tavg[0];
+            V.tausjpkp = c->tavg[1];
+            V.tausipkp = c->tavg[2];
+            for (int l = 0; l < IFOS_MAX_L; ++l) V.eta[l] = c->eta[l];
+            V.L = c->L;
+            V.lstride = (int64_t)c->fe;
+            A.V = &V;
+        }
+        const bool force = s->src_type >= 2 && s->src_type <= 5;
+        A.src = c->src;
+        A.srccls = c->srccls;
+        A.sig = c->sig;
+        A.force_slab = force && c->slab_src;
+        A.force_in = force && !c->slab_src;
+        A.explosive = s->src_type == 1;
+        A.rec = c->rec;
+        A.chain = c->chain;
+        A.rcls = c->rcls;
+        A.adj = c->adj;
+        A.syn = d_syn;
+        A.ntr = s->ntr;
+        A.slab_rec = c->slab_rec;
+        A.cfg_v = plain_cfg();
+        A.cfg_v.group = A.cfg_v.split = 0;
+        A.cfg_v.kb = A.cfg_v.sb = 1;
+        A.cfg_s = A.cfg_v;
     }
-    if (!rc && g->free_surf) rc = ifos_surface(g, &f, &m, st);
-    if (!rc && !back && d_syn) rc = ifos_seismo(g, &f, c->rec, s->ntr, nt, g->nt, d_syn, st);
-    return rc;
-}
+    CtxStep(const CtxStep &) = delete;
+    int operator()(int back, int nt, const Snap *N, hipStream_t st) const
+    {
+        return launch_step(A, back, nt, N, !back && A.syn, st);
+    }
+};
 
 // NaN probe of ifos3d.c:761 on vy of state S (the reference checks every
 // step on the host; here every 64 steps)
@@ -638,28 +649,76 @@ static int probe_nan(ifos_ctx *c, const ShotState &S, int nt, hipStream_t st)
     return rc;
 }
 
+// the snapshot ring of the chunked DFT, allocated by the first shot that
+// samples: 16 snapshots (the 6 nf accumulators of a cell cross HBM once per
+// chunk instead of once per sample: at 276^3 with 6 frequencies 0.5 ms per
+// sample against 1.4 ms), fewer where they would take more than a quarter of
+// the free memory, none (one pass per sample) where 4 would, or where one
+// snapshot exceeds the 4 GiB of a buffer descriptor
+static int ring_alloc(ifos_ctx *c)
+{
+    if (c->chunk >= 0) return IFOS_OK;
+    size_t free_b = 0, total_b = 0;
+    const size_t snap = 3 * c->fe * 4;
+    int rc = hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+    if (rc) return rc;
+    for (int ch = 16; ch >= 4; ch /= 2) {
+        if (snap >= 4294967295u || ch * snap > free_b / 4) continue;
+        if (hipMalloc((void **)&c->ring, ch * snap) != hipSuccess) {
+            (void)hipGetLastError();
+            c->ring = nullptr;
+            continue;
+        }
+        c->allocs.push_back(c->ring);
+        c->chunk = ch;
+        return IFOS_OK;
+    }
+    c->chunk = 0;
+    return IFOS_OK;
+}
+
 // one propagation of NT steps; back = 0 forward (sources), 1 adjoint
 static int propagate(ifos_ctx *c, int back, const ifos_shot *s, int ntast, float *d_syn, hipStream_t st)
 {
+    const ifos_geom *g = &c->g;
     const ShotState S = ctx_state(c);
+    const CtxStep step(c, S, s, d_syn);
     const bool dft = s->want_adjoint != 0;
-    for (int nt = 1; nt <= c->g.nt; ++nt) {
+    float *const *F = c->F + (back ? 6 : 0);
+    float *const *C = c->prec == IFOS_DFT_KAHAN ? c->C + (back ? 6 : 0) : nullptr;
+    int nsnap = 0, q0 = 0;
+    auto chunk = [&] {
+        const double *tr = c->trig + ((size_t)back * c->nsamp + q0) * c->nf * 2;
+        const int rc = launch_dft_chunk(g, 1, c->ring, c->chunk, nsnap, F, C, 0, tr, c->nf, q0 == 0, st);
+        q0 += nsnap;
+        nsnap = 0;
+        return rc;
+    };
+    for (int nt = 1; nt <= g->nt; ++nt) {
+        const bool samp = dft && nt % ntast == 0;
+        Snap N = {nullptr, 0, 0, 0};
+        if (samp && c->chunk > 0) N = Snap{c->ring + (size_t)nsnap * 3 * c->fe, 0, (uint32_t)(3 * c->fe * 4), 0};
         int rc = (nt & 63) == 0 ? probe_nan(c, S, nt, st) : IFOS_OK;
-        if (!rc) rc = step(c, S, back, s, nt, dft, ntast, d_syn, st);
+        if (!rc) rc = step(back, nt, N.ring ? &N : nullptr, st);
+        if (!rc && samp && c->chunk > 0 && ++nsnap == c->chunk) rc = chunk();
+        if (!rc && samp && c->chunk == 0)
+            rc = ifos_discfourier(g, &step.A.f, F, C, c->finv, c->nf, nt, ntast, back, c->prec, st);
         if (rc) return rc;
     }
-    return IFOS_OK;
+    return nsnap ? chunk() : IFOS_OK;
 }
 
 static int zero_wavefield(ifos_ctx *c, hipStream_t st)
 {
-    int rc = 0;
-    for (int n = 0; n < 9 && !rc; ++n) rc = ifos_fill(c->fields[n], c->fe, 0.0f, st);
-    for (int n = 0; n < 9 && !rc; ++n) rc = ifos_fill(c->psi_s[n], ifos_psi_elems(&c->g, n), 0.0f, st);
-    for (int n = 0; n < 9 && !rc; ++n) rc = ifos_fill(c->psi_v[n], ifos_psi_elems(&c->g, n), 0.0f, st);
+    MoveList M;
+    for (int n = 0; n < 9; ++n) {
+        M.add(c->fields[n], nullptr, c->fe);
+        M.add(c->psi_s[n], nullptr, ifos_psi_elems(&c->g, n));
+        M.add(c->psi_v[n], nullptr, ifos_psi_elems(&c->g, n));
+    }
     if (c->L)  // zero_wavefield.c:80-95
-        for (int n = 0; n < 6 && !rc; ++n) rc = ifos_fill(c->r[n], c->fe * (size_t)c->L, 0.0f, st);
-    return rc;
+        for (int n = 0; n < 6; ++n) M.add(c->r[n], nullptr, c->fe * (size_t)c->L);
+    return launch_moves(M, st);
 }
 
 // checks a shot and uploads its wavelet, source and receivers
@@ -700,6 +759,29 @@ static int prepare_shot(ifos_ctx *c, const ifos_shot *s, hipStream_t st, const c
     if (!rc && s->ntr > 0)
         rc = hip_check(hipMemcpyAsync(c->chain, chain.data(), 2 * sizeof(int) * s->ntr, hipMemcpyHostToDevice, st),
                        "upload receiver chain");
+    const int cls = point_class(g, s->src_i, s->src_j, s->src_k);
+    std::vector<int> rcls((size_t)(s->ntr > 0 ? s->ntr : 1));
+    c->slab_src = cls != 0;
+    c->slab_rec = false;
+    for (int r = 0; r < s->ntr; ++r) {
+        rcls[r] = point_class(g, s->rec_ijk[3 * r], s->rec_ijk[3 * r + 1], s->rec_ijk[3 * r + 2]);
+        c->slab_rec |= rcls[r] != 0;
+    }
+    if (!rc) rc = hip_check(hipMemcpyAsync(c->srccls, &cls, sizeof cls, hipMemcpyHostToDevice, st), "upload source class");
+    if (!rc && s->ntr > 0)
+        rc = hip_check(hipMemcpyAsync(c->rcls, rcls.data(), sizeof(int) * s->ntr, hipMemcpyHostToDevice, st),
+                       "upload receiver classes");
+    std::vector<double> trig;
+    if (!rc && need_freqs && s->want_adjoint) {
+        const int ntast = ifos_ntast(c->finv[c->nf - 1], c->tast, g->dt);
+        trig.resize(4 * (size_t)(g->nt / ntast) * c->nf + 1);
+        c->nsamp = dft_trig(g, c->finv, c->nf, ntast, trig.data());
+        if (c->nsamp > 0) rc = ring_alloc(c);
+        if (!rc && c->nsamp > 0)
+            rc = hip_check(hipMemcpyAsync(c->trig, trig.data(), 4 * sizeof(double) * (size_t)c->nsamp * c->nf,
+                                          hipMemcpyHostToDevice, st),
+                           "upload trig");
+    }
     if (!rc) rc = hip_check(hipStreamSynchronize(st), "sync uploads");
     return rc;
 }
@@ -715,7 +797,10 @@ extern "C" int ifos_ctx_run_shot(ifos_ctx *c, const ifos_shot *s, float *d_syn, 
     const int ntast = s->want_adjoint ? ifos_ntast(c->finv[c->nf - 1], c->tast, g->dt) : 1;
     // ifos3d.c:738-739: zero wavefield and DFT accumulators
     rc = zero_wavefield(c, st);
-    for (int n = 0; n < 12 && !rc; ++n) {
+    // (the first chunk of a pass writes the frequencies in use without reading
+    // them)
+    const bool chunked = s->want_adjoint && c->chunk > 0 && c->nsamp > 0 && c->nf == c->nf_max;
+    for (int n = 0; n < 12 && !rc && !chunked; ++n) {
         rc = ifos_fill(c->F[n], c->fe * c->nf_max, 0.0f, st);
         if (!rc && c->C[n]) rc = ifos_fill(c->C[n], c->fe * c->nf_max, 0.0f, st);
     }
@@ -756,7 +841,7 @@ struct TdBufs {
     int K = 0, nck = 0, L = 0;  // L: memory-variable mechanisms of the states
     std::vector<ShotState> ck;  // state after steps 0, K, 2K, ...
     ShotState work;             // the recomputed forward state
-    std::vector<float *> seg;   // [K][3] forward velocities of one segment
+    float *seg;                 // [K][3][fe] forward velocities of one segment
     float *uf[3], *ub[3];       // running displacements, forward and adjoint
     double *acc[3];             // lambda, mu, rho sums
     std::vector<void *> allocs;
@@ -807,8 +892,9 @@ static int td_alloc(ifos_ctx *c, int K)
     int rc = IFOS_OK;
     for (int q = 0; q < nck && !rc; ++q) rc = td_alloc_state(c, T, T->ck[q]);
     if (!rc) rc = td_alloc_state(c, T, T->work);
-    T->seg.assign(3 * (size_t)K, nullptr);
-    for (size_t q = 0; q < T->seg.size() && !rc; ++q) rc = td_alloc_one(T, (void **)&T->seg[q], c->fe * 4);
+    // (the marches write the snapshots' cells of [1..N]^3 only: halos stay 0)
+    if (!rc) rc = td_alloc_one(T, (void **)&T->seg, 3 * (size_t)K * c->fe * 4);
+    if (!rc) rc = hip_check(hipMemset(T->seg, 0, 3 * (size_t)K * c->fe * 4), "hipMemset");
     for (int n = 0; n < 3 && !rc; ++n) rc = td_alloc_one(T, (void **)&T->uf[n], c->fe * 4);
     for (int n = 0; n < 3 && !rc; ++n) rc = td_alloc_one(T, (void **)&T->ub[n], c->fe * 4);
     for (int n = 0; n < 3 && !rc; ++n) rc = td_alloc_one(T, (void **)&T->acc[n], c->fe * 8);
@@ -818,22 +904,15 @@ static int td_alloc(ifos_ctx *c, int K)
 
 static int copy_state(ifos_ctx *c, const ShotState &dst, const ShotState &src, hipStream_t st)
 {
-    int rc = IFOS_OK;
-    for (int n = 0; n < 9 && !rc; ++n)
-        rc = hip_check(hipMemcpyAsync(dst.fields[n], src.fields[n], c->fe * 4, hipMemcpyDeviceToDevice, st),
-                       "checkpoint copy");
-    for (int n = 0; n < 9 && !rc; ++n) {
-        const size_t b = ifos_psi_elems(&c->g, n) * 4;
-        rc = hip_check(hipMemcpyAsync(dst.psi_s[n], src.psi_s[n], b, hipMemcpyDeviceToDevice, st), "checkpoint copy");
-        if (!rc)
-            rc = hip_check(hipMemcpyAsync(dst.psi_v[n], src.psi_v[n], b, hipMemcpyDeviceToDevice, st),
-                           "checkpoint copy");
+    MoveList M;
+    for (int n = 0; n < 9; ++n) {
+        M.add(dst.fields[n], src.fields[n], c->fe);
+        M.add(dst.psi_s[n], src.psi_s[n], ifos_psi_elems(&c->g, n));
+        M.add(dst.psi_v[n], src.psi_v[n], ifos_psi_elems(&c->g, n));
     }
     if (c->L)
-        for (int n = 0; n < 6 && !rc; ++n)
-            rc = hip_check(hipMemcpyAsync(dst.r[n], src.r[n], c->fe * 4 * (size_t)c->L, hipMemcpyDeviceToDevice, st),
-                           "checkpoint copy");
-    return rc;
+        for (int n = 0; n < 6; ++n) M.add(dst.r[n], src.r[n], c->fe * (size_t)c->L);
+    return launch_moves(M, st);
 }
 
 extern "C" size_t ifos_td_bytes(const ifos_geom *g, int every, int L)
@@ -866,13 +945,14 @@ extern "C" int ifos_ctx_run_shot_td(ifos_ctx *c, const ifos_shot *s, int every, 
     if (rc) return rc;
     TdBufs *T = c->td;
     const ShotState S = ctx_state(c);
+    const CtxStep fwd(c, S, s, d_syn), again(c, T->work, s, nullptr), back(c, S, s, nullptr);
     // forward (ifos3d.c:754-814) with the state stored after steps 0, K, 2K, ...
     rc = zero_wavefield(c, st);
     if (!rc) rc = ifos_fill(d_syn, 3 * (size_t)s->ntr * (N + 1), 0.0f, st);
     if (!rc) rc = copy_state(c, T->ck[0], S, st);
     for (int nt = 1; nt <= N && !rc; ++nt) {
         if ((nt & 63) == 0) rc = probe_nan(c, S, nt, st);
-        if (!rc) rc = step(c, S, 0, s, nt, false, 1, d_syn, st);
+        if (!rc) rc = fwd(0, nt, nullptr, st);
         if (!rc && nt % K == 0 && nt / K < T->nck) rc = copy_state(c, T->ck[nt / K], S, st);
     }
     // residual -> adjoint sources (ifos3d.c:837-866)
@@ -891,20 +971,26 @@ extern "C" int ifos_ctx_run_shot_td(ifos_ctx *c, const ifos_shot *s, int every, 
         // recompute the segment's forward velocities from its checkpoint
         rc = copy_state(c, T->work, T->ck[q], st);
         for (int n = a + 1; n <= b && !rc; ++n) {
-            rc = step(c, T->work, 0, s, n, false, 1, nullptr, st);
-            for (int d = 0; d < 3 && !rc; ++d)
-                rc = hip_check(hipMemcpyAsync(T->seg[3 * (n - a - 1) + d], T->work.fields[d], c->fe * 4,
+            // v(n) goes into the segment as the march's snapshot, or by copies
+            // where three fields exceed the 4 GiB of a buffer descriptor
+            float *v = T->seg + 3 * (size_t)(n - a - 1) * c->fe;
+            const bool snap = 3 * c->fe * 4 < 4294967295u;
+            const Snap N = {v, 0, (uint32_t)(snap ? 3 * c->fe * 4 : 0), 0};
+            rc = again(0, n, snap ? &N : nullptr, st);
+            for (int d = 0; d < 3 && !rc && !snap; ++d)
+                rc = hip_check(hipMemcpyAsync(v + (size_t)d * c->fe, T->work.fields[d], c->fe * 4,
                                               hipMemcpyDeviceToDevice, st),
                                "segment copy");
         }
         // the segment backwards, the adjoint forwards (ifos3d.c:905-960)
         for (int n = b; n > a && !rc; --n) {
-            const float *vf[3] = {T->seg[3 * (n - a - 1)], T->seg[3 * (n - a - 1) + 1], T->seg[3 * (n - a - 1) + 2]};
+            const float *v0 = T->seg + 3 * (size_t)(n - a - 1) * c->fe;
+            const float *vf[3] = {v0, v0 + c->fe, v0 + 2 * c->fe};
             rc = launch_td_integrate(g, T->uf, vf, dt, st);
             if (rc || n > N - 2) continue;
             const int m = N - 1 - n;
             if ((m & 63) == 0) rc = probe_nan(c, S, m, st);
-            if (!rc) rc = step(c, S, 1, s, m, false, 1, nullptr, st);
+            if (!rc) rc = back(1, m, nullptr, st);
             if (!rc) rc = launch_td_integrate(g, T->ub, vb, dt, st);
             if (!rc) rc = launch_td_sample(g, T->uf, vf, T->ub, vb, (double)dt, T->acc, st);
         }
@@ -1034,13 +1120,14 @@ extern "C" int ifos_ctx_run_shot_adj(ifos_ctx *c, const ifos_shot *s, int every,
     if (rc) return rc;
     AdjBufs *A = c->cadj;
     const ShotState S = ctx_state(c);
+    const CtxStep fwd(c, S, s, d_syn), again(c, A->work, s, nullptr);
     // forward (ifos3d.c:754-814) with the state stored after steps 0, K, 2K, ...
     rc = zero_wavefield(c, st);
     if (!rc) rc = ifos_fill(d_syn, 3 * (size_t)s->ntr * (N + 1), 0.0f, st);
     if (!rc) rc = copy_state(c, A->ck[0], S, st);
     for (int nt = 1; nt <= N && !rc; ++nt) {
         if ((nt & 63) == 0) rc = probe_nan(c, S, nt, st);
-        if (!rc) rc = step(c, S, 0, s, nt, false, 1, d_syn, st);
+        if (!rc) rc = fwd(0, nt, nullptr, st);
         if (!rc && nt % K == 0 && nt / K < A->nck) rc = copy_state(c, A->ck[nt / K], S, st);
     }
     if (!rc) rc = probe_nan(c, S, N, st);
@@ -1057,21 +1144,16 @@ extern "C" int ifos_ctx_run_shot_adj(ifos_ctx *c, const ifos_shot *s, int every,
         rc = copy_state(c, A->work, A->ck[q], st);
         for (int n = a + 1; n <= b && !rc; ++n) {
             const size_t e = (size_t)(n - a - 1);
-            for (int m = 0; m < 6 && !rc; ++m)
-                rc = hip_check(hipMemcpyAsync(A->rs[6 * e + m], A->work.fields[3 + m], c->fe * 4,
-                                              hipMemcpyDeviceToDevice, st), "ring copy");
-            if (!rc) rc = step(c, A->work, 0, s, n, false, 1, nullptr, st);
-            for (int m = 0; m < 3 && !rc; ++m)
-                rc = hip_check(hipMemcpyAsync(A->rv[3 * e + m], A->work.fields[m], c->fe * 4, hipMemcpyDeviceToDevice,
-                                              st), "ring copy");
-            for (int m = 0; m < 9 && !rc; ++m) {
-                const size_t pb = ifos_psi_elems(g, m) * 4;
-                rc = hip_check(hipMemcpyAsync(A->rps[9 * e + m], A->work.psi_s[m], pb, hipMemcpyDeviceToDevice, st),
-                               "ring copy");
-                if (!rc)
-                    rc = hip_check(hipMemcpyAsync(A->rpv[9 * e + m], A->work.psi_v[m], pb, hipMemcpyDeviceToDevice,
-                                                  st), "ring copy");
+            MoveList before, after;
+            for (int m = 0; m < 6; ++m) before.add(A->rs[6 * e + m], A->work.fields[3 + m], c->fe);
+            for (int m = 0; m < 3; ++m) after.add(A->rv[3 * e + m], A->work.fields[m], c->fe);
+            for (int m = 0; m < 9; ++m) {
+                after.add(A->rps[9 * e + m], A->work.psi_s[m], ifos_psi_elems(g, m));
+                after.add(A->rpv[9 * e + m], A->work.psi_v[m], ifos_psi_elems(g, m));
             }
+            rc = launch_moves(before, st);
+            if (!rc) rc = again(0, n, nullptr, st);
+            if (!rc) rc = launch_moves(after, st);
         }
         for (int n = b; n > a && !rc; --n) {
             const size_t e = (size_t)(n - a - 1);

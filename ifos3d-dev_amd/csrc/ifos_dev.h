@@ -192,17 +192,76 @@ __device__ inline void bstore_cp(float v, rsrc_t r, uint32_t voff, uint32_t soff
 
 DevGeom make_dev_geom(const ifos_geom *g);
 
-// multi-shot fused (interior + CPML) updates over [1..N]^3 for the batched
-// path (stencil.hip): f and psi point at shot 0; snap may be null
+// multi-shot fused (interior + CPML) updates over [1..N]^3 (stencil.hip): f
+// and psi point at shot 0; snap may be null
 int launch_v_shots(const ifos_geom *g, const ifos_fields *f, const ifos_model *m, const float *d_prof,
                    const ifos_psi *psi, const Shots &S, const Snap *snap, const MarchCfg &c, hipStream_t s);
 int launch_s_shots(const ifos_geom *g, const ifos_fields *f, const ifos_model *m, const float *d_prof,
                    const ifos_psi *psi, const Shots &S, const MarchCfg &c, hipStream_t s,
                    const ViscoF *V = nullptr);
+// the tile shape of the one-shot march launches (ifos_set_plain_tiles)
+const MarchCfg &plain_cfg();
+
+// one time step of ns shots of one model (batch.hip): what the shots of a
+// launch share, and which point operations any of them needs
+struct StepArgs {
+    const ifos_geom *g;
+    int ns;
+    ifos_fields f;              // shot 0; shot s at + s * S.fstride
+    ifos_psi ps, pv;            // stress- and velocity-derivative memory
+    ifos_model m;
+    const float *prof;
+    Shots S;
+    const ViscoF *V;            // null: elastic
+    const int *src, *srccls;    // [ns][4] i j k type; point_class of each
+    const float *sig;           // [ns][nt + 2]
+    bool force_slab, force_in;  // a body force in a CPML slab, in the interior
+    bool explosive;             // an explosive source
+    const int *rec, *chain, *rcls;  // [ns][ntr][3], [ns][ntr][2], [ns][ntr]
+    const float *adj;           // [ns][3][ntr][nt + 2]
+    float *syn;                 // [ns][3][ntr][nt + 1]
+    int ntr;
+    bool slab_rec;              // a receiver in a CPML slab
+    MarchCfg cfg_v, cfg_s;
+};
+// class of a point: 1 = in a CPML slab, 0 = in the interior box
+int point_class(const ifos_geom *g, int i, int j, int k);
+// step nt of a propagation (ifos3d.c:754-814, back = 0; :905-960, back = 1);
+// N: the snapshot slot that receives the step's velocities, or null; seis:
+// write the seismograms
+int launch_step(const StepArgs &A, int back, int nt, const Snap *N, bool seis, hipStream_t st);
+// accumulates nsnap (<= chunk <= 32) velocity snapshots of ns shots into their
+// DFT fields: shot s's snapshot c at ring + (s * chunk + c) * 3 fields, its
+// accumulators at F[n] + s * fshot (C: their Kahan compensations, or null),
+// frequency l + field l; trig[(c * nf + l) * 2 + {0, 1}] the factors of
+// disc_fourier.c:42-44.  first: the accumulators start at 0 and are not read.
+int launch_dft_chunk(const ifos_geom *g, int ns, const float *ring, int chunk, int nsnap, float *const F[6],
+                     float *const C[6], int64_t fshot, const double *trig, int nf, bool first, hipStream_t st);
+// the factors of every sampling step of both directions (disc_fourier.c:36-44):
+// out[back][sample][frequency][cos, sin], samples of one direction
+int dft_trig(const ifos_geom *g, const float *finv, int nf, int ntast, double *out);
 // gradient_F of ns shots in shot order into d_grad (aux.hip); shot s's DFT
 // fields at d_F*[n] + s*fshot
 int launch_gradient_shots(const ifos_geom *g, float *const d_Ff[6], float *const d_Fb[6], int64_t fshot, int ns,
                           const ifos_model *m, const float *finv, int nf, float *const d_grad[3], hipStream_t st);
+// copies (src set) and fills with 0 (src null) of up to 40 arrays in one
+// launch (aux.hip): the state of a shot is 27 arrays and more, and a launch of
+// its own for each costs 3-5 us on the small ones
+struct MoveList {
+    static constexpr int kMax = 40;
+    int n = 0;
+    const float *src[kMax];
+    float *dst[kMax];
+    int64_t len[kMax];    // floats
+    int start[kMax + 1];  // first workgroup of each array
+    void add(float *d, const float *s, size_t elems)
+    {
+        dst[n] = d;
+        src[n] = s;
+        len[n++] = (int64_t)elems;
+    }
+};
+int launch_moves(MoveList &L, hipStream_t st);
 // arguments of the fused stress(n) + velocity(n+1) step (stencil.hip)
 struct FusedArgs {
     const float *vx, *vy, *vz, *sxx, *syy, *szz, *sxy, *syz, *sxz;  // v^n, sigma^(n-1)

@@ -2191,6 +2191,10 @@ int launch_vs_fused(const ifos_geom *g, const FusedArgs &A, const float *d_prof,
 }
 }  // namespace ifos
 
+namespace ifos {
+const MarchCfg &plain_cfg() { return g_default_cfg; }
+}  // namespace ifos
+
 extern "C" int ifos_set_plain_tiles(const int cfg[IFOS_TILE_FIELDS])
 {
     if (!cfg) return IFOS_EINVAL;
