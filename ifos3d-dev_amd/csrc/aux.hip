@@ -297,13 +297,6 @@ __global__ __launch_bounds__(256) void k_copy(v4f *__restrict__ dst, const v4f *
 }
 
 // ---------------------------------------------------------------------------
-// gradient_F.c:70-72: 1 / (4 pi^2 f^2) of each frequency, the double
-// product rounded to float before the reciprocal
-struct GradFreq {
-    float fdummy[IFOS_MAX_NF];
-};
-
-// ---------------------------------------------------------------------------
 // matcopy.c:31-307 (single rank): three passes, y faces then x then z
 __global__ void k_wrap_y(DevGeom g, float *m)
 {
@@ -588,27 +581,7 @@ extern "C" int ifos_gradient_F(const ifos_geom *g, float *const d_Ff[6], float *
         set_error("ifos_gradient_F: nf=%d outside [1,%d]", nf, IFOS_MAX_NF);
         return IFOS_EINVAL;
     }
-    DevGeom G = make_dev_geom(g);
-    GradFreq GF;
-    for (int l = 0; l < nf; ++l) {
-        // gradient_F.c:70-72: double product stored to float, then 1/x in float
-        float fd = (float)(2.0 * 2.0 * finv[l] * finv[l] * M_PI * M_PI);
-        GF.fdummy[l] = 1 / fd;
-    }
-    (void)G;
-    // one march launch per frequency, in order (gradient_F.c:66-139)
-    const size_t fe = ifos_field_elems(g);
-    ProfScope ps_(IFOS_K_GRADIENT, (hipStream_t)stream);
-    for (int l = 0; l < nf; ++l) {
-        const float *f[12];
-        for (int n = 0; n < 6; ++n) {
-            f[n] = d_Ff[n] + (size_t)l * fe;
-            f[6 + n] = d_Fb[n] + (size_t)l * fe;
-        }
-        int rc = launch_grad_march(g, f, GF.fdummy[l], m, d_grad, (hipStream_t)stream);
-        if (rc) return rc;
-    }
-    return IFOS_OK;
+    return launch_gradient_shots(g, d_Ff, d_Fb, 0, 1, m, finv, nf, d_grad, (hipStream_t)stream);
 }
 
 extern "C" int ifos_hess_F(const ifos_geom *g, float *const d_Ff[6], float *const d_Fb[6], int ntr_hess,
@@ -618,50 +591,30 @@ extern "C" int ifos_hess_F(const ifos_geom *g, float *const d_Ff[6], float *cons
         set_error("ifos_hess_F: nf=%d outside [1,%d] or ntr_hess=%d < 0", nf, IFOS_MAX_NF, ntr_hess);
         return IFOS_EINVAL;
     }
-    const size_t fe = ifos_field_elems(g);
-    ProfScope ps_(IFOS_K_GRADIENT, (hipStream_t)stream);
-    // hess_F.c:72-77: receivers outer, frequencies inner, one march per pair
-    for (int n = 1; n <= ntr_hess; ++n)
-        for (int l = 1; l <= nf; ++l) {
-            const float fdummy = (float)(finv[l - 1] * M_PI * 2);
-            const float fd = 1 / fdummy;
-            const size_t mb = (size_t)(n * nf + l - 1);
-            const float *f[12];
-            for (int c = 0; c < 6; ++c) {
-                f[c] = d_Ff[c] + (size_t)(l - 1) * fe;
-                f[6 + c] = d_Fb[c] + mb * fe;
-            }
-            int rc = launch_grad_march(g, f, fd, m, d_hess, (hipStream_t)stream, true);
-            if (rc) return rc;
-        }
-    return IFOS_OK;
+    float fd[IFOS_MAX_NF];
+    for (int l = 0; l < nf; ++l) {  // hess_F.c:75-77
+        const float fdummy = (float)(finv[l] * M_PI * 2);
+        fd[l] = 1 / fdummy;
+    }
+    // hess_F.c:72-77: receivers n = 1.. outer, their fields of frequency l at
+    // n * nf + l
+    const int64_t set = (int64_t)nf * (int64_t)ifos_field_elems(g);
+    float *Fb[6];
+    for (int n = 0; n < 6; ++n) Fb[n] = d_Fb[n] + set;
+    return launch_gradient(g, d_Ff, Fb, 0, set, ntr_hess, fd, nf, m, d_hess, true, (hipStream_t)stream);
 }
 
 namespace ifos {
 int launch_gradient_shots(const ifos_geom *g, float *const d_Ff[6], float *const d_Fb[6], int64_t fshot, int ns,
                           const ifos_model *m, const float *finv, int nf, float *const d_grad[3], hipStream_t st)
 {
-    DevGeom G = make_dev_geom(g);
-    GradFreq GF;
+    float fd[IFOS_MAX_NF];
     for (int l = 0; l < nf; ++l) {
-        float fd = (float)(2.0 * 2.0 * finv[l] * finv[l] * M_PI * M_PI);
-        GF.fdummy[l] = 1 / fd;
+        // gradient_F.c:70-72: double product stored to float, then 1/x in float
+        const float f = (float)(2.0 * 2.0 * finv[l] * finv[l] * M_PI * M_PI);
+        fd[l] = 1 / f;
     }
-    (void)G;
-    // shots in order, frequencies in order: one march launch each
-    const size_t fe = ifos_field_elems(g);
-    ProfScope ps_(IFOS_K_GRADIENT, st);
-    for (int s = 0; s < ns; ++s)
-        for (int l = 0; l < nf; ++l) {
-            const float *f[12];
-            for (int n = 0; n < 6; ++n) {
-                f[n] = d_Ff[n] + (size_t)s * fshot + (size_t)l * fe;
-                f[6 + n] = d_Fb[n] + (size_t)s * fshot + (size_t)l * fe;
-            }
-            int rc = launch_grad_march(g, f, GF.fdummy[l], m, d_grad, st);
-            if (rc) return rc;
-        }
-    return IFOS_OK;
+    return launch_gradient(g, d_Ff, d_Fb, fshot, fshot, ns, fd, nf, m, d_grad, false, st);
 }
 }  // namespace ifos
 

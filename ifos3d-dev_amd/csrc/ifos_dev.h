@@ -280,10 +280,12 @@ struct FTiles {
 int launch_vs_fused(const ifos_geom *g, const FusedArgs &A, const float *d_prof, const Shots &S, const Snap *snap,
                     int ti, int jc, hipStream_t s);
 
-// gradient_F for one frequency of one shot, march kernel (stencil.hip); with
-// hess, hess_F for one frequency of one receiver-side set
-int launch_grad_march(const ifos_geom *g, const float *const f[12], float fd, const ifos_model *m,
-                      float *const d_grad[3], hipStream_t s, bool hess = false);
+// gradient_F (hess: hess_F) of nouter shots (receiver-side sets) x nf
+// frequencies in one launch (stencil.hip): item o's fields of frequency l at
+// d_Ff[n] + o * fouter + l fields and d_Fb[n] + o * bouter + l fields
+int launch_gradient(const ifos_geom *g, float *const d_Ff[6], float *const d_Fb[6], int64_t fouter, int64_t bouter,
+                    int nouter, const float *fd, int nf, const ifos_model *m, float *const d_grad[3], bool hess,
+                    hipStream_t s);
 // time-domain gradient (stencil.hip, aux.hip): one time sample of the
 // lambda / mu / rho sums; u += v dt; the sums to the vp, vs, rho gradients
 int launch_td_sample(const ifos_geom *g, const float *const uf[3], const float *const vf[3],

@@ -1086,153 +1086,175 @@ __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields 
 #undef LBN
 }
 // ---------------------------------------------------------------------------
-// gradient_F.c:79-139 for one frequency of one shot as a march over j: the
-// y-derivatives of the 12 DFT fields come from 4-deep register queues and the
-// three gradients are read, updated and written once per call.  Calls in
-// frequency order (and shot order) repeat the reference's per-cell
-// accumulation order exactly.  f[0..2] forward Re x y z, f[3..5] forward Im,
-// f[6..8] adjoint Re, f[9..11] adjoint Im.
+// gradient_F.c:79-139 and hess_F.c:28-192: one thread per cell, every shot
+// (or receiver-side set) and frequency in one launch, the three sums of the
+// cell in registers.  The terms are added in the reference's order (shots or
+// receivers outer, frequencies inner), so each cell sees the same sequence of
+// roundings as one pass per frequency, without reading and writing the sums
+// and the model (9 of 21 array passes) and forming two FP64 square roots for
+// each of them.  A workgroup covers 64 k x 4 i x 4 j cells, so that the i and
+// j neighbours, 20 of a field's 30 loads, are mostly its own rows and come
+// from L1, and its 16 wavefronts keep some 1900 loads in flight; workgroups
+// are numbered so that an XCD's stretch is contiguous.  The vector-memory
+// path bounds it (120 loads per cell and frequency).
 struct GradArgs {
-    const float *f[12];
-    float fd;  // 1 / (4 pi^2 f^2) as gradient_F.c:70-72 rounds it
+    const float *f[12];  // forward Re x y z, Im x y z, adjoint (receiver side) Re, Im
+    int64_t fouter, bouter;  // elements from one outer item's forward / adjoint fields to the next
+    int64_t fe;              // elements of one field: the next frequency
+    int nouter, nf;
+    float fd[IFOS_MAX_NF];   // 1 / (4 pi^2 f^2) (gradient_F.c:70-72); hess: 1 / (2 pi f) (hess_F.c:75-77)
     const float *rho, *pi, *u;
     float *g1, *g2, *g3;
-    double *acc[3];  // GRAD_TD: lambda, mu and rho sums, one double per cell of the device layout
-    double w;        // GRAD_TD: weight of the time sample (the time step)
+    uint32_t ntk, nti, total, per;
 };
 
-// MODE GRAD_HESS: hess_F.c:28-192 instead, the same fields read as the
-// forward set (f, fi) and one receiver-side set (b, bi), fd = 1 / (2 pi f) as
-// hess_F.c:75-77 rounds it, the three Hessian diagonals in place of g1..g3.
-// MODE GRAD_TD: one time sample of the time-domain gradient: f[0..2] the
-// forward displacement, f[3..5] the forward velocity, f[6..8] the adjoint
-// displacement, f[9..11] the adjoint velocity; the products of
-// gradient_F.c:122-132 (displacement derivatives for lambda and mu, the
-// velocities for rho, no frequency factor) are added, times w, to acc[0..2].
-enum { GRAD_F = 0, GRAD_HESS = 1, GRAD_TD = 2 };
+// the nine derivatives xx xy xz yx yy yz zx zy zz of three fields at a cell,
+// and the cell's values c
+struct Strain {
+    float d[9], c[3];
+};
+__device__ __forceinline__ Strain cell_strain(const DevGeom &g, rsrc_t fx, rsrc_t fy, rsrc_t fz, uint32_t vo,
+                                              uint32_t SJ, uint32_t SI)
+{
+    const float b1 = g.b1, b2 = g.b2;
+    Strain s;
+    const float x = LD(fx, 0, 0, 0), y = LD(fy, 0, 0, 0), z = LD(fz, 0, 0, 0);
+    s.d[0] = D4B(b1, b2, LD(fx, 0, -2, 0), LD(fx, 0, -1, 0), x, LD(fx, 0, 1, 0));
+    s.d[1] = D4F(b1, b2, LD(fx, -1, 0, 0), x, LD(fx, 1, 0, 0), LD(fx, 2, 0, 0));
+    s.d[2] = D4F(b1, b2, LD(fx, 0, 0, -1), x, LD(fx, 0, 0, 1), LD(fx, 0, 0, 2));
+    s.d[3] = D4F(b1, b2, LD(fy, 0, -1, 0), y, LD(fy, 0, 1, 0), LD(fy, 0, 2, 0));
+    s.d[4] = D4B(b1, b2, LD(fy, -2, 0, 0), LD(fy, -1, 0, 0), y, LD(fy, 1, 0, 0));
+    s.d[5] = D4F(b1, b2, LD(fy, 0, 0, -1), y, LD(fy, 0, 0, 1), LD(fy, 0, 0, 2));
+    s.d[6] = D4F(b1, b2, LD(fz, 0, -1, 0), z, LD(fz, 0, 1, 0), LD(fz, 0, 2, 0));
+    s.d[7] = D4F(b1, b2, LD(fz, -1, 0, 0), z, LD(fz, 1, 0, 0), LD(fz, 2, 0, 0));
+    s.d[8] = D4B(b1, b2, LD(fz, 0, 0, -2), LD(fz, 0, 0, -1), z, LD(fz, 0, 0, 1));
+    div_spacing(g, s.d[0], s.d[1], s.d[2], s.d[3], s.d[4], s.d[5], s.d[6], s.d[7], s.d[8]);
+    s.c[0] = x;
+    s.c[1] = y;
+    s.c[2] = z;
+    return s;
+}
 
-template <int TI, int MODE>
-__global__ __launch_bounds__(64 * TI) void k_grad_march(DevGeom g, MTiles T, GradArgs A)
+constexpr int kGradTI = 2, kGradTJ = 4;
+
+template <bool HESS>
+__global__ __launch_bounds__(64 * kGradTI * kGradTJ) void k_grad_cells(DevGeom g, GradArgs A)
+{
+    const uint32_t L = (blockIdx.x & 7u) * A.per + (blockIdx.x >> 3);
+    if (L >= A.total) return;
+    const int k = (int)(L % A.ntk) * 64 + (int)threadIdx.x + 1;
+    const uint32_t t = L / A.ntk;
+    const int i = (int)(t % A.nti) * kGradTI + (int)threadIdx.y + 1;
+    const int j = (int)(t / A.nti) * kGradTJ + (int)threadIdx.z + 1;
+    if (k > g.nz || i > g.nx || j > g.ny) return;
+    const uint32_t SJ = (uint32_t)g.sj * 4u, SI = (uint32_t)g.si * 4u;
+    const uint32_t vo = (uint32_t)((int64_t)j * g.sj + (int64_t)i * g.si + k + IFOS_KOFF - 2) * 4u;
+    const int64_t c = at(g, j, i, k);
+    const float r = A.rho[c], p = A.pi[c], m = A.u[c];
+    float a1 = A.g1[c], a2 = A.g2[c], a3 = A.g3[c];
+    const double srp = HESS ? 0.0 : sqrt((double)(r * p)), sru = HESS ? 0.0 : sqrt((double)(r * m));
+    for (int o = 0; o < A.nouter; ++o)
+        for (int l = 0; l < A.nf; ++l) {
+            const int64_t of = o * A.fouter + l * A.fe, ob = o * A.bouter + l * A.fe;
+            rsrc_t rf[12];
+#pragma unroll
+            for (int n = 0; n < 12; ++n) rf[n] = make_rsrc(A.f[n] + (n < 6 ? of : ob), g.fbytes);
+            const Strain F = cell_strain(g, rf[0], rf[1], rf[2], vo, SJ, SI),
+                         FI = cell_strain(g, rf[3], rf[4], rf[5], vo, SJ, SI),
+                         B = cell_strain(g, rf[6], rf[7], rf[8], vo, SJ, SI),
+                         BI = cell_strain(g, rf[9], rf[10], rf[11], vo, SJ, SI);
+            const float *f = F.d, *fi = FI.d, *bb = B.d, *bi = BI.d;
+            const float fd = A.fd[l];
+            if (HESS) {
+                // hess_F.c:135-182
+                const float fdiv = f[0] + f[4] + f[8], fidiv = fi[0] + fi[4] + fi[8];
+                const float bdiv = bb[0] + bb[4] + bb[8], bidiv = bi[0] + bi[4] + bi[8];
+                float relam = fidiv * bdiv + fdiv * bidiv;
+                relam = fd * relam;
+                float imlam = fidiv * bidiv - fdiv * bdiv;
+                imlam = fd * imlam;
+                float remu = 2.0f * fi[0] * bb[0] + 2.0f * fi[4] * bb[4] + 2.0f * fi[8] * bb[8] +
+                             2.0f * f[0] * bi[0] + 2.0f * f[4] * bi[4] + 2.0f * f[8] * bi[8] +
+                             (fi[1] + fi[3]) * (bb[1] + bb[3]) + (f[1] + f[3]) * (bi[1] + bi[3]) +
+                             (fi[2] + fi[6]) * (bb[2] + bb[6]) + (f[2] + f[6]) * (bi[2] + bi[6]) +
+                             (fi[5] + fi[7]) * (bb[5] + bb[7]) + (f[5] + f[7]) * (bi[5] + bi[7]);
+                remu = fd * remu;
+                float immu = 2.0f * fi[0] * bi[0] + 2.0f * fi[4] * bi[4] + 2.0f * fi[8] * bi[8] -
+                             2.0f * f[0] * bb[0] - 2.0f * f[4] * bb[4] - 2.0f * f[8] * bb[8] +
+                             (fi[1] + fi[3]) * (bi[1] + bi[3]) - (f[1] + f[3]) * (bb[1] + bb[3]) +
+                             (fi[2] + fi[6]) * (bi[2] + bi[6]) - (f[2] + f[6]) * (bb[2] + bb[6]) +
+                             (fi[5] + fi[7]) * (bi[5] + bi[7]) - (f[5] + f[7]) * (bb[5] + bb[7]);
+                immu = fd * immu;
+                const float rerho = (F.c[0] * B.c[0] + F.c[1] * B.c[1] + F.c[2] * B.c[2]) -
+                                    (FI.c[0] * BI.c[0] + FI.c[1] * BI.c[1] + FI.c[2] * BI.c[2]);
+                const float imrho = (F.c[0] * BI.c[0] + F.c[1] * BI.c[1] + F.c[2] * BI.c[2]) +
+                                    (FI.c[0] * B.c[0] + FI.c[1] * B.c[1] + FI.c[2] * B.c[2]);
+                const float revs = -2.0f * relam + remu, imvs = -2.0f * imlam + immu;
+                const float rerho1 = rerho + relam * (p - 2.0f * m) / r + remu * m / r;
+                const float imrho1 = imrho + imlam * (p - 2.0f * m) / r + immu * m / r;
+                a1 += (relam * relam + imlam * imlam) * r * p * 4.0f;
+                a2 += (revs * revs + imvs * imvs) * 4.0f * r * m;
+                a3 += rerho1 * rerho1 + imrho1 * imrho1;
+            } else {
+                // gradient_F.c:122-139
+                float gl = (f[0] + f[4] + f[8]) * (bb[0] + bb[4] + bb[8]) +
+                           (fi[0] + fi[4] + fi[8]) * (bi[0] + bi[4] + bi[8]);
+                gl = -gl * fd;
+                float gm = 2.0f * f[0] * bb[0] + 2.0f * f[4] * bb[4] + 2.0f * f[8] * bb[8] + 2.0f * fi[0] * bi[0] +
+                           2.0f * fi[4] * bi[4] + 2.0f * fi[8] * bi[8] + (f[1] + f[3]) * (bb[1] + bb[3]) +
+                           (fi[1] + fi[3]) * (bi[1] + bi[3]) + (f[2] + f[6]) * (bb[2] + bb[6]) +
+                           (fi[2] + fi[6]) * (bi[2] + bi[6]) + (f[5] + f[7]) * (bb[5] + bb[7]) +
+                           (fi[5] + fi[7]) * (bi[5] + bi[7]);
+                gm = -gm * fd;
+                const float gr = (F.c[0] * B.c[0] + F.c[1] * B.c[1] + F.c[2] * B.c[2]) +
+                                 (FI.c[0] * BI.c[0] + FI.c[1] * BI.c[1] + FI.c[2] * BI.c[2]);
+                a1 = (float)(a1 + srp * 2 * gl);
+                a2 = (float)(a2 + (-4 * sru * gl + 2 * sru * gm));
+                a3 += gr + m / r * gm + (p - 2.0f * m) / r * gl;
+            }
+        }
+    A.g1[c] = a1;
+    A.g2[c] = a2;
+    A.g3[c] = a3;
+}
+
+// one time sample of the time-domain gradient as a march over j: the
+// products of gradient_F.c:122-132 (displacement derivatives for lambda and
+// mu, the velocities for rho, no frequency factor), times w, added to acc.
+// f[0..2] the forward displacement, f[3..5] the forward velocity, f[6..8]
+// the adjoint displacement, f[9..11] the adjoint velocity.
+struct TdArgs {
+    const float *f[12];
+    double *acc[3];  // lambda, mu and rho sums, one double per cell of the device layout
+    double w;        // weight of the time sample (the time step)
+};
+
+template <int TI>
+__global__ __launch_bounds__(64 * TI) void k_td_march(DevGeom g, MTiles T, TdArgs A)
 {
     int k, i, jb, je, shot;
     Box R;
     if (!decode_tile(T, TI, k, i, jb, je, shot, R)) return;
     const uint32_t SJ = (uint32_t)g.sj * 4u, SI = (uint32_t)g.si * 4u;
-    const float b1 = g.b1, b2 = g.b2;
+    uint32_t vo = (uint32_t)((int64_t)jb * g.sj + (int64_t)i * g.si + k + IFOS_KOFF - 2) * 4u;
     rsrc_t rf[12];
 #pragma unroll
     for (int n = 0; n < 12; ++n) rf[n] = make_rsrc(A.f[n], g.fbytes);
-    const rsrc_t rrho = make_rsrc(A.rho, g.fbytes), rpi = make_rsrc(A.pi, g.fbytes), ru = make_rsrc(A.u, g.fbytes),
-                 rg1 = make_rsrc(A.g1, g.fbytes), rg2 = make_rsrc(A.g2, g.fbytes), rg3 = make_rsrc(A.g3, g.fbytes);
-    uint32_t vo = (uint32_t)((int64_t)jb * g.sj + (int64_t)i * g.si + k + IFOS_KOFF - 2) * 4u;
-    // queues per triple t: x component at j-1..j+2, y at j-2..j+1, z at j-1..j+2
-    float qx[4][4], qy[4][4], qz[4][4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        qx[t][0] = LD(rf[3 * t], -1, 0, 0); qx[t][1] = LD(rf[3 * t], 0, 0, 0); qx[t][2] = LD(rf[3 * t], 1, 0, 0);
-        qy[t][0] = LD(rf[3 * t + 1], -2, 0, 0); qy[t][1] = LD(rf[3 * t + 1], -1, 0, 0);
-        qy[t][2] = LD(rf[3 * t + 1], 0, 0, 0);
-        qz[t][0] = LD(rf[3 * t + 2], -1, 0, 0); qz[t][1] = LD(rf[3 * t + 2], 0, 0, 0);
-        qz[t][2] = LD(rf[3 * t + 2], 1, 0, 0);
-    }
     for (int j = jb; j <= je; ++j, vo += SJ) {
-        float d[4][9];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const rsrc_t fx = rf[3 * t], fy = rf[3 * t + 1], fz = rf[3 * t + 2];
-            qx[t][3] = LD(fx, 2, 0, 0);
-            qy[t][3] = LD(fy, 1, 0, 0);
-            qz[t][3] = LD(fz, 2, 0, 0);
-            if (MODE == GRAD_TD && (t & 1)) continue;  // velocities: cell values only
-            const float x_c = qx[t][1], y_c = qy[t][2], z_c = qz[t][1];
-            d[t][0] = b1 * (x_c - LD(fx, 0, -1, 0)) + b2 * (LD(fx, 0, 1, 0) - LD(fx, 0, -2, 0));
-            d[t][1] = b1 * (qx[t][2] - x_c) + b2 * (qx[t][3] - qx[t][0]);
-            d[t][2] = b1 * (LD(fx, 0, 0, 1) - x_c) + b2 * (LD(fx, 0, 0, 2) - LD(fx, 0, 0, -1));
-            d[t][3] = b1 * (LD(fy, 0, 1, 0) - y_c) + b2 * (LD(fy, 0, 2, 0) - LD(fy, 0, -1, 0));
-            d[t][4] = b1 * (y_c - qy[t][1]) + b2 * (qy[t][3] - qy[t][0]);
-            d[t][5] = b1 * (LD(fy, 0, 0, 1) - y_c) + b2 * (LD(fy, 0, 0, 2) - LD(fy, 0, 0, -1));
-            d[t][6] = b1 * (LD(fz, 0, 1, 0) - z_c) + b2 * (LD(fz, 0, 2, 0) - LD(fz, 0, -1, 0));
-            d[t][7] = b1 * (qz[t][2] - z_c) + b2 * (qz[t][3] - qz[t][0]);
-            d[t][8] = b1 * (z_c - LD(fz, 0, 0, -1)) + b2 * (LD(fz, 0, 0, 1) - LD(fz, 0, 0, -2));
-            div_spacing(g, d[t][0], d[t][1], d[t][2], d[t][3], d[t][4], d[t][5], d[t][6], d[t][7], d[t][8]);
-        }
-        // d[t] = xx xy xz yx yy yz zx zy zz of f (t 0), fi (1), b (2), bi (3)
-        const float *f = d[0], *fi = d[1], *bb = d[2], *bi = d[3];
-        if (MODE == GRAD_TD) {
-            float gl = (f[0] + f[4] + f[8]) * (bb[0] + bb[4] + bb[8]);
-            gl = -gl;
-            float gm = 2.0f * f[0] * bb[0] + 2.0f * f[4] * bb[4] + 2.0f * f[8] * bb[8] + (f[1] + f[3]) * (bb[1] + bb[3]) +
-                       (f[2] + f[6]) * (bb[2] + bb[6]) + (f[5] + f[7]) * (bb[5] + bb[7]);
-            gm = -gm;
-            const float gr = qx[1][1] * qx[3][1] + qy[1][2] * qy[3][2] + qz[1][1] * qz[3][1];
-            const int64_t c = at(g, j, i, k);
-            A.acc[0][c] += (double)gl * A.w;
-            A.acc[1][c] += (double)gm * A.w;
-            A.acc[2][c] += (double)gr * A.w;
-        } else if (MODE == GRAD_HESS) {
-            // hess_F.c:135-182, values of the cell: qx[t][1], qy[t][2], qz[t][1]
-            const float fdiv = f[0] + f[4] + f[8], fidiv = fi[0] + fi[4] + fi[8];
-            const float bdiv = bb[0] + bb[4] + bb[8], bidiv = bi[0] + bi[4] + bi[8];
-            float relam = fidiv * bdiv + fdiv * bidiv;
-            relam = A.fd * relam;
-            float imlam = fidiv * bidiv - fdiv * bdiv;
-            imlam = A.fd * imlam;
-            float remu = 2.0f * fi[0] * bb[0] + 2.0f * fi[4] * bb[4] + 2.0f * fi[8] * bb[8] + 2.0f * f[0] * bi[0] +
-                         2.0f * f[4] * bi[4] + 2.0f * f[8] * bi[8] + (fi[1] + fi[3]) * (bb[1] + bb[3]) +
-                         (f[1] + f[3]) * (bi[1] + bi[3]) + (fi[2] + fi[6]) * (bb[2] + bb[6]) +
-                         (f[2] + f[6]) * (bi[2] + bi[6]) + (fi[5] + fi[7]) * (bb[5] + bb[7]) +
-                         (f[5] + f[7]) * (bi[5] + bi[7]);
-            remu = A.fd * remu;
-            float immu = 2.0f * fi[0] * bi[0] + 2.0f * fi[4] * bi[4] + 2.0f * fi[8] * bi[8] - 2.0f * f[0] * bb[0] -
-                         2.0f * f[4] * bb[4] - 2.0f * f[8] * bb[8] + (fi[1] + fi[3]) * (bi[1] + bi[3]) -
-                         (f[1] + f[3]) * (bb[1] + bb[3]) + (fi[2] + fi[6]) * (bi[2] + bi[6]) -
-                         (f[2] + f[6]) * (bb[2] + bb[6]) + (fi[5] + fi[7]) * (bi[5] + bi[7]) -
-                         (f[5] + f[7]) * (bb[5] + bb[7]);
-            immu = A.fd * immu;
-            const float fx = qx[0][1], fy = qy[0][2], fz = qz[0][1], fix = qx[1][1], fiy = qy[1][2], fiz = qz[1][1];
-            const float bx = qx[2][1], by = qy[2][2], bz = qz[2][1], bix = qx[3][1], biy = qy[3][2], biz = qz[3][1];
-            const float rerho = (fx * bx + fy * by + fz * bz) - (fix * bix + fiy * biy + fiz * biz);
-            const float imrho = (fx * bix + fy * biy + fz * biz) + (fix * bx + fiy * by + fiz * bz);
-            const float revs = -2.0f * relam + remu, imvs = -2.0f * imlam + immu;
-            const float r = LD(rrho, 0, 0, 0), p = LD(rpi, 0, 0, 0), m = LD(ru, 0, 0, 0);
-            const float rerho1 = rerho + relam * (p - 2.0f * m) / r + remu * m / r;
-            const float imrho1 = imrho + imlam * (p - 2.0f * m) / r + immu * m / r;
-            float h1 = LD(rg1, 0, 0, 0), h2 = LD(rg2, 0, 0, 0), h3 = LD(rg3, 0, 0, 0);
-            h1 += (relam * relam + imlam * imlam) * r * p * 4.0f;
-            h2 += (revs * revs + imvs * imvs) * 4.0f * r * m;
-            h3 += rerho1 * rerho1 + imrho1 * imrho1;
-            ST(h1, rg1);
-            ST(h2, rg2);
-            ST(h3, rg3);
-        } else {
-        float gl = (f[0] + f[4] + f[8]) * (bb[0] + bb[4] + bb[8]) + (fi[0] + fi[4] + fi[8]) * (bi[0] + bi[4] + bi[8]);
-        gl = -gl * A.fd;
-        float gm = 2.0f * f[0] * bb[0] + 2.0f * f[4] * bb[4] + 2.0f * f[8] * bb[8] + 2.0f * fi[0] * bi[0] +
-                   2.0f * fi[4] * bi[4] + 2.0f * fi[8] * bi[8] + (f[1] + f[3]) * (bb[1] + bb[3]) +
-                   (fi[1] + fi[3]) * (bi[1] + bi[3]) + (f[2] + f[6]) * (bb[2] + bb[6]) +
-                   (fi[2] + fi[6]) * (bi[2] + bi[6]) + (f[5] + f[7]) * (bb[5] + bb[7]) +
-                   (fi[5] + fi[7]) * (bi[5] + bi[7]);
-        gm = -gm * A.fd;
-        const float gr = (qx[0][1] * qx[2][1] + qy[0][2] * qy[2][2] + qz[0][1] * qz[2][1]) +
-                         (qx[1][1] * qx[3][1] + qy[1][2] * qy[3][2] + qz[1][1] * qz[3][1]);
-        const float r = LD(rrho, 0, 0, 0), p = LD(rpi, 0, 0, 0), m = LD(ru, 0, 0, 0);
-        float a1 = LD(rg1, 0, 0, 0), a2 = LD(rg2, 0, 0, 0), a3 = LD(rg3, 0, 0, 0);
-        const double srp = sqrt((double)(r * p)), sru = sqrt((double)(r * m));
-        a1 = (float)(a1 + srp * 2 * gl);
-        a2 = (float)(a2 + (-4 * sru * gl + 2 * sru * gm));
-        a3 += gr + m / r * gm + (p - 2.0f * m) / r * gl;
-        ST(a1, rg1);
-        ST(a2, rg2);
-        ST(a3, rg3);
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                qx[t][q] = qx[t][q + 1];
-                qy[t][q] = qy[t][q + 1];
-                qz[t][q] = qz[t][q + 1];
-            }
+        const Strain F = cell_strain(g, rf[0], rf[1], rf[2], vo, SJ, SI),
+                     B = cell_strain(g, rf[6], rf[7], rf[8], vo, SJ, SI);
+        const float *f = F.d, *bb = B.d;
+        float gl = (f[0] + f[4] + f[8]) * (bb[0] + bb[4] + bb[8]);
+        gl = -gl;
+        float gm = 2.0f * f[0] * bb[0] + 2.0f * f[4] * bb[4] + 2.0f * f[8] * bb[8] + (f[1] + f[3]) * (bb[1] + bb[3]) +
+                   (f[2] + f[6]) * (bb[2] + bb[6]) + (f[5] + f[7]) * (bb[5] + bb[7]);
+        gm = -gm;
+        const float gr = LD(rf[3], 0, 0, 0) * LD(rf[9], 0, 0, 0) + LD(rf[4], 0, 0, 0) * LD(rf[10], 0, 0, 0) +
+                         LD(rf[5], 0, 0, 0) * LD(rf[11], 0, 0, 0);
+        const int64_t c = at(g, j, i, k);
+        A.acc[0][c] += (double)gl * A.w;
+        A.acc[1][c] += (double)gm * A.w;
+        A.acc[2][c] += (double)gr * A.w;
     }
 }
 
@@ -1844,36 +1866,47 @@ int launch_s_shots(const ifos_geom *g, const ifos_fields *f, const ifos_model *m
 namespace ifos {
 // gradient_F over [1..N]^3 for one frequency: f[12] point at that
 // frequency's fields (forward Re xyz, Im xyz, adjoint Re xyz, Im xyz)
-int launch_grad_march(const ifos_geom *g, const float *const f[12], float fd, const ifos_model *m,
-                      float *const d_grad[3], hipStream_t s, bool hess)
+int launch_gradient(const ifos_geom *g, float *const d_Ff[6], float *const d_Fb[6], int64_t fouter, int64_t bouter,
+                    int nouter, const float *fd, int nf, const ifos_model *m, float *const d_grad[3], bool hess,
+                    hipStream_t s)
 {
-    DevGeom G = make_dev_geom(g);
+    if (nouter < 1 || nf < 1) return IFOS_OK;
+    const DevGeom G = make_dev_geom(g);
     GradArgs A;
-    for (int n = 0; n < 12; ++n) A.f[n] = f[n];
-    A.fd = fd;
+    for (int n = 0; n < 6; ++n) {
+        A.f[n] = d_Ff[n];
+        A.f[6 + n] = d_Fb[n];
+    }
+    A.fouter = fouter;
+    A.bouter = bouter;
+    A.fe = (int64_t)ifos_field_elems(g);
+    A.nouter = nouter;
+    A.nf = nf;
+    for (int l = 0; l < nf; ++l) A.fd[l] = fd[l];
     A.rho = m->rho;
     A.pi = m->pi;
     A.u = m->u;
     A.g1 = d_grad[0];
     A.g2 = d_grad[1];
     A.g3 = d_grad[2];
-    const Box all = region_box(g, IFOS_REGION_ALL);
-    const MTiles T = make_tiles(&all, 1, 4, 0, 1, 0);
+    A.ntk = (uint32_t)((g->nz + 63) / 64);
+    A.nti = (uint32_t)((g->nx + kGradTI - 1) / kGradTI);
+    A.total = A.ntk * A.nti * (uint32_t)((g->ny + kGradTJ - 1) / kGradTJ);
+    A.per = (A.total + 7) / 8;
+    const dim3 grid(A.per * 8), block(64, kGradTI, kGradTJ);
+    ProfScope ps_(IFOS_K_GRADIENT, s);
     if (hess)
-        hipLaunchKernelGGL((k_grad_march<4, GRAD_HESS>), dim3((unsigned)(T.per * 8)), dim3(64, 4), 0, s, G, T, A);
+        hipLaunchKernelGGL((k_grad_cells<true>), grid, block, 0, s, G, A);
     else
-        hipLaunchKernelGGL((k_grad_march<4, GRAD_F>), dim3((unsigned)(T.per * 8)), dim3(64, 4), 0, s, G, T, A);
-    return hip_check(hipGetLastError(), "k_grad_march");
+        hipLaunchKernelGGL((k_grad_cells<false>), grid, block, 0, s, G, A);
+    return hip_check(hipGetLastError(), "k_grad_cells");
 }
-
-// one time sample of the time-domain gradient over [1..N]^3: uf, vf forward
-// displacement and velocity, ub, vb adjoint displacement and velocity
 int launch_td_sample(const ifos_geom *g, const float *const uf[3], const float *const vf[3],
                      const float *const ub[3], const float *const vb[3], double w, double *const acc[3],
                      hipStream_t s)
 {
     DevGeom G = make_dev_geom(g);
-    GradArgs A = {};
+    TdArgs A = {};
     for (int n = 0; n < 3; ++n) {
         A.f[n] = uf[n];
         A.f[3 + n] = vf[n];
@@ -1885,9 +1918,9 @@ int launch_td_sample(const ifos_geom *g, const float *const uf[3], const float *
     const Box all = region_box(g, IFOS_REGION_ALL);
     const MTiles T = make_tiles(&all, 1, 4, 0, 1, 0);
     { ProfScope ps_(IFOS_K_GRADIENT, s);
-    hipLaunchKernelGGL((k_grad_march<4, GRAD_TD>), dim3((unsigned)(T.per * 8)), dim3(64, 4), 0, s, G, T, A);
+    hipLaunchKernelGGL((k_td_march<4>), dim3((unsigned)(T.per * 8)), dim3(64, 4), 0, s, G, T, A);
     }
-    return hip_check(hipGetLastError(), "k_grad_march td");
+    return hip_check(hipGetLastError(), "k_td_march");
 }
 }  // namespace ifos
 
