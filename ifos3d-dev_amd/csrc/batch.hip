@@ -36,8 +36,6 @@
 
 namespace ifos {
 
-#define IFOS_CHUNK_MAX 32
-
 int point_class(const ifos_geom *g, int i, int j, int k)
 {
     return (slab_h(i, g->nx, g->fw, 1) || slab_h(j, g->ny, g->fw, !g->free_surf) || slab_h(k, g->nz, g->fw, 1)) ? 1
@@ -191,181 +189,11 @@ __global__ void k_bsurface(DevGeom g, BFields F, float *sxy, float *syz, const f
     szz[c] += h;
 }
 
-// chunked DFT: nsnap (<= CH) snapshots of one shot's v, every accumulator
-// of the cell updated nsnap times in registers.  trig[(c*tstride + l)*2 +
-// {0,1}] are the cos/sin factors of snapshot c (disc_fourier.c:42-44).  One thread
-// per cell of [1..N]^3, shot and velocity component (blockIdx.z = shot * ny
-// + j - 1, blockIdx.y = 3 * (i row block) + component), so a thread holds
-// one component's snapshots and its two accumulators; the frequencies are
-// walked in order with the next frequency's accumulators loaded while the
-// current one is updated.  FIRST: the accumulators start at 0 and are not
-// read, which saves their zeroing as well.
-struct FBase {
-    float *p[6];
-};
-
-template <int NF, int CH, bool KAHAN, bool FIRST>
-__global__ __launch_bounds__(256) void k_dft_chunk(DevGeom g, const float *ring, int64_t rstride, int nsnap,
-                                                  FBase F, FBase Cc, int64_t fshot, uint32_t tot,
-                                                  const double *__restrict__ trig, int tstride)
-{
-    const int q = (int)(blockIdx.y % 3u);  // velocity component: accumulators q (Re) and 3 + q (Im)
-    const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int i = (int)(blockIdx.y / 3u) * blockDim.y + threadIdx.y + 1;
-    const int j = (int)(blockIdx.z % (unsigned)g.ny) + 1;
-    const int s = (int)(blockIdx.z / (unsigned)g.ny);
-    if (k > g.nz || i > g.nx) return;
-    const int64_t cell = at(g, j, i, k);
-    const uint32_t vo = (uint32_t)cell * 4u;
-    const int64_t fe = g.fbytes / 4;
-    const float *rp = ring + (int64_t)s * rstride + (int64_t)q * fe + cell;
-    float v[CH];
-#pragma unroll
-    for (int c = 0; c < CH; ++c)
-        if (c < nsnap) v[c] = __builtin_nontemporal_load(rp + 3 * c * fe);
-    rsrc_t r[2], rc[2];
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-        r[n] = make_rsrc(F.p[q + 3 * n] + (int64_t)s * fshot, tot);
-        if (KAHAN) rc[n] = make_rsrc(Cc.p[q + 3 * n] + (int64_t)s * fshot, tot);
-    }
-    float a[2], cm[2], an[2], cn[2];
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-        a[n] = FIRST ? 0.0f : bload(r[n], vo, 0);
-        cm[n] = KAHAN && !FIRST ? bload(rc[n], vo, 0) : 0.0f;
-    }
-#pragma unroll
-    for (int l = 0; l < NF; ++l) {
-        if (l + 1 < NF) {
-#pragma unroll
-            for (int n = 0; n < 2; ++n) {
-                an[n] = FIRST ? 0.0f : bload(r[n], vo, (uint32_t)(l + 1) * g.fbytes);
-                cn[n] = KAHAN && !FIRST ? bload(rc[n], vo, (uint32_t)(l + 1) * g.fbytes) : 0.0f;
-            }
-        }
-#pragma unroll
-        for (int n = 0; n < 2; ++n) {  // n = 0: cos (Re), 1: sin (Im)
-            float acc = a[n], cmp = cm[n];
-#pragma unroll
-            for (int c = 0; c < CH; ++c)
-                if (c < nsnap) {
-                    const double term = (double)v[c] * trig[(c * tstride + l) * 2 + n];
-                    if (KAHAN) {
-                        const float yv = (float)(term - (double)cmp);
-                        const float t = acc + yv;
-                        cmp = (t - acc) - yv;
-                        acc = t;
-                    } else {
-                        acc = (float)(acc + term);
-                    }
-                }
-            bstore(acc, r[n], vo, (uint32_t)l * g.fbytes);
-            if (KAHAN) bstore(cmp, rc[n], vo, (uint32_t)l * g.fbytes);
-        }
-        if (l + 1 < NF) {
-#pragma unroll
-            for (int n = 0; n < 2; ++n) {
-                a[n] = an[n];
-                cm[n] = cn[n];
-            }
-        }
-    }
-}
-
 static __global__ void k_bfill(float *d, int64_t n, float v)
 {
     int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (; t < n; t += stride) d[t] = v;
-}
-
-int dft_trig(const ifos_geom *g, const float *finv, int nf, int ntast, double *out)
-{
-    const int nsamp = g->nt / ntast;
-    for (int back = 0; back < 2; ++back)
-        for (int q = 0; q < nsamp; ++q) {
-            const int nt = (q + 1) * ntast;
-            float t = 0.0f;
-            if (back == 0) t = nt * g->dt;
-            if (back == 1) t = g->time - nt * g->dt;
-            double *o = out + ((size_t)back * nsamp + q) * nf * 2;
-            for (int l = 0; l < nf; ++l) {
-                o[2 * l + 0] = cos(2.0 * t * finv[l] * M_PI) * g->dt * ntast;
-                o[2 * l + 1] = sin(2.0 * t * finv[l] * M_PI) * g->dt * ntast;
-            }
-        }
-    return nsamp;
-}
-
-template <int NF>
-static void dft_chunk_nf(int chunk, bool kahan, bool first, dim3 grid, dim3 block, hipStream_t st, const DevGeom &G,
-                         const float *ring, int64_t rstride, int nsnap, const FBase &F, const FBase &C,
-                         int64_t fshot, uint32_t tot, const double *trig, int tstride)
-{
-    auto go = [&](auto ch) {
-        constexpr int CH = decltype(ch)::value;
-        if (kahan && first)
-            hipLaunchKernelGGL((k_dft_chunk<NF, CH, true, true>), grid, block, 0, st, G, ring, rstride, nsnap, F, C,
-                               fshot, tot, trig, tstride);
-        else if (kahan)
-            hipLaunchKernelGGL((k_dft_chunk<NF, CH, true, false>), grid, block, 0, st, G, ring, rstride, nsnap, F, C,
-                               fshot, tot, trig, tstride);
-        else if (first)
-            hipLaunchKernelGGL((k_dft_chunk<NF, CH, false, true>), grid, block, 0, st, G, ring, rstride, nsnap, F, C,
-                               fshot, tot, trig, tstride);
-        else
-            hipLaunchKernelGGL((k_dft_chunk<NF, CH, false, false>), grid, block, 0, st, G, ring, rstride, nsnap, F,
-                               C, fshot, tot, trig, tstride);
-    };
-    if (chunk <= 4) go(std::integral_constant<int, 4>{});
-    else if (chunk <= 8) go(std::integral_constant<int, 8>{});
-    else if (chunk <= 16) go(std::integral_constant<int, 16>{});
-    else if (chunk <= 24) go(std::integral_constant<int, 24>{});
-    else go(std::integral_constant<int, 32>{});
-}
-
-int launch_dft_chunk(const ifos_geom *g, int ns, const float *ring, int chunk, int nsnap, float *const Fp[6],
-                     float *const Cp[6], int64_t fshot, const double *trig, int nf, bool first, hipStream_t st)
-{
-    DevGeom G = make_dev_geom(g);
-    const size_t fe = ifos_field_elems(g);
-    const int64_t rstride = (int64_t)chunk * 3 * (int64_t)fe;
-    dim3 block(64, 4), grid((unsigned)((g->nz + 63) / 64), (unsigned)(3 * ((g->nx + 3) / 4)), (unsigned)(ns * g->ny));
-    ProfScope ps_(IFOS_K_DFT, st);
-    // up to 8 frequencies a launch, and their fields below 4 GiB (the
-    // accumulators' buffer offsets are 32-bit)
-    const int most = (int)std::min<size_t>(8, 4294967295u / (fe * 4));
-    for (int l0 = 0; l0 < nf; l0 += most) {
-        const int n = std::min(most, nf - l0);
-        FBase F, C = {};
-        for (int q = 0; q < 6; ++q) {
-            F.p[q] = Fp[q] + (size_t)l0 * fe;
-            if (Cp) C.p[q] = Cp[q] + (size_t)l0 * fe;
-        }
-        const uint32_t tot = (uint32_t)(n * fe * 4);
-        const double *tr = trig + 2 * l0;
-#define IFOS_CHUNK_CASE(NFV)                                                                                    \
-    case NFV:                                                                                                   \
-        dft_chunk_nf<NFV>(chunk, Cp != nullptr, first, grid, block, st, G, ring, rstride, nsnap, F, C, fshot,    \
-                          tot, tr, nf);                                                                         \
-        break;
-        switch (n) {
-            IFOS_CHUNK_CASE(1)
-            IFOS_CHUNK_CASE(2)
-            IFOS_CHUNK_CASE(3)
-            IFOS_CHUNK_CASE(4)
-            IFOS_CHUNK_CASE(5)
-            IFOS_CHUNK_CASE(6)
-            IFOS_CHUNK_CASE(7)
-            IFOS_CHUNK_CASE(8)
-        default: set_error("dft_chunk: nf=%d", n); return IFOS_EINVAL;
-        }
-#undef IFOS_CHUNK_CASE
-        const int rc = hip_check(hipGetLastError(), "k_dft_chunk");
-        if (rc) return rc;
-    }
-    return IFOS_OK;
 }
 
 int launch_step(const StepArgs &A, int back, int nt, const Snap *N, bool seis, hipStream_t st)

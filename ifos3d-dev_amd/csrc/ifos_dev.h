@@ -11,6 +11,8 @@
 
 // largest number of DFT frequencies per call (kernel-argument arrays)
 #define IFOS_MAX_NF 32
+// longest snapshot ring of the chunked DFT
+#define IFOS_CHUNK_MAX 32
 
 namespace ifos {
 
