@@ -6,21 +6,23 @@
 // partial sums, so a call's result does not depend on scheduling.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 #include "ifos_dev.h"
 
 namespace ifos {
 
-constexpr int kRedBlocks = 512;   // partial sums per dot product
-constexpr int kRedThreads = 256;
+constexpr int kRedBlocks = 1024;  // partial sums per dot product
+constexpr int kRedThreads = 256;  // 4 wavefronts
 
-// block-wide FP64 sum of one value per thread (fixed tree order)
-__device__ inline double block_sum(double v, double *sh)
+// block-wide FP64 sum of one value per thread (fixed tree order); t: the
+// thread's index in the block
+__device__ inline double block_sum(double v, double *sh, int t)
 {
-    sh[threadIdx.x] = v;
+    sh[t] = v;
     __syncthreads();
     for (int s = kRedThreads / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
+        if (t < s) sh[t] += sh[t + s];
         __syncthreads();
     }
     const double r = sh[0];
@@ -28,67 +30,122 @@ __device__ inline double block_sum(double v, double *sh)
     return r;
 }
 
-// ---- compact vectors: [numpar][NY][NX][NZ], cell l = ((j-1)*NX + i-1)*NZ + k-1
+// Cells are walked a row (j, i) of the grid per wavefront, 64 k at a time: no
+// index divisions, and a row of 276 cells fills 86 % of the lanes (256
+// threads side by side along k: 54 %).
+struct Rows {
+    int64_t r, step, n;
+};
+__device__ inline Rows wave_rows(const DevGeom &g)
+{
+    const int y = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    return Rows{(int64_t)blockIdx.x * blockDim.y + y, (int64_t)gridDim.x * blockDim.y, (int64_t)g.nx * g.ny};
+}
+__device__ inline int64_t row_at(const DevGeom &g, int64_t r)
+{
+    const int j = (int)(r / g.nx) + 1, i = (int)(r % g.nx) + 1;
+    return at(g, j, i, 1);
+}
+
+// ---- L-BFGS on compact vectors: [numpar][NY][NX][NZ], cell l = ((j-1)*NX +
+// i-1)*NZ + k-1.  The two-loop recursion is a chain of passes over q, each
+// pass applying the update of one pair and forming the dot product that the
+// next needs, with the coefficients in device memory: 9 r + 1 vectors moved
+// for r pairs instead of 10 r + 12, and no host round trip inside.
+// The scalars of an update: state[0] y.s, [1] y.y, [2] the last dot product,
+// [3] h0, [4 + w] alpha of slot w, [4 + bfgsnum + w] scale of slot w
+// (bfgsscale, 1 / y.s)
 struct Pack {
-    const float *g1, *g2;  // device-layout gradients (g2 used when numpar == 2)
+    float *g1, *g2;  // device-layout gradients (g2 used when numpar == 2)
     int numpar;
-    int64_t n1;            // NX*NY*NZ
+    int64_t n1;      // NX*NY*NZ
 };
 
-__device__ inline int64_t compact_to_field(const DevGeom &g, int64_t l)
+// lbfgs_save.c:31-53: y = grad
+__global__ __launch_bounds__(kRedThreads) void k_lb_save(DevGeom g, Pack P, float *y)
 {
-    const int k = (int)(l % g.nz) + 1;
-    const int64_t r = l / g.nz;
-    const int i = (int)(r % g.nx) + 1, j = (int)(r / g.nx) + 1;
-    return at(g, j, i, k);
-}
-
-// mode 0, lbfgs_save.c:31-53: y = grad.  mode 1, lbfgs.c:47-71:
-// y += -grad, q = grad.
-__global__ __launch_bounds__(256) void k_lb_pack(DevGeom g, Pack P, float *q, float *y, int mode)
-{
-    const int64_t n = P.n1 * P.numpar;
-    for (int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; l < n; l += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t c = compact_to_field(g, l % P.n1);
-        const float v = l < P.n1 ? P.g1[c] : P.g2[c];
-        if (mode == 0) {
-            y[l] = +v;
-        } else {
-            y[l] += -v;
-            q[l] = v;
-        }
+    for (Rows R = wave_rows(g); R.r < R.n; R.r += R.step) {
+        const int64_t c = row_at(g, R.r), l = R.r * g.nz;
+        for (int q = 0; q < P.numpar; ++q)
+            for (int k = threadIdx.x; k < g.nz; k += 64) y[q * P.n1 + l + k] = +(q ? P.g2 : P.g1)[c + k];
     }
 }
 
-// lbfgs.c:157-178: bfgsgrad[w] = grad, grad = q
-__global__ __launch_bounds__(256) void k_lb_unpack(DevGeom g, float *g1, float *g2, int numpar, int64_t n1,
-                                                  const float *q, float *y)
-{
-    const int64_t n = n1 * numpar;
-    for (int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; l < n; l += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t c = compact_to_field(g, l % n1);
-        float *G = l < n1 ? g1 : g2;
-        y[l] = G[c];
-        G[c] = q[l];
-    }
-}
-
-// part[b*2 + 0] = sum a*b, part[b*2 + 1] = sum c*d (when c) over this
-// block's share of the compact vectors
-__global__ __launch_bounds__(kRedThreads) void k_lb_dot2(const float *a, const float *b, const float *c,
-                                                         const float *d, int64_t n, double *part)
+// lbfgs.c:45-71: y += -grad, q = grad, and the sums y.s, y.y (:74-88) and s.q
+// (the first of the recursion, :94-116, whose newest pair this is)
+__global__ __launch_bounds__(kRedThreads) void k_lb_first(DevGeom g, Pack P, float *q, float *y, const float *s,
+                                                          double *part)
 {
     __shared__ double sh[kRedThreads];
-    double s0 = 0.0, s1 = 0.0;
-    for (int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; l < n; l += (int64_t)gridDim.x * blockDim.x) {
-        s0 += (double)a[l] * (double)b[l];
-        if (c) s1 += (double)c[l] * (double)d[l];
+    double d[3] = {0.0, 0.0, 0.0};
+    for (Rows R = wave_rows(g); R.r < R.n; R.r += R.step) {
+        const int64_t c = row_at(g, R.r), l = R.r * g.nz;
+        for (int m = 0; m < P.numpar; ++m)
+            for (int k = threadIdx.x; k < g.nz; k += 64) {
+                const int64_t o = m * P.n1 + l + k;
+                const float v = (m ? P.g2 : P.g1)[c + k], sv = s[o];
+                const float yv = y[o] + -v;
+                y[o] = yv;
+                q[o] = v;
+                d[0] += (double)yv * (double)sv;
+                d[1] += (double)yv * (double)yv;
+                d[2] += (double)sv * (double)v;
+            }
     }
-    s0 = block_sum(s0, sh);
-    s1 = block_sum(s1, sh);
-    if (threadIdx.x == 0) {
-        part[2 * blockIdx.x] = s0;
-        part[2 * blockIdx.x + 1] = s1;
+    const int t = (int)(threadIdx.y * 64 + threadIdx.x);
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+        const double x = block_sum(d[m], sh, t);
+        if (t == 0) part[3 * blockIdx.x + m] = x;
+    }
+}
+
+// one pass of the recursion over the compact vectors, V floats at a time:
+// q += a x (lbfgs.c:115: x = y_w, a = -alpha_w; :149: x = s_w, a = alpha_w -
+// beta_w), q *= h0 where SCALE (:120-124), and the partial sums of z.q
+template <int V, bool SCALE>
+__global__ __launch_bounds__(kRedThreads) void k_lb_pass(float *q, const float *x, const float *z, int64_t n,
+                                                         const double *state, int ia, int is, int up, double *part)
+{
+    typedef float vec __attribute__((ext_vector_type(V)));
+    __shared__ double sh[kRedThreads];
+    // the dot product this pass's coefficient comes from is state[2]: alpha =
+    // scale * (s.q) on the way down, beta = scale * (y.q) on the way up
+    const double co = state[is] * state[2];
+    const float a = up ? (float)(state[ia] - co) : (float)(-co);
+    const float h0 = SCALE ? (float)state[3] : 0.0f;
+    double s = 0.0;
+    const int64_t nv = n / V, step = (int64_t)gridDim.x * kRedThreads;
+    for (int64_t l = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; l < nv; l += step) {
+        vec qv = ((const vec *)q)[l];
+        const vec xv = ((const vec *)x)[l], zv = ((const vec *)z)[l];
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            float w = qv[e] + (a * xv[e]);
+            if (SCALE) w = w * h0;
+            qv[e] = w;
+            s += (double)zv[e] * (double)w;
+        }
+        ((vec *)q)[l] = qv;
+    }
+    s = block_sum(s, sh, threadIdx.x);
+    if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+
+// lbfgs.c:149 for the newest pair, then :157-178: bfgsgrad[w] = grad, grad = q
+__global__ __launch_bounds__(kRedThreads) void k_lb_last(DevGeom g, Pack P, const float *q, const float *s, float *y,
+                                                         const double *state, int ia, int is)
+{
+    const float a = (float)(state[ia] - state[is] * state[2]);
+    for (Rows R = wave_rows(g); R.r < R.n; R.r += R.step) {
+        const int64_t c = row_at(g, R.r), l = R.r * g.nz;
+        for (int m = 0; m < P.numpar; ++m)
+            for (int k = threadIdx.x; k < g.nz; k += 64) {
+                const int64_t o = m * P.n1 + l + k;
+                float *G = m ? P.g2 : P.g1;
+                y[o] = G[c + k];
+                G[c + k] = q[o] + (s[o] * a);
+            }
     }
 }
 
@@ -99,52 +156,40 @@ __global__ __launch_bounds__(kRedThreads) void k_red_final(const double *part, i
     for (int m = 0; m < nd; ++m) {
         double s = 0.0;
         for (int b = threadIdx.x; b < nblk; b += blockDim.x) s += part[b * nd + m];
-        s = block_sum(s, sh);
+        s = block_sum(s, sh, threadIdx.x);
         if (threadIdx.x == 0) out[m] = s;
     }
 }
 
-// q += a * y (the FP32 update of lbfgs.c:115 and :149 with the coefficient
-// already formed); a_first: q += y * a as lbfgs.c:149 orders it
-__global__ __launch_bounds__(256) void k_lb_axpy(float *q, const float *y, float a, int64_t n, int a_first)
+// after the first pass: the scalars of the new pair (lbfgs.c:74-88); ia >= 0
+// (down the recursion): alpha of the slot whose dot product just arrived
+__global__ void k_lb_scalars(double *state, int first, int ia, int is)
 {
-    for (int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; l < n; l += (int64_t)gridDim.x * blockDim.x)
-        q[l] = a_first ? q[l] + (a * y[l]) : q[l] + (y[l] * a);
+    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    if (first) {
+        state[is] = 1.0 / state[0];
+        state[3] = state[0] / state[1];
+    }
+    if (ia >= 0) state[ia] = state[is] * state[2];
 }
 
-// lbfgs.c:120-124: q = q * h0
-__global__ __launch_bounds__(256) void k_lb_scale(float *q, float h0, int64_t n)
-{
-    for (int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; l < n; l += (int64_t)gridDim.x * blockDim.x)
-        q[l] = q[l] * h0;
-}
-
-// ---- conjugategrad.c on the device-layout fields: rows (j,i) over blocks,
-// k over threads
+// ---- conjugategrad.c on the device-layout fields
 struct CgArgs {
     float *g[3], *p[6];
 };
 
-__device__ inline bool cg_row(const DevGeom &g, int64_t r, int &j, int &i)
-{
-    if (r >= (int64_t)g.nx * g.ny) return false;
-    j = (int)(r / g.nx) + 1;
-    i = (int)(r % g.nx) + 1;
-    return true;
-}
-
 // conjugategrad.c:42-54 (cdf == 1): all six priors = grad
-__global__ __launch_bounds__(256) void k_cg_copy(DevGeom g, CgArgs A)
+__global__ __launch_bounds__(kRedThreads) void k_cg_copy(DevGeom g, CgArgs A)
 {
-    for (int64_t r = blockIdx.x; r < (int64_t)g.nx * g.ny; r += gridDim.x) {
-        int j, i;
-        cg_row(g, r, j, i);
-        for (int k = 1 + (int)threadIdx.x; k <= g.nz; k += blockDim.x) {
-            const int64_t c = at(g, j, i, k);
+    for (Rows R = wave_rows(g); R.r < R.n; R.r += R.step) {
+        const int64_t c0 = row_at(g, R.r);
+        for (int k = threadIdx.x; k < g.nz; k += 64) {
+            const int64_t c = c0 + k;
 #pragma unroll
             for (int n = 0; n < 3; ++n) {
-                A.p[n][c] = A.g[n][c];
-                A.p[n + 3][c] = A.g[n][c];
+                const float v = A.g[n][c];
+                A.p[n][c] = v;
+                A.p[n + 3][c] = v;
             }
         }
     }
@@ -155,50 +200,57 @@ __global__ __launch_bounds__(kRedThreads) void k_cg_dots(DevGeom g, CgArgs A, do
 {
     __shared__ double sh[kRedThreads];
     double s[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t r = blockIdx.x; r < (int64_t)g.nx * g.ny; r += gridDim.x) {
-        int j, i;
-        cg_row(g, r, j, i);
-        for (int k = 1 + (int)threadIdx.x; k <= g.nz; k += blockDim.x) {
-            const int64_t c = at(g, j, i, k);
+    for (Rows R = wave_rows(g); R.r < R.n; R.r += R.step) {
+        const int64_t c0 = row_at(g, R.r);
+        for (int k = threadIdx.x; k < g.nz; k += 64) {
+            const int64_t c = c0 + k;
+            float gv[3], pv[3];
 #pragma unroll
             for (int n = 0; n < 3; ++n) {
-                const double gn = A.g[n][c], pn = A.p[n][c];
-                s[2 * n] += gn * (double)(A.g[n][c] - A.p[n][c]);
-                s[2 * n + 1] += pn * pn;
-                A.p[n][c] = A.g[n][c];
+                gv[n] = A.g[n][c];
+                pv[n] = A.p[n][c];
+            }
+#pragma unroll
+            for (int n = 0; n < 3; ++n) {
+                s[2 * n] += (double)gv[n] * (double)(gv[n] - pv[n]);
+                s[2 * n + 1] += (double)pv[n] * (double)pv[n];
+                A.p[n][c] = gv[n];
             }
         }
     }
+    const int t = (int)(threadIdx.y * 64 + threadIdx.x);
 #pragma unroll
     for (int m = 0; m < 6; ++m) {
-        const double t = block_sum(s[m], sh);
-        if (threadIdx.x == 0) part[6 * blockIdx.x + m] = t;
+        const double x = block_sum(s[m], sh, t);
+        if (t == 0) part[6 * blockIdx.x + m] = x;
     }
 }
 
 // conjugategrad.c:93-106: grad = prior4..6 * beta + grad; prior4..6 = grad
-__global__ __launch_bounds__(256) void k_cg_update(DevGeom g, CgArgs A, float b0, float b1, float b2)
+__global__ __launch_bounds__(kRedThreads) void k_cg_update(DevGeom g, CgArgs A, float b0, float b1, float b2)
 {
     const float b[3] = {b0, b1, b2};
-    for (int64_t r = blockIdx.x; r < (int64_t)g.nx * g.ny; r += gridDim.x) {
-        int j, i;
-        cg_row(g, r, j, i);
-        for (int k = 1 + (int)threadIdx.x; k <= g.nz; k += blockDim.x) {
-            const int64_t c = at(g, j, i, k);
+    for (Rows R = wave_rows(g); R.r < R.n; R.r += R.step) {
+        const int64_t c0 = row_at(g, R.r);
+        for (int k = threadIdx.x; k < g.nz; k += 64) {
+            const int64_t c = c0 + k;
+            float v[3];
+#pragma unroll
+            for (int n = 0; n < 3; ++n) v[n] = (A.p[n + 3][c] * b[n]) + A.g[n][c];
 #pragma unroll
             for (int n = 0; n < 3; ++n) {
-                const float v = (A.p[n + 3][c] * b[n]) + A.g[n][c];
-                A.g[n][c] = v;
-                A.p[n + 3][c] = v;
+                A.g[n][c] = v[n];
+                A.p[n + 3][c] = v[n];
             }
         }
     }
 }
 
-static unsigned grid_for(int64_t n)
+// workgroups of a row-walking kernel without partial sums
+static unsigned row_grid(const ifos_geom *g)
 {
-    const int64_t b = (n + 255) / 256;
-    return (unsigned)(b < 4096 ? (b < 1 ? 1 : b) : 4096);
+    const int64_t b = ((int64_t)g->nx * g->ny + 3) / 4;
+    return (unsigned)(b < 8192 ? b : 8192);
 }
 
 }  // namespace ifos
@@ -213,9 +265,9 @@ struct ifos_lbfgs {
     float *grad = nullptr;    // bfgsgrad [bfgsnum][n] (slot w at w-1)
     float *mod = nullptr;     // bfgsmod  [bfgsnum][n]
     float *q = nullptr;       // [n]
-    double *part = nullptr;   // [kRedBlocks * 2]
-    double *out = nullptr;    // [2]
-    std::vector<double> scale;  // bfgsscale[1..bfgsnum] (index w-1)
+    double *part = nullptr;   // [kRedBlocks * 3]
+    double *state = nullptr;  // [4 + 2 * bfgsnum] scalars of an update
+    std::vector<double> scale;  // bfgsscale[1..bfgsnum] (index w-1), as state holds it
 };
 
 static int lb_slot(const ifos_lbfgs *b, int v)
@@ -223,16 +275,6 @@ static int lb_slot(const ifos_lbfgs *b, int v)
     int w = v % b->bfgsnum;
     if (w == 0) w = b->bfgsnum;
     return w - 1;
-}
-
-// two dot products of compact vectors, reduced in FP64: (a.b, c.d)
-static int lb_dot2(ifos_lbfgs *b, const float *x0, const float *y0, const float *x1, const float *y1, double r[2])
-{
-    hipLaunchKernelGGL(k_lb_dot2, dim3(kRedBlocks), dim3(kRedThreads), 0, 0, x0, y0, x1, y1, b->n, b->part);
-    hipLaunchKernelGGL(k_red_final, dim3(1), dim3(kRedThreads), 0, 0, b->part, kRedBlocks, 2, b->out);
-    int rc = hip_check(hipGetLastError(), "lbfgs dot");
-    if (!rc) rc = hip_check(hipMemcpy(r, b->out, 2 * sizeof(double), hipMemcpyDeviceToHost), "lbfgs dot copy");
-    return rc;
 }
 
 extern "C" int ifos_lbfgs_create(const ifos_geom *g, int numpar, int bfgsnum, ifos_lbfgs **out)
@@ -254,8 +296,10 @@ extern "C" int ifos_lbfgs_create(const ifos_geom *g, int numpar, int bfgsnum, if
     int rc = hip_check(hipMalloc(&b->grad, vb * bfgsnum), "lbfgs grad");
     if (!rc) rc = hip_check(hipMalloc(&b->mod, vb * bfgsnum), "lbfgs mod");
     if (!rc) rc = hip_check(hipMalloc(&b->q, vb), "lbfgs q");
-    if (!rc) rc = hip_check(hipMalloc(&b->part, kRedBlocks * 6 * sizeof(double)), "lbfgs partials");
-    if (!rc) rc = hip_check(hipMalloc(&b->out, 6 * sizeof(double)), "lbfgs sums");
+    const size_t sb = (4 + 2 * (size_t)bfgsnum) * sizeof(double);
+    if (!rc) rc = hip_check(hipMalloc(&b->part, kRedBlocks * 3 * sizeof(double)), "lbfgs partials");
+    if (!rc) rc = hip_check(hipMalloc(&b->state, sb), "lbfgs scalars");
+    if (!rc) rc = hip_check(hipMemset(b->state, 0, sb), "lbfgs zero");
     // ifos3d.c:373-379: fmatrix / vector zero-fill
     if (!rc) rc = hip_check(hipMemset(b->grad, 0, vb * bfgsnum), "lbfgs zero");
     if (!rc) rc = hip_check(hipMemset(b->mod, 0, vb * bfgsnum), "lbfgs zero");
@@ -274,7 +318,7 @@ extern "C" void ifos_lbfgs_destroy(ifos_lbfgs *b)
     (void)hipFree(b->mod);
     (void)hipFree(b->q);
     (void)hipFree(b->part);
-    (void)hipFree(b->out);
+    (void)hipFree(b->state);
     delete b;
 }
 
@@ -300,9 +344,9 @@ extern "C" int ifos_lbfgs_scale(const ifos_lbfgs *b, double *scale)
 extern "C" int ifos_lbfgs_savegrad(ifos_lbfgs *b, const float *d_grad1, const float *d_grad2)
 {
     if (!b || !d_grad1 || (b->numpar == 2 && !d_grad2)) return IFOS_EINVAL;
-    const Pack P = {d_grad1, d_grad2, b->numpar, b->n1};
-    hipLaunchKernelGGL(k_lb_pack, dim3(grid_for(b->n)), dim3(256), 0, 0, b->G, P, nullptr, b->grad, 0);
-    int rc = hip_check(hipGetLastError(), "k_lb_pack");
+    const Pack P = {const_cast<float *>(d_grad1), const_cast<float *>(d_grad2), b->numpar, b->n1};
+    hipLaunchKernelGGL(k_lb_save, dim3(row_grid(&b->g)), dim3(64, 4), 0, 0, b->G, P, b->grad);
+    int rc = hip_check(hipGetLastError(), "k_lb_save");
     if (!rc) rc = hip_check(hipStreamSynchronize(0), "lbfgs_savegrad");
     return rc;
 }
@@ -314,56 +358,64 @@ extern "C" int ifos_lbfgs_update(ifos_lbfgs *b, float *d_grad1, float *d_grad2, 
         return IFOS_EINVAL;
     }
     const int64_t n = b->n;
-    const unsigned gr = grid_for(n);
-    int m = iteration - b->bfgsnum;
+    const int M = b->bfgsnum;
+    int m = iteration - M;
     if (m < 1) m = 1;
-    // lbfgs.c:45-71: y_w = g_prev - g, q = g
-    int w = lb_slot(b, iteration - 1);
-    float *yw = b->grad + (size_t)w * n, *sw = b->mod + (size_t)w * n;
+    double *st = b->state;
+    auto grad = [&](int w) { return b->grad + (size_t)w * n; };
+    auto mod = [&](int w) { return b->mod + (size_t)w * n; };
+    auto red = [&](int nd, double *out) {
+        hipLaunchKernelGGL(k_red_final, dim3(1), dim3(kRedThreads), 0, 0, b->part, kRedBlocks, nd, out);
+    };
+    auto scalars = [&](int first, int w) {
+        hipLaunchKernelGGL(k_lb_scalars, dim3(1), dim3(64), 0, 0, st, first, w >= 0 ? 4 + w : -1, 4 + M + (w >= 0 ? w : 0));
+    };
+    // q += (up: alpha_w - beta_w, else -alpha_w) x, (* h0), then state[2] = z.q
+    auto pass = [&](bool up, bool scale, int w, const float *x, const float *z) {
+        // 16-byte vectors where every slot starts on such a boundary
+        auto go = [&](auto v, auto sc) {
+            hipLaunchKernelGGL((k_lb_pass<decltype(v)::value, decltype(sc)::value>), dim3(kRedBlocks),
+                               dim3(kRedThreads), 0, 0, b->q, x, z, n, st, 4 + w, 4 + M + w, up ? 1 : 0, b->part);
+        };
+        if (n % 4 == 0 && scale) go(std::integral_constant<int, 4>{}, std::true_type{});
+        else if (n % 4 == 0) go(std::integral_constant<int, 4>{}, std::false_type{});
+        else if (scale) go(std::integral_constant<int, 1>{}, std::true_type{});
+        else go(std::integral_constant<int, 1>{}, std::false_type{});
+        red(1, st + 2);
+    };
+    // lbfgs.c:45-88: y_w = g_prev - g, q = g, rho_w = 1 / (y.s), h0 = (y.s) /
+    // (y.y), and s_w.q
+    const int wn = lb_slot(b, iteration - 1);
     const Pack P = {d_grad1, d_grad2, b->numpar, b->n1};
-    hipLaunchKernelGGL(k_lb_pack, dim3(gr), dim3(256), 0, 0, b->G, P, b->q, yw, 1);
-    int rc = hip_check(hipGetLastError(), "k_lb_pack");
-    // lbfgs.c:74-88: rho_w = 1 / (y.s), h0 = (y.s) / (y.y)
-    double r[2];
-    if (!rc) rc = lb_dot2(b, yw, sw, yw, yw, r);
-    if (rc) return rc;
-    b->scale[w] = 1.0 / r[0];
-    const double h0 = r[0] / r[1];
-    if (h0_out) *h0_out = h0;
-    // lbfgs.c:94-116: newest to oldest, alpha_w = rho_w s_w.q, q -= alpha_w y_w
-    std::vector<double> alpha(b->bfgsnum, 0.0);
-    for (int v = iteration - 1; v >= m && !rc; --v) {
-        w = lb_slot(b, v);
-        rc = lb_dot2(b, b->mod + (size_t)w * n, b->q, nullptr, nullptr, r);
-        if (rc) break;
-        alpha[w] = b->scale[w] * r[0];
-        hipLaunchKernelGGL(k_lb_axpy, dim3(gr), dim3(256), 0, 0, b->q, b->grad + (size_t)w * n,
-                           (float)(-alpha[w]), n, 1);
-        rc = hip_check(hipGetLastError(), "k_lb_axpy");
-    }
-    // lbfgs.c:120-124
-    if (!rc) {
-        hipLaunchKernelGGL(k_lb_scale, dim3(gr), dim3(256), 0, 0, b->q, (float)h0, n);
-        rc = hip_check(hipGetLastError(), "k_lb_scale");
+    hipLaunchKernelGGL(k_lb_first, dim3(kRedBlocks), dim3(64, 4), 0, 0, b->G, P, b->q, grad(wn), mod(wn), b->part);
+    red(3, st);
+    scalars(1, wn);
+    // lbfgs.c:94-116: newest to oldest, alpha_w = rho_w s_w.q, q -= alpha_w y_w;
+    // the oldest also multiplies by h0 (:120-124) and starts the way back
+    for (int v = iteration - 1; v >= m; --v) {
+        const int w = lb_slot(b, v);
+        if (v > m) {
+            pass(false, false, w, grad(w), mod(lb_slot(b, v - 1)));
+            scalars(0, lb_slot(b, v - 1));
+        } else {
+            pass(false, true, w, grad(w), grad(w));
+        }
     }
     // lbfgs.c:136-151: oldest to newest, beta = rho_w y_w.q, q += s_w (alpha_w - beta)
-    for (int v = m; v <= iteration - 1 && !rc; ++v) {
-        w = lb_slot(b, v);
-        rc = lb_dot2(b, b->grad + (size_t)w * n, b->q, nullptr, nullptr, r);
-        if (rc) break;
-        const double beta = b->scale[w] * r[0];
-        hipLaunchKernelGGL(k_lb_axpy, dim3(gr), dim3(256), 0, 0, b->q, b->mod + (size_t)w * n,
-                           (float)(alpha[w] - beta), n, 0);
-        rc = hip_check(hipGetLastError(), "k_lb_axpy");
+    for (int v = m; v < iteration - 1; ++v) {
+        const int w = lb_slot(b, v);
+        pass(true, false, w, mod(w), grad(lb_slot(b, v + 1)));
     }
-    // lbfgs.c:154-178: save this gradient in slot iteration, grad = q
-    if (!rc) {
-        w = lb_slot(b, iteration);
-        hipLaunchKernelGGL(k_lb_unpack, dim3(gr), dim3(256), 0, 0, b->G, d_grad1, d_grad2, b->numpar, b->n1, b->q,
-                           b->grad + (size_t)w * n);
-        rc = hip_check(hipGetLastError(), "k_lb_unpack");
-    }
-    if (!rc) rc = hip_check(hipStreamSynchronize(0), "ifos_lbfgs_update");
+    // the newest pair, and lbfgs.c:154-178: save this gradient in slot
+    // iteration, grad = q
+    hipLaunchKernelGGL(k_lb_last, dim3(row_grid(&b->g)), dim3(64, 4), 0, 0, b->G, P, b->q, mod(wn),
+                       grad(lb_slot(b, iteration)), st, 4 + wn, 4 + M + wn);
+    int rc = hip_check(hipGetLastError(), "ifos_lbfgs_update");
+    std::vector<double> h(4 + 2 * (size_t)M);
+    if (!rc) rc = hip_check(hipMemcpy(h.data(), st, h.size() * sizeof(double), hipMemcpyDeviceToHost), "lbfgs scalars");
+    if (rc) return rc;
+    b->scale[wn] = h[4 + M + wn];
+    if (h0_out) *h0_out = h[3];
     return rc;
 }
 
@@ -403,11 +455,10 @@ extern "C" int ifos_conjugate(const ifos_geom *g, float *const d_grad[3], float 
     CgArgs A;
     for (int n = 0; n < 3; ++n) A.g[n] = d_grad[n];
     for (int n = 0; n < 6; ++n) A.p[n] = d_prior[n];
-    const int64_t rows = (int64_t)g->nx * g->ny;
-    const unsigned gr = (unsigned)(rows < 4096 ? rows : 4096);
+    const unsigned gr = row_grid(g);
     beta[0] = beta[1] = beta[2] = 0.0f;  // conjugategrad.c:37
     if (cdf == 1) {
-        hipLaunchKernelGGL(k_cg_copy, dim3(gr), dim3(256), 0, 0, G, A);
+        hipLaunchKernelGGL(k_cg_copy, dim3(gr), dim3(64, 4), 0, 0, G, A);
         int rc = hip_check(hipGetLastError(), "k_cg_copy");
         if (!rc) rc = hip_check(hipStreamSynchronize(0), "ifos_conjugate");
         return rc;
@@ -416,7 +467,7 @@ extern "C" int ifos_conjugate(const ifos_geom *g, float *const d_grad[3], float 
     int rc = cg_buffers(&part, &out);
     double s[6] = {0, 0, 0, 0, 0, 0};
     if (!rc) {
-        hipLaunchKernelGGL(k_cg_dots, dim3(kRedBlocks), dim3(kRedThreads), 0, 0, G, A, part);
+        hipLaunchKernelGGL(k_cg_dots, dim3(kRedBlocks), dim3(64, 4), 0, 0, G, A, part);
         hipLaunchKernelGGL(k_red_final, dim3(1), dim3(kRedThreads), 0, 0, part, kRedBlocks, 6, out);
         rc = hip_check(hipGetLastError(), "k_cg_dots");
     }
@@ -437,7 +488,7 @@ extern "C" int ifos_conjugate(const ifos_geom *g, float *const d_grad[3], float 
     if (beta[0] > 0.5f) beta[0] = 0.5f;
     if (beta[0] > 0.5f) beta[1] = 0.5f;
     if (beta[0] > 0.5f) beta[2] = 0.5f;
-    hipLaunchKernelGGL(k_cg_update, dim3(gr), dim3(256), 0, 0, G, A, beta[0], beta[1], beta[2]);
+    hipLaunchKernelGGL(k_cg_update, dim3(gr), dim3(64, 4), 0, 0, G, A, beta[0], beta[1], beta[2]);
     rc = hip_check(hipGetLastError(), "k_cg_update");
     if (!rc) rc = hip_check(hipStreamSynchronize(0), "ifos_conjugate");
     return rc;
@@ -595,60 +646,85 @@ __global__ __launch_bounds__(kRedThreads) void k_mu_max(DevGeom g, const float *
 {
     __shared__ float sh[6][kRedThreads];
     float m[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t r = blockIdx.x; r < (int64_t)g.nx * g.ny; r += gridDim.x) {
-        const int j = (int)(r / g.nx) + 1, i = (int)(r % g.nx) + 1;
-        for (int k = 1 + (int)threadIdx.x; k <= g.nz; k += blockDim.x) {
-            const int64_t c = at(g, j, i, k);
-            const float vp = (float)sqrt((double)(pi[c] / rho[c]));
-            const float vs = (float)sqrt((double)(u[c] / rho[c]));
+    for (Rows R = wave_rows(g); R.r < R.n; R.r += R.step) {
+        const int64_t c0 = row_at(g, R.r);
+        for (int k = threadIdx.x; k < g.nz; k += 64) {
+            const int64_t c = c0 + k;
+            const float r = rho[c];
+            const float vp = (float)sqrt((double)(pi[c] / r));
+            const float vs = (float)sqrt((double)(u[c] / r));
             if (vp > m[0]) m[0] = vp;
             if (vs > m[1]) m[1] = vs;
-            if (rho[c] > m[2]) m[2] = rho[c];
+            if (r > m[2]) m[2] = r;
             if (fabsf(g1[c]) > m[3]) m[3] = fabsf(g1[c]);
             if (fabsf(g2[c]) > m[4]) m[4] = fabsf(g2[c]);
             if (fabsf(g3[c]) > m[5]) m[5] = fabsf(g3[c]);
         }
     }
-    for (int q = 0; q < 6; ++q) sh[q][threadIdx.x] = m[q];
+    const int t = (int)(threadIdx.y * 64 + threadIdx.x);
+    for (int q = 0; q < 6; ++q) sh[q][t] = m[q];
     __syncthreads();
     for (int s = kRedThreads / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s)
-            for (int q = 0; q < 6; ++q) sh[q][threadIdx.x] = fmaxf(sh[q][threadIdx.x], sh[q][threadIdx.x + s]);
+        if (t < s)
+            for (int q = 0; q < 6; ++q) sh[q][t] = fmaxf(sh[q][t], sh[q][t + s]);
         __syncthreads();
     }
-    if (threadIdx.x < 6) part[6 * blockIdx.x + threadIdx.x] = sh[threadIdx.x][0];
+    if (t < 6) part[6 * blockIdx.x + t] = sh[t][0];
+}
+
+// the six maxima over the blocks (none below 0): max[0..5]
+__global__ __launch_bounds__(kRedThreads) void k_mu_final(const float *part, int nblk, float *max6)
+{
+    __shared__ float sh[kRedThreads];
+    for (int q = 0; q < 6; ++q) {
+        float m = 0.0f;
+        for (int b = threadIdx.x; b < nblk; b += kRedThreads) m = fmaxf(m, part[6 * b + q]);
+        sh[threadIdx.x] = m;
+        __syncthreads();
+        for (int s = kRedThreads / 2; s > 0; s >>= 1) {
+            if ((int)threadIdx.x < s) sh[threadIdx.x] = fmaxf(sh[threadIdx.x], sh[threadIdx.x + s]);
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) max6[q] = sh[0];
+        __syncthreads();
+    }
 }
 
 struct MuArgs {
     float *g[3], *rho, *pi, *u, *mod;  // mod: bfgsmod slot (compact) or null
-    float step, s1, s2, s3, vp0, vs0, rho0, n1, n2, n3;  // n*: gradient normalisers (1 when none)
-    int numpar;
+    float step, s1, s2, s3, vp0, vs0, rho0;
+    const float *max6;  // maxima of vp, vs, rho and of the gradients
+    int lbfgs, numpar;
     int64_t ncell;
 };
 
-// modelupdate.c:97-157 (the gradient normalisation folded in as a division)
-__global__ __launch_bounds__(256) void k_modelupdate(DevGeom g, MuArgs A, int normalise)
+// modelupdate.c:97-157 (the gradient normalisation folded in as a division:
+// modelupdate.c:84-115, without L-BFGS, by the gradients' maxima, when the vp
+// and vs maxima are both nonzero)
+__global__ __launch_bounds__(kRedThreads) void k_modelupdate(DevGeom g, MuArgs A)
 {
-    for (int64_t r = blockIdx.x; r < (int64_t)g.nx * g.ny; r += gridDim.x) {
-        const int j = (int)(r / g.nx) + 1, i = (int)(r % g.nx) + 1;
-        for (int k = 1 + (int)threadIdx.x; k <= g.nz; k += blockDim.x) {
-            const int64_t c = at(g, j, i, k);
+    const float n1 = A.max6[3], n2 = A.max6[4], m5 = A.max6[5], n3 = m5 == 0.0f ? 1.0f : m5;
+    const bool normalise = !A.lbfgs && n1 > 0.0f && n2 > 0.0f;
+    for (Rows R = wave_rows(g); R.r < R.n; R.r += R.step) {
+        const int64_t c0 = row_at(g, R.r), l0 = R.r * g.nz;
+        for (int k = threadIdx.x; k < g.nz; k += 64) {
+            const int64_t c = c0 + k;
             float gvp = A.g[0][c], gvs = A.g[1][c], grho = A.g[2][c];
+            const float rho = A.rho[c], pi = A.pi[c], u = A.u[c];
             if (normalise) {
-                gvp = gvp / A.n1;
-                gvs = gvs / A.n2;
-                grho = grho / A.n3;
+                gvp = gvp / n1;
+                gvs = gvs / n2;
+                grho = grho / n3;
                 A.g[0][c] = gvp;
                 A.g[1][c] = gvs;
                 A.g[2][c] = grho;
             }
-            const float rho = A.rho[c], pi = A.pi[c], u = A.u[c];
             const double vp = sqrt((double)(pi / rho)), vs = sqrt((double)(u / rho));
             const float vpnew = (float)(vp + (double)(((A.step * A.s1) * gvp) * A.vp0));
             const float vsnew = (float)(vs + (double)(((A.step * A.s2) * gvs) * A.vs0));
             const float rhonew = rho + (((A.s3 * A.step) * grho) * A.rho0);
             if (A.mod) {
-                const int64_t l = ((int64_t)(j - 1) * g.nx + (i - 1)) * g.nz + (k - 1);
+                const int64_t l = l0 + k;
                 A.mod[l] = (float)(((double)vpnew - vp) / (double)A.vp0);
                 if (A.numpar > 1) A.mod[A.ncell + l] = (float)(((double)vsnew - vs) / (double)A.vs0);
             }
@@ -723,23 +799,9 @@ extern "C" int ifos_modelupdate(const ifos_geom *g, float *const d_grad[3], floa
     }
     const hipStream_t st = (hipStream_t)stream;
     const DevGeom G = make_dev_geom(g);
-    float *part = nullptr;
-    float m[6] = {0, 0, 0, 0, 0, 0};
-    int rc = hip_check(hipMalloc(&part, kRedBlocks * 6 * sizeof(float)), "modelupdate partials");
-    if (!rc) {
-        hipLaunchKernelGGL(k_mu_max, dim3(kRedBlocks), dim3(kRedThreads), 0, st, G, d_rho, d_pi, d_u, d_grad[0],
-                           d_grad[1], d_grad[2], part);
-        rc = hip_check(hipGetLastError(), "k_mu_max");
-    }
-    std::vector<float> h(kRedBlocks * 6);
-    if (!rc) rc = hip_check(hipMemcpyAsync(h.data(), part, h.size() * sizeof(float), hipMemcpyDeviceToHost, st), "max");
-    if (!rc) rc = hip_check(hipStreamSynchronize(st), "modelupdate max");
-    (void)hipFree(part);
+    float *part = nullptr, m[6] = {0, 0, 0, 0, 0, 0};
+    int rc = hip_check(hipMallocAsync((void **)&part, (kRedBlocks + 1) * 6 * sizeof(float), st), "modelupdate partials");
     if (rc) return rc;
-    for (int b = 0; b < kRedBlocks; ++b)
-        for (int q = 0; q < 6; ++q) m[q] = std::max(m[q], h[6 * b + q]);
-    if (maxima)
-        for (int q = 0; q < 3; ++q) maxima[q] = m[q];
     MuArgs A;
     for (int n = 0; n < 3; ++n) A.g[n] = d_grad[n];
     A.rho = d_rho;
@@ -753,19 +815,21 @@ extern "C" int ifos_modelupdate(const ifos_geom *g, float *const d_grad[3], floa
     A.vp0 = vp0;
     A.vs0 = vs0;
     A.rho0 = rho0;
+    A.max6 = part + 6 * kRedBlocks;
+    A.lbfgs = lbfgs;
     A.numpar = numpar;
     A.ncell = (int64_t)g->nx * g->ny * g->nz;
-    // modelupdate.c:84-115: without L-BFGS the gradients are divided by their
-    // maxima, when the vp and vs maxima are both nonzero
-    int normalise = 0;
-    A.n1 = m[3];
-    A.n2 = m[4];
-    A.n3 = m[5] == 0.0f ? 1.0f : m[5];
-    if (!lbfgs && A.n1 > 0.0f && A.n2 > 0.0f) normalise = 1;
-    const int64_t rows = (int64_t)g->nx * g->ny;
-    hipLaunchKernelGGL(k_modelupdate, dim3((unsigned)(rows < 8192 ? rows : 8192)), dim3(256), 0, st, G, A, normalise);
+    hipLaunchKernelGGL(k_mu_max, dim3(kRedBlocks), dim3(64, 4), 0, st, G, d_rho, d_pi, d_u, d_grad[0], d_grad[1],
+                       d_grad[2], part);
+    hipLaunchKernelGGL(k_mu_final, dim3(1), dim3(kRedThreads), 0, st, part, kRedBlocks, part + 6 * kRedBlocks);
+    hipLaunchKernelGGL(k_modelupdate, dim3(row_grid(g)), dim3(64, 4), 0, st, G, A);
     rc = hip_check(hipGetLastError(), "k_modelupdate");
+    if (!rc) rc = hip_check(hipMemcpyAsync(m, part + 6 * kRedBlocks, sizeof m, hipMemcpyDeviceToHost, st), "max");
     if (!rc) rc = hip_check(hipStreamSynchronize(st), "ifos_modelupdate");
+    (void)hipFreeAsync(part, st);
+    if (rc) return rc;
+    if (maxima)
+        for (int q = 0; q < 3; ++q) maxima[q] = m[q];
     return rc;
 }
 
