@@ -38,16 +38,16 @@ namespace ifos {
 // szz sxy syz sxz), axis, forward (1) / backward (0) difference, half-grid
 // CPML profile, CPML memory array (update_v_ssg_CPML.c:84-130,
 // update_s_ssg_CPML_elastic.c:63-115)
-__constant__ int c_vq_field[9] = {3, 6, 8, 4, 6, 7, 5, 8, 7};
-__constant__ int c_vq_axis[9] = {0, 1, 2, 1, 0, 2, 2, 0, 1};
-__constant__ int c_vq_fwd[9] = {1, 0, 0, 1, 0, 0, 1, 0, 0};
-__constant__ int c_vq_half[9] = {1, 0, 0, 1, 0, 0, 1, 0, 0};
-__constant__ int c_vq_psi[9] = {0, 3, 6, 4, 1, 7, 8, 2, 5};
-__constant__ int c_sq_field[9] = {0, 0, 0, 1, 1, 1, 2, 2, 2};
-__constant__ int c_sq_axis[9] = {0, 1, 2, 0, 1, 2, 0, 1, 2};
-__constant__ int c_sq_fwd[9] = {0, 1, 1, 1, 0, 1, 1, 1, 0};
-__constant__ int c_sq_half[9] = {0, 1, 1, 1, 0, 1, 1, 1, 0};
-__constant__ int c_sq_psi[9] = {0, 3, 6, 1, 4, 7, 2, 5, 8};
+static constexpr __device__ int c_vq_field[9] = {3, 6, 8, 4, 6, 7, 5, 8, 7};
+static constexpr __device__ int c_vq_axis[9] = {0, 1, 2, 1, 0, 2, 2, 0, 1};
+static constexpr __device__ int c_vq_fwd[9] = {1, 0, 0, 1, 0, 0, 1, 0, 0};
+static constexpr __device__ int c_vq_half[9] = {1, 0, 0, 1, 0, 0, 1, 0, 0};
+static constexpr __device__ int c_vq_psi[9] = {0, 3, 6, 4, 1, 7, 8, 2, 5};
+static constexpr __device__ int c_sq_field[9] = {0, 0, 0, 1, 1, 1, 2, 2, 2};
+static constexpr __device__ int c_sq_axis[9] = {0, 1, 2, 0, 1, 2, 0, 1, 2};
+static constexpr __device__ int c_sq_fwd[9] = {0, 1, 1, 1, 0, 1, 1, 1, 0};
+static constexpr __device__ int c_sq_half[9] = {0, 1, 1, 1, 0, 1, 1, 1, 0};
+static constexpr __device__ int c_sq_psi[9] = {0, 3, 6, 1, 4, 7, 2, 5, 8};
 
 struct AdjS {
     float *L[9];                 // adjoint of vx vy vz sxx syy szz sxy syz sxz
@@ -228,20 +228,26 @@ __global__ __launch_bounds__(256) void k_ca_v_T(DevGeom g, AdjV A)
     for (int n = 3; n < 9; ++n) A.L[n][c] += acc[n];
 }
 
-// lambda_v += syn(n) - obs(n) at every receiver, in receiver order (one
-// thread: receivers may share a cell)
-__global__ void k_ca_inject(DevGeom g, float *Lx, float *Ly, float *Lz, const int *rec, int ntr, const float *res,
-                            int ldres, int n)
+// lambda_v += syn(n) - obs(n): one thread per receiver, the first receiver of
+// a cell adding for all that share it, in receiver order (chain as
+// ifos_rec_chain makes it).  One thread for all receivers took 1.2 us each.
+__global__ __launch_bounds__(256) void k_ca_inject(DevGeom g, float *Lx, float *Ly, float *Lz, const int *rec,
+                                                   const int *chain, int ntr, const float *res, int ldres, int n)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= ntr || !chain[2 * r]) return;
     const int64_t comp = (int64_t)ntr * ldres;
-    for (int r = 0; r < ntr; ++r) {
-        const int *p = rec + 3 * r;
-        const int64_t c = at(g, p[1], p[0], p[2]), o = (int64_t)r * ldres + n;
-        Lx[c] += res[o];
-        Ly[c] += res[comp + o];
-        Lz[c] += res[2 * comp + o];
+    const int64_t c = at(g, rec[3 * r + 1], rec[3 * r], rec[3 * r + 2]);
+    float x = Lx[c], y = Ly[c], z = Lz[c];
+    for (int q = r; q >= 0 && q < ntr; q = chain[2 * q + 1]) {
+        const int64_t o = (int64_t)q * ldres + n;
+        x += res[o];
+        y += res[comp + o];
+        z += res[2 * comp + o];
     }
+    Lx[c] = x;
+    Ly[c] = y;
+    Lz[c] = z;
 }
 
 // res = syn - obs (samples 1..nt of [3][ntr][nt+1]) and J = 1/2 sum res^2 in
@@ -348,8 +354,8 @@ int launch_ca_step(const ifos_geom *g, const float *d_prof, const CaStep &S, hip
     const Prof P = {d_prof, 2 * g->fw + 1};
     const dim3 blk(64, 4), grd = cells_grid(g);
     if (S.ntr > 0) {
-        hipLaunchKernelGGL(k_ca_inject, dim3(1), dim3(64), 0, st, G, S.L[0], S.L[1], S.L[2], S.rec, S.ntr, S.res,
-                           g->nt + 1, S.n);
+        hipLaunchKernelGGL(k_ca_inject, dim3((unsigned)((S.ntr + 255) / 256)), dim3(256), 0, st, G, S.L[0], S.L[1],
+                           S.L[2], S.rec, S.chain, S.ntr, S.res, g->nt + 1, S.n);
     }
     AdjS A;
     for (int q = 0; q < 9; ++q) {

@@ -1172,6 +1172,7 @@ extern "C" int ifos_ctx_run_shot_adj(ifos_ctx *c, const ifos_shot *s, int every,
             for (int m = 0; m < 9; ++m) C.model[m] = mp[m];
             for (int m = 0; m < 8; ++m) C.G[m] = A->G[m];
             C.rec = c->rec;
+            C.chain = c->chain;
             C.ntr = s->ntr;
             C.res = A->res;
             C.n = n;

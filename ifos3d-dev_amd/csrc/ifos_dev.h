@@ -304,7 +304,7 @@ struct CaStep {
     float *mu_v[9], *mu_s[9];    // their adjoints
     const float *model[9];       // rho pi u uipjp ujpkp uipkp rjp rkp rip
     double *G[8];                // dJ / d rip rjp rkp pi u uipjp ujpkp uipkp
-    const int *rec;
+    const int *rec, *chain;      // [ntr][3]; [ntr][2] (ifos_rec_chain)
     int ntr;
     const float *res;            // [3][ntr][nt+1]
     int n;
