@@ -305,6 +305,7 @@ struct MTiles {
     int start[7];  // cumulative tile counts per box
     int nb, jc, ns, group, total, per;
     int sb, nsg;  // shots per workgroup (one wavefront row each), shot groups
+    int lds, ti;  // host: tiled for the LDS-staged marches; wavefronts per workgroup
 };
 
 __device__ inline bool decode_tile(const MTiles &T, int TI, int &k, int &i, int &jb, int &je, int &shot,
@@ -1416,10 +1417,23 @@ static Box region_box(const ifos_geom *g, int region)
     return B;
 }
 
-// tiles of boxes for TI i-rows per block and at most jc j-planes (<= 0: 64)
-static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, int ns, int group, int kb = 1, int sb = 1)
+// lanes of a wavefront along k (the others take further i-rows): a row of nk
+// cells in pieces of 64, or of 32 (one 128-byte line; two rows a wavefront)
+// where that leaves fewer lanes idle; rows below 64 cells whole
+static int row_lanes(int nk, bool lds)
+{
+    const auto padded = [&](int w) { return (nk + w - 1) / w * w; };
+    if (nk < 64) return nk;
+    return !lds && padded(32) < padded(64) ? 32 : 64;
+}
+
+// tiles of boxes for TI i-rows per block and at most jc j-planes (<= 0: 64);
+// lds: for the LDS-staged marches
+static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, int ns, int group, int kb = 1, int sb = 1,
+                         bool lds = false)
 {
     MTiles T = {};
+    T.lds = lds;
     T.nb = 0;
     T.ns = ns;
     // shots side by side in a workgroup share its model loads
@@ -1432,7 +1446,7 @@ static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, int ns, int g
         const Box &B = boxes[q];
         if (B.i1 < B.i0 || B.j1 < B.j0 || B.k1 < B.k0) continue;
         const int nk = B.k1 - B.k0 + 1, ni = B.i1 - B.i0 + 1;
-        const int kw = nk >= 64 ? 64 : nk, rpw = 64 / kw;
+        const int kw = row_lanes(nk, lds), rpw = 64 / kw;
         const int nwk = (nk + kw - 1) / kw;  // wavefront columns along k
         int kbq = kb < 1 ? 1 : kb;
         while (kbq > 1 && (kbq > nwk || (ti / sbq) % kbq)) kbq /= 2;
@@ -1497,38 +1511,60 @@ int check_tile_cfg(const int *c, const char *who)
     return IFOS_OK;
 }
 
-// shape of a launch beyond its tiles: register marches one plane ahead
-// (pipe), LDS staging, streaming policy
-struct MarchMode {
-    bool lds, pipe, nt;
-};
-
-// the LDS-staged marches need 64-lane rows (every box at least 64 cells deep
-// in k), one k column and one shot per workgroup, and TI >= 2
-static bool lds_ok(const MarchCfg &c, const MTiles &T)
+// A time step reads 9 fields of every shot and 8 of the model (more with L
+// mechanisms).  While these fit the 256 MB Infinity Cache the next launch
+// finds this launch's words there, and the streaming hint only costs.
+static bool step_cached(const DevGeom &g, int ns, int L)
 {
-    if (!c.lds || c.ti < 2 || T.sb != 1) return false;
-    for (int q = 0; q < T.nb; ++q)
-        if (T.kw[q] != 64 || T.kb[q] != 1) return false;
-    return true;
+    return 4.0 * g.nx * g.ny * g.nz * ((9.0 + 6.0 * L) * ns + (L ? 13.0 : 8.0)) <= 256e6;
 }
 
-// A time step reads 9 fields of every shot and 8 of the model.  While these
-// fit the 256 MB Infinity Cache the next launch finds this launch's words
-// there: the streaming hint then only costs, and the register marches, whose
-// neighbour loads are cache hits, beat the LDS staging and its barrier; past
-// it the LDS marches with streamed own words win.  v / s whole-domain
-// marches, LDS + streaming -> register + default policy: one shot at 84^3
-// (10 MB) 24.3 / 25.8 -> 18.9 / 19.5 us, 148^3 (220 MB) 66.4 / 70.8 -> 56.4 /
-// 64.2, 202 x 106 x 202 (294 MB) 89.6 / 96.2 -> 93.7 / 109.2, 4 shots at 84^3
-// (104 MB) 63.2 / 67.2 -> 53.7 / 55.0, 3 at 148^3 (454 MB) with LDS 195 / 196
-// -> 197 / 208.  A tile shape that a caller or the autotuner set keeps its
-// lds choice.
-static MarchMode march_mode(const MarchCfg &c, const MTiles &T, const DevGeom &g, int ns, bool whole, int L = 0)
+// The march of a launch.  The LDS-staged marches take rows of 64 lanes (every
+// box at least 64 cells deep in k), one k column and one shot per workgroup,
+// and TI >= 2.  They save cache misses, so in a default shape they are left
+// out where a step is cached, and where rows of 64 leave many lanes idle: the
+// register marches with two rows of 32 per wavefront then win.  v / s, us,
+// LDS -> register, whole-domain, both with the better cache policy: one shot
+// at 84^3 23.2 / 23.8 -> 17.3 / 17.9, 148^3 63 / 66 -> 47 / 59, 202 x 106 x 202
+// (rows 1.14 x longer in 64s) 90 / 96 -> 75 / 88; 4 shots at 84^3 59 / 57 ->
+// 41 / 45, 3 at 148^3 (1.2 x) 195 / 194 -> 168 / 190; but 4 at 276^3 (1.11 x)
+// 1208 / 1452 -> 1222 / 1550, 536 x 280 x 536 (1.06 x) 1230 / 1540 -> 1275 /
+// 1595.  A shape that a caller or the autotuner set keeps its lds choice.
+static bool use_lds(const MarchCfg &c, const Box *boxes, int nb, const DevGeom &g, int ns, int kb, int sb, int L)
 {
-    const double set = 4.0 * g.nx * g.ny * g.nz * ((9.0 + 6.0 * L) * ns + (L ? 13.0 : 8.0));
-    const bool cached = set <= 256e6;
-    return MarchMode{lds_ok(c, T) && !(c.dflt && cached), c.pipe != 0, whole && !cached};
+    if (!c.lds || c.ti < 2 || kb > 1 || sb > 1) return false;
+    for (int q = 0; q < nb; ++q) {
+        const int nk = boxes[q].k1 - boxes[q].k0 + 1;
+        if (nk < 64) return false;
+        if (c.dflt && (nk + 63) / 64 * 64 > 1.12 * ((nk + 31) / 32 * 32)) return false;
+    }
+    return !(c.dflt && step_cached(g, ns, L));
+}
+
+// the tiles of a launch of shape c over boxes; kb, sb: c's, or 1 for one shot
+static MTiles march_tiles(const MarchCfg &c, const Box *boxes, int nb, const DevGeom &g, int ns, int group, int kb,
+                          int sb, bool velocity, int L = 0)
+{
+    const bool lds = use_lds(c, boxes, nb, g, ns, kb, sb, L);
+    MTiles T = make_tiles(boxes, nb, c.ti, c.jc, ns, group, kb, sb, lds);
+    // half the rows per workgroup suit the velocity march with rows of 32
+    // (3 shots at 148^3: 176 -> 168 us; the stress march: no difference)
+    if (c.dflt && velocity && !lds && c.ti == 4 && T.nb == 1 && T.kw[0] == 32) {
+        T = make_tiles(boxes, nb, 2, c.jc, ns, group, kb, sb, false);
+        T.ti = 2;
+    } else {
+        T.ti = c.ti;
+    }
+    return T;
+}
+
+// register marches one plane ahead (pipe), streaming policy (nt)
+struct MarchMode {
+    bool pipe, nt;
+};
+static MarchMode march_mode(const MarchCfg &c, const DevGeom &g, int ns, bool whole, int L = 0)
+{
+    return MarchMode{c.pipe != 0, whole && !step_cached(g, ns, L)};
 }
 
 template <int TI, bool CPML, bool SNAP, bool NT>
@@ -1536,7 +1572,7 @@ static void launch_v_one(const MarchMode &m, dim3 grid, const MTiles &T, const D
                          const Prof &P, const Psi9 &psi, const Shots &S, const Snap &N, hipStream_t s)
 {
     if constexpr (TI >= 2)
-        if (m.lds) {
+        if (T.lds) {
             hipLaunchKernelGGL((k_v_lds<TI, CPML, SNAP, NT>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, N);
             return;
         }
@@ -1552,7 +1588,7 @@ static int launch_v(const MarchCfg &c, const MTiles &T, const DevGeom &G, const 
 {
     if (T.total == 0) return IFOS_OK;
     const dim3 grid((unsigned)(T.per * 8));
-    const MarchMode m = march_mode(c, T, G, S.n, CPML);
+    const MarchMode m = march_mode(c, G, S.n, CPML);
     auto go = [&](auto ti) {
         constexpr int TI = decltype(ti)::value;
         if constexpr (CPML)
@@ -1562,12 +1598,12 @@ static int launch_v(const MarchCfg &c, const MTiles &T, const DevGeom &G, const 
             }
         launch_v_one<TI, CPML, SNAP, false>(m, grid, T, G, F, P, psi, S, N, s);
     };
-    switch (c.ti) {
+    switch (T.ti) {
     case 1: go(std::integral_constant<int, 1>{}); break;
     case 2: go(std::integral_constant<int, 2>{}); break;
     case 4: go(std::integral_constant<int, 4>{}); break;
     case 8: go(std::integral_constant<int, 8>{}); break;
-    default: set_error("march: TI=%d not in {1,2,4,8}", c.ti); return IFOS_EINVAL;
+    default: set_error("march: TI=%d not in {1,2,4,8}", T.ti); return IFOS_EINVAL;
     }
     return hip_check(hipGetLastError(), "velocity march");
 }
@@ -1577,7 +1613,7 @@ static void launch_s_one(const MarchMode &m, dim3 grid, const MTiles &T, const D
                          const Prof &P, const Psi9 &psi, const Shots &S, const ViscoF &V, hipStream_t s)
 {
     if constexpr (TI >= 2)
-        if (m.lds) {
+        if (T.lds) {
             hipLaunchKernelGGL((k_s_lds<TI, CPML, VM, NT>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, V);
             return;
         }
@@ -1593,7 +1629,7 @@ static int launch_s(const MarchCfg &c, const MTiles &T, const DevGeom &G, const 
 {
     if (T.total == 0) return IFOS_OK;
     const dim3 grid((unsigned)(T.per * 8));
-    const MarchMode m = march_mode(c, T, G, S.n, CPML, VM ? V.L : 0);
+    const MarchMode m = march_mode(c, G, S.n, CPML, VM ? V.L : 0);
     auto go = [&](auto ti) {
         constexpr int TI = decltype(ti)::value;
         if constexpr (CPML)
@@ -1603,12 +1639,12 @@ static int launch_s(const MarchCfg &c, const MTiles &T, const DevGeom &G, const 
             }
         launch_s_one<TI, CPML, VM, false>(m, grid, T, G, F, P, psi, S, V, s);
     };
-    switch (c.ti) {
+    switch (T.ti) {
     case 1: go(std::integral_constant<int, 1>{}); break;
     case 2: go(std::integral_constant<int, 2>{}); break;
     case 4: go(std::integral_constant<int, 4>{}); break;
     case 8: go(std::integral_constant<int, 8>{}); break;
-    default: set_error("march: TI=%d not in {1,2,4,8}", c.ti); return IFOS_EINVAL;
+    default: set_error("march: TI=%d not in {1,2,4,8}", T.ti); return IFOS_EINVAL;
     }
     return hip_check(hipGetLastError(), "stress march");
 }
@@ -1670,7 +1706,7 @@ static int update_v_region(const ifos_geom *g, int region, const Box *box, const
     }
     Box boxes[1];
     boxes[0] = box ? *box : region_box(g, region);
-    const MTiles T = make_tiles(boxes, 1, c.ti, c.jc, 1, 0);
+    const MTiles T = march_tiles(c, boxes, 1, G, 1, 0, 1, 1, true);
     const int cat = region == IFOS_REGION_ALL ? IFOS_K_V_FUSED : IFOS_K_V_INTERIOR;
     ProfScope ps_(cat, s);
     if (region == IFOS_REGION_INTERIOR) return launch_v<false, false>(c, T, G, F, P, psi, one, none, s);
@@ -1703,7 +1739,7 @@ static int update_s_region(const ifos_geom *g, int region, const Box *box, const
     }
     Box boxes[1];
     boxes[0] = box ? *box : region_box(g, region);
-    const MTiles T = make_tiles(boxes, 1, c.ti, c.jc, 1, 0);
+    const MTiles T = march_tiles(c, boxes, 1, G, 1, 0, 1, 1, false, visco ? visco->L : 0);
     const int cat = region == IFOS_REGION_ALL ? IFOS_K_S_FUSED : IFOS_K_S_INTERIOR;
     ProfScope ps_(cat, s);
     if (visco) {
@@ -1817,15 +1853,15 @@ int launch_v_shots(const ifos_geom *g, const ifos_fields *f, const ifos_model *m
     ProfScope ps_(IFOS_K_V_FUSED, s);
     if (!c.split) {
         const Box all = region_box(g, IFOS_REGION_ALL);
-        const MTiles T = make_tiles(&all, 1, c.ti, c.jc, S.n, c.group, c.kb, c.sb);
+        const MTiles T = march_tiles(c, &all, 1, G, S.n, c.group, c.kb, c.sb, true);
         return snap ? launch_v<true, true>(c, T, G, F, P, psi, S, N, s)
                     : launch_v<true, false>(c, T, G, F, P, psi, S, N, s);
     }
     const Box in = region_box(g, IFOS_REGION_INTERIOR);
     Box sl[6];
     const int nb = slab_boxes(g, sl);
-    const MTiles Ti = make_tiles(&in, 1, c.ti, c.jc, S.n, c.group, c.kb, c.sb);
-    const MTiles Ts = make_tiles(sl, nb, c.ti, c.jc, S.n, c.group, c.kb, c.sb);
+    const MTiles Ti = march_tiles(c, &in, 1, G, S.n, c.group, c.kb, c.sb, true);
+    const MTiles Ts = march_tiles(c, sl, nb, G, S.n, c.group, c.kb, c.sb, true);
     int rc = snap ? launch_v<false, true>(c, Ti, G, F, P, psi, S, N, s)
                   : launch_v<false, false>(c, Ti, G, F, P, psi, S, N, s);
     if (!rc)
@@ -1842,7 +1878,8 @@ int launch_s_shots(const ifos_geom *g, const ifos_fields *f, const ifos_model *m
     const Prof P = {d_prof, 2 * g->fw + 1};
     const Psi9 psi = psi9(psi_v);
     ProfScope ps_(IFOS_K_S_FUSED, s);
-    auto go = [&](const MTiles &T, bool cpml) {
+    auto go = [&](const Box *boxes, int nb, bool cpml) {
+        const MTiles T = march_tiles(c, boxes, nb, G, S.n, c.group, c.kb, c.sb, false, V ? V->L : 0);
         if (!V) return cpml ? launch_s<true>(c, T, G, F, P, psi, S, s) : launch_s<false>(c, T, G, F, P, psi, S, s);
         if (V->L == 1)
             return cpml ? launch_s<true, 1>(c, T, G, F, P, psi, S, s, *V)
@@ -1851,21 +1888,19 @@ int launch_s_shots(const ifos_geom *g, const ifos_fields *f, const ifos_model *m
     };
     if (!c.split) {
         const Box all = region_box(g, IFOS_REGION_ALL);
-        return go(make_tiles(&all, 1, c.ti, c.jc, S.n, c.group, c.kb, c.sb), true);
+        return go(&all, 1, true);
     }
     const Box in = region_box(g, IFOS_REGION_INTERIOR);
     Box sl[6];
     const int nb = slab_boxes(g, sl);
-    int rc = go(make_tiles(&in, 1, c.ti, c.jc, S.n, c.group, c.kb, c.sb), false);
-    if (!rc) rc = go(make_tiles(sl, nb, c.ti, c.jc, S.n, c.group, c.kb, c.sb), true);
+    int rc = go(&in, 1, false);
+    if (!rc) rc = go(sl, nb, true);
     return rc;
 }
 
 }  // namespace ifos
 
 namespace ifos {
-// gradient_F over [1..N]^3 for one frequency: f[12] point at that
-// frequency's fields (forward Re xyz, Im xyz, adjoint Re xyz, Im xyz)
 int launch_gradient(const ifos_geom *g, float *const d_Ff[6], float *const d_Fb[6], int64_t fouter, int64_t bouter,
                     int nouter, const float *fd, int nf, const ifos_model *m, float *const d_grad[3], bool hess,
                     hipStream_t s)

@@ -417,7 +417,8 @@ int ifos_levels_run(ifos_batch *const *lv, int nlev, const ifos_shot *const *sho
  * the in-plane neighbours are staged in LDS (used where every row is 64 k
  * wide and kb = sb = 1, TI >= 2; elsewhere ignored).  NULL leaves a shape
  * unchanged.  A new batch starts with {4, 32, 0, 0, 0, 1, 1, 1} for both,
- * with lds left out while a step's working set fits the Infinity Cache. */
+ * with lds left out while a step's working set fits the Infinity Cache or
+ * rows of 64 k leave many lanes idle. */
 #define IFOS_TILE_FIELDS 8
 int ifos_batch_set_tiles(ifos_batch *b, const int cfg_v[IFOS_TILE_FIELDS], const int cfg_s[IFOS_TILE_FIELDS]);
 /* the tile shape (same fields; group, split and sb have no effect) of the
