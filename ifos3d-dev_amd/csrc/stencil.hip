@@ -522,14 +522,14 @@ __global__ __launch_bounds__(64 * TI) void k_v_march(DevGeom g, MTiles T, VField
 // i0+TI), sxz, syz and szz for their k-neighbours (the row's halo words).
 // sxx, sxz and szz are read at the plane itself, sxy and syz come from the
 // j-queues.  Same arithmetic, in the same order, as k_v_march.
-template <int TI, bool CPML, bool SNAP, bool NT>
+template <int TI, bool CPML, bool SNAP, bool NT, int KW>
 __global__ __launch_bounds__(64 * TI) void k_v_lds(DevGeom g, MTiles T, VFields F, Prof P, Psi9 psi, Shots S,
                                                   Snap N)
 {
-    constexpr int RW = TI + 4;
-    constexpr int NH = (9 + TI - 1) / TI;
+    constexpr int RPW = 64 / KW, NR = TI * RPW, RW = NR + 4;
+    constexpr int NS = KW == 64 ? 9 : 6, NH = (NS + TI - 1) / TI;
     constexpr int CPN = NT ? IFOS_CPOL_NT : 0;
-    __shared__ float sh[2][5][RW][68];  // sxx, sxy, sxz, syz, szz
+    __shared__ float sh[2][5][RW][KW + 4];  // sxx, sxy, sxz, syz, szz
     const int b = blockIdx.x;
     const int L = (b & 7) * T.per + (b >> 3);
     if (L >= T.total) return;  // whole workgroup
@@ -545,9 +545,11 @@ __global__ __launch_bounds__(64 * TI) void k_v_lds(DevGeom g, MTiles T, VFields 
     const int tk = t % T.ntk[q];
     t /= T.ntk[q];
     const int ti = t % T.nti[q], tj = t / T.nti[q];
-    const int lane = (int)threadIdx.x;
-    const int y = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
-    const int k0 = R.k0 + tk * 64, i0 = R.i0 + ti * TI;
+    const int lane = (int)threadIdx.x & (KW - 1);  // along k
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    const int sub = KW == 64 ? 0 : (int)threadIdx.x / KW;
+    const int y = w * RPW + sub;  // row of the workgroup (KW 64: one per wavefront)
+    const int k0 = R.k0 + tk * KW, i0 = R.i0 + ti * NR;
     const int k = k0 + lane, i = i0 + y;
     const int jb = R.j0 + tj * T.jc, je = min(jb + T.jc - 1, R.j1);
     const bool act = k <= R.k1 && i <= R.i1;
@@ -566,20 +568,21 @@ __global__ __launch_bounds__(64 * TI) void k_v_lds(DevGeom g, MTiles T, VFields 
     if (SNAP) rring = make_rsrc(N.ring + (int64_t)shot * N.rstride, N.rbytes);
     if (CPML) shift_psi(psi, S, shot);
     uint32_t vb = (uint32_t)((int64_t)jb * g.sj + (int64_t)i0 * g.si + kc + IFOS_KOFF - 2) * 4u;
-    const uint32_t own = (uint32_t)(yc + 2) * SI;
-#define LB(r, dj) bload(r, vb + 8u, (uint32_t)((dj) + 2) * SJ + own)
-#define LBN(r, dj) bload_cp<CPN>(r, vb + 8u, (uint32_t)((dj) + 2) * SJ + own)
-    const int kh = lane < 2 ? k0 - 2 + lane : lane < 32 ? k0 - 1 : lane < 63 ? k0 + 64 : k0 + 65;
-    const int hcol = lane < 62 ? (lane < 2 ? lane : lane + 2) : lane + 4;
+    // own row: KW 64 in the scalar offset, else in the lane's (vo)
+    const uint32_t own = KW == 64 ? (uint32_t)(yc + 2) * SI : 2u * SI, ro = KW == 64 ? 0u : (uint32_t)yc * SI;
+#define LB(r, dj) bload(r, vb + ro + 8u, (uint32_t)((dj) + 2) * SJ + own)
+#define LBN(r, dj) bload_cp<CPN>(r, vb + ro + 8u, (uint32_t)((dj) + 2) * SJ + own)
+    const int kh = lane < 2 ? k0 - 2 + lane : lane < KW / 2 ? k0 - 1 : lane < KW - 1 ? k0 + KW : k0 + KW + 1;
+    const int hcol = lane < KW - 2 ? (lane < 2 ? lane : lane + 2) : lane + 4;
     const uint32_t hd = (uint32_t)((min(kh, g.nz + 2) - kc) * 4);
     // outside rows: e = min(y + n TI, 8) is (stress e / 3: sxx, sxy, sxz; row i0 + orow)
     int oc[NH], orow[NH];
     uint32_t ooff[NH];
 #pragma unroll
     for (int n = 0; n < NH; ++n) {
-        const int e = min(y + n * TI, 8);
-        const int c = e < 3 ? 0 : (e < 6 ? 1 : 2), m = e - 3 * c;
-        const int r = c == 0 ? (m == 0 ? -1 : (m == 1 ? TI : TI + 1)) : (m == 0 ? -2 : (m == 1 ? -1 : TI));
+        const int p = min(w + n * TI, NS - 1);
+        const int c = KW == 64 ? p / 3 : p / 2, m = KW == 64 ? p - 3 * c : min(2 * (p & 1) + sub, 2);
+        const int r = c == 0 ? (m == 0 ? -1 : (m == 1 ? NR : NR + 1)) : (m == 0 ? -2 : (m == 1 ? -1 : NR));
         oc[n] = c;
         orow[n] = r;
         ooff[n] = (uint32_t)(min(i0 + r, g.nx + 2) - i0 + 2) * SI;
@@ -602,13 +605,13 @@ __global__ __launch_bounds__(64 * TI) void k_v_lds(DevGeom g, MTiles T, VFields 
     auto load_ops = [&](Ops &O, int D) {
         const uint32_t pj = (uint32_t)(D + 2) * SJ;
         O.sxx = LB(rsxx, D); O.sxz = LB(rsxz, D); O.szz = LB(rszz, D);
-        O.hk[0] = bload(rsxz, vb + 8u + hd, pj + own);
-        O.hk[1] = bload(rsyz, vb + 8u + hd, pj + own);
-        O.hk[2] = bload(rszz, vb + 8u + hd, pj + own);
+        O.hk[0] = bload(rsxz, vb + ro + 8u + hd, pj + own);
+        O.hk[1] = bload(rsyz, vb + ro + 8u + hd, pj + own);
+        O.hk[2] = bload(rszz, vb + ro + 8u + hd, pj + own);
 #pragma unroll
         for (int n = 0; n < NH; ++n) {
             const rsrc_t rc = oc[n] == 0 ? rsxx : (oc[n] == 1 ? rsxy : rsxz);
-            O.ho[n] = bload(rc, vb + 8u, pj + ooff[n]);
+            O.ho[n] = KW == 64 ? bload(rc, vb + 8u, pj + ooff[n]) : bload(rc, vb + ooff[n] + 8u, pj);
         }
     };
 
@@ -627,7 +630,7 @@ __global__ __launch_bounds__(64 * TI) void k_v_lds(DevGeom g, MTiles T, VFields 
         load_ops(nxt, 1);
         load_cell(cur, 0);
         const uint32_t q3 = (uint32_t)(min(j + 3, g.ny + 2) - j + 2) * SJ + own;
-        const float sxy_n = LB(rsxy, 2), syz_n = LB(rsyz, 2), syy_n = bload(rsyy, vb + 8u, q3);
+        const float sxy_n = LB(rsxy, 2), syz_n = LB(rsyz, 2), syy_n = bload(rsyy, vb + ro + 8u, q3);
         // stage plane j: halo words first, then the rows over them
         sh[p][2][y + 2][hcol] = cur.hk[0];
         sh[p][3][y + 2][hcol] = cur.hk[1];
@@ -641,11 +644,11 @@ __global__ __launch_bounds__(64 * TI) void k_v_lds(DevGeom g, MTiles T, VFields 
         for (int n = 0; n < NH; ++n) sh[p][oc[n]][orow[n] + 2][lane + 2] = cur.ho[n];
         __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (act) {
-            const float(*XX)[68] = sh[p][0];
-            const float(*XY)[68] = sh[p][1];
-            const float(*XZ)[68] = sh[p][2];
-            const float(*YZ)[68] = sh[p][3];
-            const float(*ZZ)[68] = sh[p][4];
+            const float(*XX)[KW + 4] = sh[p][0];
+            const float(*XY)[KW + 4] = sh[p][1];
+            const float(*XZ)[KW + 4] = sh[p][2];
+            const float(*YZ)[KW + 4] = sh[p][3];
+            const float(*ZZ)[KW + 4] = sh[p][4];
             const int c0 = lane + 2, r0_ = y + 2;
             PsiCell pc;
             const int hy = CPML ? slab_h(j, g.ny, g.fw, !g.free_surf) : 0;
@@ -665,13 +668,13 @@ __global__ __launch_bounds__(64 * TI) void k_v_lds(DevGeom g, MTiles T, VFields 
             const float nvy = cur.vy0 + (syy_y + sxy_x + syz_z) / cur.rjp;
             const float nvz = cur.vz0 + (szz_z + sxz_x + syz_y) / cur.rkp;
             const uint32_t st = 2u * SJ + own;
-            bstore_cp<CPN>(nvx, rvx, vb + 8u, st);
-            bstore_cp<CPN>(nvy, rvy, vb + 8u, st);
-            bstore_cp<CPN>(nvz, rvz, vb + 8u, st);
+            bstore_cp<CPN>(nvx, rvx, vb + ro + 8u, st);
+            bstore_cp<CPN>(nvy, rvy, vb + ro + 8u, st);
+            bstore_cp<CPN>(nvz, rvz, vb + ro + 8u, st);
             if (SNAP) {
-                bstore_cp<CPN>(nvx, rring, vb + 8u, st + N.soff);
-                bstore_cp<CPN>(nvy, rring, vb + 8u, st + N.soff + g.fbytes);
-                bstore_cp<CPN>(nvz, rring, vb + 8u, st + N.soff + 2 * g.fbytes);
+                bstore_cp<CPN>(nvx, rring, vb + ro + 8u, st + N.soff);
+                bstore_cp<CPN>(nvy, rring, vb + ro + 8u, st + N.soff + g.fbytes);
+                bstore_cp<CPN>(nvz, rring, vb + ro + 8u, st + N.soff + 2 * g.fbytes);
             }
         }
         sxy_m2 = sxy_m1; sxy_m1 = sxy_0; sxy_0 = sxy_p1; sxy_p1 = sxy_n;
@@ -839,8 +842,10 @@ __global__ __launch_bounds__(64 * TI) void k_s_march(DevGeom g, MTiles T, SField
 #undef SLOAD
 
 // ---------------------------------------------------------------------------
-// Stress march with the in-plane neighbours staged in LDS.  Tiles of 64
-// k-lanes (one row per wavefront, one shot per workgroup): at each plane j
+// Stress march with the in-plane neighbours staged in LDS.  Rows of KW = 64
+// k-lanes (one row per wavefront) or 32 (two rows per wavefront), one shot per
+// workgroup; the text is for 64, where 32 differs NR = 2 TI rows take TI's
+// place and the halo words are those of each half.  At each plane j
 // every wavefront writes its row of vx, vy, vz (the centre of its j-queues)
 // to LDS, the halo words of its row (k0-2, k0-1, k0+64, k0+65), and its share
 // of the rows just outside the workgroup (vx at i0-2, i0-1, i0+TI; vy and vz
@@ -862,14 +867,16 @@ __global__ __launch_bounds__(64 * TI) void k_s_march(DevGeom g, MTiles T, SField
 // update and store.  The barrier waits for LDS only (s_waitcnt lgkmcnt(0)):
 // the loads in flight for the next plane stay in flight across it.  Same
 // arithmetic, in the same order, as k_s_march.
-template <int TI, bool CPML, int VM, bool NT>
+template <int TI, bool CPML, int VM, bool NT, int KW>
 __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields F, Prof P, Psi9 psi, Shots S,
                                                   ViscoF V)
 {
-    constexpr int RW = TI + 4;              // LDS rows: i0-2 .. i0+TI+1
-    constexpr int NH = (9 + TI - 1) / TI;   // outside rows per wavefront (9 per workgroup)
+    constexpr int RPW = 64 / KW;            // rows of a wavefront
+    constexpr int NR = TI * RPW, RW = NR + 4;  // rows of the workgroup; LDS rows i0-2 .. i0+NR+1
+    // loads of outside rows per wavefront: 9 rows, or 6 pairs of one field
+    constexpr int NS = KW == 64 ? 9 : 6, NH = (NS + TI - 1) / TI;
     constexpr int CPN = NT ? IFOS_CPOL_NT : 0;
-    __shared__ float sh[2][3][RW][68];
+    __shared__ float sh[2][3][RW][KW + 4];
     const int b = blockIdx.x;
     const int L = (b & 7) * T.per + (b >> 3);
     if (L >= T.total) return;  // whole workgroup
@@ -885,14 +892,16 @@ __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields 
     const int tk = t % T.ntk[q];
     t /= T.ntk[q];
     const int ti = t % T.nti[q], tj = t / T.nti[q];
-    const int lane = (int)threadIdx.x;
-    const int y = __builtin_amdgcn_readfirstlane((int)threadIdx.y);  // one row per wavefront
-    const int k0 = R.k0 + tk * 64, i0 = R.i0 + ti * TI;
+    const int lane = (int)threadIdx.x & (KW - 1);  // along k
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    const int sub = KW == 64 ? 0 : (int)threadIdx.x / KW;
+    const int y = w * RPW + sub;  // row of the workgroup (KW 64: one per wavefront)
+    const int k0 = R.k0 + tk * KW, i0 = R.i0 + ti * NR;
     const int k = k0 + lane, i = i0 + y;
     const int jb = R.j0 + tj * T.jc, je = min(jb + T.jc - 1, R.j1);
     const bool act = k <= R.k1 && i <= R.i1;  // updates and stores
     const int kc = min(k, g.nz + 2);          // clamped load cell
-    const int yc = min(i, g.nx + 2) - i0;     // clamped own row (wavefront-uniform)
+    const int yc = min(i, g.nx + 2) - i0;     // clamped own row (KW 64: wavefront-uniform)
     const uint32_t SJ = (uint32_t)g.sj * 4u, SI = (uint32_t)g.si * 4u;
     const float b1 = g.b1, b2 = g.b2, DT = g.dt;
     const int64_t so = (int64_t)shot * S.fstride;
@@ -918,29 +927,31 @@ __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields 
     // byte offset of (j-2, i0-2, kc-2) at plane j: operand (j+dj, i0+r, kc)
     // at vb + 8 + (dj+2)*SJ + (r+2)*SI
     uint32_t vb = (uint32_t)((int64_t)jb * g.sj + (int64_t)i0 * g.si + kc + IFOS_KOFF - 2) * 4u;
-    const uint32_t own = (uint32_t)(yc + 2) * SI;
-#define LB(r, dj) bload(r, vb + 8u, (uint32_t)((dj) + 2) * SJ + own)
-#define LBN(r, dj) bload_cp<CPN>(r, vb + 8u, (uint32_t)((dj) + 2) * SJ + own)
+    // own row: KW 64 in the scalar offset, else in the lane's (vo)
+    const uint32_t own = KW == 64 ? (uint32_t)(yc + 2) * SI : 2u * SI, ro = KW == 64 ? 0u : (uint32_t)yc * SI;
+#define LB(r, dj) bload(r, vb + ro + 8u, (uint32_t)((dj) + 2) * SJ + own)
+#define LBN(r, dj) bload_cp<CPN>(r, vb + ro + 8u, (uint32_t)((dj) + 2) * SJ + own)
     // halo words of the own row: lane l loads k0-2+l (lanes 0, 1), k0+64 and
     // k0+65 (lanes 62, 63); lanes 2-31 repeat lane 1's word and lanes 32-61
     // lane 62's (the load touches two lines).  Lanes 2-61 write theirs to
     // their own column, which the row write after it overwrites, so the 64
     // lanes write 64 different words.  hd is the word's byte offset from the
     // lane's own word (>= -4 (lane + 2): the sum vb + 8 + hd stays >= 0).
-    const int kh = lane < 2 ? k0 - 2 + lane : lane < 32 ? k0 - 1 : lane < 63 ? k0 + 64 : k0 + 65;
-    const int hcol = lane < 62 ? (lane < 2 ? lane : lane + 2) : lane + 4;
+    const int kh = lane < 2 ? k0 - 2 + lane : lane < KW / 2 ? k0 - 1 : lane < KW - 1 ? k0 + KW : k0 + KW + 1;
+    const int hcol = lane < KW - 2 ? (lane < 2 ? lane : lane + 2) : lane + 4;
     const uint32_t hd = (uint32_t)((min(kh, g.nz + 2) - kc) * 4);
-    // outside rows of this wavefront: e = min(y + n TI, 8) is (component e / 3,
-    // row i0 + orow[e]); the load row is clamped to nx+2.  The 9 rows take
-    // NH TI slots; the spare slots repeat row 8 (the same words, written with
-    // the same values), so no wavefront branches around a load or a write.
+    // outside rows of this wavefront: piece p = min(w + n TI, NS - 1) is row p %
+    // 3 of component p / 3, or (KW 32) rows 2 (p % 2) and 2 (p % 2) + 1 of
+    // component p / 2, the third row twice; the load row is clamped to nx+2.
+    // The spare slots repeat the last piece (the same words, written with the
+    // same values), so no wavefront branches around a load or a write.
     int oc[NH], orow[NH];
     uint32_t ooff[NH];
 #pragma unroll
     for (int n = 0; n < NH; ++n) {
-        const int e = min(y + n * TI, 8);
-        const int c = e < 3 ? 0 : (e < 6 ? 1 : 2), m = e - 3 * c;
-        const int r = c == 0 ? (m == 0 ? -2 : (m == 1 ? -1 : TI)) : (m == 0 ? -1 : (m == 1 ? TI : TI + 1));
+        const int p = min(w + n * TI, NS - 1);
+        const int c = KW == 64 ? p / 3 : p / 2, m = KW == 64 ? p - 3 * c : min(2 * (p & 1) + sub, 2);
+        const int r = c == 0 ? (m == 0 ? -2 : (m == 1 ? -1 : NR)) : (m == 0 ? -1 : (m == 1 ? NR : NR + 1));
         oc[n] = c;
         orow[n] = r;
         ooff[n] = (uint32_t)(min(i0 + r, g.nx + 2) - i0 + 2) * SI;
@@ -972,13 +983,13 @@ __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields 
             O.ts = LB(rtaus, D); O.tp = LB(rtaup, D);
             O.tsipjp = LB(rtsipjp, D); O.tsjpkp = LB(rtsjpkp, D); O.tsipkp = LB(rtsipkp, D);
         }
-        O.hk[0] = bload(rvx, vb + 8u + hd, pj + own);
-        O.hk[1] = bload(rvy, vb + 8u + hd, pj + own);
-        O.hk[2] = bload(rvz, vb + 8u + hd, pj + own);
+        O.hk[0] = bload(rvx, vb + ro + 8u + hd, pj + own);
+        O.hk[1] = bload(rvy, vb + ro + 8u + hd, pj + own);
+        O.hk[2] = bload(rvz, vb + ro + 8u + hd, pj + own);
 #pragma unroll
         for (int n = 0; n < NH; ++n) {
             const rsrc_t rc = oc[n] == 0 ? rvx : (oc[n] == 1 ? rvy : rvz);
-            O.ho[n] = bload(rc, vb + 8u, pj + ooff[n]);
+            O.ho[n] = KW == 64 ? bload(rc, vb + 8u, pj + ooff[n]) : bload(rc, vb + ooff[n] + 8u, pj);
         }
     };
 
@@ -999,7 +1010,7 @@ __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields 
         load_ops(nxt, 1);
         load_cell(cur, 0);
         const uint32_t q3 = (uint32_t)(min(j + 3, g.ny + 2) - j + 2) * SJ + own;
-        const float vx_n = bload(rvx, vb + 8u, q3), vz_n = bload(rvz, vb + 8u, q3), vy_n = LB(rvy, 2);
+        const float vx_n = bload(rvx, vb + ro + 8u, q3), vz_n = bload(rvz, vb + ro + 8u, q3), vy_n = LB(rvy, 2);
         // stage plane j: halo words first, then the row over them
         sh[p][0][y + 2][hcol] = cur.hk[0];
         sh[p][1][y + 2][hcol] = cur.hk[1];
@@ -1011,9 +1022,9 @@ __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields 
         for (int n = 0; n < NH; ++n) sh[p][oc[n]][orow[n] + 2][lane + 2] = cur.ho[n];
         __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (act) {
-            const float(*X)[68] = sh[p][0];
-            const float(*Y)[68] = sh[p][1];
-            const float(*Z)[68] = sh[p][2];
+            const float(*X)[KW + 4] = sh[p][0];
+            const float(*Y)[KW + 4] = sh[p][1];
+            const float(*Z)[KW + 4] = sh[p][2];
             const int c0 = lane + 2, r0_ = y + 2;
             PsiCell pc;
             const int hy = CPML ? slab_h(j, g.ny, g.fw, !g.free_surf) : 0;
@@ -1056,10 +1067,10 @@ __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields 
                 } else {
                     const uint32_t sto = 2u * SJ + own;
                     auto ldm = [&](int l, int n) {
-                        return bload_cp<CPN>(rr[n], vb + 8u, sto + (uint32_t)l * g.fbytes);
+                        return bload_cp<CPN>(rr[n], vb + ro + 8u, sto + (uint32_t)l * g.fbytes);
                     };
                     auto stm = [&](int l, int n, float v) {
-                        bstore_cp<CPN>(v, rr[n], vb + 8u, sto + (uint32_t)l * g.fbytes);
+                        bstore_cp<CPN>(v, rr[n], vb + ro + 8u, sto + (uint32_t)l * g.fbytes);
                     };
                     stress_visco_n(DT, V, cur.pi, cur.u, cur.uipjp, cur.ujpkp, cur.uipkp, cur.ts, cur.tp,
                                    cur.tsipjp, cur.tsjpkp, cur.tsipkp, vxyyx, vyzzy, vxzzx, vxxyyzz, vyyzz, vxxzz,
@@ -1067,15 +1078,15 @@ __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields 
                 }
             }
             const uint32_t st = 2u * SJ + own;
-            bstore_cp<CPN>(sn[3], rsxy, vb + 8u, st);
-            bstore_cp<CPN>(sn[4], rsyz, vb + 8u, st);
-            bstore_cp<CPN>(sn[5], rsxz, vb + 8u, st);
-            bstore_cp<CPN>(sn[0], rsxx, vb + 8u, st);
-            bstore_cp<CPN>(sn[1], rsyy, vb + 8u, st);
-            bstore_cp<CPN>(sn[2], rszz, vb + 8u, st);
+            bstore_cp<CPN>(sn[3], rsxy, vb + ro + 8u, st);
+            bstore_cp<CPN>(sn[4], rsyz, vb + ro + 8u, st);
+            bstore_cp<CPN>(sn[5], rsxz, vb + ro + 8u, st);
+            bstore_cp<CPN>(sn[0], rsxx, vb + ro + 8u, st);
+            bstore_cp<CPN>(sn[1], rsyy, vb + ro + 8u, st);
+            bstore_cp<CPN>(sn[2], rszz, vb + ro + 8u, st);
             if (VM) {
 #pragma unroll
-                for (int n = 0; n < 6; ++n) bstore_cp<CPN>(rn[n], rr[n], vb + 8u, st);
+                for (int n = 0; n < 6; ++n) bstore_cp<CPN>(rn[n], rr[n], vb + ro + 8u, st);
             }
         }
         vx_m1 = vx_0; vx_0 = vx_p1; vx_p1 = vx_p2; vx_p2 = vx_n;
@@ -1417,20 +1428,22 @@ static Box region_box(const ifos_geom *g, int region)
     return B;
 }
 
+// cells of a row of nk padded to pieces of w lanes
+static int padded(int nk, int w) { return (nk + w - 1) / w * w; }
+
 // lanes of a wavefront along k (the others take further i-rows): a row of nk
 // cells in pieces of 64, or of 32 (one 128-byte line; two rows a wavefront)
 // where that leaves fewer lanes idle; rows below 64 cells whole
-static int row_lanes(int nk, bool lds)
+static int row_lanes(int nk)
 {
-    const auto padded = [&](int w) { return (nk + w - 1) / w * w; };
     if (nk < 64) return nk;
-    return !lds && padded(32) < padded(64) ? 32 : 64;
+    return padded(nk, 32) < padded(nk, 64) ? 32 : 64;
 }
 
 // tiles of boxes for TI i-rows per block and at most jc j-planes (<= 0: 64);
-// lds: for the LDS-staged marches
+// lds: for the LDS-staged marches with rows of that many lanes
 static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, int ns, int group, int kb = 1, int sb = 1,
-                         bool lds = false)
+                         int lds = 0)
 {
     MTiles T = {};
     T.lds = lds;
@@ -1446,7 +1459,7 @@ static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, int ns, int g
         const Box &B = boxes[q];
         if (B.i1 < B.i0 || B.j1 < B.j0 || B.k1 < B.k0) continue;
         const int nk = B.k1 - B.k0 + 1, ni = B.i1 - B.i0 + 1;
-        const int kw = row_lanes(nk, lds), rpw = 64 / kw;
+        const int kw = lds ? lds : row_lanes(nk), rpw = 64 / kw;
         const int nwk = (nk + kw - 1) / kw;  // wavefront columns along k
         int kbq = kb < 1 ? 1 : kb;
         while (kbq > 1 && (kbq > nwk || (ti / sbq) % kbq)) kbq /= 2;
@@ -1519,38 +1532,54 @@ static bool step_cached(const DevGeom &g, int ns, int L)
     return 4.0 * g.nx * g.ny * g.nz * ((9.0 + 6.0 * L) * ns + (L ? 13.0 : 8.0)) <= 256e6;
 }
 
-// The march of a launch.  The LDS-staged marches take rows of 64 lanes (every
-// box at least 64 cells deep in k), one k column and one shot per workgroup,
-// and TI >= 2.  They save cache misses, so in a default shape they are left
-// out where a step is cached, and where rows of 64 leave many lanes idle: the
-// register marches with two rows of 32 per wavefront then win.  v / s, us,
-// LDS -> register, whole-domain, both with the better cache policy: one shot
-// at 84^3 23.2 / 23.8 -> 17.3 / 17.9, 148^3 63 / 66 -> 47 / 59, 202 x 106 x 202
-// (rows 1.14 x longer in 64s) 90 / 96 -> 75 / 88; 4 shots at 84^3 59 / 57 ->
-// 41 / 45, 3 at 148^3 (1.2 x) 195 / 194 -> 168 / 190; but 4 at 276^3 (1.11 x)
-// 1208 / 1452 -> 1222 / 1550, 536 x 280 x 536 (1.06 x) 1230 / 1540 -> 1275 /
-// 1595.  A shape that a caller or the autotuner set keeps its lds choice.
-static bool use_lds(const MarchCfg &c, const Box *boxes, int nb, const DevGeom &g, int ns, int kb, int sb, int L)
+// The march of a launch: 0 the register march, else the LDS-staged one with
+// rows of that many lanes.  The LDS marches take boxes at least 64 cells deep
+// in k, one k column and one shot per workgroup, and TI >= 2.  They save cache
+// misses, so a default shape leaves them out where a step is cached (one shot
+// at 84^3, v / s us: 23 / 24 against 17 / 18, 148^3 63 / 66 against 47 / 59).
+// Past that, rows of 32 where they leave fewer lanes idle; the stress march
+// only where they save more than 12 %, as two rows' halo words cost it more
+// cache lines than the velocity march, of whose six stresses three have them.
+// v / s us: register, 64, 32 -- 3 shots at 212^3 (rows 1.14 x longer in 64s)
+// 465 / 577, 517 / 601, 455 / 564; 202 x 106 x 202 (1.14) 88 / 100, 102 / 107,
+// 85 / 99; 4 at 276^3 (1.11) 1222 / 1547, 1209 / 1427, 1172 / 1459; 536 x 280
+// x 536 (1.06) 1264 / 1624, 1231 / 1520, 1217 / 1543.  A shape that a caller
+// or the autotuner set keeps its lds choice.
+static int use_lds(const MarchCfg &c, const Box *boxes, int nb, const DevGeom &g, int ns, int kb, int sb,
+                   bool velocity, int L)
 {
-    if (!c.lds || c.ti < 2 || kb > 1 || sb > 1) return false;
+    if (!c.lds || c.ti < 2 || kb > 1 || sb > 1 || (c.dflt && step_cached(g, ns, L))) return 0;
+    int kw = 64;
     for (int q = 0; q < nb; ++q) {
         const int nk = boxes[q].k1 - boxes[q].k0 + 1;
-        if (nk < 64) return false;
-        if (c.dflt && (nk + 63) / 64 * 64 > 1.12 * ((nk + 31) / 32 * 32)) return false;
+        if (nk < 64) return 0;
+        if (padded(nk, 64) > (velocity ? 1.0 : 1.12) * padded(nk, 32)) kw = 32;
     }
-    return !(c.dflt && step_cached(g, ns, L));
+    return kw;
+}
+
+// j-planes of a tile of the default shape, of which make_tiles takes fewer
+// for small launches: the 3-5 planes that neighbouring chunks both read come
+// from the Infinity Cache while the chunks in flight, one on each of 8 XCDs,
+// fit it: chunks of 8 there (4 shots at 276^3, v / s: 1136 / 1390 us against
+// 1172 / 1427 with 16 and 1180 / 1456 with 32), 16 past it (536 x 280 x 536:
+// 1217 / 1520 against 1275 / 1527 with 8 and 1223 / 1535 with 32)
+static int march_chunk(const MarchCfg &c, const DevGeom &g)
+{
+    if (!c.dflt) return c.jc;
+    return 8.0 * 8.0 * 12.0 * 4.0 * g.nx * g.nz <= 256e6 ? 8 : 16;
 }
 
 // the tiles of a launch of shape c over boxes; kb, sb: c's, or 1 for one shot
 static MTiles march_tiles(const MarchCfg &c, const Box *boxes, int nb, const DevGeom &g, int ns, int group, int kb,
                           int sb, bool velocity, int L = 0)
 {
-    const bool lds = use_lds(c, boxes, nb, g, ns, kb, sb, L);
-    MTiles T = make_tiles(boxes, nb, c.ti, c.jc, ns, group, kb, sb, lds);
+    const int lds = use_lds(c, boxes, nb, g, ns, kb, sb, velocity, L), jc = march_chunk(c, g);
+    MTiles T = make_tiles(boxes, nb, c.ti, jc, ns, group, kb, sb, lds);
     // half the rows per workgroup suit the velocity march with rows of 32
     // (3 shots at 148^3: 176 -> 168 us; the stress march: no difference)
     if (c.dflt && velocity && !lds && c.ti == 4 && T.nb == 1 && T.kw[0] == 32) {
-        T = make_tiles(boxes, nb, 2, c.jc, ns, group, kb, sb, false);
+        T = make_tiles(boxes, nb, 2, jc, ns, group, kb, sb);
         T.ti = 2;
     } else {
         T.ti = c.ti;
@@ -1573,7 +1602,10 @@ static void launch_v_one(const MarchMode &m, dim3 grid, const MTiles &T, const D
 {
     if constexpr (TI >= 2)
         if (T.lds) {
-            hipLaunchKernelGGL((k_v_lds<TI, CPML, SNAP, NT>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, N);
+            if (T.lds == 32)
+                hipLaunchKernelGGL((k_v_lds<TI, CPML, SNAP, NT, 32>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, N);
+            else
+                hipLaunchKernelGGL((k_v_lds<TI, CPML, SNAP, NT, 64>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, N);
             return;
         }
     if (m.pipe)
@@ -1614,7 +1646,10 @@ static void launch_s_one(const MarchMode &m, dim3 grid, const MTiles &T, const D
 {
     if constexpr (TI >= 2)
         if (T.lds) {
-            hipLaunchKernelGGL((k_s_lds<TI, CPML, VM, NT>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, V);
+            if (T.lds == 32)
+                hipLaunchKernelGGL((k_s_lds<TI, CPML, VM, NT, 32>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, V);
+            else
+                hipLaunchKernelGGL((k_s_lds<TI, CPML, VM, NT, 64>), grid, dim3(64, TI), 0, s, G, T, F, P, psi, S, V);
             return;
         }
     if (m.pipe)
