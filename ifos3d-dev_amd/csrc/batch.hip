@@ -1085,7 +1085,7 @@ static const MarchCfg k_candidates[] = {
     {2, 0, 0, 0, 1, 1, 1, 0},  {1, 0, 0, 0, 1, 1, 1, 0},  {4, 0, 0, 1, 1, 1, 1, 0}, {4, 32, 0, 0, 0, 1, 2, 0},
     {4, 32, 0, 0, 1, 1, 2, 0}, {8, 32, 0, 0, 0, 1, 2, 0}, {4, 32, 0, 0, 0, 1, 4, 0}, {2, 32, 0, 0, 1, 1, 2, 0},
     {4, 32, 0, 0, 0, 1, 1, 1}, {8, 32, 0, 0, 0, 1, 1, 1}, {2, 32, 0, 0, 0, 1, 1, 1}, {4, 0, 0, 0, 0, 1, 1, 1},
-    {8, 0, 0, 0, 0, 1, 1, 1},  {4, 64, 0, 0, 0, 1, 1, 1}, {8, 16, 0, 0, 0, 1, 1, 1}, {2, 0, 0, 0, 0, 1, 1, 1},
+    {8, 0, 0, 0, 0, 1, 1, 1},  {4, 16, 0, 0, 0, 1, 1, 1}, {8, 16, 0, 0, 0, 1, 1, 1}, {4, 8, 0, 0, 0, 1, 1, 1},
 };
 
 extern "C" int ifos_batch_autotune(ifos_batch *b, int ns, int reps, int *best_v, int *best_s, float *ms_v,
