@@ -99,6 +99,17 @@ def test_receiver_chain():
     assert ig.rec_chain(np.zeros((0, 3), np.int32)).shape == (0, 2)
 
 
+@pytest.mark.parametrize("ntr,cells", [(1, 1), (8, 1), (9, 200), (300, 40), (2000, 5000)])
+def test_receiver_chain_of_many(ntr, cells):
+    """against the definition, all pairs compared"""
+    import ifosgpu as ig
+    rng = np.random.default_rng(ntr)
+    rec = rng.integers(-3, 500, (cells, 3)).astype(np.int32)[rng.integers(0, cells, ntr)]
+    same = (rec[:, None] == rec[None]).all(-1)
+    want = [[int(not same[r, :r].any()), next((q for q in range(r + 1, ntr) if same[r, q]), -1)] for r in range(ntr)]
+    assert ig.rec_chain(rec).tolist() == want
+
+
 def test_entry_points_reject_bad_arguments_before_any_device_call():
     """argument checks of the SU I/O, grid-level and time-domain entry points
     return IFOS_EINVAL with a message and touch no device"""
