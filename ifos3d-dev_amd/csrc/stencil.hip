@@ -1098,17 +1098,8 @@ __global__ __launch_bounds__(64 * TI) void k_s_lds(DevGeom g, MTiles T, SFields 
 #undef LBN
 }
 // ---------------------------------------------------------------------------
-// gradient_F.c:79-139 and hess_F.c:28-192: one thread per cell, every shot
-// (or receiver-side set) and frequency in one launch, the three sums of the
-// cell in registers.  The terms are added in the reference's order (shots or
-// receivers outer, frequencies inner), so each cell sees the same sequence of
-// roundings as one pass per frequency, without reading and writing the sums
-// and the model (9 of 21 array passes) and forming two FP64 square roots for
-// each of them.  A workgroup covers 64 k x 4 i x 4 j cells, so that the i and
-// j neighbours, 20 of a field's 30 loads, are mostly its own rows and come
-// from L1, and its 16 wavefronts keep some 1900 loads in flight; workgroups
-// are numbered so that an XCD's stretch is contiguous.  The vector-memory
-// path bounds it (120 loads per cell and frequency).
+// gradient_F.c:79-139 and hess_F.c:28-192 in one launch over every shot (or
+// receiver-side set) and frequency, described at the kernel below.
 struct GradArgs {
     const float *f[12];  // forward Re x y z, Im x y z, adjoint (receiver side) Re, Im
     int64_t fouter, bouter;  // elements from one outer item's forward / adjoint fields to the next
@@ -1117,7 +1108,6 @@ struct GradArgs {
     float fd[IFOS_MAX_NF];   // 1 / (4 pi^2 f^2) (gradient_F.c:70-72); hess: 1 / (2 pi f) (hess_F.c:75-77)
     const float *rho, *pi, *u;
     float *g1, *g2, *g3;
-    uint32_t ntk, nti, total, per;
 };
 
 // the nine derivatives xx xy xz yx yy yz zx zy zz of three fields at a cell,
@@ -1147,55 +1137,222 @@ __device__ __forceinline__ Strain cell_strain(const DevGeom &g, rsrc_t fx, rsrc_
     return s;
 }
 
-constexpr int kGradTI = 2, kGradTJ = 4;
-
-template <bool HESS>
-__global__ __launch_bounds__(64 * kGradTI * kGradTJ) void k_grad_cells(DevGeom g, GradArgs A)
+// a field by its address in scalar registers and a 32-bit offset: half the
+// scalar registers of a descriptor, of which a dozen do not fit
+typedef const __attribute__((address_space(1))) char *gfield;
+__device__ __forceinline__ gfield field(const float *p) { return (gfield)(uintptr_t)p; }
+__device__ __forceinline__ float gload(gfield f, uint32_t off)
 {
-    const uint32_t L = (blockIdx.x & 7u) * A.per + (blockIdx.x >> 3);
-    if (L >= A.total) return;
-    const int k = (int)(L % A.ntk) * 64 + (int)threadIdx.x + 1;
-    const uint32_t t = L / A.ntk;
-    const int i = (int)(t % A.nti) * kGradTI + (int)threadIdx.y + 1;
-    const int j = (int)(t / A.nti) * kGradTJ + (int)threadIdx.z + 1;
-    if (k > g.nz || i > g.nx || j > g.ny) return;
-    const uint32_t SJ = (uint32_t)g.sj * 4u, SI = (uint32_t)g.si * 4u;
-    const uint32_t vo = (uint32_t)((int64_t)j * g.sj + (int64_t)i * g.si + k + IFOS_KOFF - 2) * 4u;
-    const int64_t c = at(g, j, i, k);
-    const float r = A.rho[c], p = A.pi[c], m = A.u[c];
-    float a1 = A.g1[c], a2 = A.g2[c], a3 = A.g3[c];
-    const double srp = HESS ? 0.0 : sqrt((double)(r * p)), sru = HESS ? 0.0 : sqrt((double)(r * m));
-    for (int o = 0; o < A.nouter; ++o)
-        for (int l = 0; l < A.nf; ++l) {
-            const int64_t of = o * A.fouter + l * A.fe, ob = o * A.bouter + l * A.fe;
-            rsrc_t rf[12];
+    return *(const __attribute__((address_space(1))) float *)(f + off);
+}
+
+// The strains of a plane of three fields from LDS, as k_s_lds stages it: the
+// workgroup's tile, and what a lane loads of it.
+template <int TI, int KW>
+struct StrainTile {
+    static constexpr int RPW = 64 / KW, NR = TI * RPW, RW = NR + 4;
+    static constexpr int NS = KW == 64 ? 9 : 6, NH = (NS + TI - 1) / TI;
+    struct Ops {
+        float n[3], hk[3], ho[NH];  // next queue entries; halo words; outside rows
+    };
+    struct Queue {
+        float x[3], y[3], z[3];  // x, z at j-1..j+1, y at j-2..j
+    };
+    struct Out {
+        float xx, yy, zz, xy, xz, yz, c[3];  // xy: the sum of both shear terms; c: the fields
+    };
+    typedef float Stage[3][RW][KW + 4];
+    int lane, y, k, i, jb, je, hcol, oc[NH], orow[NH];
+    bool act;
+    uint32_t SJ, vl, vh, vo[NH];  // offsets at plane jb - 2: own cell, halo word, outside rows
+
+    // false: no tile (the whole workgroup)
+    __device__ bool init(const DevGeom &g, const MTiles &T)
+    {
+        const int b = blockIdx.x;
+        int t = (b & 7) * T.per + (b >> 3);
+        if (t >= T.total || t >= T.start[1]) return false;
+        const Box R = T.b[0];
+        const int tk = t % T.ntk[0];
+        t /= T.ntk[0];
+        const int ti = t % T.nti[0], tj = t / T.nti[0];
+        lane = (int)threadIdx.x & (KW - 1);
+        const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+        const int sub = KW == 64 ? 0 : (int)threadIdx.x / KW;
+        y = w * RPW + sub;
+        const int k0 = R.k0 + tk * KW, i0 = R.i0 + ti * NR;
+        k = k0 + lane;
+        i = i0 + y;
+        jb = R.j0 + tj * T.jc;
+        je = min(jb + T.jc - 1, R.j1);
+        act = k <= R.k1 && i <= R.i1;
+        const int kc = min(k, g.nz + 2), yc = min(i, g.nx + 2) - i0;
+        const uint32_t SI = (uint32_t)g.si * 4u;
+        SJ = (uint32_t)g.sj * 4u;
+        const uint32_t v0 = (uint32_t)((int64_t)jb * g.sj + (int64_t)i0 * g.si + kc + IFOS_KOFF) * 4u;
+        vl = v0 + (uint32_t)(yc + 2) * SI;
+        const int kh = lane < 2 ? k0 - 2 + lane : lane < KW / 2 ? k0 - 1 : lane < KW - 1 ? k0 + KW : k0 + KW + 1;
+        hcol = lane < KW - 2 ? (lane < 2 ? lane : lane + 2) : lane + 4;
+        vh = vl + (uint32_t)((min(kh, g.nz + 2) - kc) * 4);
 #pragma unroll
-            for (int n = 0; n < 12; ++n) rf[n] = make_rsrc(A.f[n] + (n < 6 ? of : ob), g.fbytes);
-            const Strain F = cell_strain(g, rf[0], rf[1], rf[2], vo, SJ, SI),
-                         FI = cell_strain(g, rf[3], rf[4], rf[5], vo, SJ, SI),
-                         B = cell_strain(g, rf[6], rf[7], rf[8], vo, SJ, SI),
-                         BI = cell_strain(g, rf[9], rf[10], rf[11], vo, SJ, SI);
-            const float *f = F.d, *fi = FI.d, *bb = B.d, *bi = BI.d;
-            const float fd = A.fd[l];
+        for (int n = 0; n < NH; ++n) {
+            const int p = min(w + n * TI, NS - 1);
+            const int c = KW == 64 ? p / 3 : p / 2, m = KW == 64 ? p - 3 * c : min(2 * (p & 1) + sub, 2);
+            const int r = c == 0 ? (m == 0 ? -2 : (m == 1 ? -1 : NR)) : (m == 0 ? -1 : (m == 1 ? NR : NR + 1));
+            oc[n] = c;
+            orow[n] = r;
+            vo[n] = v0 + (uint32_t)(min(i0 + r, g.nx + 2) - i0 + 2) * SI;
+        }
+        return true;
+    }
+    // planes from jb - 2 to j + d, in bytes
+    __device__ uint32_t plane(int j, int d) const { return (uint32_t)(j + d - jb + 2) * SJ; }
+    __device__ void first(Queue &q, gfield fx, gfield fy, gfield fz) const
+    {
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            q.x[n] = gload(fx, vl + plane(jb, n - 1));
+            q.y[n] = gload(fy, vl + plane(jb, n - 2));
+            q.z[n] = gload(fz, vl + plane(jb, n - 1));
+        }
+    }
+    // operands of plane j
+    __device__ void load(Ops &O, gfield fx, gfield fy, gfield fz, int j) const
+    {
+        const uint32_t p0 = plane(j, 0);
+        // (opaque, so that each block's loads see a 32-bit offset)
+        uint32_t l1 = vl + plane(j, 1), l2 = vl + plane(j, 2), h = vh + p0;
+        __asm__ volatile("" : "+v"(l1), "+v"(l2), "+v"(h));
+        O.n[0] = gload(fx, l2);
+        O.n[1] = gload(fy, l1);
+        O.n[2] = gload(fz, l2);
+        O.hk[0] = gload(fx, h);
+        O.hk[1] = gload(fy, h);
+        O.hk[2] = gload(fz, h);
+#pragma unroll
+        for (int n = 0; n < NH; ++n) {
+            uint32_t r = vo[n] + p0;
+            __asm__ volatile("" : "+v"(r));
+            O.ho[n] = gload(oc[n] == 0 ? fx : (oc[n] == 1 ? fy : fz), r);
+        }
+    }
+    __device__ void stage(Stage &sh, const Ops &O, const Queue &q) const
+    {
+#pragma unroll
+        for (int n = 0; n < 3; ++n) sh[n][y + 2][hcol] = O.hk[n];
+        sh[0][y + 2][lane + 2] = q.x[1];
+        sh[1][y + 2][lane + 2] = q.y[2];
+        sh[2][y + 2][lane + 2] = q.z[1];
+#pragma unroll
+        for (int n = 0; n < NH; ++n) sh[oc[n]][orow[n] + 2][lane + 2] = O.ho[n];
+    }
+    // of the staged plane; moves the queue to the next plane
+    __device__ Out strain(const DevGeom &g, const Stage &sh, Queue &q, const float (&n)[3]) const
+    {
+        const float b1 = g.b1, b2 = g.b2;
+        const float(*X)[KW + 4] = sh[0], (*Y)[KW + 4] = sh[1], (*Z)[KW + 4] = sh[2];
+        const int c0 = lane + 2, r0 = y + 2;
+        const float x = q.x[1], yv = q.y[2], z = q.z[1];
+        float xx = D4B(b1, b2, X[r0 - 2][c0], X[r0 - 1][c0], x, X[r0 + 1][c0]);
+        float xy = D4F(b1, b2, q.x[0], x, q.x[2], n[0]);
+        float xz = D4F(b1, b2, X[r0][c0 - 1], x, X[r0][c0 + 1], X[r0][c0 + 2]);
+        float yx = D4F(b1, b2, Y[r0 - 1][c0], yv, Y[r0 + 1][c0], Y[r0 + 2][c0]);
+        float yy = D4B(b1, b2, q.y[0], q.y[1], yv, n[1]);
+        float yz = D4F(b1, b2, Y[r0][c0 - 1], yv, Y[r0][c0 + 1], Y[r0][c0 + 2]);
+        float zx = D4F(b1, b2, Z[r0 - 1][c0], z, Z[r0 + 1][c0], Z[r0 + 2][c0]);
+        float zy = D4F(b1, b2, q.z[0], z, q.z[2], n[2]);
+        float zz = D4B(b1, b2, Z[r0][c0 - 2], Z[r0][c0 - 1], z, Z[r0][c0 + 1]);
+        div_spacing(g, xx, xy, xz, yx, yy, yz, zx, zy, zz);
+        q.x[0] = q.x[1]; q.x[1] = q.x[2]; q.x[2] = n[0];
+        q.y[0] = q.y[1]; q.y[1] = q.y[2]; q.y[2] = n[1];
+        q.z[0] = q.z[1]; q.z[1] = q.z[2]; q.z[2] = n[2];
+        return Out{xx, yy, zz, xy + yx, xz + zx, yz + zy, {x, yv, z}};
+    }
+};
+
+// A workgroup takes a tile of kGradTJ planes through all shots and frequencies
+// (outer, inner: the reference's order, so each cell sees the same sequence of
+// roundings as one pass per frequency), its three sums in LDS meanwhile; along
+// the planes it marches as k_s_lds does, the four strains of a plane (forward
+// and adjoint, Re and Im) one after the other through two LDS stages, each
+// strain's operands loaded a plane ahead.  A thread per cell that loads its
+// 120 neighbours itself misses L1 three times as often and waits.
+// 276^3, 6 frequencies, gradient / Hessian: 4.43 / 4.30 -> 3.07 / 3.22 ms
+// (2 GB/ms of fields at least once).  Bound by the vector units (420
+// instructions a cell and frequency, 40 of them FP64) and by the lines at the
+// tile's edges, which neighbouring tiles read at another time.  Rows of 64:
+// 3.49 / 3.49, 16 planes a tile 3.30 / 3.36, 12 wavefronts 3.63 / 3.65 ms.
+constexpr int kGradTI = 4, kGradTJ = 8;
+
+template <bool HESS, int KW>
+__global__ __launch_bounds__(64 * kGradTI) void k_grad_lds(DevGeom g, MTiles T, GradArgs A)
+{
+    typedef StrainTile<kGradTI, KW> Tile;
+    __shared__ typename Tile::Stage sh[2];
+    __shared__ float sums[3][kGradTJ][64 * kGradTI];
+    Tile t;
+    if (!t.init(g, T)) return;  // whole workgroup
+    const int tid = (int)(threadIdx.y * 64 + threadIdx.x);
+    const int64_t cb = at(g, t.jb, t.act ? t.i : 1, t.act ? t.k : 1);
+    for (int j = t.jb; j <= t.je; ++j) {
+        const int64_t c = cb + (j - t.jb) * g.sj;
+        sums[0][j - t.jb][tid] = A.g1[c];
+        sums[1][j - t.jb][tid] = A.g2[c];
+        sums[2][j - t.jb][tid] = A.g3[c];
+    }
+    const int items = A.nouter * A.nf;
+    for (int q = 0, o = 0, l = 0; q < items; ++q, l = l + 1 == A.nf ? 0 : l + 1, o += l == 0) {
+        const int64_t of = o * A.fouter + l * A.fe, ob = o * A.bouter + l * A.fe;
+        gfield rf[4][3];  // forward, adjoint Re; forward, adjoint Im
+#pragma unroll
+        for (int n = 0; n < 12; ++n)
+            rf[n / 3][n % 3] = field(A.f[n % 3 + 6 * (n / 3 % 2) + 3 * (n / 6)] + (n / 3 % 2 ? ob : of));
+        typename Tile::Queue Q[4];
+        typename Tile::Ops O[4];
+        typename Tile::Out S[4];
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            t.first(Q[n], rf[n][0], rf[n][1], rf[n][2]);
+            t.load(O[n], rf[n][0], rf[n][1], rf[n][2], t.jb);
+        }
+        const float fd = A.fd[l];
+        for (int j = t.jb; j <= t.je; ++j) {
+            const uint32_t co = t.vl + t.plane(j, 0);
+            const float r = gload(field(A.rho), co), p = gload(field(A.pi), co), m = gload(field(A.u), co);
+            // four stages in two buffers, one barrier each: a buffer is written
+            // again after the barrier of the stage between, which every
+            // wavefront reaches with its reads of it done
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                t.stage(sh[n & 1], O[n], Q[n]);
+                const float nx[3] = {O[n].n[0], O[n].n[1], O[n].n[2]};
+                // the next plane's (the last plane: its own again, unused)
+                t.load(O[n], rf[n][0], rf[n][1], rf[n][2], min(j + 1, t.je));
+                __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                S[n] = t.strain(g, sh[n & 1], Q[n], nx);
+            }
+            const typename Tile::Out &F = S[0], &B = S[1], &FI = S[2], &BI = S[3];
+            float a1 = sums[0][j - t.jb][tid], a2 = sums[1][j - t.jb][tid], a3 = sums[2][j - t.jb][tid];
+            const double srp = HESS ? 0.0 : sqrt((double)(r * p)), sru = HESS ? 0.0 : sqrt((double)(r * m));
             if (HESS) {
                 // hess_F.c:135-182
-                const float fdiv = f[0] + f[4] + f[8], fidiv = fi[0] + fi[4] + fi[8];
-                const float bdiv = bb[0] + bb[4] + bb[8], bidiv = bi[0] + bi[4] + bi[8];
+                const float fdiv = F.xx + F.yy + F.zz, fidiv = FI.xx + FI.yy + FI.zz;
+                const float bdiv = B.xx + B.yy + B.zz, bidiv = BI.xx + BI.yy + BI.zz;
                 float relam = fidiv * bdiv + fdiv * bidiv;
                 relam = fd * relam;
                 float imlam = fidiv * bidiv - fdiv * bdiv;
                 imlam = fd * imlam;
-                float remu = 2.0f * fi[0] * bb[0] + 2.0f * fi[4] * bb[4] + 2.0f * fi[8] * bb[8] +
-                             2.0f * f[0] * bi[0] + 2.0f * f[4] * bi[4] + 2.0f * f[8] * bi[8] +
-                             (fi[1] + fi[3]) * (bb[1] + bb[3]) + (f[1] + f[3]) * (bi[1] + bi[3]) +
-                             (fi[2] + fi[6]) * (bb[2] + bb[6]) + (f[2] + f[6]) * (bi[2] + bi[6]) +
-                             (fi[5] + fi[7]) * (bb[5] + bb[7]) + (f[5] + f[7]) * (bi[5] + bi[7]);
+                float remu = 2.0f * FI.xx * B.xx + 2.0f * FI.yy * B.yy + 2.0f * FI.zz * B.zz +
+                             2.0f * F.xx * BI.xx + 2.0f * F.yy * BI.yy + 2.0f * F.zz * BI.zz +
+                             FI.xy * B.xy + F.xy * BI.xy +
+                             FI.xz * B.xz + F.xz * BI.xz +
+                             FI.yz * B.yz + F.yz * BI.yz;
                 remu = fd * remu;
-                float immu = 2.0f * fi[0] * bi[0] + 2.0f * fi[4] * bi[4] + 2.0f * fi[8] * bi[8] -
-                             2.0f * f[0] * bb[0] - 2.0f * f[4] * bb[4] - 2.0f * f[8] * bb[8] +
-                             (fi[1] + fi[3]) * (bi[1] + bi[3]) - (f[1] + f[3]) * (bb[1] + bb[3]) +
-                             (fi[2] + fi[6]) * (bi[2] + bi[6]) - (f[2] + f[6]) * (bb[2] + bb[6]) +
-                             (fi[5] + fi[7]) * (bi[5] + bi[7]) - (f[5] + f[7]) * (bb[5] + bb[7]);
+                float immu = 2.0f * FI.xx * BI.xx + 2.0f * FI.yy * BI.yy + 2.0f * FI.zz * BI.zz -
+                             2.0f * F.xx * B.xx - 2.0f * F.yy * B.yy - 2.0f * F.zz * B.zz +
+                             FI.xy * BI.xy - F.xy * B.xy +
+                             FI.xz * BI.xz - F.xz * B.xz +
+                             FI.yz * BI.yz - F.yz * B.yz;
                 immu = fd * immu;
                 const float rerho = (F.c[0] * B.c[0] + F.c[1] * B.c[1] + F.c[2] * B.c[2]) -
                                     (FI.c[0] * BI.c[0] + FI.c[1] * BI.c[1] + FI.c[2] * BI.c[2]);
@@ -1209,14 +1366,14 @@ __global__ __launch_bounds__(64 * kGradTI * kGradTJ) void k_grad_cells(DevGeom g
                 a3 += rerho1 * rerho1 + imrho1 * imrho1;
             } else {
                 // gradient_F.c:122-139
-                float gl = (f[0] + f[4] + f[8]) * (bb[0] + bb[4] + bb[8]) +
-                           (fi[0] + fi[4] + fi[8]) * (bi[0] + bi[4] + bi[8]);
+                float gl = (F.xx + F.yy + F.zz) * (B.xx + B.yy + B.zz) +
+                           (FI.xx + FI.yy + FI.zz) * (BI.xx + BI.yy + BI.zz);
                 gl = -gl * fd;
-                float gm = 2.0f * f[0] * bb[0] + 2.0f * f[4] * bb[4] + 2.0f * f[8] * bb[8] + 2.0f * fi[0] * bi[0] +
-                           2.0f * fi[4] * bi[4] + 2.0f * fi[8] * bi[8] + (f[1] + f[3]) * (bb[1] + bb[3]) +
-                           (fi[1] + fi[3]) * (bi[1] + bi[3]) + (f[2] + f[6]) * (bb[2] + bb[6]) +
-                           (fi[2] + fi[6]) * (bi[2] + bi[6]) + (f[5] + f[7]) * (bb[5] + bb[7]) +
-                           (fi[5] + fi[7]) * (bi[5] + bi[7]);
+                float gm = 2.0f * F.xx * B.xx + 2.0f * F.yy * B.yy + 2.0f * F.zz * B.zz + 2.0f * FI.xx * BI.xx +
+                           2.0f * FI.yy * BI.yy + 2.0f * FI.zz * BI.zz + F.xy * B.xy +
+                           FI.xy * BI.xy + F.xz * B.xz +
+                           FI.xz * BI.xz + F.yz * B.yz +
+                           FI.yz * BI.yz;
                 gm = -gm * fd;
                 const float gr = (F.c[0] * B.c[0] + F.c[1] * B.c[1] + F.c[2] * B.c[2]) +
                                  (FI.c[0] * BI.c[0] + FI.c[1] * BI.c[1] + FI.c[2] * BI.c[2]);
@@ -1224,10 +1381,18 @@ __global__ __launch_bounds__(64 * kGradTI * kGradTJ) void k_grad_cells(DevGeom g
                 a2 = (float)(a2 + (-4 * sru * gl + 2 * sru * gm));
                 a3 += gr + m / r * gm + (p - 2.0f * m) / r * gl;
             }
+            sums[0][j - t.jb][tid] = a1;
+            sums[1][j - t.jb][tid] = a2;
+            sums[2][j - t.jb][tid] = a3;
         }
-    A.g1[c] = a1;
-    A.g2[c] = a2;
-    A.g3[c] = a3;
+    }
+    if (!t.act) return;
+    for (int j = t.jb; j <= t.je; ++j) {
+        const int64_t c = cb + (j - t.jb) * g.sj;
+        A.g1[c] = sums[0][j - t.jb][tid];
+        A.g2[c] = sums[1][j - t.jb][tid];
+        A.g3[c] = sums[2][j - t.jb][tid];
+    }
 }
 
 // one time sample of the time-domain gradient as a march over j: the
@@ -1959,17 +2124,23 @@ int launch_gradient(const ifos_geom *g, float *const d_Ff[6], float *const d_Fb[
     A.g1 = d_grad[0];
     A.g2 = d_grad[1];
     A.g3 = d_grad[2];
-    A.ntk = (uint32_t)((g->nz + 63) / 64);
-    A.nti = (uint32_t)((g->nx + kGradTI - 1) / kGradTI);
-    A.total = A.ntk * A.nti * (uint32_t)((g->ny + kGradTJ - 1) / kGradTJ);
-    A.per = (A.total + 7) / 8;
-    const dim3 grid(A.per * 8), block(64, kGradTI, kGradTJ);
+    const Box all = region_box(g, IFOS_REGION_ALL);
+    // rows of 32 where they leave fewer lanes idle, as in the marches
+    const int kw = padded(g->nz, 32) < padded(g->nz, 64) ? 32 : 64;
+    const MTiles T = make_tiles(&all, 1, kGradTI, kGradTJ, 1, 0, 1, 1, kw);
+    const dim3 grid((unsigned)T.per * 8), block(64, kGradTI);
     ProfScope ps_(IFOS_K_GRADIENT, s);
+    auto go = [&](auto h, auto w) {
+        hipLaunchKernelGGL((k_grad_lds<h(), w()>), grid, block, 0, s, G, T, A);
+    };
+    using std::integral_constant;
+    const integral_constant<int, 32> w32;
+    const integral_constant<int, 64> w64;
     if (hess)
-        hipLaunchKernelGGL((k_grad_cells<true>), grid, block, 0, s, G, A);
+        kw == 32 ? go(std::true_type(), w32) : go(std::true_type(), w64);
     else
-        hipLaunchKernelGGL((k_grad_cells<false>), grid, block, 0, s, G, A);
-    return hip_check(hipGetLastError(), "k_grad_cells");
+        kw == 32 ? go(std::false_type(), w32) : go(std::false_type(), w64);
+    return hip_check(hipGetLastError(), "k_grad_lds");
 }
 int launch_td_sample(const ifos_geom *g, const float *const uf[3], const float *const vf[3],
                      const float *const ub[3], const float *const vb[3], double w, double *const acc[3],
