@@ -136,7 +136,7 @@ struct Box {
 };
 struct BoxList {
     Box b[6];
-    int64_t start[7];  // cumulative cell counts
+    uint32_t start[7];  // cumulative cell counts (a field is below 2^30 elements)
     int n;
 };
 
