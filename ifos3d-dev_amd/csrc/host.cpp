@@ -650,9 +650,11 @@ static int probe_nan(ifos_ctx *c, const ShotState &S, int nt, hipStream_t st)
 }
 
 // the snapshot ring of the chunked DFT, allocated by the first shot that
-// samples: 16 snapshots (the 6 nf accumulators of a cell cross HBM once per
+// samples: 32 snapshots (the 6 nf accumulators of a cell cross HBM once per
 // chunk instead of once per sample: at 276^3 with 6 frequencies 0.5 ms per
-// sample against 1.4 ms), fewer where they would take more than a quarter of
+// sample against 1.4 ms; a shot of 100 steps and samples 193.8 ms with 16, 191.0
+// with 32, and with compensated sums of 8 frequencies on 202 x 106 x 202 100.0
+// and 94.8), fewer where they would take more than a quarter of
 // the free memory, none (one pass per sample) where 4 would, or where one
 // snapshot exceeds the 4 GiB of a buffer descriptor
 static int ring_alloc(ifos_ctx *c)
@@ -662,7 +664,7 @@ static int ring_alloc(ifos_ctx *c)
     const size_t snap = 3 * c->fe * 4;
     int rc = hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
     if (rc) return rc;
-    for (int ch = 16; ch >= 4; ch /= 2) {
+    for (int ch = 32; ch >= 4; ch /= 2) {
         if (snap >= 4294967295u || ch * snap > free_b / 4) continue;
         if (hipMalloc((void **)&c->ring, ch * snap) != hipSuccess) {
             (void)hipGetLastError();
