@@ -1110,33 +1110,6 @@ struct GradArgs {
     float *g1, *g2, *g3;
 };
 
-// the nine derivatives xx xy xz yx yy yz zx zy zz of three fields at a cell,
-// and the cell's values c
-struct Strain {
-    float d[9], c[3];
-};
-__device__ __forceinline__ Strain cell_strain(const DevGeom &g, rsrc_t fx, rsrc_t fy, rsrc_t fz, uint32_t vo,
-                                              uint32_t SJ, uint32_t SI)
-{
-    const float b1 = g.b1, b2 = g.b2;
-    Strain s;
-    const float x = LD(fx, 0, 0, 0), y = LD(fy, 0, 0, 0), z = LD(fz, 0, 0, 0);
-    s.d[0] = D4B(b1, b2, LD(fx, 0, -2, 0), LD(fx, 0, -1, 0), x, LD(fx, 0, 1, 0));
-    s.d[1] = D4F(b1, b2, LD(fx, -1, 0, 0), x, LD(fx, 1, 0, 0), LD(fx, 2, 0, 0));
-    s.d[2] = D4F(b1, b2, LD(fx, 0, 0, -1), x, LD(fx, 0, 0, 1), LD(fx, 0, 0, 2));
-    s.d[3] = D4F(b1, b2, LD(fy, 0, -1, 0), y, LD(fy, 0, 1, 0), LD(fy, 0, 2, 0));
-    s.d[4] = D4B(b1, b2, LD(fy, -2, 0, 0), LD(fy, -1, 0, 0), y, LD(fy, 1, 0, 0));
-    s.d[5] = D4F(b1, b2, LD(fy, 0, 0, -1), y, LD(fy, 0, 0, 1), LD(fy, 0, 0, 2));
-    s.d[6] = D4F(b1, b2, LD(fz, 0, -1, 0), z, LD(fz, 0, 1, 0), LD(fz, 0, 2, 0));
-    s.d[7] = D4F(b1, b2, LD(fz, -1, 0, 0), z, LD(fz, 1, 0, 0), LD(fz, 2, 0, 0));
-    s.d[8] = D4B(b1, b2, LD(fz, 0, 0, -2), LD(fz, 0, 0, -1), z, LD(fz, 0, 0, 1));
-    div_spacing(g, s.d[0], s.d[1], s.d[2], s.d[3], s.d[4], s.d[5], s.d[6], s.d[7], s.d[8]);
-    s.c[0] = x;
-    s.c[1] = y;
-    s.c[2] = z;
-    return s;
-}
-
 // a field by its address in scalar registers and a 32-bit offset: half the
 // scalar registers of a descriptor, of which a dozen do not fit
 typedef const __attribute__((address_space(1))) char *gfield;
@@ -1278,7 +1251,7 @@ struct StrainTile {
 // strain's operands loaded a plane ahead.  A thread per cell that loads its
 // 120 neighbours itself misses L1 three times as often and waits.
 // 276^3, 6 frequencies, gradient / Hessian: 4.43 / 4.30 -> 3.07 / 3.22 ms
-// (2 GB/ms of fields at least once).  Bound by the vector units (420
+// (6.1 GB of fields at least once).  Bound by the vector units (420
 // instructions a cell and frequency, 40 of them FP64) and by the lines at the
 // tile's edges, which neighbouring tiles read at another time.  Rows of 64:
 // 3.49 / 3.49, 16 planes a tile 3.30 / 3.36, 12 wavefronts 3.63 / 3.65 ms.
@@ -1395,43 +1368,65 @@ __global__ __launch_bounds__(64 * kGradTI) void k_grad_lds(DevGeom g, MTiles T, 
     }
 }
 
-// one time sample of the time-domain gradient as a march over j: the
+// one time sample of the time-domain gradient, marched as k_grad_lds: the
 // products of gradient_F.c:122-132 (displacement derivatives for lambda and
 // mu, the velocities for rho, no frequency factor), times w, added to acc.
 // f[0..2] the forward displacement, f[3..5] the forward velocity, f[6..8]
-// the adjoint displacement, f[9..11] the adjoint velocity.
+// the adjoint displacement, f[9..11] the adjoint velocity.  148^3: 93 -> 72 us
+// (a thread per row of cells that loads its 66 neighbours itself), 0.31 GB at
+// least once; bound by memory and, at this size, by the chain of 4 planes.
 struct TdArgs {
     const float *f[12];
     double *acc[3];  // lambda, mu and rho sums, one double per cell of the device layout
     double w;        // weight of the time sample (the time step)
 };
 
-template <int TI>
-__global__ __launch_bounds__(64 * TI) void k_td_march(DevGeom g, MTiles T, TdArgs A)
+template <int KW>
+__global__ __launch_bounds__(64 * kGradTI) void k_td_lds(DevGeom g, MTiles T, TdArgs A)
 {
-    int k, i, jb, je, shot;
-    Box R;
-    if (!decode_tile(T, TI, k, i, jb, je, shot, R)) return;
-    const uint32_t SJ = (uint32_t)g.sj * 4u, SI = (uint32_t)g.si * 4u;
-    uint32_t vo = (uint32_t)((int64_t)jb * g.sj + (int64_t)i * g.si + k + IFOS_KOFF - 2) * 4u;
-    rsrc_t rf[12];
+    typedef StrainTile<kGradTI, KW> Tile;
+    __shared__ typename Tile::Stage sh[2];
+    Tile t;
+    if (!t.init(g, T)) return;  // whole workgroup
+    gfield f[12];  // forward, adjoint displacement; forward, adjoint velocity
 #pragma unroll
-    for (int n = 0; n < 12; ++n) rf[n] = make_rsrc(A.f[n], g.fbytes);
-    for (int j = jb; j <= je; ++j, vo += SJ) {
-        const Strain F = cell_strain(g, rf[0], rf[1], rf[2], vo, SJ, SI),
-                     B = cell_strain(g, rf[6], rf[7], rf[8], vo, SJ, SI);
-        const float *f = F.d, *bb = B.d;
-        float gl = (f[0] + f[4] + f[8]) * (bb[0] + bb[4] + bb[8]);
+    for (int n = 0; n < 12; ++n) f[n] = field(A.f[n % 3 + 6 * (n / 3 % 2) + 3 * (n / 6)]);
+    typename Tile::Queue Q[2];
+    typename Tile::Ops O[2];
+    typename Tile::Out S[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+        t.first(Q[n], f[3 * n], f[3 * n + 1], f[3 * n + 2]);
+        t.load(O[n], f[3 * n], f[3 * n + 1], f[3 * n + 2], t.jb);
+    }
+    int64_t c = at(g, t.jb, t.act ? t.i : 1, t.act ? t.k : 1);
+    for (int j = t.jb; j <= t.je; ++j, c += g.sj) {
+        const uint32_t co = t.vl + t.plane(j, 0);
+        float v[6];
+#pragma unroll
+        for (int n = 0; n < 6; ++n) v[n] = gload(f[6 + n], co);
+        const double a0 = A.acc[0][c], a1 = A.acc[1][c], a2 = A.acc[2][c];
+        // a stage each, written again after the other's barrier (k_grad_lds)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            t.stage(sh[n], O[n], Q[n]);
+            const float nx[3] = {O[n].n[0], O[n].n[1], O[n].n[2]};
+            t.load(O[n], f[3 * n], f[3 * n + 1], f[3 * n + 2], min(j + 1, t.je));
+            __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            S[n] = t.strain(g, sh[n], Q[n], nx);
+        }
+        const typename Tile::Out &F = S[0], &B = S[1];
+        float gl = (F.xx + F.yy + F.zz) * (B.xx + B.yy + B.zz);
         gl = -gl;
-        float gm = 2.0f * f[0] * bb[0] + 2.0f * f[4] * bb[4] + 2.0f * f[8] * bb[8] + (f[1] + f[3]) * (bb[1] + bb[3]) +
-                   (f[2] + f[6]) * (bb[2] + bb[6]) + (f[5] + f[7]) * (bb[5] + bb[7]);
+        float gm = 2.0f * F.xx * B.xx + 2.0f * F.yy * B.yy + 2.0f * F.zz * B.zz + F.xy * B.xy + F.xz * B.xz +
+                   F.yz * B.yz;
         gm = -gm;
-        const float gr = LD(rf[3], 0, 0, 0) * LD(rf[9], 0, 0, 0) + LD(rf[4], 0, 0, 0) * LD(rf[10], 0, 0, 0) +
-                         LD(rf[5], 0, 0, 0) * LD(rf[11], 0, 0, 0);
-        const int64_t c = at(g, j, i, k);
-        A.acc[0][c] += (double)gl * A.w;
-        A.acc[1][c] += (double)gm * A.w;
-        A.acc[2][c] += (double)gr * A.w;
+        const float gr = v[0] * v[3] + v[1] * v[4] + v[2] * v[5];
+        if (t.act) {
+            A.acc[0][c] = a0 + (double)gl * A.w;
+            A.acc[1][c] = a1 + (double)gm * A.w;
+            A.acc[2][c] = a2 + (double)gr * A.w;
+        }
     }
 }
 
@@ -1653,8 +1648,7 @@ static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, int ns, int g
     // 4-6 extra planes a tile loads cost what the shorter chain gains).
     // One shot, v / s march, chunk 32 -> this rule: 84^3 97 / 102 -> 25 / 27
     // us (chunk 4), 148^3 117 / 130 -> 65 / 71 us (4), 276^3 404 / 485 ->
-    // 345 / 417 us (8).  4 shots at 276^3 and 536 x 280 x 536 have the
-    // workgroups and keep 32 planes (8-16 planes: 0-9 % slower there).
+    // 345 / 417 us (8).  Launches with the workgroups keep the caller's chunk.
     constexpr int64_t kTileMin = 8192;
     if (jc <= 0) jc = 64;
     while (jc > 4 && count(jc) * T.nsg < kTileMin) jc = jc / 2 > 4 ? jc / 2 : 4;
@@ -1671,10 +1665,8 @@ static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, int ns, int g
 }
 
 // default tile shape of the march kernels (i-rows per block, j chunk,
-// shot grouping, ..., LDS staging where every box row holds 64 k-lanes);
-// the batched path's autotuner overrides it per kernel.  On the 256^3
-// interior of a 276^3 grid the LDS marches with 32-plane chunks run 4-8 %
-// faster than the register marches over the whole j extent.
+// shot grouping, ..., LDS staging); use_lds and march_chunk fit it to the
+// grid, the batched path's autotuner overrides it per kernel
 static MarchCfg g_default_cfg = {4, 32, 0, 0, 0, 1, 1, 1, 1};
 
 // the shape checks of ifos_batch_set_tiles and ifos_set_plain_tiles
@@ -2159,11 +2151,16 @@ int launch_td_sample(const ifos_geom *g, const float *const uf[3], const float *
     }
     A.w = w;
     const Box all = region_box(g, IFOS_REGION_ALL);
-    const MTiles T = make_tiles(&all, 1, 4, 0, 1, 0);
+    const int kw = padded(g->nz, 32) < padded(g->nz, 64) ? 32 : 64;
+    const MTiles T = make_tiles(&all, 1, kGradTI, 16, 1, 0, 1, 1, kw);
+    const dim3 grid((unsigned)T.per * 8), block(64, kGradTI);
     { ProfScope ps_(IFOS_K_GRADIENT, s);
-    hipLaunchKernelGGL((k_td_march<4>), dim3((unsigned)(T.per * 8)), dim3(64, 4), 0, s, G, T, A);
+    if (kw == 32)
+        hipLaunchKernelGGL(k_td_lds<32>, grid, block, 0, s, G, T, A);
+    else
+        hipLaunchKernelGGL(k_td_lds<64>, grid, block, 0, s, G, T, A);
     }
-    return hip_check(hipGetLastError(), "k_td_march");
+    return hip_check(hipGetLastError(), "k_td_lds");
 }
 }  // namespace ifos
 

@@ -197,6 +197,33 @@ def test_gradient_and_hessian_tiles(nx, ny, nz):
         assert max_ulp(g.interior(G.from_dev(dev[n])), g.interior(ref[n])) == 0, f"grad{n + 1}"
 
 
+@pytest.mark.parametrize("nx,ny,nz", [(17, 19, 47), (19, 17, 64), (15, 16, 65)])
+def test_time_domain_gradient_tiles(nx, ny, nz):
+    """the sample kernel's tiles: rows of 64 (nz 47, 64) and 32 lanes, rows and
+    planes past a tile; bits, as the other test of this gradient"""
+    import ifosgpu as ig
+    import test_gpu_td as tt
+    g = small_grid(nx=nx, ny=ny, nz=nz, fw=4, nt=40)
+    _note(f"time-domain gradient tiles {nx}x{ny}x{nz}")
+    src, rec = (8, 8, nz // 2, 0.0, 60.0, 1.0, 1), np.array([[3 + 2 * n, 6, nz // 2 + n] for n in range(6)], np.int32)
+    o = Oracle("f32")
+    start, true = tt._models(g, 3)
+    obs = o.run_shot(g, *true, src, rec, [40.0], want_adjoint=False)["syn"]
+    ref = o.run_shot(g, *start, src, rec, [40.0], obs=obs, want_history=True)
+    want = [o.zeros(g) for _ in range(3)]
+    o.td_gradient(g, ref["vfwd"], ref["vadj"], *start, want)
+    G = tk._geom(ig, g)
+    ctx = ig.ShotContext(G, 1, len(rec))
+    ctx.set_cpml(4000.0, 50.0)
+    ctx.set_model(*[G.to_dev(a) for a in start])
+    grads = [G.empty() for _ in range(3)]
+    ctx.run_shot_td(src, rec, ig.DBuf((3, len(rec), g.nt + 1)), grads, ig.DBuf.from_numpy(np.stack(obs)))
+    ig.sync()
+    for n in range(3):
+        assert max_ulp(g.interior(G.from_dev(grads[n])), g.interior(want[n])) == 0, f"gradient {n + 1}"
+    ctx.close()
+
+
 @pytest.mark.parametrize("ntr", [1, 64, 200])
 def test_precon_points(ntr):
     """tapers of many points, most of them far from a cell; the bound of the
