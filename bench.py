@@ -40,35 +40,36 @@ sys.path.insert(0, os.path.join(ROOT, "ifos3d-dev_amd"))
 
 METRIC = "gradient shots/sec at 256³ (batched vs plain); Gcell-updates/s; % HBM peak"
 HBM_PEAK_GBS = 8000.0
-# kernel (as rocprofv3 names it) behind each launch-timer category; the
-# march kernels' template arguments follow the tile shape in use
+PLAIN_CHUNK = 32  # velocity snapshots a one-shot context folds into its DFT sums at once, memory permitting
 
 
-def kernel_names(path, nf, chunk, tiles=None):
+def kernel_names(w, S, chunk, tiles=None):
+    """the kernel, as rocprofv3 names it, behind each launch-timer category of
+    a whole-domain run of S shots (the march kernels' template arguments follow
+    the tile shape in use; cache policy and lanes per row as the library
+    chooses them)"""
+    nz, nt = w.nz, "true" if 4.0 * w.cells * (9 * S + 8) > 256e6 else "false"
     b = lambda x: "true" if x else "false"
-    if path == "plain":
-        # interior boxes at least 64 cells deep in k take the LDS marches
-        return {"v_interior": "ifos::k_v_lds<4, false, false>",
-                "s_interior": "ifos::k_s_lds<4, false, 0>",
-                "v_cpml": "ifos::k_v_slabs", "s_cpml": "ifos::k_s_slabs<0>",
-                "dft": f"ifos::k_dft_nf<{nf}>", "dft_kahan": f"ifos::k_dft_kahan_nf<{nf}>",
-                "gradient": "ifos::k_grad_march<4, 0>"}
-    tv, ts = tiles
+    tv, ts = tiles or ((4, 0, 0, 0, 0, 1, 1, 1),) * 2
     # the LDS-staged marches run when asked for with TI >= 2, one k column
     # and one shot per workgroup
-    lds = lambda t: len(t) > 7 and t[7] and t[0] >= 2 and t[5] <= 1 and t[6] == 1
-    return {"v_fused": f"ifos::k_v_lds<{tv[0]}, true, false>" if lds(tv)
-            else f"ifos::k_v_march<{tv[0]}, true, false, {b(tv[4])}>",
-            "s_fused": f"ifos::k_s_lds<{ts[0]}, true, 0>" if lds(ts)
-            else f"ifos::k_s_march<{ts[0]}, true, 0, {b(ts[4])}>",
+    lds = lambda t: len(t) > 7 and t[7] and t[0] >= 2 and t[5] <= 1 and t[6] == 1 and nz >= 64
+    pad = lambda n: -(-nz // n) * n
+    kw = lambda least: 32 if pad(64) > least * pad(32) else 64
+    ch = next(c for c in (4, 8, 16, 24, 32) if chunk <= c)
+    return {"v_fused": f"ifos::k_v_lds<{tv[0]}, true, false, {nt}, {kw(1.0)}>" if lds(tv)
+            else f"ifos::k_v_march<{tv[0]}, true, false, {b(tv[4])}, {nt}>",
+            "s_fused": f"ifos::k_s_lds<{ts[0]}, true, 0, {nt}, {kw(1.12)}>" if lds(ts)
+            else f"ifos::k_s_march<{ts[0]}, true, 0, {b(ts[4])}, {nt}>",
             "vs_fused": "ifos::k_vs_fused<16, false>",
-            "dft": f"ifos::k_dft_chunk<{nf}, {chunk}, false>", "dft_kahan": f"ifos::k_dft_chunk<{nf}, {chunk}, true>",
-            "gradient": "ifos::k_grad_march<4, 0>"}
+            "dft": f"ifos::k_dft_chunk<{ch}, false, false, true>",
+            "dft_kahan": f"ifos::k_dft_chunk<{ch}, true, false, true>",
+            "gradient": f"ifos::k_grad_lds<false, {kw(1.0)}>"}
 
 
 # tile shapes {TI, jc, group, split, pipe} used without the autotuner (its
 # usual choice on grad276)
-DEFAULT_TILES = ((4, 32, 0, 0, 0, 1, 1, 1), (4, 32, 0, 0, 0, 1, 1, 1))
+DEFAULT_TILES = ((4, 8, 0, 0, 0, 1, 1, 1), (4, 8, 0, 0, 0, 1, 1, 1))
 CATS = ["v_interior", "v_cpml", "v_fused", "s_interior", "s_cpml", "s_fused", "dft", "gradient", "sources", "other",
         "vs_fused"]
 
@@ -87,17 +88,20 @@ def slab_stats(w, free_surf=0):
     return bi, slab, axes
 
 
-def algorithmic_bytes(w, nf, kahan=False):
-    """bytes each kernel category must move per launch (FP32, each array
-    counted once per pass): v 60 B/cell, sigma 80 B/cell, +24 B per active
-    CPML axis, DFT 12 + 48*nf B/cell (x2 accumulators with Kahan),
-    gradient 48*nf + 36 B/cell"""
-    bi, slab, axes = slab_stats(w)
+def algorithmic_bytes(w, nf, kahan=False, ntast=0, visco=0):
+    """bytes each kernel category of the plain path must move per launch
+    (FP32, each array counted once per pass): v 60 B/cell, sigma 80 B/cell
+    (+ visco), +24 B per active CPML axis, at the sampling steps 12 B/cell of
+    velocity snapshot; a DFT chunk of c snapshots 12*c + 48*nf B/cell (x2
+    accumulators with Kahan), gradient 48*nf + 36 B/cell"""
+    _, _, axes = slab_stats(w)
     acc = 96 if kahan else 48
+    nsamp = w.nt // ntast if ntast else 0
+    nchunks = max(1, -(-nsamp // PLAIN_CHUNK))
     return {
-        "v_interior": 60 * bi, "v_cpml": 60 * slab + 24 * axes, "v_fused": 60 * w.cells + 24 * axes,
-        "s_interior": 80 * bi, "s_cpml": 80 * slab + 24 * axes, "s_fused": 80 * w.cells + 24 * axes,
-        "dft": (12 + acc * nf) * w.cells, "gradient": (48 * nf + 36) * w.cells,
+        "v_fused": (60 + 12 * nsamp / w.nt) * w.cells + 24 * axes,
+        "s_fused": (80 + visco) * w.cells + 24 * axes,
+        "dft": (12 * nsamp / nchunks + acc * nf) * w.cells, "gradient": (48 * nf + 36) * w.cells,
     }
 
 
@@ -503,12 +507,10 @@ def run_visco(args):
     b.close()
     log(f"batched gradient shot (one shot, Kahan): {res['batched'][0]:.2f} s")
     cells = w.cells
-    bi, slab, axes = slab_stats(w)
+    _, _, axes = slab_stats(w)
     vis = 68 + 48 * (L - 1)   # per cell of the stress update: tau arrays, the memory variables
-    ab_p = {"v_interior": 60 * bi, "v_cpml": 60 * slab + 24 * axes,
-            "s_interior": (80 + vis) * bi, "s_cpml": (80 + vis) * slab + 24 * axes,
-            "dft": (12 + 48 * nf) * cells, "gradient": (48 * nf + 36) * cells}
-    ab_k = dict(ab_p, dft=(12 + 96 * nf) * cells)
+    ab_p = algorithmic_bytes(w, nf, False, ntast, vis)
+    ab_k = algorithmic_bytes(w, nf, True, ntast, vis)
     # the batched DFT: a chunk of c snapshots, 12 B per cell each, folded
     # into 2 x 48 B per cell and frequency of Kahan accumulators
     nchunks = -(-(w.nt // ntast) // args.chunk)
@@ -518,7 +520,7 @@ def run_visco(args):
     out_k = {}
     for name, ab in (("compat", ab_p), ("kahan", ab_k), ("batched", ab_b)):
         el, prof = res[name]
-        dom = "s_interior" if name != "batched" else "s_fused"
+        dom = "s_fused"
         avg = prof[dom][0] / prof[dom][1]
         out_k[name] = {"gradient_shot_s": round(el, 3), "gcell_updates_per_s": round(cells * 2 * w.nt / el / 1e9, 3),
                        "stress_kernel_ms": round(avg, 4),
@@ -973,7 +975,7 @@ def main():
     if args.path == "batched":
         ab = algorithmic_bytes_batched(w, nf, S, args.chunk, ntast, kahan)
     else:
-        ab = algorithmic_bytes(w, nf, kahan)
+        ab = algorithmic_bytes(w, nf, kahan, ntast)
     roof = None
     kernels = None
     if res["prof"] is not None:
@@ -986,7 +988,8 @@ def main():
         if args.path == "batched":
             tune = batched.get("tune")
             tiles = (tuple(tune["v"]), tuple(tune["s"])) if tune else DEFAULT_TILES
-        kname = kernel_names(path_tag, nf, args.chunk, tiles).get("dft_kahan" if dom == "dft" and kahan else dom, "")
+        kname = kernel_names(w, S if tiles else 1, args.chunk if tiles else PLAIN_CHUNK, tiles).get(
+            "dft_kahan" if dom == "dft" and kahan else dom, "")
         if os.path.exists(tpath) and kname:
             import profsum
             traffic = profsum.read_traffic(tpath).get(kname)
@@ -1046,7 +1049,7 @@ def main():
         "td_kernels_ms": {k: round(v[0], 1) for k, v in td["prof"].items() if v[1]} if td else None,
         "roofline": roof,
         "kernels": kernels,
-        "plain_kernels": kernel_table(plain["prof"], algorithmic_bytes(w, nf, kahan))
+        "plain_kernels": kernel_table(plain["prof"], algorithmic_bytes(w, nf, kahan, ntast))
         if (plain and args.path == "batched") else None,
         "autotune": batched.get("tune") if batched else None,
         "copy_probe": copy,
