@@ -411,21 +411,21 @@ int ifos_levels_run(ifos_batch *const *lv, int nlev, const ifos_shot *const *sho
  * the next shot (1: shots fastest, <= 0: one shot after the other); split:
  * 1 = interior box and CPML slabs in separate launches, 0 = one CPML-aware
  * launch; pipe: 1 = the next plane's operands are loaded one plane ahead;
- * kb: the workgroup's wavefronts stand kb side by side along k (64 k each);
+ * kb: the workgroup's wavefronts stand kb side by side along k (64 or 32 k each);
  * sb: sb shots of one tile share a workgroup (and its model loads); the
  * remaining TI / (kb sb) wavefronts go along i (kb sb divides TI); lds: 1 =
- * the in-plane neighbours are staged in LDS (used where every row is 64 k
- * wide and kb = sb = 1, TI >= 2; elsewhere ignored).  NULL leaves a shape
- * unchanged.  A new batch starts with {4, 32, 0, 0, 0, 1, 1, 1} for both,
- * with lds left out while a step's working set fits the Infinity Cache or
- * rows of 64 k leave many lanes idle. */
+ * the in-plane neighbours are staged in LDS (used where every row is at least
+ * 64 k long and kb = sb = 1, TI >= 2; elsewhere ignored).  NULL leaves a shape
+ * unchanged.  A new batch starts with {4, 32, 0, 0, 0, 1, 1, 1} for both, but
+ * with jc 8 or 16 as the planes in flight fit the Infinity Cache or not, and
+ * with lds left out while a step's working set fits it. */
 #define IFOS_TILE_FIELDS 8
 int ifos_batch_set_tiles(ifos_batch *b, const int cfg_v[IFOS_TILE_FIELDS], const int cfg_s[IFOS_TILE_FIELDS]);
 /* the tile shape (same fields; group, split and sb have no effect) of the
  * one-shot march launches: ifos_update_v / ifos_update_s(_visco) on the
  * interior or the whole domain, the shot contexts and the drop-in.
- * Process-wide, default {4, 32, 0, 0, 0, 1, 1, 1}; set it between launches,
- * not while another thread launches. */
+ * Process-wide, default {4, 32, 0, 0, 0, 1, 1, 1} with jc and lds as a new
+ * batch's; set it between launches, not while another thread launches. */
 int ifos_set_plain_tiles(const int cfg[IFOS_TILE_FIELDS]);
 int ifos_get_plain_tiles(int cfg[IFOS_TILE_FIELDS]);
 /* the autotuner's candidate shapes (IFOS_TILE_FIELDS ints each, at most
