@@ -97,22 +97,32 @@ __global__ __launch_bounds__(256) void k_badjoint(DevGeom g, BFields F, const in
     const int s = blockIdx.y;
     if (r >= ntr) return;
     const int64_t rs = (int64_t)s * ntr;
-    if (!chain[2 * (rs + r)]) return;
-    const int cls = rcls[rs + r];
-    if (before && !cls) return;
-    const int *p = rec + 3 * (rs + r);
-    const int64_t c = at(g, p[1], p[0], p[2]);
-    const int64_t so = (int64_t)s * F.fstride;
     const int64_t comp = (int64_t)ntr * ldadj;
     const float *a = adj + (int64_t)s * 3 * comp;
+    // the receiver's indices and its own samples in one wait: a launch this
+    // small costs its chain of dependent loads (with a wait before each branch,
+    // and the source behind the first receivers in k_bpoints, a shot of 600
+    // steps at 84^3 with 32 receivers took 49.4 ms, now 48.5)
+    const int64_t o = (int64_t)r * ldadj + nt;
+    int first = chain[2 * (rs + r)], next = chain[2 * (rs + r) + 1], cls = rcls[rs + r];
+    int p0 = rec[3 * (rs + r)], p1 = rec[3 * (rs + r) + 1], p2 = rec[3 * (rs + r) + 2];
+    float ax = a[o], ay = a[comp + o], az = a[2 * comp + o];
+    __asm__ volatile("" : "+v"(first), "+v"(next), "+v"(cls), "+v"(p0), "+v"(p1), "+v"(p2), "+v"(ax), "+v"(ay), "+v"(az));
+    if (!first || (before && !cls)) return;
+    const int64_t c = at(g, p1, p0, p2);
+    const int64_t so = (int64_t)s * F.fstride;
     float x = F.vx[so + c], y = F.vy[so + c], z = F.vz[so + c];
-    for (int times = before || cls ? 1 : 2; times > 0; --times)
-        for (int q = r; q >= 0 && q < ntr; q = chain[2 * (rs + q) + 1]) {
-            const int64_t o = (int64_t)q * ldadj + nt;
-            x += a[o];
-            z += a[2 * comp + o];
-            y += a[comp + o];
+    for (int times = before || cls ? 1 : 2; times > 0; --times) {
+        x += ax;
+        z += az;
+        y += ay;
+        for (int q = next; q >= 0 && q < ntr; q = chain[2 * (rs + q) + 1]) {
+            const int64_t oq = (int64_t)q * ldadj + nt;
+            x += a[oq];
+            z += a[2 * comp + oq];
+            y += a[comp + oq];
         }
+    }
     F.vx[so + c] = x;
     F.vy[so + c] = y;
     F.vz[so + c] = z;
@@ -125,8 +135,9 @@ __global__ __launch_bounds__(256) void k_badjoint(DevGeom g, BFields F, const in
     }
 }
 
-// explosive sources (psource.c:26-54, the first thread of each shot, sources
-// in order) and seismograms (seismo_ssg.c:51-53, thread per receiver and
+// explosive sources (psource.c:26-54, one thread of each shot, sources in
+// order; of the second wavefront, so that they do not wait for the first
+// receivers) and seismograms (seismo_ssg.c:51-53, thread per receiver and
 // shot; sec [S][3][ntr][ldsec], or null) in one launch: the one writes
 // stresses, the other reads velocities
 __global__ __launch_bounds__(256) void k_bpoints(DevGeom g, BFields F, const int *src, const float *sig, int nsrc,
@@ -145,7 +156,7 @@ __global__ __launch_bounds__(256) void k_bpoints(DevGeom g, BFields F, const int
         o[comp] = F.vy[c];
         o[2 * comp] = F.vz[c];
     }
-    if (r != 0) return;
+    if (r != 64) return;  // workgroups have 256 threads
     float amp = 0.0f;
     const double den = 2.0 * g.dx * g.dy * g.dz;
     for (int l = 0; l < nsrc; ++l) {
