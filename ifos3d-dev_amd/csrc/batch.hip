@@ -317,7 +317,7 @@ static int balloc(ifos_batch *b, void **p, size_t bytes)
         return IFOS_ENOMEM;
     }
     b->allocs.push_back(*p);
-    return hip_check(hipMemset(*p, 0, bytes), "hipMemset");
+    return zero_new(*p, bytes);
 }
 
 static void drop_graphs(ifos_batch *b)

@@ -74,6 +74,12 @@ DevGeom make_dev_geom(const ifos_geom *g)
     return d;
 }
 
+int zero_new(void *p, size_t bytes)
+{
+    const int rc = hip_check(hipMemset(p, 0, bytes), "hipMemset");
+    return rc ? rc : hip_check(hipStreamSynchronize(nullptr), "hipMemset");
+}
+
 }  // namespace ifos
 
 using namespace ifos;
@@ -383,8 +389,7 @@ static int dalloc(ifos_ctx *c, void **p, size_t bytes)
         return IFOS_ENOMEM;
     }
     c->allocs.push_back(*p);
-    e = hipMemset(*p, 0, bytes);
-    return hip_check(e, "hipMemset");
+    return zero_new(*p, bytes);
 }
 
 extern "C" int ifos_ctx_destroy(ifos_ctx *c)
@@ -896,7 +901,7 @@ static int td_alloc(ifos_ctx *c, int K)
     if (!rc) rc = td_alloc_state(c, T, T->work);
     // (the marches write the snapshots' cells of [1..N]^3 only: halos stay 0)
     if (!rc) rc = td_alloc_one(T, (void **)&T->seg, 3 * (size_t)K * c->fe * 4);
-    if (!rc) rc = hip_check(hipMemset(T->seg, 0, 3 * (size_t)K * c->fe * 4), "hipMemset");
+    if (!rc) rc = zero_new(T->seg, 3 * (size_t)K * c->fe * 4);
     for (int n = 0; n < 3 && !rc; ++n) rc = td_alloc_one(T, (void **)&T->uf[n], c->fe * 4);
     for (int n = 0; n < 3 && !rc; ++n) rc = td_alloc_one(T, (void **)&T->ub[n], c->fe * 4);
     for (int n = 0; n < 3 && !rc; ++n) rc = td_alloc_one(T, (void **)&T->acc[n], c->fe * 8);
@@ -1036,7 +1041,7 @@ static int adj_one(AdjBufs *A, void **p, size_t bytes)
         return IFOS_ENOMEM;
     }
     A->allocs.push_back(*p);
-    return hip_check(hipMemset(*p, 0, bytes ? bytes : 4), "hipMemset");
+    return zero_new(*p, bytes ? bytes : 4);
 }
 
 static int adj_alloc(ifos_ctx *c, int K, int ntr)

@@ -299,10 +299,10 @@ extern "C" int ifos_lbfgs_create(const ifos_geom *g, int numpar, int bfgsnum, if
     const size_t sb = (4 + 2 * (size_t)bfgsnum) * sizeof(double);
     if (!rc) rc = hip_check(hipMalloc(&b->part, kRedBlocks * 3 * sizeof(double)), "lbfgs partials");
     if (!rc) rc = hip_check(hipMalloc(&b->state, sb), "lbfgs scalars");
-    if (!rc) rc = hip_check(hipMemset(b->state, 0, sb), "lbfgs zero");
+    if (!rc) rc = zero_new(b->state, sb);
     // ifos3d.c:373-379: fmatrix / vector zero-fill
-    if (!rc) rc = hip_check(hipMemset(b->grad, 0, vb * bfgsnum), "lbfgs zero");
-    if (!rc) rc = hip_check(hipMemset(b->mod, 0, vb * bfgsnum), "lbfgs zero");
+    if (!rc) rc = zero_new(b->grad, vb * bfgsnum);
+    if (!rc) rc = zero_new(b->mod, vb * bfgsnum);
     if (rc) {
         ifos_lbfgs_destroy(b);
         return rc;

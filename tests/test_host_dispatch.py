@@ -1,0 +1,93 @@
+"""The library's host code against a stand-in for the HIP runtime
+(tests/standin/standin.c): which memory it holds, which launches it makes and
+what it waits for, without a GPU.  The library's own objects are linked
+against the stand-in; kernels do not run.
+"""
+import ctypes as C
+import gc
+import glob
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+OBJ = os.path.join(os.path.dirname(HERE), "ifos3d-dev_amd", "lib", "obj")
+
+
+@pytest.fixture(scope="module")
+def standin(tmp_path_factory):
+    objs = [o for o in glob.glob(os.path.join(OBJ, "*.o")) if "dropin" not in o]
+    if not objs:
+        pytest.skip("the library's objects are not built here")
+    d = tmp_path_factory.mktemp("standin")
+    c, so = str(d / "standin.o"), str(d / "libifos3d_standin.so")
+    subprocess.run(["gcc", "-O1", "-fPIC", "-Wall", "-c", os.path.join(HERE, "standin", "standin.c"), "-o", c],
+                   check=True)
+    subprocess.run(["g++", "-shared", "-fPIC", "-Wl,-Bsymbolic", "-o", so, *objs, c], check=True)
+    return so
+
+
+@pytest.fixture
+def ig(standin):
+    """ifosgpu on the stand-in library, with its log as ig.lib().standin_log()"""
+    import ifosgpu
+    old = ifosgpu._lib, ifosgpu.LIBPATH
+    ifosgpu._lib, ifosgpu.LIBPATH = None, standin
+    lib = ifosgpu.lib()
+    lib.standin_log.restype = C.c_char_p
+    lib.standin_held.restype = C.c_size_t
+    lib.standin_clear()
+    try:
+        yield ifosgpu
+    finally:
+        gc.collect()
+        ifosgpu._lib, ifosgpu.LIBPATH = old
+
+
+def _log(ig):
+    return [line.split() for line in ig.lib().standin_log().decode().splitlines()]
+
+
+STREAM = C.c_void_p(0x5150)  # a stream other than the null stream
+SRC = (10, 11, 12, 0.0, 60.0, 1.0, 1)
+REC = np.array([[8, 9, 10], [12, 9, 14]], np.int32)
+
+
+def _context(ig, nt=12, nf=2):
+    G = ig.Geom(24, 22, 26, 5, 2.0, 2.0, 2.0, 2e-4, nt)
+    ctx = ig.ShotContext(G, nf, len(REC))
+    ctx.set_cpml(4000.0, 50.0)
+    ctx.set_freqs([40.0 + 20.0 * n for n in range(nf)], 10)
+    return G, ctx
+
+
+def test_new_memory_is_zeroed_before_another_stream_sees_it(ig):
+    """every fill of new memory on the null stream has been waited for before
+    the call returns, and before the call's next work on another stream"""
+    G, ctx = _context(ig)
+    obs, syn = ig.DBuf((3, len(REC), G.nt + 1)), ig.DBuf((3, len(REC), G.nt + 1))
+    grads, model = [G.empty() for _ in range(3)], [G.empty() for _ in range(3)]
+    eta = np.array([0.1, 0.2], np.float32)
+    calls = {
+        "context": lambda: ig.ShotContext(G, 2, 4),
+        "set_visco": lambda: ig.ShotContext(G, 1, 1).set_visco(model[0], model[1], eta, stream=STREAM),
+        "time-domain": lambda: ctx.run_shot_td(SRC, REC, syn, grads, obs, stream=STREAM),
+        "exact adjoint": lambda: ctx.run_shot_adj(SRC, REC, syn, grads, obs, stream=STREAM),
+        "batch": lambda: ig.BatchContext(G, 2, 2, 2).set_model(*model),
+        "l-bfgs": lambda: ig.Lbfgs(G, 2, 2),
+    }
+    for what, call in calls.items():
+        ig.lib().standin_clear()
+        keep = call()
+        pending, fills = None, 0
+        for line in _log(ig) + [["end"]]:
+            if line[0] == "fill":
+                pending, fills = line, fills + 1
+            elif line[0] == "wait" and line[1] in ("all", "(nil)"):
+                pending = None
+            elif line[0] in ("launch", "copy") and line[-1] != "(nil)" or line[0] == "end":
+                assert pending is None, f"{what}: {line} behind {pending}"
+        assert fills > 0, what
+        del keep
