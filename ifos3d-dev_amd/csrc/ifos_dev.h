@@ -141,8 +141,8 @@ struct BoxList {
 };
 
 // Tile shape of a march launch: TI i-rows per block (1, 2, 4, 8), jc
-// j-planes per tile at most (<= 0: 64; fewer where the launch would have
-// too few workgroups), `group` consecutive tiles per shot
+// j-planes per tile (<= 0: 64, or fewer where the launch would have too few
+// workgroups), `group` consecutive tiles per shot
 // before the next shot (1: shots fastest, <= 0: one shot after the other),
 // split: interior box and CPML slabs in separate launches; pipe: the next
 // plane's operands are loaded one iteration ahead (two planes in flight).

@@ -1602,10 +1602,11 @@ static int row_lanes(int nk)
     return padded(nk, 32) < padded(nk, 64) ? 32 : 64;
 }
 
-// tiles of boxes for TI i-rows per block and at most jc j-planes (<= 0: 64);
-// lds: for the LDS-staged marches with rows of that many lanes
-static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, int ns, int group, int kb = 1, int sb = 1,
-                         int lds = 0)
+// tiles of boxes for TI i-rows per block and jc j-planes, or with fit (and
+// for jc <= 0: 64) at most jc; lds: for the LDS-staged marches with rows of
+// that many lanes
+static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, bool fit, int ns, int group, int kb = 1,
+                         int sb = 1, int lds = 0)
 {
     MTiles T = {};
     T.lds = lds;
@@ -1648,10 +1649,14 @@ static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, int ns, int g
     // 4-6 extra planes a tile loads cost what the shorter chain gains).
     // One shot, v / s march, chunk 32 -> this rule: 84^3 97 / 102 -> 25 / 27
     // us (chunk 4), 148^3 117 / 130 -> 65 / 71 us (4), 276^3 404 / 485 ->
-    // 345 / 417 us (8).  Launches with the workgroups keep the caller's chunk.
+    // 345 / 417 us (8).  Launches with the workgroups keep the chunk, and so
+    // does a shape whose chunk a caller set.
     constexpr int64_t kTileMin = 8192;
-    if (jc <= 0) jc = 64;
-    while (jc > 4 && count(jc) * T.nsg < kTileMin) jc = jc / 2 > 4 ? jc / 2 : 4;
+    if (jc <= 0) {
+        jc = 64;
+        fit = true;
+    }
+    while (fit && jc > 4 && count(jc) * T.nsg < kTileMin) jc = jc / 2 > 4 ? jc / 2 : 4;
     T.jc = jc;
     for (int q = 0; q < T.nb; ++q)
         T.start[q + 1] = T.start[q] + T.ntk[q] * T.nti[q] * ((T.b[q].j1 - T.b[q].j0 + 1 + jc - 1) / jc);
@@ -1734,11 +1739,11 @@ static MTiles march_tiles(const MarchCfg &c, const Box *boxes, int nb, const Dev
                           int sb, bool velocity, int L = 0)
 {
     const int lds = use_lds(c, boxes, nb, g, ns, kb, sb, velocity, L), jc = march_chunk(c, g);
-    MTiles T = make_tiles(boxes, nb, c.ti, jc, ns, group, kb, sb, lds);
+    MTiles T = make_tiles(boxes, nb, c.ti, jc, c.dflt, ns, group, kb, sb, lds);
     // half the rows per workgroup suit the velocity march with rows of 32
     // (3 shots at 148^3: 176 -> 168 us; the stress march: no difference)
     if (c.dflt && velocity && !lds && c.ti == 4 && T.nb == 1 && T.kw[0] == 32) {
-        T = make_tiles(boxes, nb, 2, jc, ns, group, kb, sb);
+        T = make_tiles(boxes, nb, 2, jc, true, ns, group, kb, sb);
         T.ti = 2;
     } else {
         T.ti = c.ti;
@@ -2121,7 +2126,7 @@ int launch_gradient(const ifos_geom *g, float *const d_Ff[6], float *const d_Fb[
     const Box all = region_box(g, IFOS_REGION_ALL);
     // rows of 32 where they leave fewer lanes idle, as in the marches
     const int kw = padded(g->nz, 32) < padded(g->nz, 64) ? 32 : 64;
-    const MTiles T = make_tiles(&all, 1, kGradTI, kGradTJ, 1, 0, 1, 1, kw);
+    const MTiles T = make_tiles(&all, 1, kGradTI, kGradTJ, true, 1, 0, 1, 1, kw);
     const dim3 grid((unsigned)T.per * 8), block(64, kGradTI);
     ProfScope ps_(IFOS_K_GRADIENT, s);
     auto go = [&](auto h, auto w) {
@@ -2152,7 +2157,7 @@ int launch_td_sample(const ifos_geom *g, const float *const uf[3], const float *
     A.w = w;
     const Box all = region_box(g, IFOS_REGION_ALL);
     const int kw = padded(g->nz, 32) < padded(g->nz, 64) ? 32 : 64;
-    const MTiles T = make_tiles(&all, 1, kGradTI, 16, 1, 0, 1, 1, kw);
+    const MTiles T = make_tiles(&all, 1, kGradTI, 16, true, 1, 0, 1, 1, kw);
     const dim3 grid((unsigned)T.per * 8), block(64, kGradTI);
     { ProfScope ps_(IFOS_K_GRADIENT, s);
     if (kw == 32)

@@ -406,8 +406,8 @@ int ifos_levels_run(ifos_batch *const *lv, int nlev, const ifos_shot *const *sho
                     float *const *d_syn, int use_graph);
 /* tile shapes of the velocity and stress march launches, each
  * {TI, jc, group, split, pipe, kb, sb, lds}: TI wavefronts per workgroup (1, 2, 4, 8);
- * at most jc j-planes per tile (<= 0: 64), halved down to 4 where the launch
- * would leave the chip short of workgroups (results do not depend on it); group: tiles of one shot before
+ * jc j-planes per tile (<= 0: automatic: 64, halved down to 4 where the launch
+ * would leave the chip short of workgroups); group: tiles of one shot before
  * the next shot (1: shots fastest, <= 0: one shot after the other); split:
  * 1 = interior box and CPML slabs in separate launches, 0 = one CPML-aware
  * launch; pipe: 1 = the next plane's operands are loaded one plane ahead;
@@ -416,8 +416,9 @@ int ifos_levels_run(ifos_batch *const *lv, int nlev, const ifos_shot *const *sho
  * remaining TI / (kb sb) wavefronts go along i (kb sb divides TI); lds: 1 =
  * the in-plane neighbours are staged in LDS (used where every row is at least
  * 64 k long and kb = sb = 1, TI >= 2; elsewhere ignored).  NULL leaves a shape
- * unchanged.  A new batch starts with {4, 32, 0, 0, 0, 1, 1, 1} for both, but
- * with jc 8 or 16 as the planes in flight fit the Infinity Cache or not, and
+ * unchanged.  Results do not depend on the shape.  A new batch starts with
+ * {4, 32, 0, 0, 0, 1, 1, 1} for both, but with jc at most 8 or 16 as the planes
+ * in flight fit the Infinity Cache or not (halved as the automatic one), and
  * with lds left out while a step's working set fits it. */
 #define IFOS_TILE_FIELDS 8
 int ifos_batch_set_tiles(ifos_batch *b, const int cfg_v[IFOS_TILE_FIELDS], const int cfg_s[IFOS_TILE_FIELDS]);

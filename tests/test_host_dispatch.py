@@ -39,10 +39,12 @@ def ig(standin):
     lib.standin_log.restype = C.c_char_p
     lib.standin_held.restype = C.c_size_t
     lib.standin_clear()
+    tiles = ifosgpu.get_plain_tiles()
     try:
         yield ifosgpu
     finally:
         gc.collect()
+        ifosgpu.set_plain_tiles(tiles)
         ifosgpu._lib, ifosgpu.LIBPATH = old
 
 
@@ -91,3 +93,39 @@ def test_new_memory_is_zeroed_before_another_stream_sees_it(ig):
                 assert pending is None, f"{what}: {line} behind {pending}"
         assert fills > 0, what
         del keep
+
+
+def _marches(ig):
+    """(kernel, workgroups) of the march launches in the log"""
+    return [(line[1], int(line[2])) for line in _log(ig) if line[0] == "launch" and
+            any(k in line[1] for k in ("k_v_march", "k_s_march", "k_v_lds", "k_s_lds"))]
+
+
+def _updates(ig, G, f, m, psi, prof):
+    ig.lib().standin_clear()
+    ig.update_v(G, ig.REGION_ALL, f, m, prof, psi)
+    ig.update_s(G, ig.REGION_ALL, f, m, prof, psi)
+    return _marches(ig)
+
+
+def _region_call(ig, n=84):
+    G = ig.Geom(n, n, n, 10, 2.0, 2.0, 2.0, 2e-4, 10)
+    bufs = [G.empty() for _ in range(9)], [G.empty() for _ in range(9)], \
+        [ig.DBuf((G.psi_elems(q),)) for q in range(9)], ig.DBuf((18 * 21,))
+    return lambda: _updates(ig, G, *bufs)
+
+
+@pytest.mark.parametrize("jc", [4, 8, 10, 32, 84])
+@pytest.mark.parametrize("lds", [0, 1])
+def test_a_set_chunk_is_kept(ig, jc, lds):
+    """jc > 0 of a caller's shape is the number of planes of a tile, however
+    few workgroups that makes: 84^3 in rows of 32 lanes is 3 x 11 tiles along k
+    and i (8 rows a workgroup), grids are multiples of 8"""
+    run = _region_call(ig)
+    ig.set_plain_tiles((4, jc, 0, 0, 0, 1, 1, lds))
+    tiles = 3 * 11 * -(-84 // jc)
+    got = run()
+    assert [n for _, n in got] == [-(-tiles // 8) * 8] * 2
+    assert all(("_lds" in k) == bool(lds) for k, _ in got)
+    ig.set_plain_tiles((4, 0, 0, 0, 0, 1, 1, lds))  # automatic: 4 planes here
+    assert [n for _, n in run()] == [-(-3 * 11 * 21 // 8) * 8] * 2
