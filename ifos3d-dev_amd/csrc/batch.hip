@@ -418,7 +418,7 @@ extern "C" int ifos_batch_create(ifos_batch **out, const ifos_geom *g, int nshot
     b->nf = 0;
     b->tast = 100;
     b->ntr = 0;
-    b->cfg_v = b->cfg_s = MarchCfg{4, 32, 0, 0, 0, 1, 1, 1, 1};  // the autotuner's usual pick
+    b->cfg_v = b->cfg_s = default_cfg();
     b->fused = 0;  // opt-in; the autotuner turns it on where it beats the separate marches
     b->fz_ti = 16;
     b->fz_jc = 0;
@@ -1238,8 +1238,8 @@ extern "C" int ifos_batch_set_tiles(ifos_batch *b, const int cfg_v[IFOS_TILE_FIE
     if (!b) return IFOS_EINVAL;
     for (const int *c : {cfg_v, cfg_s})
         if (c && check_tile_cfg(c, "ifos_batch_set_tiles")) return IFOS_EINVAL;
-    if (cfg_v) b->cfg_v = MarchCfg{cfg_v[0], cfg_v[1], cfg_v[2], cfg_v[3], cfg_v[4], cfg_v[5], cfg_v[6], cfg_v[7]};
-    if (cfg_s) b->cfg_s = MarchCfg{cfg_s[0], cfg_s[1], cfg_s[2], cfg_s[3], cfg_s[4], cfg_s[5], cfg_s[6], cfg_s[7]};
+    if (cfg_v) b->cfg_v = march_cfg(cfg_v);
+    if (cfg_s) b->cfg_s = march_cfg(cfg_s);
     drop_graphs(b);
     return IFOS_OK;
 }

@@ -153,8 +153,11 @@ struct MarchCfg {
     int kb;  // wavefronts of a workgroup side by side along k (divides ti; <= 1: one)
     int sb;  // shots of a workgroup, one wavefront row each (kb * sb divides ti)
     int lds; // in-plane neighbours staged in LDS (rows of at least 64 cells, kb = sb = 1, ti >= 2)
-    int dflt; // 1: nobody set this shape: jc and lds follow the grid (march_chunk, use_lds)
+    int dflt; // 1: the default shape: jc and lds follow the grid (march_chunk, use_lds)
 };
+const MarchCfg &default_cfg();
+// the shape of IFOS_TILE_FIELDS checked ints
+MarchCfg march_cfg(const int *c);
 // TI / kb / sb checks of a tile shape {TI, jc, group, split, pipe, kb, sb, lds}
 int check_tile_cfg(const int *c, const char *who);
 

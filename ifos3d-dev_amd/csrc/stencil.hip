@@ -1672,7 +1672,21 @@ static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, bool fit, int
 // default tile shape of the march kernels (i-rows per block, j chunk,
 // shot grouping, ..., LDS staging); use_lds and march_chunk fit it to the
 // grid, the batched path's autotuner overrides it per kernel
-static MarchCfg g_default_cfg = {4, 32, 0, 0, 0, 1, 1, 1, 1};
+constexpr MarchCfg kDefaultCfg = {4, 32, 0, 0, 0, 1, 1, 1, 1};
+static MarchCfg g_default_cfg = kDefaultCfg;
+const MarchCfg &default_cfg() { return kDefaultCfg; }
+
+// The default shape's fields stand for its rules wherever they come from: a
+// caller that reads a shape and sets it again, or sets one that the autotuner
+// reported, gets the launches it had.
+MarchCfg march_cfg(const int *c)
+{
+    MarchCfg m = {c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7], 0};
+    const MarchCfg &d = kDefaultCfg;
+    m.dflt = m.ti == d.ti && m.jc == d.jc && m.group == d.group && m.split == d.split && m.pipe == d.pipe &&
+             m.kb == d.kb && m.sb == d.sb && m.lds == d.lds;
+    return m;
+}
 
 // the shape checks of ifos_batch_set_tiles and ifos_set_plain_tiles
 int check_tile_cfg(const int *c, const char *who)
@@ -2477,7 +2491,7 @@ extern "C" int ifos_set_plain_tiles(const int cfg[IFOS_TILE_FIELDS])
 {
     if (!cfg) return IFOS_EINVAL;
     if (ifos::check_tile_cfg(cfg, "ifos_set_plain_tiles")) return IFOS_EINVAL;
-    ifos::g_default_cfg = ifos::MarchCfg{cfg[0], cfg[1], cfg[2], cfg[3], cfg[4], cfg[5], cfg[6], cfg[7]};
+    ifos::g_default_cfg = ifos::march_cfg(cfg);
     return IFOS_OK;
 }
 

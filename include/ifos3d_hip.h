@@ -417,16 +417,18 @@ int ifos_levels_run(ifos_batch *const *lv, int nlev, const ifos_shot *const *sho
  * the in-plane neighbours are staged in LDS (used where every row is at least
  * 64 k long and kb = sb = 1, TI >= 2; elsewhere ignored).  NULL leaves a shape
  * unchanged.  Results do not depend on the shape.  A new batch starts with
- * {4, 32, 0, 0, 0, 1, 1, 1} for both, but with jc at most 8 or 16 as the planes
- * in flight fit the Infinity Cache or not (halved as the automatic one), and
- * with lds left out while a step's working set fits it. */
+ * {4, 32, 0, 0, 0, 1, 1, 1} for both.  This one shape, also when it is set, stands
+ * for the rule that fits it to the grid: jc at most 8 or 16 as the planes in
+ * flight fit the Infinity Cache or not (halved as the automatic one), lds left
+ * out while a step's working set fits it.  Every other shape is kept as set. */
 #define IFOS_TILE_FIELDS 8
 int ifos_batch_set_tiles(ifos_batch *b, const int cfg_v[IFOS_TILE_FIELDS], const int cfg_s[IFOS_TILE_FIELDS]);
 /* the tile shape (same fields; group, split and sb have no effect) of the
  * one-shot march launches: ifos_update_v / ifos_update_s(_visco) on the
  * interior or the whole domain, the shot contexts and the drop-in.
- * Process-wide, default {4, 32, 0, 0, 0, 1, 1, 1} with jc and lds as a new
- * batch's; set it between launches, not while another thread launches. */
+ * Process-wide, default {4, 32, 0, 0, 0, 1, 1, 1}, by the same rule as a
+ * batch's (setting what ifos_get_plain_tiles gave changes nothing); set it
+ * between launches, not while another thread launches. */
 int ifos_set_plain_tiles(const int cfg[IFOS_TILE_FIELDS]);
 int ifos_get_plain_tiles(int cfg[IFOS_TILE_FIELDS]);
 /* the autotuner's candidate shapes (IFOS_TILE_FIELDS ints each, at most

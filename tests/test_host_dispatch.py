@@ -115,7 +115,7 @@ def _region_call(ig, n=84):
     return lambda: _updates(ig, G, *bufs)
 
 
-@pytest.mark.parametrize("jc", [4, 8, 10, 32, 84])
+@pytest.mark.parametrize("jc", [4, 8, 10, 30, 84])
 @pytest.mark.parametrize("lds", [0, 1])
 def test_a_set_chunk_is_kept(ig, jc, lds):
     """jc > 0 of a caller's shape is the number of planes of a tile, however
@@ -129,3 +129,36 @@ def test_a_set_chunk_is_kept(ig, jc, lds):
     assert all(("_lds" in k) == bool(lds) for k, _ in got)
     ig.set_plain_tiles((4, 0, 0, 0, 0, 1, 1, lds))  # automatic: 4 planes here
     assert [n for _, n in run()] == [-(-3 * 11 * 21 // 8) * 8] * 2
+
+
+def test_the_default_shape_comes_back(ig):
+    """default -> another shape -> the shape read before: the launches of the
+    default's rule again (register marches with 4 planes a tile at 84^3), for
+    the region calls and for a batch"""
+    run = _region_call(ig)
+    first, old = run(), ig.get_plain_tiles()
+    assert all("_march" in k for k, _ in first)
+    ig.set_plain_tiles(old)
+    assert run() == first
+    ig.set_plain_tiles((4, 8, 0, 0, 0, 1, 1, 1))
+    assert run() != first
+    ig.set_plain_tiles(old)
+    assert run() == first
+
+    G = ig.Geom(84, 84, 84, 10, 2.0, 2.0, 2.0, 2e-4, 1)
+    b = ig.BatchContext(G, 3, 1, 2)
+
+    def shots():
+        ig.lib().standin_clear()
+        b.run([SRC] * 3, REC, want_adjoint=False)
+        return _marches(ig)
+
+    first = shots()
+    assert all("_march" in k for k, _ in first)
+    b.set_tiles(old, old)
+    assert shots() == first
+    b.set_tiles((8, 32, 0, 0, 0, 1, 1, 1), (8, 32, 0, 0, 0, 1, 1, 1))
+    assert shots() != first
+    b.set_tiles(old, old)
+    assert shots() == first
+    b.close()
