@@ -145,7 +145,7 @@ def test_the_default_shape_comes_back(ig):
     ig.set_plain_tiles(old)
     assert run() == first
 
-    G = ig.Geom(84, 84, 84, 10, 2.0, 2.0, 2.0, 2e-4, 1)
+    G = ig.Geom(84, 84, 84, 10, 2.0, 2.0, 2.0, 2e-4, 2)
     b = ig.BatchContext(G, 3, 1, 2)
 
     def shots():
