@@ -1090,12 +1090,14 @@ extern "C" int ifos_levels_run(ifos_batch *const *lv, int nlev, const ifos_shot 
 // ---------------------------------------------------------------------------
 // autotuner: times each candidate tile shape of the two march launches on
 // the batch's own buffers (ns shots, `reps` launches each) and keeps the
-// fastest.  The wavefields are zeroed afterwards.
+// fastest.  The default shape is one of them, by its rule as a batch that is
+// not tuned runs it, so that tuning does not lose to it.  The wavefields are
+// zeroed afterwards.
 static const MarchCfg k_candidates[] = {
     {4, 32, 0, 0, 0, 1, 1, 0}, {4, 32, 0, 0, 1, 1, 1, 0}, {4, 0, 0, 0, 0, 1, 1, 0}, {8, 32, 0, 0, 0, 1, 1, 0},
     {2, 0, 0, 0, 1, 1, 1, 0},  {1, 0, 0, 0, 1, 1, 1, 0},  {4, 0, 0, 1, 1, 1, 1, 0}, {4, 32, 0, 0, 0, 1, 2, 0},
     {4, 32, 0, 0, 1, 1, 2, 0}, {8, 32, 0, 0, 0, 1, 2, 0}, {4, 32, 0, 0, 0, 1, 4, 0}, {2, 32, 0, 0, 1, 1, 2, 0},
-    {4, 32, 0, 0, 0, 1, 1, 1}, {8, 32, 0, 0, 0, 1, 1, 1}, {2, 32, 0, 0, 0, 1, 1, 1}, {4, 0, 0, 0, 0, 1, 1, 1},
+    {4, 32, 0, 0, 0, 1, 1, 1, 1}, {8, 32, 0, 0, 0, 1, 1, 1}, {2, 32, 0, 0, 0, 1, 1, 1}, {4, 0, 0, 0, 0, 1, 1, 1},
     {8, 0, 0, 0, 0, 1, 1, 1},  {4, 16, 0, 0, 0, 1, 1, 1}, {8, 16, 0, 0, 0, 1, 1, 1}, {4, 8, 0, 0, 0, 1, 1, 1},
 };
 

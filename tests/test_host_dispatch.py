@@ -162,3 +162,31 @@ def test_the_default_shape_comes_back(ig):
     b.set_tiles(old, old)
     assert shots() == first
     b.close()
+
+
+def test_the_autotuner_times_and_keeps_the_default(ig):
+    """where the default shape is the fastest candidate, the tuned batch makes
+    the launches of one that was not tuned; set again from the tuner's answer too"""
+    G = ig.Geom(84, 84, 84, 10, 2.0, 2.0, 2.0, 2e-4, 2)
+    b = ig.BatchContext(G, 3, 1, 2)
+    cands = b.tune_candidates()
+    assert cands.count((4, 32, 0, 0, 0, 1, 1, 1)) == 1 and len(set(cands)) == len(cands)
+    d = cands.index((4, 32, 0, 0, 0, 1, 1, 1))
+
+    def shots():
+        ig.lib().standin_clear()
+        b.run([SRC] * 3, REC, want_adjoint=False)
+        return _marches(ig)
+
+    first = shots()
+    ms = [2.0] * 2 * len(cands) + [100.0] * 16  # v and s of each candidate, then the fused step's
+    ms[2 * d] = ms[2 * d + 1] = 1.0
+    ig.lib().standin_times((C.c_float * len(ms))(*ms), len(ms))
+    ig.lib().standin_clear()
+    bv, bs, _ = b.autotune(reps=1)
+    assert set(first) <= set(_marches(ig))
+    assert bv == bs == cands[d]
+    assert shots() == first
+    b.set_tiles(bv, bs)
+    assert shots() == first
+    b.close()
