@@ -361,8 +361,8 @@ struct ifos_ctx {
     int *srccls, *rcls;    // [1], [ntr] point_class of the source and the receivers
     bool slab_src, slab_rec;
     float *adj;            // [3][ntr][nt+2]
-    float *ring;           // [chunk][3][fe] velocity snapshots of the chunked DFT
-    int chunk;             // snapshots of the ring; 0: one DFT pass per sample; -1: not decided
+    float *ring;           // [chunk][3][fe] velocity snapshots of the chunked DFT, while a shot runs
+    int chunk;             // snapshots of the ring; 0: one DFT pass per sample
     double *trig;          // [2][nsamp][nf][2] (dft_trig)
     int nsamp;
     float finv[IFOS_MAX_NF];
@@ -440,7 +440,7 @@ extern "C" int ifos_ctx_create(ifos_ctx **out, const ifos_geom *g, int nf_max, i
         return rc;
     }
     c->ring = nullptr;
-    c->chunk = -1;
+    c->chunk = 0;
     c->nsamp = 0;
     c->slab_src = c->slab_rec = false;
     c->nf = 0;
@@ -654,19 +654,23 @@ static int probe_nan(ifos_ctx *c, const ShotState &S, int nt, hipStream_t st)
     return rc;
 }
 
-// the snapshot ring of the chunked DFT, allocated by the first shot that
-// samples: 32 snapshots (the 6 nf accumulators of a cell cross HBM once per
-// chunk instead of once per sample: at 276^3 with 6 frequencies 0.5 ms per
-// sample against 1.4 ms; a shot of 100 steps and samples 193.8 ms with 16, 191.0
-// with 32, and with compensated sums of 8 frequencies on 202 x 106 x 202 100.0
-// and 94.8), fewer where they would take more than a quarter of
-// the free memory, none (one pass per sample) where 4 would, or where one
-// snapshot exceeds the 4 GiB of a buffer descriptor
+// the snapshot ring of the chunked DFT, held while a shot runs: 32 snapshots
+// (the 6 nf accumulators of a cell cross HBM once per chunk instead of once per
+// sample: at 276^3 with 6 frequencies 0.5 ms per sample against 1.4 ms; a shot
+// of 100 steps and samples 193.8 ms with 16, 191.0 with 32, and with
+// compensated sums of 8 frequencies on 202 x 106 x 202 100.0 and 94.8), fewer
+// where they would take more than a quarter of the free memory, none (one pass
+// per sample) where 4 would, or where one snapshot exceeds the 4 GiB of a buffer
+// descriptor.  Given back at the shot's end, so that a context keeps nothing
+// that its caller did not size: 0.3 ms to take and 0.35 ms to give back the 8 GB
+// of 276^3.  Not from the stream's memory pool, which kept freed blocks behind
+// waits for the stream and the device, now and then.
 static int ring_alloc(ifos_ctx *c)
 {
-    if (c->chunk >= 0) return IFOS_OK;
     size_t free_b = 0, total_b = 0;
     const size_t snap = 3 * c->fe * 4;
+    c->ring = nullptr;
+    c->chunk = 0;
     int rc = hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
     if (rc) return rc;
     for (int ch = 32; ch >= 4; ch /= 2) {
@@ -676,12 +680,18 @@ static int ring_alloc(ifos_ctx *c)
             c->ring = nullptr;
             continue;
         }
-        c->allocs.push_back(c->ring);
         c->chunk = ch;
         return IFOS_OK;
     }
-    c->chunk = 0;
     return IFOS_OK;
+}
+
+static int ring_free(ifos_ctx *c)
+{
+    const int rc = c->ring ? hip_check(hipFree(c->ring), "hipFree") : IFOS_OK;  // waits for the work on it
+    c->ring = nullptr;
+    c->chunk = 0;
+    return rc;
 }
 
 // one propagation of NT steps; back = 0 forward (sources), 1 adjoint
@@ -793,17 +803,13 @@ static int prepare_shot(ifos_ctx *c, const ifos_shot *s, hipStream_t st, const c
     return rc;
 }
 
-extern "C" int ifos_ctx_run_shot(ifos_ctx *c, const ifos_shot *s, float *d_syn, float *const d_grad[3],
-                                 double *l2, void *stream)
+// the shot that prepare_shot has set up
+static int run_shot(ifos_ctx *c, const ifos_shot *s, float *d_syn, float *const d_grad[3], double *l2, hipStream_t st)
 {
-    if (!c || !s) return IFOS_EINVAL;
     const ifos_geom *g = &c->g;
-    hipStream_t st = (hipStream_t)stream;
-    int rc = prepare_shot(c, s, st, "ifos_ctx_run_shot", true);
-    if (rc) return rc;
     const int ntast = s->want_adjoint ? ifos_ntast(c->finv[c->nf - 1], c->tast, g->dt) : 1;
     // ifos3d.c:738-739: zero wavefield and DFT accumulators
-    rc = zero_wavefield(c, st);
+    int rc = zero_wavefield(c, st);
     // (the first chunk of a pass writes the frequencies in use without reading
     // them)
     const bool chunked = s->want_adjoint && c->chunk > 0 && c->nsamp > 0 && c->nf == c->nf_max;
@@ -828,6 +834,17 @@ extern "C" int ifos_ctx_run_shot(ifos_ctx *c, const ifos_shot *s, float *d_syn, 
         Fb[n] = c->F[6 + n];
     }
     return ifos_gradient_F(g, Ff, Fb, &m, c->finv, c->nf, d_grad, st);
+}
+
+extern "C" int ifos_ctx_run_shot(ifos_ctx *c, const ifos_shot *s, float *d_syn, float *const d_grad[3],
+                                 double *l2, void *stream)
+{
+    if (!c || !s) return IFOS_EINVAL;
+    hipStream_t st = (hipStream_t)stream;
+    int rc = prepare_shot(c, s, st, "ifos_ctx_run_shot", true);
+    if (!rc) rc = run_shot(c, s, d_syn, d_grad, l2, st);
+    const int rc2 = ring_free(c);
+    return rc ? rc : rc2;
 }
 
 // ---------------------------------------------------------------------------

@@ -312,7 +312,11 @@ int ifos_ctx_set_visco(ifos_ctx *c, const float *d_taus, const float *d_taup,
 int ifos_ctx_set_visco_n(ifos_ctx *c, const float *d_taus, const float *d_taup,
                          const float *eta, int L, void *stream);
 /* runs one shot; d_syn [3][ntr][nt+1] (device, written); d_grad[3]
- * (device layout, accumulated); *l2 (host, accumulated) */
+ * (device layout, accumulated); *l2 (host, accumulated).  A shot with
+ * want_adjoint also holds velocity snapshots while it runs: 32 times three
+ * fields, 16, 8 or 4 where more would be over a quarter of the free device
+ * memory, or none (slower); it frees them, which waits for the device, before
+ * it returns */
 int ifos_ctx_run_shot(ifos_ctx *c, const ifos_shot *s, float *d_syn,
                       float *const d_grad[3], double *l2, void *stream);
 /* Time-domain gradient with checkpoints (no counterpart in the reference,

@@ -190,3 +190,25 @@ def test_the_autotuner_times_and_keeps_the_default(ig):
     b.set_tiles(bv, bs)
     assert shots() == first
     b.close()
+
+
+@pytest.mark.parametrize("stream", [None, STREAM])
+def test_a_shot_gives_its_snapshot_ring_back(ig, stream):
+    """a sampling shot holds no more memory after it than before, whether it
+    ends well or not; by hipFree, as a stream's pool may keep what it is given"""
+    G, ctx = _context(ig)
+    obs, syn = ig.DBuf((3, len(REC), G.nt + 1)), ig.DBuf((3, len(REC), G.nt + 1))
+    grads = [G.empty() for _ in range(3)]
+    before = ig.lib().standin_held()
+    for rec, ok in ((REC, True), (REC, True), (np.array([[99, 1, 1]] * 2, np.int32), False)):
+        ig.lib().standin_clear()
+        if ok:
+            ctx.run_shot(SRC, rec, syn, grads, d_obs=obs, stream=stream)
+            log = _log(ig)
+            assert 32 * 3 * 4 * G.field_elems() in [int(line[2]) for line in log if line[0] == "malloc"]
+            assert any("k_dft_chunk" in line[1] for line in log if line[0] == "launch")
+            assert [line[0] for line in log[-2:]] == ["wait", "free"] and log[-2][1] == "all"
+        else:
+            with pytest.raises(ig.IfosError):
+                ctx.run_shot(SRC, rec, syn, grads, d_obs=obs, stream=stream)
+        assert ig.lib().standin_held() == before
