@@ -410,6 +410,7 @@ extern "C" int ifos_batch_create(ifos_batch **out, const ifos_geom *g, int nshot
     if (!rc) rc = balloc(b, (void **)&b->adj, S * 3 * ntr * nt2 * 4);
     if (!rc) rc = balloc(b, (void **)&b->syn, S * 3 * ntr * (nt2 - 1) * 4);
     if (!rc) rc = balloc(b, (void **)&b->probe, S * 4);
+    if (!rc) rc = zero_wait();
     b->trig[0] = b->trig[1] = nullptr;
     if (rc) {
         ifos_batch_destroy(b);
@@ -474,10 +475,12 @@ extern "C" int ifos_batch_set_visco_n(ifos_batch *b, const float *d_taus, const 
         if (!rc) rc = balloc(b, (void **)&b->taus, b->fe * 4);
         if (!rc) rc = balloc(b, (void **)&b->taup, b->fe * 4);
         for (int n = 0; n < 3 && !rc; ++n) rc = balloc(b, (void **)&b->tavg[n], b->fe * 4);
+        if (!rc) rc = zero_wait();
         if (rc) return rc;
     }
     if (b->L_alloc < L) {  // [S][L][fe] per component (the old arrays stay with the context)
         for (int n = 0; n < 6 && !rc; ++n) rc = balloc(b, (void **)&b->r[n], (size_t)b->S * L * b->fe * 4);
+        if (!rc) rc = zero_wait();
         if (rc) return rc;
         b->L_alloc = L;
     }

@@ -74,11 +74,8 @@ DevGeom make_dev_geom(const ifos_geom *g)
     return d;
 }
 
-int zero_new(void *p, size_t bytes)
-{
-    const int rc = hip_check(hipMemset(p, 0, bytes), "hipMemset");
-    return rc ? rc : hip_check(hipStreamSynchronize(nullptr), "hipMemset");
-}
+int zero_new(void *p, size_t bytes) { return hip_check(hipMemset(p, 0, bytes), "hipMemset"); }
+int zero_wait() { return hip_check(hipStreamSynchronize(nullptr), "hipMemset"); }
 
 }  // namespace ifos
 
@@ -435,6 +432,7 @@ extern "C" int ifos_ctx_create(ifos_ctx **out, const ifos_geom *g, int nf_max, i
     if (!rc) rc = dalloc(c, (void **)&c->rcls, sizeof(int) * (size_t)(ntr_max > 0 ? ntr_max : 1));
     if (!rc) rc = dalloc(c, (void **)&c->trig, 4 * sizeof(double) * (size_t)g->nt * (size_t)nf_max);
     if (!rc) rc = dalloc(c, (void **)&c->adj, 3 * (size_t)(ntr_max > 0 ? ntr_max : 1) * (g->nt + 2) * 4);
+    if (!rc) rc = zero_wait();
     if (rc) {
         ifos_ctx_destroy(c);
         return rc;
@@ -476,10 +474,12 @@ extern "C" int ifos_ctx_set_visco_n(ifos_ctx *c, const float *d_taus, const floa
         if (!rc) rc = dalloc(c, (void **)&c->taus, c->fe * 4);
         if (!rc) rc = dalloc(c, (void **)&c->taup, c->fe * 4);
         for (int n = 0; n < 3 && !rc; ++n) rc = dalloc(c, (void **)&c->tavg[n], c->fe * 4);
+        if (!rc) rc = zero_wait();
         if (rc) return rc;
     }
     if (c->L_alloc < L) {  // memory variables: L fields per component (the old ones stay with the context)
         for (int n = 0; n < 6 && !rc; ++n) rc = dalloc(c, (void **)&c->r[n], c->fe * 4 * (size_t)L);
+        if (!rc) rc = zero_wait();
         if (rc) return rc;
         c->L_alloc = L;
         td_free(c);  // its checkpoint states hold memory variables of the old count
@@ -922,6 +922,7 @@ static int td_alloc(ifos_ctx *c, int K)
     for (int n = 0; n < 3 && !rc; ++n) rc = td_alloc_one(T, (void **)&T->uf[n], c->fe * 4);
     for (int n = 0; n < 3 && !rc; ++n) rc = td_alloc_one(T, (void **)&T->ub[n], c->fe * 4);
     for (int n = 0; n < 3 && !rc; ++n) rc = td_alloc_one(T, (void **)&T->acc[n], c->fe * 8);
+    if (!rc) rc = zero_wait();
     if (rc) td_free(c);
     return rc;
 }
@@ -1105,6 +1106,7 @@ static int adj_alloc(ifos_ctx *c, int K, int ntr)
     if (!rc) rc = adj_one(A, (void **)&A->Gu, fe * 8);
     if (!rc) rc = adj_one(A, (void **)&A->J, 8);
     if (!rc) rc = adj_one(A, (void **)&A->res, 3 * (size_t)(ntr > 0 ? ntr : 1) * (c->g.nt + 1) * 4);
+    if (!rc) rc = zero_wait();
     if (rc) adj_free(c);
     return rc;
 }

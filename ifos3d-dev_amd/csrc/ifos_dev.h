@@ -196,10 +196,13 @@ __device__ inline void bstore_cp(float v, rsrc_t r, uint32_t voff, uint32_t soff
 }
 
 DevGeom make_dev_geom(const ifos_geom *g);
-// fills a new allocation with 0 and waits: hipMemset may return before it has
-// run, and the null stream is not ordered with a non-blocking one, on which a
-// caller (or the batch's own stream) writes the memory next
+// fills a new allocation with 0, and waits for all such fills: hipMemset may
+// return before it has run, and the null stream is not ordered with a
+// non-blocking one, on which a caller (or the batch's own stream) writes the
+// memory next.  One wait behind a creation's allocations: behind each of them
+// it made the creation of a context 1 to 2 ms longer.
 int zero_new(void *p, size_t bytes);
+int zero_wait();
 
 // multi-shot fused (interior + CPML) updates over [1..N]^3 (stencil.hip): f
 // and psi point at shot 0; snap may be null

@@ -303,6 +303,7 @@ extern "C" int ifos_lbfgs_create(const ifos_geom *g, int numpar, int bfgsnum, if
     // ifos3d.c:373-379: fmatrix / vector zero-fill
     if (!rc) rc = zero_new(b->grad, vb * bfgsnum);
     if (!rc) rc = zero_new(b->mod, vb * bfgsnum);
+    if (!rc) rc = zero_wait();
     if (rc) {
         ifos_lbfgs_destroy(b);
         return rc;
