@@ -89,14 +89,6 @@ struct Prof {
     __device__ float BH(int ax, int h) const { return p[(6 * ax + 5) * len + h]; }
 };
 
-// psi <- b*psi + a*d ;  d <- d/K + psi   (update_v_ssg_CPML.c:85-90)
-__device__ inline void cpml_apply(float *psi, int64_t at_, float &d, float K, float a, float b)
-{
-    float p = b * psi[at_] + a * d;
-    psi[at_] = p;
-    d = d / K + p;
-}
-
 struct Psi9 {
     float *p[9];
 };
