@@ -1,12 +1,13 @@
-"""The batched path against the plain path, shot for shot.
+"""The batched path against the plain routines, shot for shot.
 
 ifos_batch_run propagates several shots of one model together (fused
 interior+CPML updates over all shots, chunked DFT from a snapshot ring,
 optionally replayed from a hipGraph).  Every number it produces must be
-bit-identical to running the same shots one by one through
-ifos_ctx_run_shot, which is itself bit-identical to the oracle
-(test_gpu_shot.py): seismograms, per-shot misfits, DFT accumulators and the
-gradient accumulated over the shots in order.
+bit-identical to running the same shots one by one through the per-routine
+entry points (routine_shots.py; ifos_ctx_run_shot runs the batch's kernels
+itself, and is compared with the oracle in test_gpu_shot.py): seismograms,
+per-shot misfits, DFT accumulators and the gradient accumulated over the
+shots in order.
 
 The cases put sources and receivers both inside the interior box and inside
 CPML slabs, with two receivers sharing a cell, because the batched path
@@ -19,6 +20,7 @@ import numpy as np
 import pytest
 
 from helpers import max_ulp, rel_l2, small_grid
+from routine_shots import RoutineShots
 
 pytestmark = pytest.mark.gpu
 
@@ -44,9 +46,10 @@ def _setup(ig, g, finv, tast, prec):
     return G
 
 
-def _plain(ig, G, g, true, start, srcs, rec, finv, tast, prec, visco=None):
-    """observed data, seismograms, misfits and accumulated gradient, one shot at a time"""
-    ctx = ig.ShotContext(G, len(finv), len(rec), prec)
+def _plain(ig, G, g, true, start, srcs, rec, finv, tast, prec, visco=None, one_shot=False):
+    """observed data, seismograms, misfits and accumulated gradient, one shot
+    at a time: through the per-routine entry points, or (one_shot) the context"""
+    ctx = ig.ShotContext(G, len(finv), len(rec), prec) if one_shot else RoutineShots(ig, G, len(finv), len(rec), prec)
     ctx.set_cpml(4000.0, 50.0)
     ctx.set_freqs(finv, tast)
     if visco is not None:

@@ -88,11 +88,12 @@ def test_bandwidth_case_shape_matches_oracle():
 @pytest.mark.timeout(900)
 def test_gradient_workload_shape_batched_matches_plain():
     """the 276^3 gradient workload's grid, model, receivers and frequencies (a
-    200-step record): two shots through the batched path (autotuned tiles)
-    give the plain path's seismograms, misfits and accumulated gradient bit
-    for bit"""
+    200-step record): two shots through the one-shot context and through the
+    batched path (autotuned tiles) give the per-routine entry points'
+    seismograms, misfits and accumulated gradient bit for bit"""
     import ifosgpu as ig
     import workloads as wl
+    from routine_shots import RoutineShots
     w = wl.grad276()
     w.nt = 200
     true, start = wl.random_models(w)
@@ -101,27 +102,29 @@ def test_gradient_workload_shape_batched_matches_plain():
     d_start = [G.to_dev(a) for a in start]
     del true, start
     shots = [w.shots[0], w.shots[5]]
-    ntr = len(w.receivers)
-    _note(f"grad276 grid, NT={w.nt}: observed data")
-    ctx = ig.ShotContext(G, len(w.finv), ntr)
-    ctx.set_cpml(w.vppml, w.fpml)
-    ctx.set_freqs(w.finv, w.tast)
+    ntr, nf = len(w.receivers), len(w.finv)
     d_syn = ig.DBuf((3, ntr, w.nt + 1))
-    ctx.set_model(*d_true)
-    obs = []
-    for s in shots:
-        ctx.run_shot(s, w.receivers, d_syn, None, want_adjoint=False)
-        obs.append(d_syn.clone())
-    _note("plain path, two gradient shots")
-    ctx.set_model(*d_start)
-    gp = [G.empty() for _ in range(3)]
-    l2p, synp = [], []
-    for n, s in enumerate(shots):
-        l2p.append(ctx.run_shot(s, w.receivers, d_syn, gp, d_obs=obs[n]))
-        synp.append(d_syn.numpy())
-    ctx.close()
+    res = {}
+    for name in ("routines", "context"):
+        _note(f"grad276 grid, NT={w.nt}: {name}, observed data and two gradient shots")
+        ctx = RoutineShots(ig, G, nf, ntr, ig.DFT_COMPAT) if name == "routines" else ig.ShotContext(G, nf, ntr)
+        ctx.set_cpml(w.vppml, w.fpml)
+        ctx.set_freqs(w.finv, w.tast)
+        if name == "routines":
+            ctx.set_model(*d_true)
+            obs = []
+            for s in shots:
+                ctx.run_shot(s, w.receivers, d_syn, None, want_adjoint=False)
+                obs.append(d_syn.clone())
+        ctx.set_model(*d_start)
+        grads, l2, syn = [G.empty() for _ in range(3)], [], []
+        for n, s in enumerate(shots):
+            l2.append(ctx.run_shot(s, w.receivers, d_syn, grads, d_obs=obs[n]))
+            syn.append(d_syn.numpy())
+        res[name] = l2, syn, [G.from_dev(t) for t in grads]
+        ctx.close()
     _note("batched path, the same two shots")
-    b = ig.BatchContext(G, 2, len(w.finv), ntr, ig.DFT_COMPAT, 8)
+    b = ig.BatchContext(G, 2, nf, ntr, ig.DFT_COMPAT, 8)
     b.set_cpml(w.vppml, w.fpml)
     b.set_freqs(w.finv, w.tast)
     b.set_model(*d_start)
@@ -129,12 +132,14 @@ def test_gradient_workload_shape_batched_matches_plain():
     gb = [G.empty() for _ in range(3)]
     d_b = ig.DBuf((2, 3, ntr, w.nt + 1))
     l2b = b.run(shots, w.receivers, d_syn=d_b, grads=gb, d_obs=obs)
-    sb = d_b.numpy()
+    res["batch"] = l2b, list(d_b.numpy()), [G.from_dev(t) for t in gb]
     b.close()
-    for n in range(2):
-        assert max_ulp(sb[n][:, :, 1:], synp[n][:, :, 1:]) == 0, f"seismograms, shot {n}"
-        assert l2b[n] == l2p[n], f"misfit, shot {n}"
-    for q in range(3):
-        a, c = G.from_dev(gb[q]), G.from_dev(gp[q])
-        assert np.abs(c).max() > 0
-        assert max_ulp(a, c) == 0, f"gradient {q + 1}"
+    l2p, synp, gp = res["routines"]
+    for name in ("context", "batch"):
+        l2, syn, grads = res[name]
+        for n in range(2):
+            assert max_ulp(syn[n][:, :, 1:], synp[n][:, :, 1:]) == 0, f"{name}: seismograms, shot {n}"
+            assert l2[n] == l2p[n], f"{name}: misfit, shot {n}"
+        for q in range(3):
+            assert np.abs(gp[q]).max() > 0
+            assert max_ulp(grads[q], gp[q]) == 0, f"{name}: gradient {q + 1}"

@@ -105,7 +105,7 @@ def test_one_shot_chunks(prec_name, nf, nt, free_surf):
     _note(f"one-shot chunks {prec_name} nf={nf} nt={nt}")
     true, start = tb._models(g)
     G = tb._setup(ig, g, finv, tast, prec)
-    ref = tb._plain(ig, G, g, true, start, srcs, rec, finv, tast, prec)
+    ref = tb._plain(ig, G, g, true, start, srcs, rec, finv, tast, prec, one_shot=True)
     orc = tb._oracle(g, true, start, srcs, rec, finv, tast)
     for n in range(len(srcs)):
         for q in range(3):
