@@ -2,7 +2,7 @@
 wrong: march rows of 32 and 64 lanes with and without LDS staging at k depths
 around multiples of both, on grids whose step fits the last-level cache and
 past it; DFT chunks with a partial one and more frequencies than one launch
-takes; gradient tiles' edges; vector tails of the optimiser passes; receivers
+takes; gradient tiles' edges; vector forms of the optimiser passes; receivers
 that share cells.  Against the oracle; where the other tests of a kernel ask
 for equal bits, so do these.
 """
@@ -52,10 +52,12 @@ def _both_updates(ig, g, seed):
 
 
 @pytest.mark.parametrize("tiles", [None, (4, 8, 0, 0, 0, 1, 1, 1), (8, 16, 0, 0, 0, 1, 1, 1), (2, 0, 0, 0, 0, 1, 1, 1),
-                                   (4, 0, 0, 0, 1, 1, 1, 0)])
+                                   (4, 0, 0, 0, 1, 1, 1, 0), (4, 16, 0, 0, 0, 1, 1, 0)])
 @pytest.mark.parametrize("nz", [63, 64, 65, 96, 97, 130])
 def test_march_rows(nz, tiles):
-    """rows of 64 (nz 64, 97) and of 32 lanes (65, 96, 130), whole rows below 64"""
+    """rows of 64 (nz 64, 97) and of 32 lanes (65, 96, 130), whole rows below
+    64; chunks of 8 and 16 planes with 5 left over of the 21 (a set chunk is
+    kept), the automatic chunk (4 and 1 left), and the default's rule (None)"""
     import ifosgpu as ig
     _note(f"march rows nz={nz} tiles={tiles}")
     old = ig.get_plain_tiles()
@@ -68,10 +70,11 @@ def test_march_rows(nz, tiles):
 
 
 # 17 words of 4 bytes a cell: past 256e6 bytes from 3.77e6 cells on
-@pytest.mark.parametrize("nx,nz", [(157, 160), (122, 200), (126, 192)])
+@pytest.mark.parametrize("nx,nz", [(157, 160), (122, 200), (126, 192), (90, 276)])
 def test_march_rows_past_the_cache(nx, nz):
     """the default shape where a step is not cached: LDS staging with rows of
-    32 (nz 160: both updates; 200: velocity only) and of 64"""
+    32 (nz 160, 200: both updates, rows in 64s 1.2 and 1.14 x longer; 276:
+    velocity only, 1.11 x) and of 64 (192)"""
     import ifosgpu as ig
     _note(f"large march {nx}x157x{nz}")
     _both_updates(ig, small_grid(nx=nx, ny=157, nz=nz, fw=9), 77)
@@ -126,35 +129,38 @@ def test_one_shot_chunks(prec_name, nf, nt, free_surf):
     out["ctx"].close()
 
 
-@pytest.mark.parametrize("nx,ny,nz", [(17, 18, 19), (18, 16, 20), (19, 17, 21)])
-def test_optimiser_tails(nx, ny, nz):
-    """L-BFGS where the number of cells leaves 0 to 3 words past the last
-    vector of four (5814, 5760, 6783 cells); the FP64 sums' order is the
-    only difference, so to the few ulp of the other L-BFGS test"""
+@pytest.mark.parametrize("nx,ny,nz", [(18, 16, 20), (17, 17, 21), (17, 18, 19), (19, 17, 21)])
+@pytest.mark.parametrize("numpar", [1, 2])
+def test_optimiser_vectors(nx, ny, nz, numpar):
+    """L-BFGS passes by vectors of four words, where they divide the history's
+    slots (5760 words, 11520, ...), and by single words (6069, 5814, 6783: 1 to
+    3 over); the FP64 sums' order is the only difference, so to the few ulp of
+    the other L-BFGS test"""
     import ifosgpu as ig
     g = small_grid(nx=nx, ny=ny, nz=nz, fw=4)
-    _note(f"optimiser tails {nx}x{ny}x{nz}")
+    _note(f"optimiser vectors {nx}x{ny}x{nz} numpar={numpar}")
     G = to._geom(ig, g)
     rng = np.random.default_rng(nx)
-    n1 = g.nx * g.ny * g.nz
-    o = LbfgsOracle(2 * n1, 2, dot="f64", vec=np.float32)
-    lb = ig.Lbfgs(G, 2, 2)
+    n = numpar * g.nx * g.ny * g.nz
+    o = LbfgsOracle(n, 2, dot="f64", vec=np.float32)
+    lb = ig.Lbfgs(G, numpar, 2)
     try:
-        grads = [to._field(g, rng) for _ in range(2)]
+        grads = [to._field(g, rng) for _ in range(numpar)]
         flat = lambda gs: np.concatenate([g.interior(a).ravel() for a in gs])
-        lb.savegrad(G.to_dev(grads[0]), G.to_dev(grads[1]))
+        pair = lambda gs: ([G.to_dev(a) for a in gs] + [None])[:2]
+        lb.savegrad(*pair(grads))
         o.savegrad(flat(grads))
         for it in range(1, 4):
             w = it % 2 or 2
-            s = (0.01 * rng.standard_normal(2 * n1)).astype(np.float32)
+            s = (0.01 * rng.standard_normal(n)).astype(np.float32)
             o.mod[w - 1] = s
             lb.mod(w).copy_from(ig.DBuf.from_numpy(s))
             grads = [(0.7 * a + 0.3 * to._field(g, rng)).astype(np.float32) for a in grads]
-            d = [G.to_dev(a) for a in grads]
+            d = pair(grads)
             h0 = lb.update(d[0], d[1], it + 1)
             q, h0_o = o.update(flat(grads), it + 1)
             assert h0 == pytest.approx(h0_o, rel=1e-12)
-            got = np.concatenate([g.interior(G.from_dev(t)).ravel() for t in d])
+            got = np.concatenate([g.interior(G.from_dev(t)).ravel() for t in d[:numpar]])
             assert to._close(got, q), f"direction, iteration {it + 1}"
             for v in (1, 2):
                 assert to._close(lb.grad(v).numpy(), o.grad[v - 1]), f"slot {v}"
@@ -164,16 +170,32 @@ def test_optimiser_tails(nx, ny, nz):
 
 @pytest.mark.parametrize("nx,ny,nz", [(13, 15, 63), (14, 16, 64), (15, 13, 65), (13, 17, 130)])
 def test_gradient_and_hessian_tiles(nx, ny, nz):
-    """tiles of 64 cells along k, 2 rows and 4 planes, and one past each"""
+    """rows of 64 cells (63, 64: 4 rows a tile) and of 32 (65, 130: 8 rows), rows
+    and planes past a tile; tiles of 4 planes, as few as these"""
     import ifosgpu as ig
-    g = small_grid(nx=nx, ny=ny, nz=nz)
     _note(f"gradient and Hessian tiles {nx}x{ny}x{nz}")
+    _gradient_and_hessian(ig, small_grid(nx=nx, ny=ny, nz=nz), [40.0, 60.0, 85.0], 2)
+
+
+@pytest.mark.timeout(300)
+@pytest.mark.parametrize("nx,ny,nz", [(233, 245, 276), (257, 260, 252)])
+def test_gradient_and_hessian_long_tiles(nx, ny, nz):
+    """8192 workgroups and more: tiles of 8 planes, 5 and 4 left over (ny), in
+    rows of 32 (nz 276) and of 64 (252)"""
+    import ifosgpu as ig
+    tiles = -(-nz // 32) * -(-nx // 8) if nz == 276 else -(-nz // 64) * -(-nx // 4)
+    assert tiles * -(-ny // 8) >= 8192
+    _note(f"gradient and Hessian, long tiles {nx}x{ny}x{nz}")
+    _gradient_and_hessian(ig, small_grid(nx=nx, ny=ny, nz=nz), [40.0], 1)
+
+
+def _gradient_and_hessian(ig, g, finv, ntr):
     o = Oracle("f32")
-    rng = np.random.default_rng(nz)
+    rng = np.random.default_rng(g.nz)
     rho, pi, u = tk.random_model(g, rng)
-    finv, ntr = [40.0, 60.0, 85.0], 2
-    Ff = [rng.standard_normal((3,) + g.shape).astype(np.float32) for _ in range(6)]
-    Fb = [rng.standard_normal((3 * (ntr + 1),) + g.shape).astype(np.float32) for _ in range(6)]
+    nf = len(finv)
+    Ff = [rng.standard_normal((nf,) + g.shape, np.float32) for _ in range(6)]
+    Fb = [rng.standard_normal((nf * (ntr + 1),) + g.shape, np.float32) for _ in range(6)]
     for a in Ff + Fb:  # zero halos, as the DFT fields have
         a[:, :3] = 0; a[:, 3 + g.ny:] = 0; a[:, :, :3] = 0; a[:, :, 3 + g.nx:] = 0
         a[:, :, :, :3] = 0; a[:, :, :, 3 + g.nz:] = 0
@@ -187,7 +209,7 @@ def test_gradient_and_hessian_tiles(nx, ny, nz):
     ig.sync()
     for n in range(3):
         assert max_ulp(g.interior(G.from_dev(dev[n])), g.interior(ref[n])) == 0, f"hess{n + 1}"
-    Fb = [np.ascontiguousarray(a[:3]) for a in Fb]
+    Fb = [np.ascontiguousarray(a[:nf]) for a in Fb]
     dFb = [G.to_dev(a) for a in Fb]
     ref, dev = [a.copy() for a in out], [G.to_dev(a) for a in out]
     o.gradient_F(g, Ff, Fb, ref, rho, pi, u, finv)
