@@ -4,9 +4,9 @@ FWI workload, one MI355X.
 
 A gradient shot is: forward NT=1000 steps with the on-the-fly DFT (6
 frequencies), residual against observed data, adjoint NT steps with the
-DFT, gradient_F.  A step of this benchmark is one batch: all 16 shot
-positions propagated together by the batched path (ifos_batch_run).  The
-plain one-shot path (ifos_ctx_run_shot, the drop-in's shape), the
+DFT, gradient_F.  A step of this benchmark is one gradient shot; the batched
+path (ifos_batch_run) propagates the steps together, all 16 shot positions at
+a time (20 steps: a batch of 16 and one of 4).  The plain one-shot path (ifos_ctx_run_shot, the drop-in's shape), the
 checkpointed time-domain gradient (ifos_ctx_run_shot_td) and the drop-in
 library itself (the reference prototypes called on Numerical-Recipes host
 arrays by an IFOS3D-shaped driver, host copies included) are timed on one
@@ -52,13 +52,16 @@ def kernel_names(w, S, chunk, tiles=None):
     b = lambda x: "true" if x else "false"
     tv, ts = tiles or ((4, 0, 0, 0, 0, 1, 1, 1),) * 2
     # the LDS-staged marches run when asked for with TI >= 2, one k column
-    # and one shot per workgroup
-    lds = lambda t: len(t) > 7 and t[7] and t[0] >= 2 and t[5] <= 1 and t[6] == 1 and nz >= 64
+    # and one shot per workgroup; the default shape leaves them out where a
+    # step is cached, and takes two rows of the velocity march with 32 lanes
+    rule = lambda t: tuple(t) == DEFAULT_TILE and nt == "false"
+    lds = lambda t: len(t) > 7 and t[7] and t[0] >= 2 and t[5] <= 1 and t[6] == 1 and nz >= 64 and not rule(t)
     pad = lambda n: -(-nz // n) * n
     kw = lambda least: 32 if pad(64) > least * pad(32) else 64
     ch = next(c for c in (4, 8, 16, 24, 32) if chunk <= c)
     return {"v_fused": f"ifos::k_v_lds<{tv[0]}, true, false, {nt}, {kw(1.0)}>" if lds(tv)
-            else f"ifos::k_v_march<{tv[0]}, true, false, {b(tv[4])}, {nt}>",
+            else f"ifos::k_v_march<{2 if rule(tv) and nz >= 64 and kw(1.0) == 32 else tv[0]}, true, false, {b(tv[4])}, "
+                 f"{nt}>",
             "s_fused": f"ifos::k_s_lds<{ts[0]}, true, 0, {nt}, {kw(1.12)}>" if lds(ts)
             else f"ifos::k_s_march<{ts[0]}, true, 0, {b(ts[4])}, {nt}>",
             "vs_fused": "ifos::k_vs_fused<16, false>",
@@ -67,9 +70,10 @@ def kernel_names(w, S, chunk, tiles=None):
             "gradient": f"ifos::k_grad_lds<false, {kw(1.0)}>"}
 
 
-# tile shapes {TI, jc, group, split, pipe} used without the autotuner (its
-# usual choice on grad276)
-DEFAULT_TILES = ((4, 8, 0, 0, 0, 1, 1, 1), (4, 8, 0, 0, 0, 1, 1, 1))
+# tile shapes {TI, jc, group, split, pipe, kb, sb, lds} used without the
+# autotuner: the library's default, whose fields stand for its rule
+DEFAULT_TILE = (4, 32, 0, 0, 0, 1, 1, 1)
+DEFAULT_TILES = (DEFAULT_TILE, DEFAULT_TILE)
 CATS = ["v_interior", "v_cpml", "v_fused", "s_interior", "s_cpml", "s_fused", "dft", "gradient", "sources", "other",
         "vs_fused"]
 
@@ -181,7 +185,14 @@ def observed_data(w, G, d_true, S, chunk, fused=False):
     return obs
 
 
+def batches_of(shots, S, positions):
+    """the shot positions of `shots` gradient shots, in turn, in batches of S
+    and a last one of what is left"""
+    return [[i % positions for i in range(b0, min(b0 + S, shots))] for b0 in range(0, shots, S)]
+
+
 def run_batched(w, G, d_start, obs, steps, warmup, precision, S, chunk, use_graph, autotune=True, fused=False):
+    """steps and warmup: gradient shots, in batches of S"""
     import ifosgpu as ig
     ntr = len(w.receivers)
     log(f"batched path: {S} shots per batch, DFT chunk {chunk}, graph {use_graph}, "
@@ -198,33 +209,31 @@ def run_batched(w, G, d_start, obs, steps, warmup, precision, S, chunk, use_grap
         tune = {"v": bv, "s": bs, "table": table, "fused": b.fused_table}
         log(f"autotune: velocity march {bv}, stress march {bs}, fused step {b.fused_table}")
     grads = [G.empty() for _ in range(3)]
-    batches = [list(range(b0, min(b0 + S, len(w.shots)))) for b0 in range(0, len(w.shots), S)]
 
-    def one(n):
-        ids = batches[n % len(batches)]
+    def one(ids):
         return b.run([w.shots[i] for i in ids], w.receivers, grads=grads, d_obs=[obs[i] for i in ids],
-                     use_graph=use_graph), len(ids)
+                     use_graph=use_graph)
 
-    for n in range(warmup):
-        one(n)
-        log(f"warmup batch {n + 1}/{warmup} done")
+    for ids in batches_of(warmup, S, len(w.shots)):
+        one(ids)
+        log(f"warmup batch of {len(ids)} shots done")
     ig.sync()
     if not use_graph:
         _prof_start(ig)
     t0 = time.perf_counter()
-    l2, nshots = 0.0, 0
-    for n in range(warmup, warmup + steps):
-        l2s, k = one(n)
-        l2 += sum(l2s)
-        nshots += k
-        log(f"timed batch {n - warmup + 1}/{steps}: {k} shots")
+    l2, sizes = 0.0, []
+    for ids in batches_of(steps, S, len(w.shots)):
+        l2 += sum(one(ids))
+        sizes.append(len(ids))
+        log(f"timed batch of {len(ids)} shots, {sum(sizes)}/{steps}")
     ig.sync()
     elapsed = time.perf_counter() - t0
     prof = _prof_stop(ig) if not use_graph else None
     gnorm = [float(np.linalg.norm(G.from_dev(t).astype(np.float64))) for t in grads]
     fused_used = b.last_fused()
     b.close()
-    return dict(elapsed=elapsed, shots=nshots, prof=prof, l2=l2, gnorm=gnorm, tune=tune, fused=fused_used)
+    return dict(elapsed=elapsed, shots=steps, sizes=sizes, prof=prof, l2=l2, gnorm=gnorm, tune=tune,
+                fused=fused_used)
 
 
 def run_levels(args):
@@ -858,8 +867,9 @@ def kernel_table(prof, ab):
 def main():
     ap = argparse.ArgumentParser(description=__doc__, formatter_class=argparse.RawDescriptionHelpFormatter)
     ap.add_argument("--gpus", type=int, default=1)
-    ap.add_argument("--steps", type=int, default=1, help="timed batches (batched) or shots (plain)")
-    ap.add_argument("--warmup", type=int, default=1)
+    ap.add_argument("--steps", type=int, default=0,
+                    help="timed gradient shots (grad276, toy84; default 16), or runs (levels3; default 1)")
+    ap.add_argument("--warmup", type=int, default=-1, help="untimed ones before them (defaults 16 and 1)")
     ap.add_argument("--config", default="grad276",
                     choices=["grad276", "toy84", "levels3", "fwd536", "aux276", "visco404"])
     ap.add_argument("--level-shots", type=int, default=32, help="shots per grid level (levels3)")
@@ -886,6 +896,9 @@ def main():
     ap.add_argument("--precision", default="compat", choices=["compat", "kahan"])
     ap.add_argument("--no-cpu-baseline", action="store_true")
     args = ap.parse_args()
+    each = 16 if args.config in ("grad276", "toy84") else 1
+    args.steps = args.steps if args.steps > 0 else each
+    args.warmup = args.warmup if args.warmup >= 0 else each
     if args.tiles:
         global DEFAULT_TILES
         DEFAULT_TILES = tuple(tuple(int(x) for x in part.split(",")) for part in args.tiles.split("/"))
@@ -962,7 +975,7 @@ def main():
     if args.path == "batched" and not args.no_kahan_graph and args.config == "grad276":
         Sk = min(8, len(w.shots))
         kg = leg(f"batched path, Kahan DFT, hipGraph replay, {Sk} shots per batch",
-                 lambda: run_batched(w, G, d_start, obs, max(1, len(w.shots) // Sk), 1, ig.DFT_KAHAN, Sk,
+                 lambda: run_batched(w, G, d_start, obs, len(w.shots), Sk, ig.DFT_KAHAN, Sk,
                                      args.chunk, True, autotune=False))
     td = leg("time-domain gradient", lambda: run_td(w, G, d_start, obs, args.td_shots)) if args.td_shots > 0 else None
     dropin = None
@@ -972,8 +985,9 @@ def main():
 
     res = batched if args.path == "batched" else plain
     el, value = res["elapsed"], res["value"]
-    if args.path == "batched":
-        ab = algorithmic_bytes_batched(w, nf, S, args.chunk, ntast, kahan)
+    if args.path == "batched":  # every batch makes the same launches, so the mean over the batches
+        per = [algorithmic_bytes_batched(w, nf, n, args.chunk, ntast, kahan) for n in batched["sizes"]]
+        ab = {k: sum(p[k] for p in per) / len(per) for k in per[0]}
     else:
         ab = algorithmic_bytes(w, nf, kahan, ntast)
     roof = None
@@ -990,7 +1004,8 @@ def main():
             tiles = (tuple(tune["v"]), tuple(tune["s"])) if tune else DEFAULT_TILES
         kname = kernel_names(w, S if tiles else 1, args.chunk if tiles else PLAIN_CHUNK, tiles).get(
             "dft_kahan" if dom == "dft" and kahan else dom, "")
-        if os.path.exists(tpath) and kname:
+        # (the counters were taken with whole batches)
+        if os.path.exists(tpath) and kname and set(res.get("sizes", [S])) == {S}:
             import profsum
             traffic = profsum.read_traffic(tpath).get(kname)
         roof = {"kernel": dom, "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
@@ -1035,8 +1050,8 @@ def main():
                                 f"elastic FP32 4th order, dh {w.dh} m, dt {w.dt:.4e} s, NT {w.nt}, "
                                 f"{len(w.shots)} shot positions, {len(w.receivers)} receivers, "
                                 f"{nf} DFT frequencies {w.finv[0]}-{w.finv[-1]} Hz, TAST {w.tast}"),
-                   "path": path_desc, "dft_precision": args.precision,
-                   "shots_per_step": res["shots"] // args.steps},
+                   "path": path_desc, "dft_precision": args.precision, "shots_per_step": 1,
+                   "batches": res.get("sizes")},
         "gcell_updates_per_s": round(gcells, 3),
         "hbm_frac_stencils": round(hbm_frac_stencils, 4) if hbm_frac_stencils else None,
         "plain_shots_per_s": round(plain["value"], 4) if plain else None,
