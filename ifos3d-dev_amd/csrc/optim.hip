@@ -502,8 +502,9 @@ namespace ifos {
 
 // The source and receiver tapers are functions of the squared distance, an
 // integer, and exactly 1 from kSrcD (r = 64: 1000 exp(-44.8) = 4e-17, so the
-// double quotient is 1) and kRecD (r^2 = 64, the same exponent) on; the edge
-// tapers are functions of one index each.  They are formed once per call in
+// double quotient is 1) and kRecD (r^2 = 64, the same exponent) on; rounded to
+// float, as the tables hold them, they are 1 from 1199 and 35 on already.  The
+// edge tapers are functions of one index each.  They are formed once per call in
 // tables, and a cell multiplies only the factors of the points near its row.
 constexpr int kSrcD = 4096, kRecD = 64;
 struct PreconArgs {

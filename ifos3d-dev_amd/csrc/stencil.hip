@@ -1647,9 +1647,10 @@ static MTiles make_tiles(const Box *boxes, int nb, int ti, int jc, bool fit, int
     // time is the chain and the last round's idle CUs, so the chunk is halved
     // until the launch has kTileMin workgroups, down to 4 planes (below, the
     // 4-6 extra planes a tile loads cost what the shorter chain gains).
-    // One shot, v / s march, chunk 32 -> this rule: 84^3 97 / 102 -> 25 / 27
-    // us (chunk 4), 148^3 117 / 130 -> 65 / 71 us (4), 276^3 404 / 485 ->
-    // 345 / 417 us (8).  Launches with the workgroups keep the chunk, and so
+    // One shot, v / s march of the same kernels, chunk 32 -> this rule: 84^3
+    // 69 / 70 -> 19 / 20 us (chunk 4; 8: 26 / 27), 148^3 79 / 83 -> 52 / 63 us
+    // (4; 8: 54 / 68), 276^3 330 / 422 -> 308 / 387 us (8; 4: 311 / 386).
+    // Launches with the workgroups keep the chunk, and so
     // does a shape whose chunk a caller set.
     constexpr int64_t kTileMin = 8192;
     if (jc <= 0) {
