@@ -1032,7 +1032,7 @@ def main():
                  f"{'fused stress+velocity step (one launch per time step)' if batched and batched['fused'] else 'separate velocity and stress marches'}, "
                  f"DFT in chunks of {args.chunk} samples, {'hipGraph replay' if args.graph else 'direct launches'}"
                  if args.path == "batched" else
-                 "plain (one kernel per reference routine per step, one shot per launch)")
+                 f"plain (ifos_ctx_run_shot: one shot per launch, whole-domain marches, DFT in chunks of {PLAIN_CHUNK} samples)")
     out = {
         "metric": METRIC,
         "value": round(value, 4),

@@ -276,7 +276,8 @@ int ifos_copy(float *d_dst, const float *d_src, size_t n, void *stream);
 
 /* --- one gradient shot, the plain path ---------------------------------
  * Forward NT steps, residual, adjoint NT steps, gradient_F, in the call
- * order of ifos3d.c:712-975, one kernel per reference routine per step.
+ * order of ifos3d.c:712-975: per step one velocity and one stress launch over
+ * the whole domain and the point operations, the DFT in chunks of samples.
  * A context owns every device buffer of one shot (fields, CPML memory,
  * averaged model, DFT accumulators, traces). */
 typedef struct ifos_ctx ifos_ctx;

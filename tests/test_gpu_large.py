@@ -9,10 +9,11 @@ every velocity of the grid after the last step with the oracle's, bit for
 bit; the seismograms of those steps are compared too.  The full 2000-step
 run is measured by `bench.py --config fwd536`.
 
-The gradient workload's 276^3 grid is checked the same way for the batched
-path: two gradient shots of a 200-step record through the batched kernels
-(the tiles the autotuner picks on that grid) against the plain path, which
-the oracle pins, bit for bit.
+The gradient workload's 276^3 grid is checked over two gradient shots of a
+200-step record: the one-shot context and the batched path (the tiles the
+autotuner picks on that grid) against the same shots made of the per-routine
+entry points, bit for bit.  They share gradient_F alone, which
+test_gpu_paths.py compares with the oracle at this size.
 """
 import sys
 

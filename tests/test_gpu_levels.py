@@ -5,7 +5,7 @@ and step counts, as the coarse-to-fine levels of an inversion) run their
 forward solves in one call: enqueued on the contexts' own streams, or
 captured into one graph with a branch per level and replayed.  Each level's
 seismograms must be bit-identical to ifos_batch_run on that context alone,
-and the first shot of each level to the plain one-shot path.  The graph is
+and the first shot of each level to the per-routine entry points.  The graph is
 replayed with new sources, and recaptured when a level's shot count or tile
 shape changes.
 """
@@ -16,6 +16,7 @@ import numpy as np
 import pytest
 
 from helpers import max_ulp, random_model, small_grid
+from routine_shots import RoutineShots
 
 pytestmark = pytest.mark.gpu
 
@@ -65,7 +66,7 @@ def _alone(ig, L, srcs):
 
 
 def _plain_first(ig, L, src):
-    ctx = ig.ShotContext(L["G"], 1, len(L["rec"]), ig.DFT_COMPAT)
+    ctx = RoutineShots(ig, L["G"], 1, len(L["rec"]), ig.DFT_COMPAT)
     ctx.set_cpml(4000.0, 50.0)
     ctx.set_freqs([40.0], 100)
     ctx.set_model(*[L["G"].to_dev(a) for a in L["model"]])
@@ -101,7 +102,7 @@ def test_levels_match_alone(use_graph):
             if rep == 0:
                 for n, L in enumerate(levels):
                     p = _plain_first(ig, L, srcs[n][0])
-                    assert max_ulp(got[n][0], p) == 0, f"level {n}, shot 0 against the plain path"
+                    assert max_ulp(got[n][0], p) == 0, f"level {n}, shot 0 against the routines"
         if use_graph:
             # fewer shots on one level, then another tile shape on another: both recapture
             _note("levels graph: fewer shots on level 1")

@@ -2,8 +2,8 @@
 
 A shot is the call order of ifos3d.c:712-975: forward NT steps with the DFT
 every ntast steps and seismograms every step, residual against observed
-data, adjoint NT steps, gradient_F.  The plain path (one kernel per
-reference routine per step) must reproduce the compat oracle bit for bit;
+data, adjoint NT steps, gradient_F.  The plain path (ifos_ctx_run_shot:
+whole-domain marches, chunked DFT) must reproduce the compat oracle bit for bit;
 the path's stated tolerances (seismograms rel. L2 <= 1e-5, gradients
 <= 1e-4) are asserted as well and reported.
 """
